@@ -1,0 +1,95 @@
+"""fp32 products from three bf16 parts per operand on the matrix cores (csrc/bf16_split.h): the mode GEMM at the edges of its
+tiles, steps and runs, against the oracle, and the exactness of the split itself."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+import turbofno_amd as tf
+from conftest import max_rel, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def _complex(rng, *shape):
+    return (rng.uniform(-1, 1, shape) + 1j * rng.uniform(-1, 1, shape)).astype(np.complex64)
+
+
+def _dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+# fp32 sums of 2 K products each: (2 K)^0.5 roundings of 2^-24 each as a random walk, doubled; never above the
+# sum of all K at full size
+def _bound(K):
+    return 2.0 * (2 * K) ** 0.5 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("M,K,N,beta", [
+    (64, 24, 64, 0.0),               # half a block of columns, a step of which a quarter is beyond K
+    (192, 32, 64, 0.0),              # one full step, the second block half filled
+    (128, 40, 128, 0.5 - 1j),        # two steps, the last with one quarter wavefront of channels; C read and written
+    (320, 96, 192, 0.0),             # three n tiles
+    (64, 192, 64, 0.0),              # the largest tile that stays in LDS
+    (64, 200, 64, 0.0),              # one step more: the tile is rebuilt, the last build covers one step
+    (576, 1000, 64, 1j),             # six builds per column block, a block with idle waves
+    (65536 + 64, 72, 64, 0.0),       # more than one block of 256 columns per CU, a partly filled last one
+    (524288 + 64, 72, 128, 0.0),     # 128-channel tiles, persistent walk, a partly filled last block
+    (262144 - 64, 32, 128, 0.0),     # N = 128 with 32 channels or fewer on a large grid
+])
+def test_cgemm_edges(M, K, N, beta):
+    print("split cgemm", M, K, N, beta, flush=True)
+    rng = np.random.default_rng(M + K + N)
+    gen = torch.Generator(device="cuda").manual_seed(M + K)
+    A = torch.view_as_complex(torch.rand((K, M, 2), device="cuda", generator=gen) * 2 - 1)
+    W = _complex(rng, N, K) / np.float32(np.sqrt(K))
+    C0 = torch.full((N, M), float("nan"), dtype=torch.complex64, device="cuda") if beta == 0.0 else \
+        torch.view_as_complex(torch.rand((N, M, 2), device="cuda", generator=gen) * 2 - 1)
+    C = C0.clone()
+    tf.cgemm(M, N, K, A, _dev(W), C, 0.5 + 1j, beta)
+    torch.cuda.synchronize()
+    assert not bool(torch.isnan(torch.view_as_real(C)).any()), "columns of C left unwritten"
+    picks = sorted(set(range(0, min(M, 300))) | set(range(max(0, M - 300), M)) | set(range(M // 2, min(M, M // 2 + 32))))
+    idx = torch.tensor(picks, device="cuda")
+    ref = oracle.cgemm(A.index_select(1, idx).cpu().numpy(), W, 0.5 + 1j)
+    if beta != 0.0:
+        ref = ref + beta * C0.index_select(1, idx).cpu().numpy().astype(np.complex128)
+    err = rel_l2(C.index_select(1, idx).cpu().numpy(), ref)
+    assert err < _bound(K), (err, _bound(K))
+
+
+@pytest.mark.parametrize("K", [24, 64])
+def test_split_is_exact(K):
+    """weights 1, i, -1 and 2^-20 on one channel each: nothing is rounded, so the product is the input bit for bit. Inputs over
+    the range in which all three parts are normal numbers, with full 24-bit significands."""
+    print("split exact", K, flush=True)
+    rng = np.random.default_rng(K)
+    M, N = 256, 64
+    mant = rng.integers(2 ** 23, 2 ** 24, (K, M, 2)).astype(np.float64) * rng.choice([-1.0, 1.0], (K, M, 2))
+    A = np.ldexp(mant, rng.integers(-80, 100, (K, M, 2))).astype(np.float32).view(np.complex64)[..., 0]
+    W = np.zeros((N, K), np.complex64)
+    factor = np.array([1, 1j, -1, 2.0 ** -20], np.complex64)
+    for n in range(N):
+        W[n, (5 * n) % K] = factor[n % 4]
+    C = torch.empty((N, M), dtype=torch.complex64, device="cuda")
+    tf.cgemm(M, N, K, _dev(A), _dev(W), C, 1.0, 0.0)
+    got = C.cpu().numpy()
+    for n in range(N):
+        f, a = factor[n % 4], A[(5 * n) % K]
+        want = np.empty_like(a)
+        want.real, want.imag = (-a.imag, a.real) if f == 1j else (a.real * f.real, a.imag * f.real)
+        assert np.array_equal(got[n].real, want.real) and np.array_equal(got[n].imag, want.imag), n
+
+
+@pytest.mark.parametrize("bs,DX,DY,K,N", [(2, 512, 128, 8, 64), (1, 512, 256, 40, 64), (1, 1024, 128, 24, 128), (1, 1024, 128, 104, 64),
+                                          (1, 512, 128, 64, 64), (1, 512, 128, 200, 64)])
+def test_weights_with_a_period(bs, DX, DY, K, N):
+    """whole images in 2 / 4 interleaved parts: the contraction runs over the parts with the weights of their channel, as one
+    run over all parts (K = 8, 24, 40) or as one run per part (K = 64, 104; K = 200 with a tile that is rebuilt)"""
+    print("split period", bs, DX, DY, K, N, flush=True)
+    rng = np.random.default_rng(DX + K)
+    x, W = _complex(rng, K, bs, DX, DY), _complex(rng, N, K) / np.float32(np.sqrt(K))
+    y = tf.layer_2d(_dev(x), _dev(W), algo=2, alpha=1 - 1j)
+    torch.cuda.synchronize()
+    ref = oracle.layer_2d(x, W, 1 - 1j)
+    assert rel_l2(y.cpu().numpy(), ref) < 1e-6 and max_rel(y.cpu().numpy(), ref) < 1e-5

@@ -1,0 +1,61 @@
+// fp32 products on the bf16 matrix cores without loss of precision. A float is the exact sum of three bf16 values,
+//   x = h + m + l,   h = bf16(x), m = bf16(x - h), l = x - h - m      (round to nearest: |m| <= 2^-8 |x|, |l| <= 2^-16 |x|),
+// because a bf16 holds 8 of the 24 significant bits. A product is then formed from six of the nine partial products,
+//   x w ~ l h' + h l' + m m' + m h' + h m' + h h'
+// the three that are left out (m l', l m', l l') are below 2^-23 |x w| together, half the spacing of floats there. Sums
+// are fp32, as in v_mfma_f32_16x16x4_f32, but one instruction adds 32 channels instead of 4, so there are fewer roundings.
+// Six v_mfma_f32_16x16x32_bf16 (16 cycles each) do the work of eight v_mfma_f32_16x16x4_f32 (32 cycles each): 2.7 times the
+// rate of the fp32 matrix instructions for the same real product.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace tfno {
+
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float float2_v __attribute__((ext_vector_type(2)));
+typedef float float4_v __attribute__((ext_vector_type(4)));
+typedef unsigned uint4_v __attribute__((ext_vector_type(4)));
+
+// two floats -> their three bf16 parts, packed two to a register (a in the low half)
+__device__ __forceinline__ void split_bf16_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l)
+{
+    h = __builtin_bit_cast(unsigned, __builtin_convertvector((float2_v){ a, b }, bf16x2_t));
+    float ra = a - __builtin_bit_cast(float, h << 16), rb = b - __builtin_bit_cast(float, h & 0xffff0000u);
+    m = __builtin_bit_cast(unsigned, __builtin_convertvector((float2_v){ ra, rb }, bf16x2_t));
+    ra -= __builtin_bit_cast(float, m << 16);
+    rb -= __builtin_bit_cast(float, m & 0xffff0000u);
+    l = __builtin_bit_cast(unsigned, __builtin_convertvector((float2_v){ ra, rb }, bf16x2_t));
+}
+
+// the three parts of eight consecutive channels of one row or column: operands of v_mfma_f32_16x16x32_bf16
+struct SplitOperand {
+    uint4_v h, m, l;
+};
+__device__ __forceinline__ float4_v mfma_bf16(uint4_v a, uint4_v b, float4_v c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+// c + a b, smallest products first
+__device__ __forceinline__ float4_v mac_split(const SplitOperand& a, const SplitOperand& b, float4_v c)
+{
+    c = mfma_bf16(a.l, b.h, c);
+    c = mfma_bf16(a.h, b.l, c);
+    c = mfma_bf16(a.m, b.m, c);
+    c = mfma_bf16(a.m, b.h, c);
+    c = mfma_bf16(a.h, b.m, c);
+    return mfma_bf16(a.h, b.h, c);
+}
+// c0 += a b0, c1 += a b1: two independent chains
+__device__ __forceinline__ void mac_split2(const SplitOperand& a, const SplitOperand& b0, const SplitOperand& b1, float4_v& c0, float4_v& c1)
+{
+    c0 = mfma_bf16(a.l, b0.h, c0); c1 = mfma_bf16(a.l, b1.h, c1);
+    c0 = mfma_bf16(a.h, b0.l, c0); c1 = mfma_bf16(a.h, b1.l, c1);
+    c0 = mfma_bf16(a.m, b0.m, c0); c1 = mfma_bf16(a.m, b1.m, c1);
+    c0 = mfma_bf16(a.m, b0.h, c0); c1 = mfma_bf16(a.m, b1.h, c1);
+    c0 = mfma_bf16(a.h, b0.m, c0); c1 = mfma_bf16(a.h, b1.m, c1);
+    c0 = mfma_bf16(a.h, b0.h, c0); c1 = mfma_bf16(a.h, b1.h, c1);
+}
+
+}  // namespace tfno

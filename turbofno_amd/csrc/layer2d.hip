@@ -17,6 +17,7 @@
 // The 4096 modes of an image are stored in "lane order": element mm*(64 LX) + q*LX + t holds mode
 // (p = t + LX mm, q), LX = DX/16. That order is private to the two image kernels (producer and consumer
 // lanes coincide, every access is contiguous per wavefront) and the GEMM is oblivious to it.
+#include "bf16_split.h"
 #include "group_fft.h"
 #include "kernels.h"
 #include <string>
@@ -380,144 +381,238 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
 }
 
 // ---------------------------------------------------------------------------------------------
-// Mode-space complex GEMM on the fp32 matrix cores.
+// Mode-space complex GEMM on the matrix cores.
 //   C[n][m] = alpha * sum_k W[k + n*K] * A[k][m] (+ beta C),   A: [K][Mtot], C: [N][Mtot]  (m contiguous)
 // Same contraction as the reference's cgemm / the GEMM phase of its fused kernel
-// (fusion_variants/1D_A_exp_fft+cgemm+ifft/cgemm.cuh:4-205, operand layout lda=M, ldb=K, ldc=M), with three real
-// products per complex one instead of four:
-//   P1 = c (a + b),  P2 = (d - c) a,  P3 = (c + d) b   =>   re = P1 - P3,  im = P1 + P2      (alpha W = c + i d, A = a + i b)
-// i.e. three v_mfma_f32_16x16x4_f32 per 16 n x 16 m x 4 k: 25 % less matrix work than the real-expanded product, and
-// the matrix work is the part of this kernel that nothing overlaps with (all waves of the grid load, multiply and
-// store in step). Rows of a tile are 16 output channels n, columns 16 consecutive m, contraction 4 channels.
-// A block is 16 waves; wave w owns the 16-m strip w and the whole 64-channel n tile, so every element of A is loaded
-// exactly once: the strip of a chunk sits in NG float2 registers per lane, all loads in flight while the W tile is
-// built. The n tiles are the outer loop, so each is stored as soon as it is complete and its stores drain under the
-// matrix work of the next ones.
-//   NG    = channel groups of four per chunk that can hold data (4, 8, 12, 16 for K <= 16, 32, 48, 64): a template
-//           parameter so that the loops stay unrolled and no loads or matrix work are spent on zero padding;
+// (fusion_variants/1D_A_exp_fft+cgemm+ifft/cgemm.cuh:4-205, operand layout lda=M, ldb=K, ldc=M). Four real products per
+// complex one, each from six bf16 matrix instructions per 32 channels (bf16_split.h).
+// Rows of a tile are 16 output channels n, columns 16 consecutive m, contraction in steps of 32 channels (eight per lane
+// of a quarter wavefront). A wave owns 16 m and all 16 NT output channels of its block: an element of A is loaded and split
+// once per block, and its parts meet NT fragments of W read from LDS. The W tile holds the parts of alpha W as fragments
+// in lane order, 6 x 1 KiB per (step, 16 channels): an operand is one conflict-free 16-byte read.
+// Blocks are persistent over column blocks (XCD j takes the j-th eighth of them, so that an XCD keeps to one part of the
+// memory system); the strip of the next step - of the next column block after the last - is requested before the matrix
+// work of the current one, and nothing in the walk waits at a barrier, so loads, matrix work and stores of the waves overlap.
 //   Kw    = period of W along the contraction: channel k is weighted with W[k mod Kw + n Kw] (Kw = K: the plain product;
 //           Kw = K / R: the R parts of decimated images, see above, share the weights of their image's channel);
-//   MULTI = K > 64: chunks of 4 NG = 32 channels with the twelve accumulator tiles of a wave kept across them
-//           (125 registers; 64-channel chunks would spill); otherwise one chunk and transient accumulators.
+//   Kp    = channels covered by one run over the tile (K, or Kw: the contraction then runs over the tile K / Kw times);
+//   cap   = steps that the tile can hold; with more steps in a run the tile is rebuilt as the contraction proceeds.
 // ---------------------------------------------------------------------------------------------
+constexpr int GEMM_KSTEP = 32;
+constexpr size_t kSplitStepBytes = 6 * 1024;            // LDS of one step of 16 output channels
+
+template <int NT, int THREADS>
+__global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_split_kernel(
+    const float2* __restrict__ A, const float2* __restrict__ W, float2* __restrict__ C, long Mtot, int K, float2 alpha,
+    float2 beta, long nblocks, int Kw, int Kp, int cap)
+{
+    extern __shared__ uint4_v sW4[];
+    constexpr int MBLOCK = THREADS / 4;                 // columns per block: 16 per wave
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 15, kq = lane >> 4;
+    const int n0 = blockIdx.y * (16 * NT);
+    const int steps = (Kp + GEMM_KSTEP - 1) / GEMM_KSTEP, runs = K / Kp;
+    const bool resident = steps <= cap;                 // the tile is built once
+    const bool eighths = (gridDim.x & 7) == 0 && (nblocks & 7) == 0;
+    auto block_of = [&](long v) { return eighths ? (v & 7) * (nblocks >> 3) + (v >> 3) : v; };
+    const bool has_beta = beta.x != 0.f || beta.y != 0.f;
+
+    // channels 8 kq ... 8 kq + 7 of step `step` of a run, of the lane's column. Branch free, so that the loads stay where
+    // they are issued: lanes beyond the run (its last step may be short) read the first channels of the step again - the tile
+    // holds zeros there - and waves beyond the last column read the first strip (nothing is stored from it). `live` is false
+    // after the last step of the block: every lane then reads one line.
+    const unsigned lane_row = (unsigned)(8 * kq * Mtot), lane_col = wave * 16 + col;
+    float2 bv[8];
+    auto fetch = [&](long mb, int run, int step, bool live) {
+        const bool column = mb * MBLOCK + wave * 16 < Mtot;       // Mtot is a multiple of 16; Kp of 8
+        const float2* base = A + (column ? mb * MBLOCK : 0) + (long)(run * Kp + GEMM_KSTEP * step) * Mtot;    // uniform
+        const unsigned off = live ? (column ? lane_col : (unsigned)col) + (GEMM_KSTEP * step + 8 * kq < Kp ? lane_row : 0u) : 0u;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) bv[j] = (base + j * Mtot)[off];
+    };
+    // fragments of the steps s0 ... s0 + count - 1: entry (step, tile, kq, n mod 16) = eight consecutive channels of one n
+    auto build = [&](int s0, int count) {
+        for (int e = tid; e < count * NT * 64; e += THREADS) {
+            const int l = e & 63, t = (e >> 6) % NT, s = (e >> 6) / NT;
+            const int k = GEMM_KSTEP * (s0 + s) + 8 * (l >> 4), n = n0 + 16 * t + (l & 15);
+            SplitOperand re, im;
+            float2 w[8];
+            const float2* src = W + (k % Kw) + (long)n * Kw;        // Kw is a multiple of 8
+#pragma unroll
+            for (int j = 0; j < 8; ++j) w[j] = k < Kp ? src[j] : make_float2(0.f, 0.f);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) w[j] = make_float2(w[j].x * alpha.x - w[j].y * alpha.y, w[j].x * alpha.y + w[j].y * alpha.x);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                unsigned h, m, lo;
+                split_bf16_pair(w[2 * j].x, w[2 * j + 1].x, h, m, lo);
+                re.h[j] = h; re.m[j] = m; re.l[j] = lo;
+                split_bf16_pair(w[2 * j].y, w[2 * j + 1].y, h, m, lo);
+                im.h[j] = h; im.m[j] = m; im.l[j] = lo;
+            }
+            uint4_v* dst = sW4 + (e >> 6) * 384 + l;
+            dst[0] = re.h; dst[64] = re.m; dst[128] = re.l;
+            dst[192] = im.h; dst[256] = im.m; dst[320] = im.l;
+        }
+    };
+
+    long v = blockIdx.x;                                // the grid is no larger than the number of column blocks
+    fetch(block_of(v), 0, 0, true);
+    if (resident) {
+        build(0, steps);
+        __syncthreads();
+    }
+    for (; v < nblocks; v += gridDim.x) {
+        const long mb = block_of(v);
+        const bool more = v + gridDim.x < nblocks;
+        const long nb = more ? block_of(v + gridDim.x) : mb;
+        float4_v re[NT], im[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) re[t] = im[t] = float4_v{ 0.f, 0.f, 0.f, 0.f };
+        for (int run = 0; run < runs; ++run)
+            for (int step = 0; step < steps; ++step) {
+                if (!resident && step % cap == 0) {     // uniform over the block
+                    __syncthreads();
+                    build(step, steps - step < cap ? steps - step : cap);
+                    __syncthreads();
+                }
+                SplitOperand ar, ai;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    unsigned h, m, l;
+                    split_bf16_pair(bv[2 * j].x, bv[2 * j + 1].x, h, m, l);
+                    ar.h[j] = h; ar.m[j] = m; ar.l[j] = l;
+                    split_bf16_pair(bv[2 * j].y, bv[2 * j + 1].y, h, m, l);
+                    ai.h[j] = h; ai.m[j] = m; ai.l[j] = l;
+                }
+                asm volatile("" ::: "memory");          // operand reads of the tile stay inside the loop
+                const bool same = step + 1 < steps || run + 1 < runs;         // the next step belongs to this column block
+                fetch(same ? mb : nb, step + 1 < steps ? run : (same ? run + 1 : 0), step + 1 < steps ? step + 1 : 0, same || more);
+                __builtin_amdgcn_sched_barrier(0);
+                const uint4_v* frag = sW4 + (resident ? step : step % cap) * (NT * 384) + lane;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    SplitOperand w{ frag[t * 384], frag[t * 384 + 64], frag[t * 384 + 128] };
+                    float4_v r = re[t], i = im[t];
+                    mac_split2(w, ar, ai, r, i);                        // Wr
+                    w = SplitOperand{ frag[t * 384 + 192], frag[t * 384 + 256], frag[t * 384 + 320] };
+                    i = mac_split(w, ar, i);                            // Wi
+                    w.h ^= 0x80008000u; w.m ^= 0x80008000u; w.l ^= 0x80008000u;
+                    r = mac_split(w, ai, r);                            // - Wi
+                    re[t] = r;
+                    im[t] = i;
+                }
+            }
+        if (mb * MBLOCK + wave * 16 < Mtot) {
+            // D[row = 4 kq + q][col] of tile t: output channel n0 + 16 t + 4 kq + q, the lane's column
+            float2* dst = C + mb * MBLOCK + lane_col + (long)(n0 + 4 * kq) * Mtot;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    float2* p = dst + (long)(16 * t + q) * Mtot;
+                    float2 r = make_float2(re[t][q], im[t][q]);
+                    if (has_beta) r = cadd(r, cmul(*p, beta));          // variants A, B
+                    *p = r;
+                }
+        }
+    }
+}
+
+// Few channels (K <= 16; K <= 32 in one range of sizes, see launch_cgemm_modes): a step of 32 channels would be mostly
+// padding. fp32 matrix instructions over groups of four channels instead, three real products per complex one:
+//   P1 = c (a + b),  P2 = (d - c) a,  P3 = (c + d) b   =>   re = P1 - P3,  im = P1 + P2      (alpha W = c + i d, A = a + i b)
+// A block is 16 waves; wave w owns the 16-m strip w and 64 output channels; the strip sits in NG float2 registers per
+// lane, all loads in flight while the W'' tile is built, and every n tile is stored as soon as it is complete.
+// NG = channel groups of four that can hold data.
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int GEMM_KC = 64;         // channels per LDS-resident W chunk
 constexpr int GEMM_THREADS = 1024;  // 16 waves x 16 m
 constexpr int GEMM_MBLOCK = 256;    // m per block
 
 // W'' tile in LDS: three planes (c, d - c, c + d) of floats at index (k / 4) * kW3Group + (k % 4) * kW3Row + n.
 // An operand fetch (64 lanes: 4 k x 16 n) reads 16 consecutive floats of four rows 80 apart: one bank each. The
-// build's lanes run along k, the contiguous direction of W: a group stride of 1 (mod 64 banks) puts the 64 lanes of a
-// store on 64 different banks as well.
-constexpr int kW3Row = 80, kW3Group = 4 * kW3Row + 1, kW3Plane = (GEMM_KC / 4) * kW3Group;
+// build's lanes run along k, the contiguous direction of W: a group stride of 1 (mod 64 banks) spreads the lanes of a
+// store over the banks as well.
+constexpr int kW3Row = 80, kW3Group = 4 * kW3Row + 1;
+template <int NG> constexpr int kW3Plane = NG * kW3Group;
 
-template <int NG, bool MULTI>
+template <int NG>
+__device__ __forceinline__ void build_w3_tile(float* sW, const float2* __restrict__ W, int n0, int K, int Kw, float2 alpha, int tid)
+{
+    constexpr int KC = 4 * NG, WPT = KC * 64 / GEMM_THREADS;
+    float2 wv[WPT];
+#pragma unroll
+    for (int u = 0; u < WPT; ++u) {
+        const int idx = tid + u * GEMM_THREADS, k = idx % KC, n = idx / KC;
+        wv[u] = (k < K) ? W[k % Kw + (long)(n0 + n) * Kw] : make_float2(0.f, 0.f);
+    }
+#pragma unroll
+    for (int u = 0; u < WPT; ++u) {
+        const int idx = tid + u * GEMM_THREADS, k = idx % KC, n = idx / KC;
+        const float c = wv[u].x * alpha.x - wv[u].y * alpha.y, d = wv[u].x * alpha.y + wv[u].y * alpha.x;
+        float* dstw = &sW[(k >> 2) * kW3Group + (k & 3) * kW3Row + n];
+        dstw[0] = c;
+        dstw[kW3Plane<NG>] = d - c;
+        dstw[2 * kW3Plane<NG>] = c + d;
+    }
+}
+
+// one column block per block
+template <int NG>
 __global__ __launch_bounds__(GEMM_THREADS) void cgemm_modes3m_kernel(const float2* __restrict__ A,
                                                                      const float2* __restrict__ W, float2* __restrict__ C,
                                                                      long Mtot, int N, int K, float2 alpha, float2 beta,
                                                                      int Kw)
 {
-    extern __shared__ float sW[];                     // 3 * kW3Plane floats
+    __shared__ float sW[3 * kW3Plane<NG>];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 15, kq = lane >> 4;
     const int n0 = blockIdx.y * 64;
     const unsigned lane_off = (unsigned)(kq * Mtot) + (unsigned)(wave * 16 + col);
-    // XCD j takes the j-th eighth of the column blocks: with every eighth block (2 KiB of each of the K + N rows, which
-    // lie Mtot * 8 bytes apart) an XCD keeps to one part of the memory system; 4-10 % faster once the operands exceed the
-    // Infinity Cache (bs = 128), no change below
+    // XCD j takes the j-th eighth of the column blocks, as above
     const unsigned mb = (unsigned)xcd_contiguous(blockIdx.x, gridDim.x);
     const float2* blk = A + (long)mb * GEMM_MBLOCK;
     const bool active = (long)mb * GEMM_MBLOCK + wave * 16 < Mtot;   // Mtot is a multiple of 16, not of 256
     float2* cblk = C + (long)mb * GEMM_MBLOCK;
     const bool has_beta = beta.x != 0.f || beta.y != 0.f;
 
-    floatx4 p1[4], p2[4], p3[4];
+    // the wave's whole A strip: lane (kq, col) holds channels 4 g + kq, g < NG; the loads overlap the tile build
+    float2 bv[NG];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) p1[t] = p2[t] = p3[t] = floatx4{ 0.f, 0.f, 0.f, 0.f };
-
-    // one chunk of up to 64 channels, or (MULTI) chunks of 4 NG = 32 channels with the accumulators kept across them
-    constexpr int KCH = MULTI ? 4 * NG : GEMM_KC;
-    for (int kc = 0; kc < (MULTI ? K : 1); kc += KCH) {
-        const int kn = (K - kc) < KCH ? (K - kc) : KCH;           // multiple of 8 (caller contract)
-        const bool last = !MULTI || kc + KCH >= K;
-        // the wave's whole A strip of this chunk: lane (kq, col) holds channels kc + 4 g + kq, g < NG
-        // (with one chunk the loads are issued before the tile build and overlap it; with several, the accumulators
-        // of all tiles stay live and the strip is loaded after the build to stay inside 128 registers)
-        float2 bv[NG];
-        if constexpr (!MULTI) {
+    for (int g = 0; g < NG; ++g) bv[g] = (active && 4 * g < K) ? (blk + (long)(4 * g) * Mtot)[lane_off] : make_float2(0.f, 0.f);
+    build_w3_tile<NG>(sW, W, n0, K, Kw, alpha, tid);
+    __syncthreads();
+    if (!active) return;
 #pragma unroll
-            for (int g = 0; g < NG; ++g)
-                bv[g] = (active && 4 * g < kn) ? (blk + (long)(kc + 4 * g) * Mtot)[lane_off] : make_float2(0.f, 0.f);
+    for (int t = 0; t < 4; ++t) {
+        floatx4 p1 = floatx4{ 0.f, 0.f, 0.f, 0.f }, p2 = p1, p3 = p1;
+        const float* wrow = &sW[kq * kW3Row + t * 16 + col];
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const float* w = wrow + g * kW3Group;
+            p1 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[0], bv[g].x + bv[g].y, p1, 0, 0, 0);
+            p2 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[kW3Plane<NG>], bv[g].x, p2, 0, 0, 0);
+            p3 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[2 * kW3Plane<NG>], bv[g].y, p3, 0, 0, 0);
         }
-        if constexpr (MULTI) __syncthreads();         // the previous chunk's tile is no longer read
-        // W'' tile: lanes run along k, the contiguous direction of W[k + n*K]. With a single chunk only the first
-        // BUILDERS threads build it: the waves of a block start one after the other over several microseconds, and the
-        // block can only go on when the last of them has passed the barrier below - which should then find nothing left
-        // to do there (its own part of the tile would add a round trip to L2 after its late start)
-        constexpr int BUILDERS = MULTI ? GEMM_THREADS : GEMM_THREADS / 2;
-        constexpr int WPT = KCH * 64 / BUILDERS;
-        if (MULTI || tid < BUILDERS) {
-            float2 wv[WPT];
+        // D[row = 4 kq + v][col]: output channel n0 + 16 t + 4 kq + v, column m = wave * 16 + col
 #pragma unroll
-            for (int u = 0; u < WPT; ++u) {
-                const int idx = tid + u * BUILDERS;
-                const int k = idx % KCH, n = idx / KCH;
-                wv[u] = (k < kn) ? W[(kc + k) % Kw + (long)(n0 + n) * Kw] : make_float2(0.f, 0.f);
-            }
-#pragma unroll
-            for (int u = 0; u < WPT; ++u) {
-                const int idx = tid + u * BUILDERS;
-                const int k = idx % KCH, n = idx / KCH;
-                const float c = wv[u].x * alpha.x - wv[u].y * alpha.y, d = wv[u].x * alpha.y + wv[u].y * alpha.x;
-                float* dstw = &sW[(k >> 2) * kW3Group + (k & 3) * kW3Row + n];
-                dstw[0] = c;
-                dstw[kW3Plane] = d - c;
-                dstw[2 * kW3Plane] = c + d;
-            }
-        }
-        if constexpr (MULTI) {
-#pragma unroll
-            for (int g = 0; g < NG; ++g)
-                bv[g] = (active && 4 * g < kn) ? (blk + (long)(kc + 4 * g) * Mtot)[lane_off] : make_float2(0.f, 0.f);
-        }
-        __syncthreads();
-        if (!active) continue;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            if constexpr (!MULTI) p1[t] = p2[t] = p3[t] = floatx4{ 0.f, 0.f, 0.f, 0.f };
-            const float* wrow = &sW[kq * kW3Row + t * 16 + col];
-#pragma unroll
-            for (int g = 0; g < NG; ++g) {
-                const float* w = wrow + g * kW3Group;
-                p1[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[0], bv[g].x + bv[g].y, p1[t], 0, 0, 0);
-                p2[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[kW3Plane], bv[g].x, p2[t], 0, 0, 0);
-                p3[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[2 * kW3Plane], bv[g].y, p3[t], 0, 0, 0);
-            }
-            if (last) {
-                // D[row = 4 kq + v][col]: output channel n0 + 16 t + 4 kq + v, column m = wave * 16 + col
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    float2* p = cblk + (long)(n0 + 16 * t + 4 * kq + v) * Mtot + (wave * 16 + col);
-                    float2 r = make_float2(p1[t][v] - p3[t][v], p1[t][v] + p2[t][v]);
-                    if (has_beta) r = cadd(r, cmul(*p, beta));      // C = alpha A W + beta C (variants A, B)
-                    *p = r;
-                }
-            }
+        for (int v = 0; v < 4; ++v) {
+            float2* p = cblk + (long)(n0 + 16 * t + 4 * kq + v) * Mtot + (wave * 16 + col);
+            float2 r = make_float2(p1[v] - p3[v], p1[v] + p2[v]);
+            if (has_beta) r = cadd(r, cmul(*p, beta));      // C = alpha A W + beta C (variants A, B)
+            *p = r;
         }
     }
 }
 
-// K <= 64 and several column blocks per CU: persistent. A block builds the W'' tile once and walks column blocks (XCD j the
-// j-th eighth of them, in order). There is no barrier inside the walk, so the waves of a CU drift apart, and the loads of
-// one, the matrix work of another and the stores of a third overlap; the strip of the next column block is requested
-// before the matrix work on the current one starts. C = alpha A W only (beta = 0).
+// Several column blocks per CU: persistent, beta = 0. A block builds the W'' tile once and walks column blocks; the strip of
+// the next one is requested before the matrix work on the current one ends.
 template <int NG>
 __global__ __launch_bounds__(GEMM_THREADS) void cgemm_modes3m_persistent_kernel(const float2* __restrict__ A,
                                                                                 const float2* __restrict__ W,
                                                                                 float2* __restrict__ C, long Mtot, int N, int K,
                                                                                 float2 alpha, long nblocks, int Kw)
 {
-    extern __shared__ float sW[];                     // 3 * kW3Plane floats
+    __shared__ float sW[3 * kW3Plane<NG>];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 15, kq = lane >> 4;
     const int n0 = blockIdx.y * 64;
     const unsigned lane_off = (unsigned)(kq * Mtot) + (unsigned)(wave * 16 + col);
@@ -532,26 +627,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void cgemm_modes3m_persistent_kernel(
     long v = blockIdx.x;                              // the grid is no larger than the number of column blocks
     float2 bv[NG];
     fetch(bv, block_of(v));
-    {
-        constexpr int WPT = GEMM_KC * 64 / GEMM_THREADS;
-        float2 wv[WPT];
-#pragma unroll
-        for (int u = 0; u < WPT; ++u) {
-            const int idx = tid + u * GEMM_THREADS;
-            const int k = idx % GEMM_KC, n = idx / GEMM_KC;
-            wv[u] = (k < K) ? W[k % Kw + (long)(n0 + n) * Kw] : make_float2(0.f, 0.f);
-        }
-#pragma unroll
-        for (int u = 0; u < WPT; ++u) {
-            const int idx = tid + u * GEMM_THREADS;
-            const int k = idx % GEMM_KC, n = idx / GEMM_KC;
-            const float c = wv[u].x * alpha.x - wv[u].y * alpha.y, d = wv[u].x * alpha.y + wv[u].y * alpha.x;
-            float* dstw = &sW[(k >> 2) * kW3Group + (k & 3) * kW3Row + n];
-            dstw[0] = c;
-            dstw[kW3Plane] = d - c;
-            dstw[2 * kW3Plane] = c + d;
-        }
-    }
+    build_w3_tile<NG>(sW, W, n0, K, Kw, alpha, tid);
     __syncthreads();
     for (; v < nblocks; v += gridDim.x) {
         asm volatile("" ::: "memory");                // keeps the operand fetches from the W'' tile inside the loop (192 registers otherwise)
@@ -570,8 +646,8 @@ __global__ __launch_bounds__(GEMM_THREADS) void cgemm_modes3m_persistent_kernel(
             for (int g = 0; g < NG; ++g) {
                 const float* w = wrow + g * kW3Group;
                 p1 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[0], bv[g].x + bv[g].y, p1, 0, 0, 0);
-                p2 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[kW3Plane], bv[g].x, p2, 0, 0, 0);
-                p3 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[2 * kW3Plane], bv[g].y, p3, 0, 0, 0);
+                p2 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[kW3Plane<NG>], bv[g].x, p2, 0, 0, 0);
+                p3 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[2 * kW3Plane<NG>], bv[g].y, p3, 0, 0, 0);
                 // the last n tile has used this group of the strip: its registers take the next column block's
                 if (t == 3 && more) bv[g] = (next_active && 4 * g < K) ? (nblk + (long)(4 * g) * Mtot)[lane_off] : make_float2(0.f, 0.f);
             }
@@ -582,83 +658,6 @@ __global__ __launch_bounds__(GEMM_THREADS) void cgemm_modes3m_persistent_kernel(
                     *p = make_float2(p1[vv] - p3[vv], p1[vv] + p2[vv]);
                 }
             }
-        }
-    }
-}
-
-// 64 < K <= 128, beta = 0: persistent as well. The W'' tile of ALL channels (three planes of 32 channel groups, 123 KiB:
-// one block per CU) is built once; a column block is multiplied in chunks of 32 channels with the accumulators of the
-// four n tiles kept, the strip registers of a chunk take the next chunk (or the first chunk of the next column block) as
-// soon as the last n tile has used them, and nothing inside the walk waits at a barrier.
-constexpr int GEMM_KMAX = 128;
-constexpr int kW3WidePlane = (GEMM_KMAX / 4) * kW3Group;
-__global__ __launch_bounds__(GEMM_THREADS) void cgemm_modes3m_persistent_wide_kernel(const float2* __restrict__ A,
-                                                                                     const float2* __restrict__ W,
-                                                                                     float2* __restrict__ C, long Mtot, int N, int K,
-                                                                                     float2 alpha, long nblocks, int Kw)
-{
-    extern __shared__ float sW[];                     // 3 * kW3WidePlane floats
-    constexpr int NG = 8;                             // channel groups per chunk
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 15, kq = lane >> 4;
-    const int n0 = blockIdx.y * 64;
-    const unsigned lane_off = (unsigned)(kq * Mtot) + (unsigned)(wave * 16 + col);
-    const bool eighths = (gridDim.x & 7) == 0 && (nblocks & 7) == 0;
-    auto block_of = [&](long v) { return eighths ? (v & 7) * (nblocks >> 3) + (v >> 3) : v; };
-    const int nchunks = (K + 4 * NG - 1) / (4 * NG);
-    // strip of chunk c of column block mb: lane (kq, col) holds channels 32 c + 4 g + kq
-    auto strip_elem = [&](long mb, int c, int g) {
-        const int k = 4 * NG * c + 4 * g;
-        const bool ok = mb * GEMM_MBLOCK + wave * 16 < Mtot && k < K;         // Mtot is a multiple of 16, not of 256
-        return ok ? (A + mb * GEMM_MBLOCK + (long)k * Mtot)[lane_off] : make_float2(0.f, 0.f);
-    };
-    long v = blockIdx.x;                              // the grid is no larger than the number of column blocks
-    float2 bv[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) bv[g] = strip_elem(block_of(v), 0, g);
-    for (int idx = tid; idx < GEMM_KMAX * 64; idx += GEMM_THREADS) {
-        const int k = idx % GEMM_KMAX, n = idx / GEMM_KMAX;
-        const float2 w = (k < K) ? W[k % Kw + (long)(n0 + n) * Kw] : make_float2(0.f, 0.f);
-        const float c = w.x * alpha.x - w.y * alpha.y, d = w.x * alpha.y + w.y * alpha.x;
-        float* dstw = &sW[(k >> 2) * kW3Group + (k & 3) * kW3Row + n];
-        dstw[0] = c;
-        dstw[kW3WidePlane] = d - c;
-        dstw[2 * kW3WidePlane] = c + d;
-    }
-    __syncthreads();
-    for (; v < nblocks; v += gridDim.x) {
-        asm volatile("" ::: "memory");                // keeps the operand fetches from the W'' tile inside the loop
-        const long mb = block_of(v);
-        const bool more = v + gridDim.x < nblocks;
-        const long nb = more ? block_of(v + gridDim.x) : mb;
-        floatx4 p1[4], p2[4], p3[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) p1[t] = p2[t] = p3[t] = floatx4{ 0.f, 0.f, 0.f, 0.f };
-        for (int c = 0; c < nchunks; ++c) {
-            const bool last = c + 1 == nchunks;
-            const bool refill = !last || more;
-            const long fb = last ? nb : mb;           // where the strip registers are refilled from
-            const int fc = last ? 0 : c + 1;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const float* wrow = &sW[(c * NG) * kW3Group + kq * kW3Row + t * 16 + col];
-#pragma unroll
-                for (int g = 0; g < NG; ++g) {
-                    const float* w = wrow + g * kW3Group;
-                    p1[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[0], bv[g].x + bv[g].y, p1[t], 0, 0, 0);
-                    p2[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[kW3WidePlane], bv[g].x, p2[t], 0, 0, 0);
-                    p3[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[2 * kW3WidePlane], bv[g].y, p3[t], 0, 0, 0);
-                    if (t == 3 && refill) bv[g] = strip_elem(fb, fc, g);
-                }
-            }
-        }
-        if (mb * GEMM_MBLOCK + wave * 16 < Mtot) {
-            float2* cblk = C + mb * GEMM_MBLOCK;
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int vv = 0; vv < 4; ++vv)
-                    cblk[(long)(n0 + 16 * t + 4 * kq + vv) * Mtot + (wave * 16 + col)] =
-                        make_float2(p1[t][vv] - p3[t][vv], p1[t][vv] + p2[t][vv]);
         }
     }
 }
@@ -755,76 +754,76 @@ hipError_t launch_ifft2d_pad(int logDX, int logDY, const float2* spec, float2* y
     return dispatch_image_kernel(true, logDX, logDY, spec, y, nimg, stream);
 }
 
+// Which kernel (times for the stand-alone product on operands that come from HBM, in us, column of the kernel before /
+// this one):
+//  * K <= 16: fp32 matrix instructions (M = 262,144, N = 128, K = 16: 55 against 74 with a step of 32 channels); with
+//    several column blocks per CU the persistent kernel. K <= 32 as well for N >= 128 and 8 to 16 blocks of 256 columns x 64
+//    output channels per CU (M = 262,144, N = 128, K = 32: 77 against 88 us; from 16 on the 128-channel tile below is ahead).
+//  * otherwise the split kernel. At most half a block of 256 columns x 64 output channels per CU: blocks of 128 columns
+//    (M = 16,384, N = 64, K = 64: fp32 18.6, 256 columns 14.0, 128 columns 11.1); also for N = 64 with one to two blocks per
+//    CU and more than 32 channels, where two blocks of 128 columns on a CU overlap each other's phases (M = 65,536, K = 64:
+//    22.7 / 21.5 / 19.6; M = 98,304: 36.2 / 26.9 / 24.2).
+//    N a multiple of 128, up to 96 channels and 8 or more blocks per CU: tiles of 128 output channels, A is read once
+//    (M = 524,288, K = 64: 271 / 214 / 197).
+//    Else blocks of 256 columns, tiles of 64 (M = 163,840, N = 128, K = 72: 136 -> 90; M = 262,144, N = 128, K = 128: 259 -> 182).
 hipError_t launch_cgemm_modes(const float2* A, const float2* W, float2* C, long Mtot, int N, int K, float2 alpha,
                               float2 beta, hipStream_t stream, int w_period)
 {
     if (Mtot % 16 != 0 || Mtot <= 0 || Mtot >= (1L << 27) || N % 64 != 0 || K % 8 != 0) return hipErrorInvalidValue;
     const int Kw = w_period > 0 ? w_period : K;
-    if (K % Kw != 0) return hipErrorInvalidValue;
-    dim3 grid((unsigned)((Mtot + GEMM_MBLOCK - 1) / GEMM_MBLOCK), (unsigned)(N / 64), 1);
-    constexpr size_t lds_bytes = sizeof(float) * 3 * kW3Plane;      // 61,632 B: above the static limit
-    auto launch = [&](auto ng_const, auto multi_const) -> hipError_t {
-        constexpr int NG = decltype(ng_const)::value;
-        constexpr bool MULTI = decltype(multi_const)::value;
-        static std::atomic<unsigned long long> served;
-        if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(cgemm_modes3m_kernel<NG, MULTI>), lds_bytes, served);
-            e != hipSuccess)
-            return e;
-        hipLaunchKernelGGL((cgemm_modes3m_kernel<NG, MULTI>), grid, dim3(GEMM_THREADS), lds_bytes, stream, A, W, C, Mtot, N, K,
-                           alpha, beta, Kw);
-        return hipGetLastError();
-    };
-    // several column blocks per CU, one chunk: persistent blocks, one per CU (and n tile)
+    if (K % Kw != 0 || Kw % 8 != 0) return hipErrorInvalidValue;
+    const long cus = cu_count(), columns = (Mtot + GEMM_MBLOCK - 1) / GEMM_MBLOCK, blocks = columns * (N / 64);
+    const bool no_beta = beta.x == 0.f && beta.y == 0.f;
+
     auto launch_persistent = [&](auto ng_const) -> hipError_t {
         constexpr int NG = decltype(ng_const)::value;
-        static std::atomic<unsigned long long> served;
-        if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(cgemm_modes3m_persistent_kernel<NG>), lds_bytes, served);
-            e != hipSuccess)
-            return e;
-        const long nblocks = grid.x;
-        // one block per CU and n tile; with several n tiles, 48 channels or more and up to two column blocks per CU the
-        // matrix pipes are the bound and one block per CU in all is faster (N = 128, K = 64: M = 65,536 41 -> 35 us,
-        // 131,072 71 -> 62; with fewer channels or more columns the kernel is bound by the loads in flight and loses 5-25 %)
-        long g = cu_count();
-        if (grid.y > 1 && K >= 48 && nblocks <= 2L * cu_count()) g /= (long)grid.y;
+        long g = cus;                                            // one block per CU and n tile
         if (g >= 8) g -= g % 8;                                  // whole groups of eight: every XCD the same share
-        if (g < 1) g = 1;
-        hipLaunchKernelGGL((cgemm_modes3m_persistent_kernel<NG>), dim3((unsigned)g, grid.y, 1), dim3(GEMM_THREADS), lds_bytes,
-                           stream, A, W, C, Mtot, N, K, alpha, nblocks, Kw);
+        if (g > columns) g = columns;
+        hipLaunchKernelGGL((cgemm_modes3m_persistent_kernel<NG>), dim3((unsigned)g, (unsigned)(N / 64), 1), dim3(GEMM_THREADS), 0,
+                           stream, A, W, C, Mtot, N, K, alpha, columns, Kw);
         return hipGetLastError();
     };
-    // from two column blocks per CU (K = N = 64: M = 131,072 40 -> 37 us, 262,144 75 -> 64, 524,288 164 -> 133; below that
-    // the two kernels are level)
-    // Not with beta: reading C back inside the walk waits for the strip requested just before it (K = 32, M = 262,144:
-    // 79 against 74 us).
-    if (K <= GEMM_KC && beta.x == 0.f && beta.y == 0.f &&
-        ((long)grid.x >= 2L * cu_count() || (K >= 48 && (long)grid.x * (long)grid.y >= 2L * cu_count()))) {
-        if (K <= 16) return launch_persistent(std::integral_constant<int, 4>{});
-        if (K <= 32) return launch_persistent(std::integral_constant<int, 8>{});
-        if (K <= 48) return launch_persistent(std::integral_constant<int, 12>{});
-        return launch_persistent(std::integral_constant<int, 16>{});
-    }
-    // from eight column blocks per CU (all n tiles together): 3-9 % ahead of the chunked kernel below (K = N = 128,
-    // M = 262,144: 274 -> 255 us); level at four, and up to 8 % behind on small problems (the larger tile to build)
-    if (K > GEMM_KC && K <= GEMM_KMAX && beta.x == 0.f && beta.y == 0.f && (long)grid.x * (long)grid.y >= 8L * cu_count()) {
-        constexpr size_t wide_lds = sizeof(float) * 3 * kW3WidePlane;            // 123,264 B: one block per CU
-        static std::atomic<unsigned long long> served;
-        if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(cgemm_modes3m_persistent_wide_kernel), wide_lds, served);
-            e != hipSuccess)
-            return e;
-        long g = cu_count() / (long)grid.y;
-        if (g >= 8) g -= g % 8;
-        if (g < 1) g = 1;
-        if (g > (long)grid.x) g = grid.x;
-        hipLaunchKernelGGL(cgemm_modes3m_persistent_wide_kernel, dim3((unsigned)g, grid.y, 1), dim3(GEMM_THREADS), wide_lds, stream, A,
-                           W, C, Mtot, N, K, alpha, (long)grid.x, Kw);
+    // Persistent not with beta: reading C back inside the walk waits for the strip requested just before it
+    // (K = 32, M = 262,144: 79 against 74 us).
+    if (K <= 16 && no_beta && columns >= 2 * cus) return launch_persistent(std::integral_constant<int, 4>{});
+    if (K > 16 && K <= 32 && no_beta && N >= 128 && blocks >= 8 * cus && blocks < 16 * cus)
+        return launch_persistent(std::integral_constant<int, 8>{});
+    if (K <= 16) {
+        hipLaunchKernelGGL((cgemm_modes3m_kernel<4>), dim3((unsigned)columns, (unsigned)(N / 64), 1), dim3(GEMM_THREADS), 0, stream, A,
+                           W, C, Mtot, N, K, alpha, beta, Kw);
         return hipGetLastError();
     }
-    if (K <= 16) return launch(std::integral_constant<int, 4>{}, std::false_type{});
-    if (K <= 32) return launch(std::integral_constant<int, 8>{}, std::false_type{});
-    if (K <= 48) return launch(std::integral_constant<int, 12>{}, std::false_type{});
-    if (K <= GEMM_KC) return launch(std::integral_constant<int, 16>{}, std::false_type{});
-    return launch(std::integral_constant<int, 8>{}, std::true_type{});
+
+    // cap: steps of 32 channels that the tile can hold; per_cu: blocks per CU
+    auto launch_split = [&](auto nt_const, auto threads_const, int cap, int per_cu) -> hipError_t {
+        constexpr int NT = decltype(nt_const)::value, THREADS = decltype(threads_const)::value;
+        // one run over the tile covers one period of the weights where that wastes no part of a step, or else all K
+        // channels, if the tile can hold them
+        const bool periods = Kw % GEMM_KSTEP == 0 || (K + GEMM_KSTEP - 1) / GEMM_KSTEP > cap;
+        const int Kp = periods ? Kw : K, steps = (Kp + GEMM_KSTEP - 1) / GEMM_KSTEP;
+        const size_t lds_bytes = kSplitStepBytes * NT * (steps < cap ? steps : cap);
+        static std::atomic<unsigned long long> served;
+        if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(cgemm_modes_split_kernel<NT, THREADS>), kSplitStepBytes * NT * cap, served);
+            e != hipSuccess)
+            return e;
+        const long nblocks = (Mtot + THREADS / 4 - 1) / (THREADS / 4), tiles = N / (16 * NT);
+        if (lds_bytes * per_cu > 160 * 1024) per_cu = 1;
+        long g = per_cu * cus / tiles;
+        if (g >= 8) g -= g % 8;
+        if (g < 1) g = 1;
+        if (g > nblocks) g = nblocks;
+        hipLaunchKernelGGL((cgemm_modes_split_kernel<NT, THREADS>), dim3((unsigned)g, (unsigned)tiles, 1), dim3(THREADS), lds_bytes, stream,
+                           A, W, C, Mtot, K, alpha, beta, nblocks, Kw, Kp, cap);
+        return hipGetLastError();
+    };
+    using Tiles4 = std::integral_constant<int, 4>;
+    using Tiles8 = std::integral_constant<int, 8>;
+    using Columns128 = std::integral_constant<int, 512>;
+    using Columns256 = std::integral_constant<int, 1024>;
+    if (2 * blocks <= cus || (N == 64 && K > 32 && blocks >= cus && blocks < 2 * cus)) return launch_split(Tiles4{}, Columns128{}, 6, 2);
+    if (N % 128 == 0 && (Kw + GEMM_KSTEP - 1) / GEMM_KSTEP <= 3 && blocks >= 8 * cus) return launch_split(Tiles8{}, Columns128{}, 3, 1);
+    return launch_split(Tiles4{}, Columns256{}, 6, 1);
 }
 
 }  // namespace tfno
