@@ -161,11 +161,13 @@ int turbofno_layer_2d_noalloc(int bs, int DX, int DY, int K, int N, const void* 
 /*
  * Process-wide choice of the fused 1D kernel behind turbofno_fused_fft_cgemm_ifft / turbofno_layer_1d and the Y stage
  * of the three-kernel 2D path (their reference-shaped signatures have no room for a selector): 0 = by problem size
- * (default), 1 = SIMT contraction, 2 / 3 = matrix cores with 512- / 256-thread blocks, 4 = matrix cores, 512 threads,
- * 32-channel output tiles, 5 = matrix cores, one wavefront per signal set and output tile, 6 = matrix cores, the K
- * channels of an item split over the waves of a block, 7 = matrix cores, the K channels of a signal set split over a
- * cluster of blocks (see below), 8 = matrix cores, 256-thread blocks with tiles of 128 output channels and three real
- * products per complex one (DY = 128 / 256). A value a kernel is not built for falls back to the choice by size. Meant for tests and measurements; set returns TURBOFNO_ERR_INVALID_ARG outside 0..TURBOFNO_1D_ALGO_MAX.
+ * (default), 1 = SIMT contraction, 2 = matrix cores with 512-thread blocks, 3 = matrix cores with 256-thread blocks of 64
+ * output channels, 4 = as 2 with 32-channel output tiles, 5 = as 3, laid out for four blocks per compute unit (DY = 128 with
+ * eight input channels: one wavefront per signal set and output tile), 6 = matrix cores, the K channels of an item split over
+ * the waves of a block, 7 = matrix cores, the K channels of a signal set split over a cluster of blocks (see below), 8 = as 3
+ * with 128 output channels per block where N allows and the size of the problem makes that the faster one (DY = 128 / 256).
+ * A value a kernel is not built for falls back to the choice by size. Meant for tests and measurements; set returns
+ * TURBOFNO_ERR_INVALID_ARG outside 0..TURBOFNO_1D_ALGO_MAX.
  */
 #define TURBOFNO_1D_ALGO_MAX 8
 int turbofno_set_1d_algo(int algo);

@@ -93,3 +93,36 @@ def test_weights_with_a_period(bs, DX, DY, K, N):
     torch.cuda.synchronize()
     ref = oracle.layer_2d(x, W, 1 - 1j)
     assert rel_l2(y.cpu().numpy(), ref) < 1e-6 and max_rel(y.cpu().numpy(), ref) < 1e-5
+
+
+@pytest.mark.parametrize("S,DY,K,N", [
+    (224, 256, 8, 64),               # half a round: two of four waves without a transform
+    (300, 256, 40, 192),             # a short last round, three blocks of 64 channels per signal set
+    (900, 256, 24, 64),              # four blocks per CU
+    (130, 256, 16, 256),             # a tail of two signal sets behind the groups of eight
+    (512, 256, 128, 128),            # blocks of 128 channels
+    (912, 256, 72, 128),             # the same with a short last round
+    (200, 128, 40, 64),              # DY = 128: rounds of 32 channels, the last with eight
+    (257, 128, 24, 192),             # one round of 24
+    (260, 128, 16, 64),              # half a round: the second step of the product is skipped
+    (513, 128, 104, 128),            # blocks of 128 channels, the last round with eight
+    (560, 128, 56, 256),             # the same with 24 in the last round, two blocks per signal set
+])
+def test_fused_1d_edges(S, DY, K, N):
+    """the fused 1D kernel with split products, chosen by size: every row of y written (y starts as NaN), the first, last and
+    some inner signal sets against the oracle"""
+    print("split fused 1d", S, DY, K, N, flush=True)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert tf.query_1d_kernel(DY, S, N, K, compute_units=0) in (3, 5, 8)
+    gen = torch.Generator(device="cuda").manual_seed(S + DY + K)
+    x = torch.view_as_complex(torch.rand((K, S, DY, 2), device="cuda", generator=gen) * 2 - 1)
+    W = _complex(np.random.default_rng(S), N, K) / np.float32(np.sqrt(K))
+    y = torch.full((N, S, DY), float("nan"), dtype=torch.complex64, device="cuda")
+    tf.layer_1d(x, _dev(W), y=y, alpha=0.5 - 0.75j)
+    torch.cuda.synchronize()
+    assert not bool(torch.isnan(torch.view_as_real(y)).any()), "rows of y left unwritten"
+    idx = torch.tensor(sorted({0, 1, 7, 8, S // 2, S - 9, S - 2, S - 1}), device="cuda")
+    ref = oracle.layer_1d(x.index_select(1, idx).cpu().numpy(), W, 0.5 - 0.75j)
+    # the product as above, and two transforms of eight real additions in a row per value
+    err = rel_l2(y.index_select(1, idx).cpu().numpy(), ref)
+    assert err < _bound(K) + 2 * 16 ** 0.5 * 2.0 ** -24, err

@@ -58,4 +58,15 @@ __device__ __forceinline__ void mac_split2(const SplitOperand& a, const SplitOpe
     c0 = mfma_bf16(a.h, b0.h, c0); c1 = mfma_bf16(a.h, b1.h, c1);
 }
 
+// c0 += a0 b, c1 += a1 b: two independent chains
+__device__ __forceinline__ void mac_split_pair(const SplitOperand& a0, const SplitOperand& a1, const SplitOperand& b, float4_v& c0, float4_v& c1)
+{
+    c0 = mfma_bf16(a0.h, b.l, c0); c1 = mfma_bf16(a1.h, b.l, c1);
+    c0 = mfma_bf16(a0.l, b.h, c0); c1 = mfma_bf16(a1.l, b.h, c1);
+    c0 = mfma_bf16(a0.m, b.m, c0); c1 = mfma_bf16(a1.m, b.m, c1);
+    c0 = mfma_bf16(a0.h, b.m, c0); c1 = mfma_bf16(a1.h, b.m, c1);
+    c0 = mfma_bf16(a0.m, b.h, c0); c1 = mfma_bf16(a1.m, b.h, c1);
+    c0 = mfma_bf16(a0.h, b.h, c0); c1 = mfma_bf16(a1.h, b.h, c1);
+}
+
 }  // namespace tfno

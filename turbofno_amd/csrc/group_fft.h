@@ -285,6 +285,14 @@ TFNO_DEV void pair128_backward(const cpx (&c)[8], const cpx (&tw)[16], cpx* exch
     rows128_backward(c, tw, exch, t, y);
 }
 
+#ifdef __HIPCC__
+TFNO_DEV float rotate8(float v)        // value of lane t ^ 8 of the same 16-lane row
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
+}
+TFNO_DEV cpx rotate8(cpx v) { return make_float2(rotate8(v.x), rotate8(v.y)); }
+#endif
+
 // The 16 samples t + L i of one output signal. By default y is streamed past the caches (it is written once and not read
 // again by the layer); KEEP leaves it cached for a consumer that follows at once (the X-axis backward kernel of the
 // three-kernel 2D pipeline: 895 -> 854 us for 16 images of 512 x 512, K = 32, N = 64).

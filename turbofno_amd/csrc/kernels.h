@@ -99,7 +99,7 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
                                        float2 alpha, int algo, hipStream_t stream, bool y_is_reread = false);
 // The kernel that call runs (the selector values 1 ... 8), from the sizes alone.
 enum {
-    kFused1dSimt = 1, kFused1dMfma512 = 2, kFused1dMfma256 = 3, kFused1dMfma512Tile32 = 4, kFused1dWave = 5,
+    kFused1dSimt = 1, kFused1dMfma512 = 2, kFused1dMfma256 = 3, kFused1dMfma512Tile32 = 4, kFused1dDense = 5,
     kFused1dSplit = 6, kFused1dCluster = 7, kFused1dWide = 8
 };
 int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y, long cus, bool exchange_attached);
@@ -116,10 +116,10 @@ hipError_t exchange_attach(hipStream_t stream, void* buffer, size_t bytes);   //
 bool exchange_attached(hipStream_t stream);
 hipError_t exchange_gave_up(hipStream_t stream, unsigned* count);   // waits for the stream
 
-// Large grids, DY = 128 / 256 (layer1d_wide.hip): one block per (signal set, 128 or 64 output channels), three-real-product
-// contraction.
-hipError_t launch_fused_wide(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha,
-                             hipStream_t stream, int keep_y = 0);
+// Grids of about one block per CU and more, DY = 128 / 256 (layer1d_split.hip): one block per (signal set, 64 or, if `wide` and N
+// allows, 128 output channels); `dense`: the variant for four blocks per CU.
+hipError_t launch_fused_split(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, bool wide,
+                              bool dense, hipStream_t stream, int keep_y = 0);
 
 // Halves of the fused kernel (variants B and C) and the stand-alone contiguous transforms (variant A).
 hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C,

@@ -163,24 +163,19 @@ template <int LOGDY, int THREADS_, int NT_ = 64> struct GeoMfma1D {
     static constexpr int NT = NT_;
     static constexpr int NTW = (NT / 2) / (THREADS / 64);     // 16x16 tiles per wave: one m tile x NTW n' tiles
     static constexpr int KC = THREADS / L;                    // channels per chunk = lane groups per block
-    // compact: sC shares the exchange regions too and the twiddles move to LDS: 53 KiB and 168 registers, three blocks
-    // per CU. Only for DY = 256: at DY = 128 (8 modes per lane) the register limit costs more in spills than it gains.
-    static constexpr bool COMPACT = THREADS_ == 256 && LOGDY == 8;
-    static constexpr int PA = 80, PC = COMPACT ? 66 : 72;     // pitches (complex) of sA and sC
+    static constexpr int PA = 80, PC = 72;                    // pitches (complex) of sA and sC
     static constexpr int EXCH = L * 17;
     static constexpr int REGION0 = KC * EXCH > KC * PA ? KC * EXCH : KC * PA;              // exchange | sA
     static constexpr int WTILE = (KC / 4) * kWGroup / 2;                                   // W' tile in complex units
-    static constexpr int REGION1 = COMPACT ? WTILE : (WTILE > NT * PC ? WTILE : NT * PC);  // W' | sC   (complex)
-    static_assert(!COMPACT || NT * PC <= REGION0, "sC must fit the exchange regions");
+    static constexpr int REGION1 = WTILE > NT * PC ? WTILE : NT * PC;                      // W' | sC   (complex)
     static_assert(NT == 64 || (NT == 32 && THREADS_ == 512), "32-channel tiles: 512 threads");
     static constexpr int PASSES = (NT + KC - 1) / KC;         // backward passes; the last may use only NT % KC lane groups
-    static constexpr int TWTAB = COMPACT ? kTwLdsSize : 0;    // compact: twiddles in LDS instead of 30 registers
-    static constexpr int DEPTH = COMPACT ? 1 : 2;             // chunks of loads in flight per lane group
-    static constexpr size_t LDS_BYTES = sizeof(float2) * (size_t)(REGION0 + REGION1 + TWTAB);
+    static constexpr int DEPTH = 2;                           // chunks of loads in flight per lane group
+    static constexpr size_t LDS_BYTES = sizeof(float2) * (size_t)(REGION0 + REGION1);
 };
 
 template <int LOGDY, int THREADS, int NT, bool KEEP = false>
-__global__ __launch_bounds__(THREADS, (THREADS == 256 && LOGDY == 8) ? 3 : 1) void fused_fft_mfma_ifft_kernel(int S, int N, int K, const float2* __restrict__ x,
+__global__ __launch_bounds__(THREADS, 1) void fused_fft_mfma_ifft_kernel(int S, int N, int K, const float2* __restrict__ x,
                                                                       const float2* __restrict__ W, float2* __restrict__ y,
                                                                       float2 alpha)
 {
@@ -190,7 +185,7 @@ __global__ __launch_bounds__(THREADS, (THREADS == 256 && LOGDY == 8) ? 3 : 1) vo
     extern __shared__ float2 lds[];
     float2* sA = lds;                                          // [KC][PA]; aliases the exchange regions
     float* sW = reinterpret_cast<float*>(lds + G::REGION0);    // W' tile, layout of kWGroup / kWHalf
-    float2* sC = G::COMPACT ? lds : lds + G::REGION0;          // [64][PC]; aliases sW (or sA) after the K loop
+    float2* sC = lds + G::REGION0;                             // [64][PC]; aliases sW after the K loop
 
     const int tid = threadIdx.x;
     const int g = tid / L, t = tid % L;                        // transform role: lane group = channel of the chunk
@@ -200,19 +195,13 @@ __global__ __launch_bounds__(THREADS, (THREADS == 256 && LOGDY == 8) ? 3 : 1) vo
     int ntile;
     decode_block_1d(S, N / NT, 1 << LOGDY, !KEEP, s, ntile);
     const int n0 = ntile * NT;
-    // DY = 128: signals are transformed in pairs by 16-lane groups (see the SIMT kernel); COMPACT never applies there
+    // DY = 128: signals are transformed in pairs by 16-lane groups (see the SIMT kernel)
     constexpr bool PAIR = LOGDY == 7;
     const int t16 = tid % 16, gpair = (tid / 16) * 2;
     float2* exch = PAIR ? lds + (tid / 16) * (2 * G::EXCH) : lds + g * G::EXCH;
 
     cpx tw[16];
-    const float2* twrow = lds + G::REGION0 + G::REGION1 + t * kTwLdsPitch;
-    if constexpr (G::COMPACT) {
-        fill_lds_twiddles<LOGDY>(lds + G::REGION0 + G::REGION1, tid, THREADS);
-        __syncthreads();
-    } else {
-        load_lane_twiddles<LOGDY>(PAIR ? t16 : t, tw);
-    }
+    load_lane_twiddles<LOGDY>(PAIR ? t16 : t, tw);
 
     floatx4_1d acc[NTW];
 #pragma unroll
@@ -256,8 +245,7 @@ __global__ __launch_bounds__(THREADS, (THREADS == 256 && LOGDY == 8) ? 3 : 1) vo
                 pair128_forward(w, tw, exch, t16, out);
             } else {
                 cpx gg[16];
-                if constexpr (G::COMPACT) fwd_pass1_lds(v, twrow, gg);
-                else fwd_pass1(v, tw, gg);
+                fwd_pass1(v, tw, gg);
                 if (kc + G::DEPTH * KC + g < K) issue(v, kc + G::DEPTH * KC);    // the chunk DEPTH chunks ahead
                 group_forward_finish<LOGDY>(gg, exch, t, out);
             }
@@ -303,14 +291,11 @@ __global__ __launch_bounds__(THREADS, (THREADS == 256 && LOGDY == 8) ? 3 : 1) vo
         sC[(n + 1) * PC + mt * 16 + col] = make_float2(acc[i][2], acc[i][3]);
     }
     __syncthreads();
-    // every pass takes its modes before the first backward transform: in the compact layout the exchange regions
-    // overlay sC
     cpx c[G::PASSES][MM];
 #pragma unroll
     for (int pass = 0; pass < G::PASSES; ++pass)
 #pragma unroll
         for (int a = 0; a < MM; ++a) c[pass][a] = (g + KC * pass < NT) ? sC[(g + KC * pass) * PC + t + L * a] : make_float2(0.f, 0.f);
-    if constexpr (G::COMPACT) __syncthreads();
 #pragma unroll
     for (int pass = 0; pass < G::PASSES; ++pass) {
         const int n = g + KC * pass;
@@ -321,56 +306,42 @@ __global__ __launch_bounds__(THREADS, (THREADS == 256 && LOGDY == 8) ? 3 : 1) vo
             float2* dst = y + ((long)(n0 + gpair + KC * pass) * S + s) * DY + t16;
             store_pair16<KEEP>(dst, (long)S * DY, yv);
         } else {
-            if constexpr (G::COMPACT) group_backward_lds<LOGDY>(c[pass], twrow, exch, t, yv);
-            else group_backward<LOGDY>(c[pass], tw, exch, t, yv);
+            group_backward<LOGDY>(c[pass], tw, exch, t, yv);
             float2* dst = y + ((long)(n0 + n) * S + s) * DY + t;
             store_row16<L, KEEP>(dst, yv);
         }
     }
 }
 
-// Fused 1D layer for large grids, DY = 128 / 256: ONE WAVEFRONT per (signal set, 64 output channels), no block barrier
+// Fused 1D layer for DY = 128 and eight input channels: ONE WAVEFRONT per (signal set, 64 output channels), no block barrier
 // and no staging of operands through LDS. The register layouts of the transforms and of v_mfma_f32_16x16x4_f32 coincide:
-//   * DY = 256: the four 16-lane groups of a wave transform four channels k = kc + g at a time and lane (g, t) ends up
-//     with modes t + 16 a, a < 4, of channel g: exactly the B operand (k = lane / 16, column = lane % 16) of the four
-//     m tiles a;
 //   * the A operand row n' = 16 nt + t, k = g is one element of W (times alpha, as (re, -im) or (im, re)), read
 //     straight from global memory (W is a few KiB and stays in the vector cache);
+//   * a 16-lane group transforms two channels kc + 2 g + h at a time (lane t = r + 8 h finishes channel h with modes
+//     r + 8 c, c < 8); one exchange between lanes t and t ^ 8 (a row rotation, no LDS) turns that into modes
+//     t + 16 a of each of the two channels, i.e. two B operands;
 //   * the accumulators D[row = 4 g + v][column = t] of tile (nt, a) hold, for j = 0, 1, the complex value
-//     (v = 2 j, 2 j + 1) of output channel n = 8 nt + 2 g + j at mode t + 16 a: the input layout of the zero-padded
-//     backward transform of channel n by lane group g;
-//   * DY = 128: a lane group transforms two channels kc + 2 g + h at a time (lane t = r + 8 h finishes channel h with
-//     modes r + 8 c, c < 8); one exchange between lanes t and t ^ 8 (a row rotation, no LDS) turns that into modes
-//     t + 16 a of each of the two channels, i.e. two B operands, and the same exchange leads from the accumulators to
-//     the paired backward transform of output channels 8 nt + 2 g and 8 nt + 2 g + 1.
+//     (v = 2 j, 2 j + 1) of output channel n = 8 nt + 2 g + j at mode t + 16 a; the same exchange leads to the paired
+//     backward transform of output channels 8 nt + 2 g and 8 nt + 2 g + 1.
 // 32 accumulator tiles (128 registers) per wave, two waves per SIMD; the only LDS traffic left is the exchange inside
-// the transforms. The loads of the next channels are issued as soon as the first pass has consumed the current ones
-// and travel under the exchange, the second pass and the matrix instructions (64 per four channels).
-TFNO_DEV float rotate8(float v)        // value of lane t ^ 8 of the same 16-lane row
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
-}
-TFNO_DEV cpx rotate8(cpx v) { return make_float2(rotate8(v.x), rotate8(v.y)); }
-
-template <int LOGDY, bool KEEP = false>
+// the transforms. With eight channels the split kernel (layer1d_split.hip) leaves three of four waves without a transform:
+// S = 1000, N = 64: 16.4 here against 18.8 us, N = 128: 32.5 / 33.6, S = 16384, N = 64: 198 / 201; from 16 channels on that kernel is
+// ahead (S = 1000, K = 16, N = 64: 20.5 / 18.7).
+template <bool KEEP>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void fused_fft_mfma_ifft_wave_kernel(
     int S, int N, int K, const float2* __restrict__ x, const float2* __restrict__ W, float2* __restrict__ y, float2 alpha)
 {
-    constexpr int DY = 1 << LOGDY, EXCH = 16 * 17;
-    constexpr bool PAIR = LOGDY == 7;
-    constexpr int CH = PAIR ? 8 : 4;                              // channels per round
-    constexpr int REGIONS = PAIR ? 4 : 8;                         // DY = 256: a second set for the paired backward transforms
-    __shared__ float2 lds[REGIONS * EXCH + kTwLdsSize];
+    constexpr int DY = 128, EXCH = 16 * 17, CH = 8;               // CH = channels per round
+    __shared__ float2 lds[4 * EXCH + kTwLdsSize];
     const int lane = threadIdx.x, g = lane >> 4, t = lane & 15;
     float2* exch = lds + g * EXCH;
-    float2* exch1 = exch + (PAIR ? 0 : 4 * EXCH);                 // second region: two backward transforms in flight
-    float2* twtab = lds + REGIONS * EXCH;
-    fill_lds_twiddles<LOGDY>(twtab, lane, 64);
+    float2* twtab = lds + 4 * EXCH;
+    fill_lds_twiddles<7>(twtab, lane, 64);
     const float2* twrow = twtab + t * kTwLdsPitch;
     __syncthreads();
     long s;
     int ntile;
-    decode_block_1d(S, N / 64, 1 << LOGDY, !KEEP, s, ntile);
+    decode_block_1d(S, N / 64, DY, !KEEP, s, ntile);
     const int n0 = ntile * 64;
     const bool upper = t >> 3, odd = t & 1;
 
@@ -380,17 +351,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
         for (int a = 0; a < 4; ++a) acc[nt][a] = floatx4_1d{ 0.f, 0.f, 0.f, 0.f };
 
-    // lane (g, t): samples t + 16 i of channel kc + g (DY = 256) or of channels kc + 2 g, kc + 2 g + 1 (DY = 128)
-    const float2* src = x + ((long)(PAIR ? 2 * g : g) * S + s) * DY + t;
-    const float2* wsrc = W + (PAIR ? 2 * g : g) + (long)(n0 + (t >> 1)) * K;   // W[k][n = n0 + 8 nt + t / 2]
+    // lane (g, t): samples t + 16 i of channels kc + 2 g, kc + 2 g + 1
+    const float2* src = x + ((long)(2 * g) * S + s) * DY + t;
+    const float2* wsrc = W + (2 * g) + (long)(n0 + (t >> 1)) * K;   // W[k][n = n0 + 8 nt + t / 2]
     auto issue = [&](cpx (&dst)[16]) {
-        if constexpr (PAIR) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) { dst[i] = src[16 * i]; dst[8 + i] = src[(long)S * DY + 16 * i]; }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) dst[i] = src[16 * i];
-        }
+        for (int i = 0; i < 8; ++i) { dst[i] = src[16 * i]; dst[8 + i] = src[(long)S * DY + 16 * i]; }
     };
     // one complex product row: acc += W'(row n', k) x B(k, column), W' = alpha W as (re, -im) / (im, re) by row parity
     auto contract = [&](floatx4_1d (&d)[4], float2 wk, const cpx (&b)[4]) {
@@ -409,87 +375,61 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
         for (int nt = 0; nt < 8; ++nt) {
             wv[nt] = wsrc[kc + (long)(8 * nt) * K];
-            if constexpr (PAIR) wv1[nt] = wsrc[kc + 1 + (long)(8 * nt) * K];
+            wv1[nt] = wsrc[kc + 1 + (long)(8 * nt) * K];
         }
-        if constexpr (!PAIR) {
-            cpx gg[16], out[4];
-            fwd_pass1_lds(v, twrow, gg);
-            if (kc + CH < K) { src += (long)CH * S * DY; issue(v); }
-            group_forward_finish<8>(gg, exch, t, out);
+        cpx gg[16], out[8], b8[8];
+        {
+            cpx a8[8];
 #pragma unroll
-            for (int nt = 0; nt < 8; ++nt) contract(acc[nt], wv[nt], out);
-        } else {
-            cpx gg[16], out[8], b8[8];
-            {
-                cpx a8[8];
+            for (int i = 0; i < 8; ++i) { a8[i] = v[i]; b8[i] = v[8 + i]; }
+            fft8<-1>(a8);
+            fft8<-1>(b8);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) { a8[i] = v[i]; b8[i] = v[8 + i]; }
-                fft8<-1>(a8);
-                fft8<-1>(b8);
+            for (int r = 0; r < 8; ++r) gg[r] = a8[r];
+        }
+        if (kc + CH < K) { src += (long)CH * S * DY; issue(v); }
+        gg[8] = b8[0];
 #pragma unroll
-                for (int r = 0; r < 8; ++r) gg[r] = a8[r];
-            }
-            if (kc + CH < K) { src += (long)CH * S * DY; issue(v); }
-            gg[8] = b8[0];
+        for (int r = 1; r < 8; ++r) {
+            const cpx w = twrow[r];
+            gg[r] = cmul(gg[r], w);
+            gg[8 + r] = cmul(b8[r], w);
+        }
+        rows128_forward_finish(gg, exch, t, out);             // out[c] = mode (t & 7) + 8 c of channel t >> 3
+        // lanes t < 8 keep the even c of their channel and take the even c of the other one; lanes t >= 8 the odd c
+        cpx b0[4], b1[4];
 #pragma unroll
-            for (int r = 1; r < 8; ++r) {
-                const cpx w = twrow[r];
-                gg[r] = cmul(gg[r], w);
-                gg[8 + r] = cmul(b8[r], w);
-            }
-            rows128_forward_finish(gg, exch, t, out);             // out[c] = mode (t & 7) + 8 c of channel t >> 3
-            // lanes t < 8 keep the even c of their channel and take the even c of the other one; lanes t >= 8 the odd c
-            cpx b0[4], b1[4];
+        for (int a = 0; a < 4; ++a) {
+            const cpx got = rotate8(upper ? out[2 * a] : out[2 * a + 1]);
+            b0[a] = upper ? got : out[2 * a];                 // channel kc + 2 g,     mode t + 16 a
+            b1[a] = upper ? out[2 * a + 1] : got;             // channel kc + 2 g + 1, mode t + 16 a
+        }
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const cpx got = rotate8(upper ? out[2 * a] : out[2 * a + 1]);
-                b0[a] = upper ? got : out[2 * a];                 // channel kc + 2 g,     mode t + 16 a
-                b1[a] = upper ? out[2 * a + 1] : got;             // channel kc + 2 g + 1, mode t + 16 a
-            }
-#pragma unroll
-            for (int nt = 0; nt < 8; ++nt) {
-                contract(acc[nt], wv[nt], b0);
-                contract(acc[nt], wv1[nt], b1);
-            }
+        for (int nt = 0; nt < 8; ++nt) {
+            contract(acc[nt], wv[nt], b0);
+            contract(acc[nt], wv1[nt], b1);
         }
     }
     // backward: the two output channels (j = 0, 1) a lane group owns per n tile are transformed together
 #pragma unroll
     for (int nt = 0; nt < 8; ++nt) {
-        cpx c0[4], c1[4], y0[16], y1[16];
+        cpx c0[4], c1[4], y0[16];
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
             c0[a] = make_float2(acc[nt][a][0], acc[nt][a][1]);   // channel 8 nt + 2 g,     mode t + 16 a
             c1[a] = make_float2(acc[nt][a][2], acc[nt][a][3]);   // channel 8 nt + 2 g + 1, mode t + 16 a
         }
         float2* dst = y + ((long)(n0 + 8 * nt + 2 * g) * S + s) * DY + t;
-        if constexpr (!PAIR) {
-            // each through its own exchange region, so that the LDS round trips of one overlap the arithmetic of the other
-            cpx h0[16], h1[16], e0[16], e1[16];
-            dft16_pad4<+1>(c0, h0);
-            dft16_pad4<+1>(c1, h1);
-            wave_lds_fence();
+        // lane t = r + 8 h finishes channel h: modes r + 8 c; even c come from lanes t < 8, odd c from lanes t >= 8
+        cpx c8[8];
 #pragma unroll
-            for (int tt = 0; tt < 16; ++tt) { exch[tt * 17 + t] = h0[tt]; exch1[tt * 17 + t] = h1[tt]; }
-            wave_lds_fence();
-#pragma unroll
-            for (int r = 0; r < 16; ++r) { e0[r] = exch[t * 17 + r]; e1[r] = exch1[t * 17 + r]; }
-            inv_pass2_lds(e0, twrow, y0);
-            inv_pass2_lds(e1, twrow, y1);
-            store_row16<16, KEEP>(dst, y0);
-            store_row16<16, KEEP>(dst + (long)S * DY, y1);
-        } else {
-            // lane t = r + 8 h finishes channel h: modes r + 8 c; even c come from lanes t < 8, odd c from lanes t >= 8
-            cpx c8[8];
-#pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const cpx got = rotate8(upper ? c0[a] : c1[a]);
-                c8[2 * a] = upper ? got : c0[a];
-                c8[2 * a + 1] = upper ? c1[a] : got;
-            }
-            rows128_backward(c8, twrow, exch, t, y0);
-            store_pair16<KEEP>(dst, (long)S * DY, y0);
+        for (int a = 0; a < 4; ++a) {
+            const cpx got = rotate8(upper ? c0[a] : c1[a]);
+            c8[2 * a] = upper ? got : c0[a];
+            c8[2 * a + 1] = upper ? c1[a] : got;
         }
+        rows128_backward(c8, twrow, exch, t, y0);
+        store_pair16<KEEP>(dst, (long)S * DY, y0);
     }
 }
 
@@ -731,81 +671,55 @@ static hipError_t launch_fused_mfma(long S, int N, int K, const float2* x, const
                   : launch_fused_mfma_k<LOGDY, THREADS, NT, false>(S, N, K, x, W, y, alpha, stream);
 }
 
-template <int LOGDY>
-static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha,
-                                    hipStream_t stream, int keep_y = 0)
+static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, hipStream_t stream,
+                                    int keep_y)
 {
     if (S * (N / 64) > 0x7fffffffL) return hipErrorInvalidValue;
     if (keep_y)
-        hipLaunchKernelGGL((fused_fft_mfma_ifft_wave_kernel<LOGDY, true>), dim3((unsigned)(S * (N / 64))), dim3(64), 0, stream, (int)S, N,
-                           K, x, W, y, alpha);
+        hipLaunchKernelGGL((fused_fft_mfma_ifft_wave_kernel<true>), dim3((unsigned)(S * (N / 64))), dim3(64), 0, stream, (int)S, N, K, x, W,
+                           y, alpha);
     else
-        hipLaunchKernelGGL((fused_fft_mfma_ifft_wave_kernel<LOGDY, false>), dim3((unsigned)(S * (N / 64))), dim3(64), 0, stream, (int)S,
-                           N, K, x, W, y, alpha);
+        hipLaunchKernelGGL((fused_fft_mfma_ifft_wave_kernel<false>), dim3((unsigned)(S * (N / 64))), dim3(64), 0, stream, (int)S, N, K, x, W,
+                           y, alpha);
     return hipGetLastError();
 }
 
 // Which fused 1D kernel runs for a problem: pure arithmetic on the sizes, the selector `algo`, the number of compute
 // units and whether the stream has an exchange buffer attached (no device call), so that callers and tests can ask.
-// algo: 0 = by size, 1 = SIMT kernel, 2 = matrix cores with 512-thread blocks, 3 = matrix cores with 256-thread blocks,
-// 4 = as 2 with 32-channel output tiles, 5 = matrix cores, one wavefront per (signal set, output tile),
-// 6 = matrix cores, the eight waves of a block split the K channels of one item (DY = 256),
-// 7 = matrix cores, a cluster of blocks splits the K channels of one signal set (DY = 256, N = 64 / 128, small grids),
-// 8 = matrix cores, 256-thread blocks with tiles of 128 output channels, three real products per complex one (DY = 256)
+// algo: 0 = by size, 1 = SIMT kernel, 2 = matrix cores with 512-thread blocks, 3 = matrix cores with 256-thread blocks of 64 output
+// channels, 4 = as 2 with 32-channel output tiles, 5 = as 3 for large grids: four blocks per CU, or with eight channels of
+// length 128 one wavefront per (signal set, output tile), 6 = matrix cores, the eight waves of a block split the K channels of one
+// item (DY = 256), 7 = matrix cores, a cluster of blocks splits the K channels of one signal set (DY = 256, N = 64 / 128, small
+// grids), 8 = as 3 with 128 output channels per block where N allows (DY = 128, 256)
 // The return value uses the same numbers (1 ... 8). A selector value that a kernel is not built for falls back to the
 // choice by size.
 //
-// By size (measured on MI355X):
+// By size (measured on MI355X, us, kernel of the smaller grids against the split kernel):
 //  * while every block has a CU to itself: matrix cores, 8 waves per block - the shortest chain of latencies for
 //    every K, even K = 8 where most of a chunk is padding;
-//  * grids of several items per SIMD: one wavefront per item (no barriers, nothing staged through LDS). At DY = 128
-//    it is ahead from two (K <= 16), four (K < 128) or eight items per CU; at DY = 256, where the block kernels are
-//    closer to what the access pattern allows, for K >= 128 (2-8 % from eight items per CU) and, K >= 24, on the
-//    very largest grids (4-6 % from 128 items per CU); below that the 256-thread block kernel is level or up to
-//    13 % ahead;
-//  * otherwise: matrix cores, 256-thread blocks, two or three per CU, for every K - measured 5-27 % ahead of the
-//    SIMT kernel on grids of 1 to 12 items per CU also for K < 32, where most of a chunk is padding (lengths
-//    512 / 1024: a tie within a few percent for every K, the SIMT kernel stays; on small grids the 512-thread
-//    kernel is 30-40 % ahead there too).
+//  * about one block of 64 output channels per CU and more, lengths 128 / 256: the split kernel (layer1d_split.hip). DY = 128 with
+//    32 channels or more from three quarters of the CUs on (N = 64: S = 200, K = 64: 13.8 / 12.2, S = 128: 10.9 / 11.8; N = 128:
+//    S = 100, K = 64: 13.5 / 12.1), DY = 256 from seven eighths on (N = 64: S = 256, K = 32: 14.7 / 13.2, S = 128, K = 64: 13.5 / 16.9),
+//    with N = 128 from three quarters on (S = 128, K = 64: 19.1 / 17.9; S = 64: 14.0 / 16.9);
+//  * lengths 512 / 1024: a tie within a few percent for every K on large grids, the SIMT kernel stays; on small grids
+//    the 512-thread kernel is 30-40 % ahead there too.
 int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y, long cus, bool exchange_attached)
 {
     const bool built = logDY >= 7 && logDY <= 10;
     const bool long_signal = logDY >= 9;            // 512 / 1024: on large grids the block kernels tie with the SIMT kernel
     const long items = S * (N / 64);
-    if (algo == 5 && (logDY == 7 || logDY == 8)) return kFused1dWave;
-    // N a multiple of 128, DY = 256, K >= 16: blocks with tiles of 128 output channels (every input channel transformed
-    // once per signal set, three real products per complex one): 5-20 % ahead of the kernels below on every grid that
-    // fills its two slots per CU reasonably evenly (measured from 400 blocks up; with a last round under three quarters
-    // full the 64-channel kernels, with their finer blocks, are ahead)
-    if (algo == 0 && logDY == 8 && N % 128 == 0 && K >= 16) {
-        const long blocks = S * (N / 128), slots = 2L * cus, rounds = (blocks + slots - 1) / slots;
-        if (blocks > cus && 4 * blocks >= 3 * rounds * slots) return kFused1dWide;
+    if (algo == 5 && !long_signal && built) return kFused1dDense;
+    if (algo == 0 && !long_signal && built) {
+        const long blocks = N % 128 == 0 ? S * (N / 128) : items;
+        if (blocks > cus) {
+            if (N % 128 == 0 && K >= 16) return kFused1dWide;           // 128 or 64 output channels per block: wide_tiles()
+            // blocks of 64 output channels, a few per CU
+            if (logDY == 7 && N % 128 != 0 && K >= 16 && blocks <= (K >= 128 ? 4 : 2) * cus) return kFused1dWide;
+            if (logDY == 8 && N % 128 != 0 && K >= 128 && blocks <= 4 * cus) return kFused1dWide;
+        }
+        // DY = 128: several items per SIMD
+        if (logDY == 7 && items >= (K <= 16 ? 2 : (K < 128 ? 4 : 8)) * cus) return kFused1dDense;
     }
-    // the same at DY = 128 for K >= 64 (3-21 % ahead up to 64 blocks per CU; with fewer channels, or on the very largest
-    // grids, the one-wavefront kernel below is level or ahead)
-    if (algo == 0 && logDY == 7 && N % 128 == 0 && K >= 64) {
-        const long blocks = S * (N / 128), slots = 2L * cus, rounds = (blocks + slots - 1) / slots;
-        if (blocks > cus && blocks <= 64L * cus && 4 * blocks >= 3 * rounds * slots) return kFused1dWide;
-    }
-    // DY = 128, about one wide block per CU (three quarters to all of them), 16 channels or more: 5-32 % ahead of the
-    // kernels below, whose blocks are finer than there are CUs to fill
-    if (algo == 0 && logDY == 7 && N % 128 == 0 && K >= 16) {
-        const long blocks = S * (N / 128);
-        if (4 * blocks >= 3L * cus && blocks <= cus) return kFused1dWide;
-    }
-    // DY = 128 with N not a multiple of 128 (tiles of 64, three real products): one to two blocks per CU, 16 channels or
-    // more: 6-22 % ahead; with 128 channels up to four per CU (12 %)
-    if (algo == 0 && logDY == 7 && N % 128 != 0 && K >= 16) {
-        const long blocks = S * (N / 64);
-        if (blocks >= cus && blocks <= (K >= 128 ? 4L : 2L) * cus) return kFused1dWide;
-    }
-    // DY = 256, N not a multiple of 128, 128 channels or more, up to four blocks of 64-channel tiles per CU: 6-8 % ahead
-    if (algo == 0 && logDY == 8 && N % 128 != 0 && K >= 128) {
-        const long blocks = S * (N / 64);
-        if (blocks > cus && blocks <= 4L * cus) return kFused1dWide;
-    }
-    if (algo == 0 && logDY == 7 && items >= (K <= 16 ? 2 : (K < 128 ? 4 : 8)) * cus) return kFused1dWave;
-    if (algo == 0 && logDY == 8 && (K >= 128 ? items >= 8L * cus : (K >= 24 && items >= 128L * cus))) return kFused1dWave;
     // small grids, 64 channels or more, N = 64 / 128: a cluster of blocks per signal set, no forward transform twice.
     // Only for streams that have an exchange buffer attached; without one the kernels below take over.
     if (algo == 7 || (algo == 0 && logDY == 8 && K >= 64)) {
@@ -814,6 +728,10 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y,
     }
     if (algo == 8 && (logDY == 7 || logDY == 8)) return kFused1dWide;
     if (algo == 8) algo = 0;
+    // not quite one block per CU
+    if (algo == 0 && logDY == 7 && K >= 16 && N % 128 == 0 && 2 * items >= 3 * cus && items <= 2 * cus) return kFused1dWide;
+    if (algo == 0 && logDY == 7 && K >= 32 && 4 * items >= 3 * cus && items <= cus) return kFused1dMfma256;
+    if (algo == 0 && logDY == 8 && (N % 128 == 0 ? 4 * items >= 3 * cus : 8 * items >= 7 * cus) && items <= cus) return kFused1dMfma256;
     int pick = algo == 4 ? 2 : algo;
     // lengths 512 / 1024 with 64 channels or more, x and y streamed: the 256-thread matrix-core kernel is 7-16 % ahead of
     // the SIMT kernel on grids of up to four blocks per CU (level or up to 10 % behind on larger ones)
@@ -829,6 +747,22 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y,
     return kFused1dSimt;
 }
 
+// Split kernel, N a multiple of 128: blocks of 128 output channels transform every input once per 128 outputs, blocks of 64 twice as
+// often (the second time from L2), but they are finer and four fit a CU instead of three. 128 pays where the repeated transforms or reads
+// are many (us, 64 / 128): DY = 256, S = 8192, K = 128: 1180 / 960; S = 4096, K = 40: 336 / 296, K = 32: 218 / 222; S = 1000, K = 96: 94 / 89,
+// K = 64: 77 / 78; S = 333, K = 128: 46.6 / 50.9. DY = 128, S = 8192, K = 128: 654 / 569; S = 3000, K = 64: 138 / 123, K = 32: 92 / 101; S = 1000,
+// K = 96: 66 / 62, K = 40: 41.4 / 46.1; and where 128 fills one round of the CUs that 64 would need two for (S = 700, K = 64: 37.9 / 32.9).
+static bool wide_tiles(int logDY, long S, int N, int K, long cus)
+{
+    const long blocks = S * (N / 128), volume = (long)K * S;
+    if (N % 128 != 0) return false;
+    if (logDY == 8) return volume >= 65536 && (K >= 64 || volume >= 160000);
+    return (K >= 96 && blocks >= 2 * cus) || volume >= 160000 || (K >= 40 && blocks > 2 * cus && blocks <= 3 * cus);
+}
+// Blocks of 64 output channels at DY = 256: registers and LDS for four per CU once there are more than three (S = 1000, K = N = 64:
+// 49.9 / 46.2 us); with two per CU the larger register budget is ahead (S = 512, K = 96: 37.4 / 39.3).
+static bool dense_blocks(long S, int N, long cus) { return S * (N / 64) > 3 * cus; }
+
 hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* y,
                                        float2 alpha, int algo, hipStream_t stream, bool y_is_reread)
 {
@@ -843,10 +777,11 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
         kernel = pick_fused_1d_kernel(logDY, S, N, K, algo, y_is_reread, cus, false);    // detached in between
     }
     switch (kernel) {
-    case kFused1dWave:
-        return logDY == 8 ? launch_fused_wave<8>(S, N, K, x, W, y, alpha, stream, keep_y)
-                          : launch_fused_wave<7>(S, N, K, x, W, y, alpha, stream, keep_y);
-    case kFused1dWide: return launch_fused_wide(logDY, S, N, K, x, W, y, alpha, stream, keep_y);
+    case kFused1dDense:
+        if (logDY == 7 && K <= 8) return launch_fused_wave(S, N, K, x, W, y, alpha, stream, keep_y);
+        return launch_fused_split(logDY, S, N, K, x, W, y, alpha, false, true, stream, keep_y);
+    case kFused1dWide:
+        return launch_fused_split(logDY, S, N, K, x, W, y, alpha, wide_tiles(logDY, S, N, K, cus), dense_blocks(S, N, cus), stream, keep_y);
     case kFused1dSplit: {
         static std::atomic<unsigned long long> served;
         if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(fused_fft_mfma_ifft_split_kernel), SPLIT_LDS, served);
@@ -869,8 +804,8 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
         }
     case kFused1dMfma256:
         switch (logDY) {
-        case 7: return launch_fused_mfma<7, 256>(S, N, K, x, W, y, alpha, stream, keep_y);
-        case 8: return launch_fused_mfma<8, 256>(S, N, K, x, W, y, alpha, stream, keep_y);
+        case 7:
+        case 8: return launch_fused_split(logDY, S, N, K, x, W, y, alpha, false, dense_blocks(S, N, cus), stream, keep_y);
         case 9: return launch_fused_mfma<9, 256>(S, N, K, x, W, y, alpha, stream, keep_y);
         default: return launch_fused_mfma<10, 256>(S, N, K, x, W, y, alpha, stream, keep_y);
         }
