@@ -107,6 +107,12 @@ def test_weights_with_a_period(bs, DX, DY, K, N):
     (260, 128, 16, 64),              # half a round: the second step of the product is skipped
     (513, 128, 104, 128),            # blocks of 128 channels, the last round with eight
     (560, 128, 56, 256),             # the same with 24 in the last round, two blocks per signal set
+    (260, 512, 40, 64),              # DY = 512: two passes per round, the last round with one
+    (140, 512, 32, 128),             # blocks of 64 channels with N = 128
+    (520, 512, 104, 128),            # blocks of 128 channels
+    (258, 1024, 40, 64),             # DY = 1024: four passes per round, the last round with two
+    (193, 1024, 8, 128),             # blocks of 128 channels, half a round
+    (256, 1024, 72, 128),            # the same with a short last round
 ])
 def test_fused_1d_edges(S, DY, K, N):
     """the fused 1D kernel with split products, chosen by size: every row of y written (y starts as NaN), the first, last and
@@ -126,3 +132,36 @@ def test_fused_1d_edges(S, DY, K, N):
     # the product as above, and two transforms of eight real additions in a row per value
     err = rel_l2(y.index_select(1, idx).cpu().numpy(), ref)
     assert err < _bound(K) + 2 * 16 ** 0.5 * 2.0 ** -24, err
+
+
+@pytest.mark.parametrize("S,DY,K,N", [
+    (1, 128, 8, 64), (9, 128, 40, 192), (400, 128, 56, 128),        # rounds of 32 channels: one of eight, a last one of eight, of 24
+    (1, 256, 8, 64), (9, 256, 40, 192), (400, 256, 72, 128),        # S = 400: blocks of 128 output channels
+    (3, 512, 24, 64), (400, 512, 40, 128), (2, 1024, 8, 64), (390, 1024, 24, 128),
+])
+@pytest.mark.parametrize("beta", [0.0, -1 + 1j])
+def test_halves_of_the_layer(S, DY, K, N, beta):
+    """forward transforms with the product (every value of C written, or added to with beta), product with backward transforms"""
+    print("split halves", S, DY, K, N, beta, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(S + DY + K)
+    rng = np.random.default_rng(S + K)
+    x = torch.view_as_complex(torch.rand((K, S, DY, 2), device="cuda", generator=gen) * 2 - 1)
+    W, W2 = _complex(rng, N, K) / np.float32(np.sqrt(K)), _complex(rng, N, N) / np.float32(np.sqrt(N))
+    C0 = torch.full((N, S, 64), float("nan"), dtype=torch.complex64, device="cuda") if beta == 0.0 else \
+        torch.view_as_complex(torch.rand((N, S, 64, 2), device="cuda", generator=gen) * 2 - 1)
+    C = C0.clone()
+    tf.fused_fft_cgemm(64 * S, N, K, x, _dev(W), C, 0.5 - 0.75j, beta)
+    y = torch.full((N, S, DY), float("nan"), dtype=torch.complex64, device="cuda")
+    tf.fused_cgemm_ifft(64 * S, N, N, C, _dev(W2), y, 1 - 1j)
+    torch.cuda.synchronize()
+    assert not bool(torch.isnan(torch.view_as_real(C)).any()), "values of C left unwritten"
+    assert not bool(torch.isnan(torch.view_as_real(y)).any()), "rows of y left unwritten"
+    idx = torch.tensor(sorted({0, S // 2, max(0, S - 9), S - 1}), device="cuda")
+    pick = lambda a: a.index_select(1, idx).cpu().numpy()
+    ref = oracle.cgemm(oracle.fft_trunc_contig(pick(x)).reshape(K, -1), W, 0.5 - 0.75j).reshape(N, -1, 64)
+    if beta != 0.0:
+        ref = ref + beta * pick(C0).astype(np.complex128)
+    slack = 16 ** 0.5 * 2.0 ** -24                                  # a transform, as above
+    assert rel_l2(pick(C), ref) < _bound(K) + slack
+    ref = oracle.ifft_pad_contig(oracle.cgemm(pick(C).reshape(N, -1), W2, 1 - 1j).reshape(N, -1, 64), DY)
+    assert rel_l2(pick(y), ref) < _bound(N) + slack

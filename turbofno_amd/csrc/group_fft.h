@@ -67,18 +67,15 @@ TFNO_DEV void wide_forward_finish(const cpx (&g)[16], cpx* exch, const cpx* powe
     }
 }
 
-// Backward, up to the inputs of the last pass: c[mm] = mode t + L mm; on return e[r] = first-pass input r of lane t
+// Backward, up to the inputs of the last pass: c[mm] = mode t + L mm (or, _of_stored: mode m in exch[m] already); on return e[r] = first-pass input r of lane t
 // (before the conjugate twiddle). Lane l = (t1 = l % Q, rq = l / Q), Q = L / 4, forms the inputs of the four lanes
 // t1 + Q t2 for the bins r = rq + 4 ri (wide_backward_partial_tw) and parks them for their owners at
 // [r][lane ^ (Q rq)], rows of L: the owners read a row as L consecutive elements, and the XOR puts the four rq of one
 // write Q elements apart, so that the 32 lanes of a half wavefront hit 32 different bank pairs in both directions.
 template <int L, bool FROM_ARRAY>
-TFNO_DEV void wide_backward_inputs(const cpx (&c)[64 / L], const cpx* powers, cpx* exch, int t, cpx (&e)[16])
+TFNO_DEV void wide_backward_inputs_of_stored(const cpx* powers, cpx* exch, int t, cpx (&e)[16])
 {
     constexpr int Q = L / 4;
-    wave_lds_fence();
-#pragma unroll
-    for (int mm = 0; mm < 64 / L; ++mm) exch[t + L * mm] = c[mm];
     wave_lds_fence();
     cpx part[16];
     const int t1 = t % Q, rq = t / Q;
@@ -92,6 +89,14 @@ TFNO_DEV void wide_backward_inputs(const cpx (&c)[64 / L], const cpx* powers, cp
     wave_lds_fence();
 #pragma unroll
     for (int r = 0; r < 16; ++r) e[r] = exch[r * L + (t ^ (Q * (r & 3)))];
+}
+template <int L, bool FROM_ARRAY>
+TFNO_DEV void wide_backward_inputs(const cpx (&c)[64 / L], const cpx* powers, cpx* exch, int t, cpx (&e)[16])
+{
+    wave_lds_fence();
+#pragma unroll
+    for (int mm = 0; mm < 64 / L; ++mm) exch[t + L * mm] = c[mm];
+    wide_backward_inputs_of_stored<L, FROM_ARRAY>(powers, exch, t, e);
 }
 // Mode that lane t of an L-lane group holds in out[mm] after a forward transform.
 template <int LOGDY> TFNO_DEV constexpr int forward_mode_of_lane(int t, int mm)

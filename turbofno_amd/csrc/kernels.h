@@ -121,6 +121,11 @@ hipError_t exchange_gave_up(hipStream_t stream, unsigned* count);   // waits for
 hipError_t launch_fused_split(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, bool wide,
                               bool dense, hipStream_t stream, int keep_y = 0);
 
+// The same kernel without its backward transforms (C = alpha A W + beta C) or without its forward transforms.
+hipError_t launch_split_forward(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C, float2 alpha, float2 beta,
+                                bool wide, hipStream_t stream);
+hipError_t launch_split_backward(int logDY, long S, int N, int K, const float2* A, const float2* W, float2* y, float2 alpha, hipStream_t stream);
+
 // Halves of the fused kernel (variants B and C) and the stand-alone contiguous transforms (variant A).
 hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C,
                                   float2 alpha, float2 beta, hipStream_t stream);

@@ -16,14 +16,10 @@
 
 namespace tfno {
 
-// FUSE_FWD: the A operand is produced by forward transforms of x (variants B and D); otherwise it is read from
-//           the column-major matrix A[m + k*M] (variant C).
-// FUSE_INV: the product goes straight into zero-padded backward transforms (variants C and D); otherwise it is
-//           stored as C[m + n*M] = alpha*A*W + beta*C (variant B).
-template <int LOGDY, bool FUSE_FWD, bool FUSE_INV, bool KEEP = false>
+template <int LOGDY, bool KEEP = false>
 __global__ __launch_bounds__(256) void fused_fft_cgemm_ifft_kernel(int S, int N, int K, const float2* __restrict__ x,
                                                                    const float2* __restrict__ W, float2* __restrict__ y,
-                                                                   float2 alpha, float2 beta)
+                                                                   float2 alpha)
 {
     using G = Geo1D<LOGDY>;
     constexpr int DY = G::DY, L = G::L, GROUPS = G::GROUPS, MM = G::MM, NN = G::NN;
@@ -38,7 +34,6 @@ __global__ __launch_bounds__(256) void fused_fft_cgemm_ifft_kernel(int S, int N,
     int ntile;
     decode_block_1d(S, N / 64, 1 << LOGDY, !KEEP, s, ntile);
     const int n0 = ntile * 64;
-    const long M = 64L * S;
     // signals of 128 samples are transformed in pairs by 16-lane groups (128-byte accesses): lane t16 of pair g/2 holds
     // samples t16 + 16 i of both signals, and ends up with the modes an 8-lane group would give lane (g, t)
     constexpr bool PAIR = LOGDY == 7;
@@ -55,38 +50,27 @@ __global__ __launch_bounds__(256) void fused_fft_cgemm_ifft_kernel(int S, int N,
         for (int b = 0; b < NN; ++b) acc[a][b] = make_float2(0.f, 0.f);
 
     for (int kc = 0; kc < K; kc += GROUPS) {
-        if constexpr (FUSE_FWD) {
-            const int k = kc + g;
-            cpx out[MM];
-            if (k < K) {
-                cpx v[16];
-                if constexpr (PAIR) {
-                    const float2* src = x + ((long)(kc + gpair) * S + s) * DY + t16;
+        const int k = kc + g;
+        cpx out[MM];
+        if (k < K) {
+            cpx v[16];
+            if constexpr (PAIR) {
+                const float2* src = x + ((long)(kc + gpair) * S + s) * DY + t16;
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) { v[i] = src[16 * i]; v[8 + i] = src[(long)S * DY + 16 * i]; }
-                    pair128_forward(v, tw, exch, t16, out);
-                } else {
-                    const float2* src = x + ((long)k * S + s) * DY + t;
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) v[i] = src[L * i];
-                    group_forward<LOGDY>(v, tw, exch, t, out);
-                }
+                for (int i = 0; i < 8; ++i) { v[i] = src[16 * i]; v[8 + i] = src[(long)S * DY + 16 * i]; }
+                pair128_forward(v, tw, exch, t16, out);
             } else {
+                const float2* src = x + ((long)k * S + s) * DY + t;
 #pragma unroll
-                for (int a = 0; a < MM; ++a) out[a] = make_float2(0.f, 0.f);
+                for (int i = 0; i < 16; ++i) v[i] = src[L * i];
+                group_forward<LOGDY>(v, tw, exch, t, out);
             }
-#pragma unroll
-            for (int a = 0; a < MM; ++a) sA[g * G::SA_PITCH + (PAIR ? t + L * a : forward_mode_of_lane<LOGDY>(t, a))] = out[a];
         } else {
-            // A tile of the chunk: 64 contiguous rows (this block's signal) of GROUPS columns
 #pragma unroll
-            for (int j = 0; j < (GROUPS * 64) / 256; ++j) {
-                const int idx = tid + 256 * j;
-                const int mloc = idx % 64, kk = idx / 64;
-                sA[kk * G::SA_PITCH + mloc] =
-                    (kc + kk < K) ? x[s * 64 + mloc + (long)(kc + kk) * M] : make_float2(0.f, 0.f);
-            }
+            for (int a = 0; a < MM; ++a) out[a] = make_float2(0.f, 0.f);
         }
+#pragma unroll
+        for (int a = 0; a < MM; ++a) sA[g * G::SA_PITCH + (PAIR ? t + L * a : forward_mode_of_lane<LOGDY>(t, a))] = out[a];
         // W chunk: GROUPS x 64 elements, consecutive threads read consecutive k (contiguous in memory)
 #pragma unroll
         for (int j = 0; j < (GROUPS * 64) / 256; ++j) {
@@ -115,27 +99,17 @@ __global__ __launch_bounds__(256) void fused_fft_cgemm_ifft_kernel(int S, int N,
 #pragma unroll
     for (int j = 0; j < NN; ++j) {
         const int n = n0 + g + GROUPS * j;
-        if constexpr (FUSE_INV) {
-            cpx c[MM], yv[16];
+        cpx c[MM], yv[16];
 #pragma unroll
-            for (int i = 0; i < MM; ++i) c[i] = cmul(acc[i][j], alpha);
-            if constexpr (PAIR) {
-                pair128_backward(c, tw, exch, t16, yv);
-                float2* dst = y + ((long)(n0 + gpair + GROUPS * j) * S + s) * DY + t16;
-                store_pair16<KEEP>(dst, (long)S * DY, yv);
-            } else {
-                group_backward<LOGDY>(c, tw, exch, t, yv);
-                float2* dst = y + ((long)n * S + s) * DY + t;
-                store_row16<L, KEEP>(dst, yv);
-            }
+        for (int i = 0; i < MM; ++i) c[i] = cmul(acc[i][j], alpha);
+        if constexpr (PAIR) {
+            pair128_backward(c, tw, exch, t16, yv);
+            float2* dst = y + ((long)(n0 + gpair + GROUPS * j) * S + s) * DY + t16;
+            store_pair16<KEEP>(dst, (long)S * DY, yv);
         } else {
-            float2* dst = y + s * 64 + t + (long)n * M;          // C[m + n*M], m = s*64 + t + L*i
-#pragma unroll
-            for (int i = 0; i < MM; ++i) {
-                cpx r = cmul(acc[i][j], alpha);
-                if (beta.x != 0.f || beta.y != 0.f) r = cadd(r, cmul(dst[L * i], beta));
-                dst[L * i] = r;
-            }
+            group_backward<LOGDY>(c, tw, exch, t, yv);
+            float2* dst = y + ((long)n * S + s) * DY + t;
+            store_row16<L, KEEP>(dst, yv);
         }
     }
 }
@@ -156,10 +130,10 @@ __global__ __launch_bounds__(256) void fused_fft_cgemm_ifft_kernel(int S, int N,
 // sC aliases the W' tile.
 typedef float floatx4_1d __attribute__((ext_vector_type(4)));
 
-// NT_ = output channels per block: 64, or 32 to spread a small grid over twice as many CUs (DY = 256, 512 threads).
-template <int LOGDY, int THREADS_, int NT_ = 64> struct GeoMfma1D {
+// NT_ = output channels per block: 64, or 32 to spread a small grid over twice as many CUs (DY = 128 / 256).
+template <int LOGDY, int NT_ = 64> struct GeoMfma1D {
     static constexpr int L = Geo1D<LOGDY>::L, MM = 64 / L;
-    static constexpr int THREADS = THREADS_;                  // 512: one block per CU; 256: two (LDS 72 KiB each)
+    static constexpr int THREADS = 512;                       // one block per CU
     static constexpr int NT = NT_;
     static constexpr int NTW = (NT / 2) / (THREADS / 64);     // 16x16 tiles per wave: one m tile x NTW n' tiles
     static constexpr int KC = THREADS / L;                    // channels per chunk = lane groups per block
@@ -168,18 +142,18 @@ template <int LOGDY, int THREADS_, int NT_ = 64> struct GeoMfma1D {
     static constexpr int REGION0 = KC * EXCH > KC * PA ? KC * EXCH : KC * PA;              // exchange | sA
     static constexpr int WTILE = (KC / 4) * kWGroup / 2;                                   // W' tile in complex units
     static constexpr int REGION1 = WTILE > NT * PC ? WTILE : NT * PC;                      // W' | sC   (complex)
-    static_assert(NT == 64 || (NT == 32 && THREADS_ == 512), "32-channel tiles: 512 threads");
+    static_assert(NT == 64 || NT == 32, "tiles of 64 or 32 output channels");
     static constexpr int PASSES = (NT + KC - 1) / KC;         // backward passes; the last may use only NT % KC lane groups
     static constexpr int DEPTH = 2;                           // chunks of loads in flight per lane group
     static constexpr size_t LDS_BYTES = sizeof(float2) * (size_t)(REGION0 + REGION1);
 };
 
-template <int LOGDY, int THREADS, int NT, bool KEEP = false>
-__global__ __launch_bounds__(THREADS, 1) void fused_fft_mfma_ifft_kernel(int S, int N, int K, const float2* __restrict__ x,
+template <int LOGDY, int NT, bool KEEP = false>
+__global__ __launch_bounds__(512, 1) void fused_fft_mfma_ifft_kernel(int S, int N, int K, const float2* __restrict__ x,
                                                                       const float2* __restrict__ W, float2* __restrict__ y,
                                                                       float2 alpha)
 {
-    using G = GeoMfma1D<LOGDY, THREADS, NT>;
+    using G = GeoMfma1D<LOGDY, NT>;
     constexpr int NTW = G::NTW;
     constexpr int DY = 1 << LOGDY, L = G::L, MM = G::MM, KC = G::KC, PA = G::PA, PC = G::PC;
     extern __shared__ float2 lds[];
@@ -604,71 +578,62 @@ __global__ __launch_bounds__(256) void stride_DY_kernel(const float2* __restrict
     }
 }
 
-template <int LOGDY, bool FUSE_FWD, bool FUSE_INV, bool KEEP>
-static hipError_t launch_fused_1d_k(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha,
-                                    float2 beta, hipStream_t stream)
+// keep_y: the output is read again at once (Y stage of the three-kernel 2D pipeline): plain instead of streaming stores,
+// as a template parameter of the kernels - a run-time branch around the stores cost the 1D layer up to 20 %
+template <int LOGDY, bool KEEP>
+static hipError_t launch_fused_1d_k(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, hipStream_t stream)
 {
     using G = Geo1D<LOGDY>;
     if (S * (N / 64) > 0x7fffffffL) return hipErrorInvalidValue;
     if constexpr (G::LDS_BYTES > 64 * 1024) {          // DY = 128: 32 channels per chunk, 70 KiB
         static std::atomic<unsigned long long> served;
-        if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(fused_fft_cgemm_ifft_kernel<LOGDY, FUSE_FWD, FUSE_INV, KEEP>),
-                                             G::LDS_BYTES, served);
+        if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(fused_fft_cgemm_ifft_kernel<LOGDY, KEEP>), G::LDS_BYTES, served);
             e != hipSuccess)
             return e;
     }
     dim3 grid((unsigned)(S * (N / 64)), 1, 1), block(256, 1, 1);
-    hipLaunchKernelGGL((fused_fft_cgemm_ifft_kernel<LOGDY, FUSE_FWD, FUSE_INV, KEEP>), grid, block, G::LDS_BYTES, stream, (int)S,
-                       N, K, x, W, y, alpha, beta);
+    hipLaunchKernelGGL((fused_fft_cgemm_ifft_kernel<LOGDY, KEEP>), grid, block, G::LDS_BYTES, stream, (int)S, N, K, x, W, y, alpha);
     return hipGetLastError();
 }
-
-// keep_y: the output is read again at once (Y stage of the three-kernel 2D pipeline): plain instead of streaming stores,
-// as a template parameter of the kernels - a run-time branch around the stores cost the 1D layer up to 20 %
-template <int LOGDY, bool FUSE_FWD, bool FUSE_INV>
-static hipError_t launch_fused_1d(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha,
-                                  float2 beta, hipStream_t stream, int keep_y = 0)
+template <int LOGDY>
+static hipError_t launch_fused_1d(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, hipStream_t stream, int keep_y)
 {
-    if constexpr (FUSE_FWD && FUSE_INV) {
-        if (keep_y) return launch_fused_1d_k<LOGDY, FUSE_FWD, FUSE_INV, true>(S, N, K, x, W, y, alpha, beta, stream);
-    }
-    return launch_fused_1d_k<LOGDY, FUSE_FWD, FUSE_INV, false>(S, N, K, x, W, y, alpha, beta, stream);
+    return keep_y ? launch_fused_1d_k<LOGDY, true>(S, N, K, x, W, y, alpha, stream)
+                  : launch_fused_1d_k<LOGDY, false>(S, N, K, x, W, y, alpha, stream);
 }
-
-template <bool FUSE_FWD, bool FUSE_INV>
-static hipError_t dispatch_fused_1d(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* y,
-                                    float2 alpha, float2 beta, hipStream_t stream, int keep_y = 0)
+static hipError_t dispatch_fused_1d(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha,
+                                    hipStream_t stream, int keep_y)
 {
     switch (logDY) {
-    case 7: return launch_fused_1d<7, FUSE_FWD, FUSE_INV>(S, N, K, x, W, y, alpha, beta, stream, keep_y);
-    case 8: return launch_fused_1d<8, FUSE_FWD, FUSE_INV>(S, N, K, x, W, y, alpha, beta, stream, keep_y);
-    case 9: return launch_fused_1d<9, FUSE_FWD, FUSE_INV>(S, N, K, x, W, y, alpha, beta, stream, keep_y);
-    case 10: return launch_fused_1d<10, FUSE_FWD, FUSE_INV>(S, N, K, x, W, y, alpha, beta, stream, keep_y);
+    case 7: return launch_fused_1d<7>(S, N, K, x, W, y, alpha, stream, keep_y);
+    case 8: return launch_fused_1d<8>(S, N, K, x, W, y, alpha, stream, keep_y);
+    case 9: return launch_fused_1d<9>(S, N, K, x, W, y, alpha, stream, keep_y);
+    case 10: return launch_fused_1d<10>(S, N, K, x, W, y, alpha, stream, keep_y);
     default: return hipErrorInvalidValue;
     }
 }
 
-template <int LOGDY, int THREADS, int NT, bool KEEP>
+template <int LOGDY, int NT, bool KEEP>
 static hipError_t launch_fused_mfma_k(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha,
                                       hipStream_t stream)
 {
-    using G = GeoMfma1D<LOGDY, THREADS, NT>;
+    using G = GeoMfma1D<LOGDY, NT>;
     static std::atomic<unsigned long long> served;
-    if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(fused_fft_mfma_ifft_kernel<LOGDY, THREADS, NT, KEEP>),
+    if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(fused_fft_mfma_ifft_kernel<LOGDY, NT, KEEP>),
                                          G::LDS_BYTES, served);
         e != hipSuccess)
         return e;
     if (S * (N / NT) > 0x7fffffffL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((fused_fft_mfma_ifft_kernel<LOGDY, THREADS, NT, KEEP>), dim3((unsigned)(S * (N / NT))), dim3(THREADS),
+    hipLaunchKernelGGL((fused_fft_mfma_ifft_kernel<LOGDY, NT, KEEP>), dim3((unsigned)(S * (N / NT))), dim3(G::THREADS),
                        G::LDS_BYTES, stream, (int)S, N, K, x, W, y, alpha);
     return hipGetLastError();
 }
-template <int LOGDY, int THREADS, int NT = 64>
+template <int LOGDY, int NT = 64>
 static hipError_t launch_fused_mfma(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha,
                                     hipStream_t stream, int keep_y = 0)
 {
-    return keep_y ? launch_fused_mfma_k<LOGDY, THREADS, NT, true>(S, N, K, x, W, y, alpha, stream)
-                  : launch_fused_mfma_k<LOGDY, THREADS, NT, false>(S, N, K, x, W, y, alpha, stream);
+    return keep_y ? launch_fused_mfma_k<LOGDY, NT, true>(S, N, K, x, W, y, alpha, stream)
+                  : launch_fused_mfma_k<LOGDY, NT, false>(S, N, K, x, W, y, alpha, stream);
 }
 
 static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, hipStream_t stream,
@@ -701,12 +666,15 @@ static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const
 //    32 channels or more from three quarters of the CUs on (N = 64: S = 200, K = 64: 13.8 / 12.2, S = 128: 10.9 / 11.8; N = 128:
 //    S = 100, K = 64: 13.5 / 12.1), DY = 256 from seven eighths on (N = 64: S = 256, K = 32: 14.7 / 13.2, S = 128, K = 64: 13.5 / 16.9),
 //    with N = 128 from three quarters on (S = 128, K = 64: 19.1 / 17.9; S = 64: 14.0 / 16.9);
-//  * lengths 512 / 1024: a tie within a few percent for every K on large grids, the SIMT kernel stays; on small grids
-//    the 512-thread kernel is 30-40 % ahead there too.
+//  * lengths 512 / 1024, more than one block per CU: the split kernel from the number of channels on where it is ahead of the SIMT
+//    kernel, which has less to do per channel (DY = 512, S = 2048, N = 64: K = 24 127 / 120, K = 40 185 / 170, K = 128 358 / 305; S = 512:
+//    K = 16 38 / 42, K = 40 52 / 51; N = 128, S = 1000: K = 32 144 / 123, K = 128 327 / 244; DY = 1024, N = 64: S = 2048, K = 32 325 / 318, S = 512,
+//    K = 16 68 / 68; N = 128, S = 1000: K = 32 246 / 257, K = 64 389 / 349). On small grids the 512-thread kernel (S = 128, K = 64, DY = 512:
+//    25.9 / 28.9).
 int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y, long cus, bool exchange_attached)
 {
     const bool built = logDY >= 7 && logDY <= 10;
-    const bool long_signal = logDY >= 9;            // 512 / 1024: on large grids the block kernels tie with the SIMT kernel
+    const bool long_signal = logDY >= 9;            // 512 / 1024
     const long items = S * (N / 64);
     if (algo == 5 && !long_signal && built) return kFused1dDense;
     if (algo == 0 && !long_signal && built) {
@@ -726,17 +694,21 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y,
         if (exchange_attached && cluster_size_1d(logDY, S, N, K, cus) > 0) return kFused1dCluster;
         if (algo == 7) algo = 0;                                // not applicable here: by size, as for every other value
     }
-    if (algo == 8 && (logDY == 7 || logDY == 8)) return kFused1dWide;
+    if (algo == 8 && built) return kFused1dWide;
     if (algo == 8) algo = 0;
     // not quite one block per CU
     if (algo == 0 && logDY == 7 && K >= 16 && N % 128 == 0 && 2 * items >= 3 * cus && items <= 2 * cus) return kFused1dWide;
     if (algo == 0 && logDY == 7 && K >= 32 && 4 * items >= 3 * cus && items <= cus) return kFused1dMfma256;
     if (algo == 0 && logDY == 8 && (N % 128 == 0 ? 4 * items >= 3 * cus : 8 * items >= 7 * cus) && items <= cus) return kFused1dMfma256;
+    // lengths 512 / 1024, more than one block per CU
+    if (algo == 0 && long_signal && built && items > cus) {
+        if (N % 128 == 0 && K >= (logDY == 9 ? 32 : 64)) return kFused1dWide;
+        if (N % 128 != 0 && K >= (logDY == 9 ? 40 : 32)) return kFused1dMfma256;
+        const long blocks = N % 128 == 0 ? S * (N / 128) : 0;
+        if (logDY == 10 && 4 * blocks >= 3 * cus && blocks <= cus) return kFused1dWide;
+    }
     int pick = algo == 4 ? 2 : algo;
-    // lengths 512 / 1024 with 64 channels or more, x and y streamed: the 256-thread matrix-core kernel is 7-16 % ahead of
-    // the SIMT kernel on grids of up to four blocks per CU (level or up to 10 % behind on larger ones)
-    if (pick == 0)
-        pick = (built && items <= cus) ? 2 : ((!long_signal || (K >= 64 && !keep_y && items <= 4L * cus)) ? 3 : 1);
+    if (pick == 0) pick = (built && items <= cus) ? 2 : (long_signal ? 1 : 3);
     // small grids, 64 channels or more: eight waves split the K channels of one item (10-16 % ahead of the kernel that
     // shares the spectra through LDS; level at K = 32)
     if (logDY == 8 && (algo == 6 || (algo == 0 && K >= 64 && S * (N / SPLIT_NT) <= cus))) return kFused1dSplit;
@@ -752,12 +724,18 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y,
 // are many (us, 64 / 128): DY = 256, S = 8192, K = 128: 1180 / 960; S = 4096, K = 40: 336 / 296, K = 32: 218 / 222; S = 1000, K = 96: 94 / 89,
 // K = 64: 77 / 78; S = 333, K = 128: 46.6 / 50.9. DY = 128, S = 8192, K = 128: 654 / 569; S = 3000, K = 64: 138 / 123, K = 32: 92 / 101; S = 1000,
 // K = 96: 66 / 62, K = 40: 41.4 / 46.1; and where 128 fills one round of the CUs that 64 would need two for (S = 700, K = 64: 37.9 / 32.9).
+// DY = 512, S = 2048, K = 128: 502 / 451; S = 1000, K = 64: 153 / 165. DY = 1024 (two blocks per CU either way): S = 512, K = 64: 173 / 163;
+// S = 256, K = 32: 84 / 73, S = 512, K = 32: 134 / 140.
 static bool wide_tiles(int logDY, long S, int N, int K, long cus)
 {
     const long blocks = S * (N / 128), volume = (long)K * S;
     if (N % 128 != 0) return false;
-    if (logDY == 8) return volume >= 65536 && (K >= 64 || volume >= 160000);
-    return (K >= 96 && blocks >= 2 * cus) || volume >= 160000 || (K >= 40 && blocks > 2 * cus && blocks <= 3 * cus);
+    switch (logDY) {
+    case 7: return (K >= 96 && blocks >= 2 * cus) || volume >= 160000 || (K >= 40 && blocks > 2 * cus && blocks <= 3 * cus);
+    case 8: return volume >= 65536 && (K >= 64 || volume >= 160000);
+    case 9: return (K >= 96 && blocks >= 2 * cus) || (K >= 40 && volume >= 80000);
+    default: return K >= 64 ? blocks >= cus : blocks <= cus;
+    }
 }
 // Blocks of 64 output channels at DY = 256: registers and LDS for four per CU once there are more than three (S = 1000, K = N = 64:
 // 49.9 / 46.2 us); with two per CU the larger register budget is ahead (S = 512, K = 96: 37.4 / 39.3).
@@ -793,36 +771,33 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
         return hipGetLastError();
     }
     case kFused1dMfma512Tile32:
-        return logDY == 8 ? launch_fused_mfma<8, 512, 32>(S, N, K, x, W, y, alpha, stream, keep_y)
-                          : launch_fused_mfma<7, 512, 32>(S, N, K, x, W, y, alpha, stream, keep_y);
+        return logDY == 8 ? launch_fused_mfma<8, 32>(S, N, K, x, W, y, alpha, stream, keep_y)
+                          : launch_fused_mfma<7, 32>(S, N, K, x, W, y, alpha, stream, keep_y);
     case kFused1dMfma512:
         switch (logDY) {
-        case 7: return launch_fused_mfma<7, 512>(S, N, K, x, W, y, alpha, stream, keep_y);
-        case 8: return launch_fused_mfma<8, 512>(S, N, K, x, W, y, alpha, stream, keep_y);
-        case 9: return launch_fused_mfma<9, 512>(S, N, K, x, W, y, alpha, stream, keep_y);
-        default: return launch_fused_mfma<10, 512>(S, N, K, x, W, y, alpha, stream, keep_y);
+        case 7: return launch_fused_mfma<7>(S, N, K, x, W, y, alpha, stream, keep_y);
+        case 8: return launch_fused_mfma<8>(S, N, K, x, W, y, alpha, stream, keep_y);
+        case 9: return launch_fused_mfma<9>(S, N, K, x, W, y, alpha, stream, keep_y);
+        default: return launch_fused_mfma<10>(S, N, K, x, W, y, alpha, stream, keep_y);
         }
     case kFused1dMfma256:
-        switch (logDY) {
-        case 7:
-        case 8: return launch_fused_split(logDY, S, N, K, x, W, y, alpha, false, dense_blocks(S, N, cus), stream, keep_y);
-        case 9: return launch_fused_mfma<9, 256>(S, N, K, x, W, y, alpha, stream, keep_y);
-        default: return launch_fused_mfma<10, 256>(S, N, K, x, W, y, alpha, stream, keep_y);
-        }
-    default: return dispatch_fused_1d<true, true>(logDY, S, N, K, x, W, y, alpha, make_float2(0.f, 0.f), stream, keep_y);
+        return launch_fused_split(logDY, S, N, K, x, W, y, alpha, false, logDY <= 8 && dense_blocks(S, N, cus), stream, keep_y);
+    default: return dispatch_fused_1d(logDY, S, N, K, x, W, y, alpha, stream, keep_y);
     }
 }
 
 hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C,
                                   float2 alpha, float2 beta, hipStream_t stream)
 {
-    return dispatch_fused_1d<true, false>(logDY, S, N, K, x, W, C, alpha, beta, stream);
+    // blocks of 128 output channels from one and a half per CU (N = 128, K = 64, DY = 256: S = 700 42.6 -> 34.4 us, S = 256 19.0 -> 19.9)
+    const bool wide = N % 128 == 0 && 2 * S * (N / 128) >= 3L * cu_count();
+    return launch_split_forward(logDY, S, N, K, x, W, C, alpha, beta, wide, stream);
 }
 
 hipError_t launch_fused_cgemm_ifft(int logDY, long S, int N, int K, const float2* A, const float2* W, float2* y,
                                    float2 alpha, hipStream_t stream)
 {
-    return dispatch_fused_1d<false, true>(logDY, S, N, K, A, W, y, alpha, make_float2(0.f, 0.f), stream);
+    return launch_split_backward(logDY, S, N, K, A, W, y, alpha, stream);
 }
 
 template <int LOGDY, bool INVERSE>

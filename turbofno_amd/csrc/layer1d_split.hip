@@ -1,24 +1,27 @@
-// Fused 1D spectral layer for grids of about one block per CU and more, DY = 128 and 256: one 256-thread block per
+// Fused 1D spectral layer for grids of about one block per CU and more, and its halves: one 256-thread block per
 // (signal set, 64 NTW output channels), NTW = 1 or 2, contraction on the bf16 matrix cores with exact three-way splits of both
 // operands (bf16_split.h).
 //
 // Same operands and result as fused_fft_cgemm_ifft_{7,8} of the reference
 // (fusion_variants/1D_D_exp_fused_fft_cgemm_ifft/fused_fft_cgemm_ifft_7.cuh:9-222: (S, N/64) blocks that each traverse K).
-// Per round of 16 channels (32 for DY = 128, two per group): forward transforms by the sixteen 16-lane groups; every lane splits
+// Per round of 16 channels (32 for DY = 128, two per group): forward transforms by the sixteen 16-lane groups (DY = 512 / 1024: in two / four
+// passes by eight / four groups of 32 / 64 lanes); every lane splits
 // its modes and writes them to LDS in operand order, a complex mode being one (re, im) pair of the contraction index, so that one
 // matrix instruction covers 16 channels. Wave w owns 16 NTW output channels and all 64 modes:
 //   * an element of W is used by one wave only and goes from global memory through its registers into the A operand, as the rows
 //     (re, -im) and (im, re); nothing of W passes through LDS;
 //   * the accumulators of a lane are, for each of four output channels, the modes t + 16 a: the input of the backward transform by
-//     its own 16-lane group (DY = 128: after one row rotation). The product never leaves the registers and the backward phase
-//     has no barrier.
+//     its own 16-lane group (DY = 128: after one row rotation; DY = 512 / 1024: through the exchange region of the group, inside
+//     the wave). The product never passes a block barrier, nor does the backward phase.
 // What bounds it: the chain of phases of a wave (x, transform, product, backward, stores), hidden by blocks in other phases, up to
 // the rate of a mixed read and write stream (4.5 - 4.8 TB/s here; a copy of 2 GiB: 4.9). Hence the registers are held to three blocks per CU (NTW = 2: 158;
 // NTW = 1: 144) or four (NTW = 1: 116 - 124, the operand tile sharing the exchange regions, x requested after the second pass)
 // without spills: with spills the kernel is up to 70 % slower, because a reload waits for the x in flight.
 // Measured against the fp32 kernels it replaced (us, x and y from HBM): DY = 256, K = N = 128, S = 8192: 1135 -> 960;
 // K = N = 64, S = 4096: 247 -> 213; DY = 128, K = N = 64, S = 16384: 533 -> 447; K = N = 128, S = 8192: 735 -> 569; K = 40, N = 128,
-// S = 1000: 52 -> 46. Error against 64 bits: 2.4e-7 -> 2.0e-7 (K = 64), 3.2e-7 -> 2.7e-7 (K = 128).
+// S = 1000: 52 -> 41; DY = 512, K = N = 128, S = 2048: 652 -> 451; DY = 1024, K = N = 128, S = 1000: 601 -> 462. Halves against the SIMT kernel:
+// forward DY = 256, K = N = 64, S = 2048: 103 -> 77, K = N = 128: 341 -> 171; backward 112 -> 65, 298 -> 149; S = 64, K = N = 64: 22 -> 13 both. (Forward, DY = 1024,
+// K = 8, N = 64, S = 2048 is the one shape found slower: 47.8 -> 50.1.) Error against 64 bits: 2.4e-7 -> 2.0e-7 (K = 64), 3.2e-7 -> 2.7e-7 (K = 128).
 #include "bf16_split.h"
 #include "group_fft.h"
 #include "kernels.h"
@@ -28,17 +31,21 @@ namespace tfno {
 // NTW = tiles of 16 output channels per wave (a block covers 64 NTW output channels).
 // ALIAS: the operand tile of the spectra shares the exchange regions (one more barrier per round, LDS for four blocks per CU).
 // BLOCKS: blocks per CU that the registers are held to.
-template <int LOGDY, int NTW, bool ALIAS> struct GeoSplit {
-    static constexpr bool PAIR = LOGDY == 7;
-    static constexpr int KC = PAIR ? 32 : 16;                   // channels per round: a 16-lane group transforms one, or two of length 128
-    static constexpr int EXCH = 16 * 17;
-    static constexpr int EXCH_BYTES = 16 * EXCH * (int)sizeof(float2);
+// FWD: the spectra are made by forward transforms of x; otherwise they are read from A[m + k M] (second half of the layer).
+// INV: the product goes into zero-padded backward transforms; otherwise it is stored as C[m + n M] (+ beta C, first half).
+template <int LOGDY, bool ALIAS, bool FWD> struct GeoSplit {
+    static constexpr int L = LOGDY <= 8 ? 16 : (1 << LOGDY) / 16;   // lanes per signal (DY = 128: per pair of signals)
+    static constexpr bool PAIR = LOGDY == 7 && FWD;             // two channels of length 128 per 16-lane group
+    static constexpr int CP = !FWD ? 16 : (PAIR ? 32 : 256 / L);    // channels per pass of the block
+    static constexpr int KC = CP > 16 ? CP : 16;                // channels per round
+    static constexpr int EXCH = L * 17;
+    static constexpr int EXCH_BYTES = 256 * 17 * (int)sizeof(float2);
     static constexpr int STEP_BYTES = 12 * 1024;                // operand tile of 16 channels: 4 m tiles x 3 parts x 1 KiB
     static constexpr int TILE_BYTES = (KC / 16) * STEP_BYTES;
     static constexpr int TILE_AT = ALIAS ? 0 : EXCH_BYTES;
-    static constexpr int TW_AT = ALIAS ? EXCH_BYTES : EXCH_BYTES + TILE_BYTES;
-    static constexpr size_t LDS_BYTES = TW_AT + sizeof(float2) * kTwLdsSize;
-    static_assert(!ALIAS || TILE_BYTES <= EXCH_BYTES, "the operand tile must fit the exchange regions");
+    static constexpr int TW_AT = ALIAS ? EXCH_BYTES : EXCH_BYTES + TILE_BYTES;      // first-pass twiddles, then the powers w_L^e
+    static constexpr size_t LDS_BYTES = TW_AT + sizeof(float2) * (L * kTwLdsPitch + (L > 16 ? L : 0));
+    static_assert(!ALIAS || (TILE_BYTES <= EXCH_BYTES && CP == KC), "the operand tile must fit the exchange regions, one pass per round");
 };
 
 // Makes `offset` depend on g[]: loads that are addressed with it cannot be issued before g[] has been computed. The compiler
@@ -46,48 +53,52 @@ template <int LOGDY, int NTW, bool ALIAS> struct GeoSplit {
 // registers (up to 78) come on top of those of the pass.
 template <int COUNT> TFNO_DEV void after(int& offset, const cpx (&g)[COUNT])
 {
-    static_assert(COUNT % 4 == 0, "in fours");
 #pragma unroll
-    for (int i = 0; i < COUNT; i += 4) asm volatile("" : "+v"(offset) : "v"(g[i].x), "v"(g[i + 1].x), "v"(g[i + 2].x), "v"(g[i + 3].x));
+    for (int i = 0; i < COUNT; ++i) asm volatile("" : "+v"(offset) : "v"(g[i].x));
 }
 
-template <int LOGDY, int NTW, bool ALIAS, int BLOCKS, bool KEEP>
+template <int LOGDY, int NTW, bool ALIAS, int BLOCKS, bool KEEP, bool FWD = true, bool INV = true>
 __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S, int N, int K, const float2* __restrict__ x,
                                                                              const float2* __restrict__ W, float2* __restrict__ y,
-                                                                             float2 alpha)
+                                                                             float2 alpha, float2 beta)
 {
-    using G = GeoSplit<LOGDY, NTW, ALIAS>;
-    constexpr bool PAIR = G::PAIR;
-    constexpr int DY = 1 << LOGDY, KC = G::KC;
-    // x of the next round is requested after the second pass instead of before it: 32 registers fewer at the peak
+    using G = GeoSplit<LOGDY, ALIAS, FWD>;
+    constexpr bool PAIR = G::PAIR, LONG = LOGDY >= 9;
+    constexpr int DY = 1 << LOGDY, KC = G::KC, CP = G::CP, L = G::L;
+    // x of the next pass is requested after the second stage instead of before it: 32 registers fewer at the peak
     constexpr bool LATE = NTW > 1 || BLOCKS == 4;
     extern __shared__ char lds_split[];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int grp = tid >> 4, t = tid & 15;                     // transform role: lane t of 16-lane group grp
+    const int grp = tid / L, t = tid % L;                       // transform role: lane t of L-lane group grp
     const int kq = lane >> 4, col = lane & 15;                  // matrix role
     long s;
     int ntile;
     decode_block_1d(S, N / (64 * NTW), DY, !KEEP, s, ntile);
     const int nw = (ntile * 4 + wave) * (16 * NTW);             // first output channel of the wave
+    const long M = 64L * S;
     float2* exch = reinterpret_cast<float2*>(lds_split) + grp * G::EXCH;
     char* tile = lds_split + G::TILE_AT;
     float2* twtab = reinterpret_cast<float2*>(lds_split + G::TW_AT);
-    fill_lds_twiddles<LOGDY>(twtab, tid, 256);
+    float2* powers = twtab + L * kTwLdsPitch;
+    fill_lds_twiddles<LOGDY, L>(twtab, tid, 256);
+    if (LONG && tid < L) powers[tid] = kTwiddle1024[tid * (1024 / L)];
     const float2* twrow = twtab + t * kTwLdsPitch;
 
-    const int first = PAIR ? 2 * grp : grp;                     // channel of a round that the group transforms (first of two)
-    const float2* src = x + ((long)first * S + s) * DY + t;
-    // x of the round that starts at channel kc. Branch free (a load under a condition would keep the old values alive and
+    // channel of a pass that the group brings in (PAIR: the first of two; without a forward transform 16 lanes per channel)
+    const int first = !FWD ? tid >> 4 : (PAIR ? 2 * grp : grp);
+    const float2* src = FWD ? x + ((long)first * S + s) * DY + t : x + (long)first * M + s * 64 + (tid & 15);
+    // input of the pass that starts at channel kc. Branch free (a load under a condition would keep the old values alive and
     // cost 30 registers): channels beyond K read the first row(s) of the array, cache resident, and are masked later
-    cpx v[16];
+    constexpr int HELD = FWD ? 16 : 4;
+    cpx v[HELD];
     auto issue = [&](int kc, int offset) {
-        const float2* p = (kc + first < K ? src + (long)kc * S * DY : x + t) + offset;
+        const float2* p = (kc + first < K ? src + (long)kc * (FWD ? (long)S * DY : M) : x + (FWD ? t : tid & 15)) + offset;
         if constexpr (PAIR) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) { v[i] = p[16 * i]; v[8 + i] = p[(long)S * DY + 16 * i]; }
         } else {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = p[16 * i];
+            for (int i = 0; i < HELD; ++i) v[i] = p[(FWD ? L : 16) * i];
         }
     };
     issue(0, 0);
@@ -100,16 +111,16 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
 
     // where the lane's modes go: channel c of the round, mode 16 a + column, in operand order (16 bytes per lane of the
     // operand read: four channels of one column)
-    const int c_own = PAIR ? 2 * grp + (t >> 3) : grp, col_own = PAIR ? t & 7 : t;
-    char* own = tile + (c_own >> 4) * G::STEP_BYTES + ((c_own >> 2) & 3) * 256 + col_own * 16 + (c_own & 3) * 4;
+    auto own_place = [&](int c, int a, int column) {
+        return tile + (c >> 4) * G::STEP_BYTES + a * 3072 + ((c >> 2) & 3) * 256 + column * 16 + (c & 3) * 4;
+    };
 
     for (int kc = 0; kc < K; kc += KC) {
         const int kn = (K - kc) < KC ? (K - kc) : KC;           // a multiple of 8 (caller contract)
-        const bool busy = (PAIR ? 8 : 4) * wave < kn;           // uniform over the wave
-        constexpr int MODES = PAIR ? 8 : 4, WSTEPS = PAIR && NTW == 1 && BLOCKS < 4 ? 2 : 1;
+        constexpr int MODES = !FWD ? 4 : (PAIR ? 8 : 64 / L), WSTEPS = PAIR && NTW == 1 && BLOCKS < 4 ? 2 : 1;
         // W rows of the round: lane (kq, col) holds channels 4 kq ... 4 kq + 3 of 16, output channel col of the tile (a short
         // last round reads its first channels again: the spectra of the missing ones are zero). Requested before the next
-        // round's x: loads return in order, so a later request would wait for all of x first
+        // pass's x: loads return in order, so a later request would wait for all of x first
         float2 wv[WSTEPS][NTW][4];
         auto load_w = [&](int step, float2 (&dst)[NTW][4], int offset) {
             const int k = 16 * step + 4 * kq;
@@ -119,65 +130,83 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
 #pragma unroll
                 for (int j = 0; j < 4; ++j) dst[i][j] = p[(long)(16 * i) * K + j];
         };
-        cpx out[MODES];
-        if (busy) {
-            cpx gg[16];
-            if constexpr (PAIR) {
-                cpx a8[8], b8[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) { a8[i] = v[i]; b8[i] = v[8 + i]; }
-                fft8<-1>(a8);
-                fft8<-1>(b8);
-                gg[0] = a8[0];
-                gg[8] = b8[0];
+        for (int pass = 0; pass < KC / CP; ++pass) {
+            const bool busy = pass * CP + (CP / 4) * wave < kn; // uniform over the wave: CP / 4 channels each
+            cpx out[MODES];
+            if constexpr (!FWD) {
 #pragma unroll
-                for (int r = 1; r < 8; ++r) {
-                    const cpx w = twrow[r];
-                    gg[r] = cmul(a8[r], w);
-                    gg[8 + r] = cmul(b8[r], w);
+                for (int a = 0; a < 4; ++a) out[a] = busy ? v[a] : make_float2(0.f, 0.f);
+#pragma unroll
+                for (int u = 0; u < WSTEPS; ++u) load_w(u, wv[u], 0);
+                issue(kc + CP, 0);
+            } else if (busy) {
+                cpx gg[16];
+                if constexpr (PAIR) {
+                    cpx a8[8], b8[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) { a8[i] = v[i]; b8[i] = v[8 + i]; }
+                    fft8<-1>(a8);
+                    fft8<-1>(b8);
+                    gg[0] = a8[0];
+                    gg[8] = b8[0];
+#pragma unroll
+                    for (int r = 1; r < 8; ++r) {
+                        const cpx w = twrow[r];
+                        gg[r] = cmul(a8[r], w);
+                        gg[8 + r] = cmul(b8[r], w);
+                    }
+                } else {
+                    fft16<-1>(v);
+                    int row = 0;
+                    after(row, v);
+                    const float2* tw = twrow + row;
+                    gg[0] = v[0];
+                    gg[1] = cmul(v[fft16_slot(1)], tw[1]);
+#pragma unroll
+                    for (int r = 2; r < 16; r += 2) {
+                        const float4 w = *reinterpret_cast<const float4*>(tw + r);
+                        gg[r] = cmul(v[fft16_slot(r)], make_float2(w.x, w.y));
+                        gg[r + 1] = cmul(v[fft16_slot(r + 1)], make_float2(w.z, w.w));
+                    }
                 }
-            } else {
-                fft16<-1>(v);
-                int row = 0;
-                after(row, v);
-                const float2* tw = twrow + row;
-                gg[0] = v[0];
-                gg[1] = cmul(v[fft16_slot(1)], tw[1]);
+                int later = 0;
+                after(later, gg);
+                if (pass == 0) {
 #pragma unroll
-                for (int r = 2; r < 16; r += 2) {
-                    const float4 w = *reinterpret_cast<const float4*>(tw + r);
-                    gg[r] = cmul(v[fft16_slot(r)], make_float2(w.x, w.y));
-                    gg[r + 1] = cmul(v[fft16_slot(r + 1)], make_float2(w.z, w.w));
+                    for (int u = 0; u < WSTEPS; ++u) load_w(u, wv[u], later);
                 }
+                if constexpr (!LATE) issue(kc + (pass + 1) * CP, later);
+                if constexpr (PAIR) rows128_forward_finish(gg, exch, t, out);
+                else if constexpr (LONG) wide_forward_finish<L, true>(gg, exch, powers, t, out);
+                else group_forward_finish<8>(gg, exch, t, out);
+                if constexpr (LATE) {
+                    later = 0;
+                    after(later, out);
+                    issue(kc + (pass + 1) * CP, later);
+                }
+            } else {                                            // the wave's channels are beyond K
+                if (pass == 0) {
+#pragma unroll
+                    for (int u = 0; u < WSTEPS; ++u) load_w(u, wv[u], 0);
+                }
+                issue(kc + (pass + 1) * CP, 0);
+#pragma unroll
+                for (int a = 0; a < MODES; ++a) out[a] = make_float2(0.f, 0.f);
             }
-            int later = 0;
-            after(later, gg);
+            if (pass == 0) __syncthreads();                     // the operand tile of the last round is read / the exchanges are done
 #pragma unroll
-            for (int u = 0; u < WSTEPS; ++u) load_w(u, wv[u], later);
-            if constexpr (!LATE) issue(kc + KC, later);
-            if constexpr (PAIR) rows128_forward_finish(gg, exch, t, out);
-            else group_forward_finish<8>(gg, exch, t, out);
-            if constexpr (LATE) {
-                later = 0;
-                after(later, out);
-                issue(kc + KC, later);
+            for (int a = 0; a < MODES; ++a) {
+                unsigned h, m, l;
+                split_bf16_pair(out[a].x, out[a].y, h, m, l);
+                char* dst;
+                if constexpr (PAIR) dst = own_place(2 * grp + (t >> 3), a >> 1, (t & 7) + 8 * (a & 1));
+                else if constexpr (!FWD) dst = own_place(tid >> 4, a, tid & 15);
+                else dst = own_place(pass * CP + grp, (t >> 4) + (L / 16) * a, t & 15);
+                *reinterpret_cast<unsigned*>(dst) = h;
+                *reinterpret_cast<unsigned*>(dst + 1024) = m;
+                *reinterpret_cast<unsigned*>(dst + 2048) = l;
             }
-        } else {                                                // the wave's channels are beyond K
-#pragma unroll
-            for (int u = 0; u < WSTEPS; ++u) load_w(u, wv[u], 0);
-            issue(kc + KC, 0);
-#pragma unroll
-            for (int a = 0; a < MODES; ++a) out[a] = make_float2(0.f, 0.f);
-        }
-        __syncthreads();                                        // the operand tile of the last round is read / the exchanges are done
-#pragma unroll
-        for (int a = 0; a < MODES; ++a) {
-            unsigned h, m, l;
-            split_bf16_pair(out[a].x, out[a].y, h, m, l);
-            char* dst = own + (PAIR ? (a >> 1) * 3072 + (a & 1) * 128 : a * 3072);
-            *reinterpret_cast<unsigned*>(dst) = h;
-            *reinterpret_cast<unsigned*>(dst + 1024) = m;
-            *reinterpret_cast<unsigned*>(dst + 2048) = l;
         }
         __syncthreads();
 #pragma unroll
@@ -213,8 +242,37 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
     // D[row = 4 kq + q][col] of tile (i, a): output channel nw + 16 i + 4 kq + q, mode col + 16 a
 #pragma unroll
     for (int i = 0; i < NTW; ++i) {
-        float2* dst = y + ((long)(nw + 16 * i + 4 * kq) * S + s) * DY + t;
-        if constexpr (!PAIR) {
+        if constexpr (!INV) {
+            float2* dst = y + (long)(nw + 16 * i + 4 * kq) * M + s * 64 + col;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    cpx r = make_float2(re[i][a][q], im[i][a][q]);
+                    if (beta.x != 0.f || beta.y != 0.f) r = cadd(r, cmul(dst[q * M + 16 * a], beta));
+                    dst[q * M + 16 * a] = r;
+                }
+        } else if constexpr (LONG) {
+            // one output channel per L-lane group: the lanes that hold it store its 64 modes into the group's region
+            constexpr int AT_ONCE = 64 / L;                     // channels per wave at a time
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll 1
+                for (int h = 0; h < 4 / AT_ONCE; ++h) {         // a loop: unrolled, the backward phase exceeds the instruction cache
+                    wave_lds_fence();
+                    if (kq / AT_ONCE == h) {
+                        float2* dst = reinterpret_cast<float2*>(lds_split) + (wave * AT_ONCE + kq % AT_ONCE) * G::EXCH + col;
+#pragma unroll
+                        for (int a = 0; a < 4; ++a) dst[16 * a] = make_float2(re[i][a][q], im[i][a][q]);
+                    }
+                    cpx e[16], yv[16];
+                    wide_backward_inputs_of_stored<L, true>(powers, exch, t, e);
+                    inv_pass2_lds(e, twrow, yv);
+                    const int n = nw + 16 * i + 4 * (AT_ONCE * h + lane / L) + q;
+                    store_row16<L, KEEP>(y + ((long)n * S + s) * DY + t, yv);
+                }
+        } else if constexpr (LOGDY == 8) {
+            float2* dst = y + ((long)(nw + 16 * i + 4 * kq) * S + s) * DY + t;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 cpx c[4], yv[16];
@@ -224,6 +282,7 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
                 store_row16<16, KEEP>(dst + (long)q * S * DY, yv);
             }
         } else {
+            float2* dst = y + ((long)(nw + 16 * i + 4 * kq) * S + s) * DY + t;
             const bool upper = t >> 3;
 #pragma unroll
             for (int q = 0; q < 4; q += 2) {
@@ -243,36 +302,81 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
     }
 }
 
-template <int LOGDY, int NTW, bool ALIAS, int BLOCKS>
-static hipError_t launch_split_t(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, hipStream_t stream, int keep_y)
+template <int LOGDY, int NTW, bool ALIAS, int BLOCKS, bool KEEP, bool FWD, bool INV>
+static hipError_t launch_split_k(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, float2 beta, hipStream_t stream)
 {
-    using G = GeoSplit<LOGDY, NTW, ALIAS>;
+    using G = GeoSplit<LOGDY, ALIAS, FWD>;
     const long blocks = S * (N / (64 * NTW));
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
     static_assert(G::LDS_BYTES <= 64 * 1024, "no attribute call needed below 64 KiB of dynamic LDS");
-    // keep_y: plain instead of streaming stores of y, for a consumer that reads it at once (a template parameter of the kernels)
-    if (keep_y)
-        hipLaunchKernelGGL((fused_fft_split_ifft_kernel<LOGDY, NTW, ALIAS, BLOCKS, true>), dim3((unsigned)blocks), dim3(256), G::LDS_BYTES,
-                           stream, (int)S, N, K, x, W, y, alpha);
-    else
-        hipLaunchKernelGGL((fused_fft_split_ifft_kernel<LOGDY, NTW, ALIAS, BLOCKS, false>), dim3((unsigned)blocks), dim3(256), G::LDS_BYTES,
-                           stream, (int)S, N, K, x, W, y, alpha);
+    hipLaunchKernelGGL((fused_fft_split_ifft_kernel<LOGDY, NTW, ALIAS, BLOCKS, KEEP, FWD, INV>), dim3((unsigned)blocks), dim3(256),
+                       G::LDS_BYTES, stream, (int)S, N, K, x, W, y, alpha, beta);
     return hipGetLastError();
 }
+// keep_y: plain instead of streaming stores of y, for a consumer that reads it at once (a template parameter of the kernels)
+template <int LOGDY, int NTW, bool ALIAS, int BLOCKS>
+static hipError_t launch_split_t(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, hipStream_t stream, int keep_y)
+{
+    const float2 beta = make_float2(0.f, 0.f);
+    return keep_y ? launch_split_k<LOGDY, NTW, ALIAS, BLOCKS, true, true, true>(S, N, K, x, W, y, alpha, beta, stream)
+                  : launch_split_k<LOGDY, NTW, ALIAS, BLOCKS, false, true, true>(S, N, K, x, W, y, alpha, beta, stream);
+}
 
-// DY = 128 or 256. wide: blocks of 128 output channels where N allows, else of 64; dense: the variant for four blocks per CU
-// (64 output channels; always at DY = 128, where it is level or ahead from one block per CU on).
+// wide: blocks of 128 output channels where N allows, else of 64; dense: the variant for four blocks per CU (64 output channels;
+// DY = 256 only; always at DY = 128, where it is level or ahead from one block per CU on).
 hipError_t launch_fused_split(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, bool wide,
                               bool dense, hipStream_t stream, int keep_y)
 {
     wide = wide && N % 128 == 0;
-    if (logDY == 7)
+    switch (logDY) {
+    case 7:
         return wide ? launch_split_t<7, 2, true, 3>(S, N, K, x, W, y, alpha, stream, keep_y)
                     : launch_split_t<7, 1, true, 4>(S, N, K, x, W, y, alpha, stream, keep_y);
-    if (logDY != 8) return hipErrorInvalidValue;
-    if (wide) return launch_split_t<8, 2, false, 3>(S, N, K, x, W, y, alpha, stream, keep_y);
-    return dense ? launch_split_t<8, 1, true, 4>(S, N, K, x, W, y, alpha, stream, keep_y)
-                 : launch_split_t<8, 1, false, 3>(S, N, K, x, W, y, alpha, stream, keep_y);
+    case 8:
+        if (wide) return launch_split_t<8, 2, false, 3>(S, N, K, x, W, y, alpha, stream, keep_y);
+        return dense ? launch_split_t<8, 1, true, 4>(S, N, K, x, W, y, alpha, stream, keep_y)
+                     : launch_split_t<8, 1, false, 3>(S, N, K, x, W, y, alpha, stream, keep_y);
+    case 9:
+        return wide ? launch_split_t<9, 2, false, 2>(S, N, K, x, W, y, alpha, stream, keep_y)
+                    : launch_split_t<9, 1, false, 3>(S, N, K, x, W, y, alpha, stream, keep_y);
+    case 10:
+        return wide ? launch_split_t<10, 2, false, 2>(S, N, K, x, W, y, alpha, stream, keep_y)
+                    : launch_split_t<10, 1, false, 2>(S, N, K, x, W, y, alpha, stream, keep_y);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+// The halves of the layer (variants B and C): forward transforms and product, product and backward transforms.
+hipError_t launch_split_forward(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C, float2 alpha, float2 beta,
+                                bool wide, hipStream_t stream)
+{
+    wide = wide && N % 128 == 0;
+    switch (logDY) {
+    case 7:
+        return wide ? launch_split_k<7, 2, true, 3, true, true, false>(S, N, K, x, W, C, alpha, beta, stream)
+                    : launch_split_k<7, 1, true, 4, true, true, false>(S, N, K, x, W, C, alpha, beta, stream);
+    case 8:
+        return wide ? launch_split_k<8, 2, false, 3, true, true, false>(S, N, K, x, W, C, alpha, beta, stream)
+                    : launch_split_k<8, 1, false, 3, true, true, false>(S, N, K, x, W, C, alpha, beta, stream);
+    case 9:
+        return wide ? launch_split_k<9, 2, false, 2, true, true, false>(S, N, K, x, W, C, alpha, beta, stream)
+                    : launch_split_k<9, 1, false, 3, true, true, false>(S, N, K, x, W, C, alpha, beta, stream);
+    case 10:
+        return wide ? launch_split_k<10, 2, false, 2, true, true, false>(S, N, K, x, W, C, alpha, beta, stream)
+                    : launch_split_k<10, 1, false, 2, true, true, false>(S, N, K, x, W, C, alpha, beta, stream);
+    default: return hipErrorInvalidValue;
+    }
+}
+hipError_t launch_split_backward(int logDY, long S, int N, int K, const float2* A, const float2* W, float2* y, float2 alpha, hipStream_t stream)
+{
+    const float2 beta = make_float2(0.f, 0.f);
+    switch (logDY) {
+    case 7: return launch_split_k<7, 1, true, 4, false, false, true>(S, N, K, A, W, y, alpha, beta, stream);
+    case 8: return launch_split_k<8, 1, true, 4, false, false, true>(S, N, K, A, W, y, alpha, beta, stream);
+    case 9: return launch_split_k<9, 1, true, 4, false, false, true>(S, N, K, A, W, y, alpha, beta, stream);
+    case 10: return launch_split_k<10, 1, true, 3, false, false, true>(S, N, K, A, W, y, alpha, beta, stream);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace tfno
