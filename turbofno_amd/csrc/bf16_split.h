@@ -32,6 +32,17 @@ __device__ __forceinline__ void split_bf16_pair(float a, float b, unsigned& h, u
 struct SplitOperand {
     uint4_v h, m, l;
 };
+// Element j of the two A operand rows of one complex weight times alpha, for a contraction over (re, im) pairs of the other
+// operand: (re, -im) gives the real part of the product, (im, re) the imaginary part.
+__device__ __forceinline__ void split_weight_rows(float2 w, float2 alpha, SplitOperand& real_row, SplitOperand& imag_row, int j)
+{
+    unsigned h, m, l;
+    split_bf16_pair(w.x * alpha.x - w.y * alpha.y, w.x * alpha.y + w.y * alpha.x, h, m, l);
+    real_row.h[j] = h ^ 0x80000000u; real_row.m[j] = m ^ 0x80000000u; real_row.l[j] = l ^ 0x80000000u;
+    imag_row.h[j] = __builtin_amdgcn_alignbit(h, h, 16);
+    imag_row.m[j] = __builtin_amdgcn_alignbit(m, m, 16);
+    imag_row.l[j] = __builtin_amdgcn_alignbit(l, l, 16);
+}
 __device__ __forceinline__ float4_v mfma_bf16(uint4_v a, uint4_v b, float4_v c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);

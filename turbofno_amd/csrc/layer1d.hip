@@ -11,6 +11,7 @@
 //     transform, so the GEMM result never passes through LDS (the reference stages it in 8 rounds,
 //     fused_fft_cgemm_ifft_7.cuh:203-218);
 //   * exchange buffers are padded (row pitch 17 complex) for the 64-bank LDS of CDNA4.
+#include "bf16_split.h"
 #include "group_fft.h"
 #include "kernels.h"
 
@@ -408,13 +409,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 }
 
 // Fused 1D layer for small grids (every block has a CU to itself), DY = 256: the eight waves of a block share ONE
-// item (signal set, 32 output channels) and split its K input channels. Operands as in the one-wavefront kernel above:
-// wave w transforms channels 32 r + 4 w + g in round r and multiplies them straight out of its registers into its own
-// partial accumulators (4 n' tiles x 4 m tiles), so the K loop has no barrier and stages nothing through LDS. The
-// eight partial products meet in LDS once (sP[w][n][m], pitch 72 complex: conflict-free b64 stores), every lane group
-// sums the eight partials of one output channel and runs its backward transform. The chain of latencies of an item
-// is K / 32 rounds + one reduction + one backward pass, against three barriers and two tile builds per 32 channels
-// in the kernel that shares the spectra through LDS.
+// item (signal set, 32 output channels) and split its K input channels: wave w transforms channels 32 r + 4 w + g in round r,
+// g = 16-lane group. Four rounds give a lane four channels of its modes t + 16 a: with real and imaginary part the eight
+// consecutive values of the contraction that a lane holds of the B operand of v_mfma_f32_16x16x32_bf16, so a wave multiplies its
+// 16 channels straight out of its registers (exact three-way split, bf16_split.h) into its own partial accumulators (2 tiles of 16
+// output channels x 4 m tiles). The K loop has no barrier and stages nothing through LDS. The eight partial products
+// meet in LDS once (sP[w][n][m], pitch 72 complex: conflict-free b64 stores), every lane group sums the eight partials
+// of one output channel and runs its backward transform. The chain of latencies of an item is K / 32 rounds + K / 128 products +
+// one reduction + one backward pass, against three barriers and two tile builds per 32 channels in the kernel that
+// shares the spectra through LDS. S = 64, K = N = 128: 18.7 us with fp32 matrix instructions in every round, 17.2 now (K = 64: 13.4 / 13.5).
 constexpr int SPLIT_NT = 32, SPLIT_PP = 72;
 constexpr size_t SPLIT_LDS = sizeof(float2) * 8 * SPLIT_NT * SPLIT_PP;       // 147,456 B; covers the 32 exchange regions
 
@@ -422,28 +425,27 @@ __global__ __launch_bounds__(512) void fused_fft_mfma_ifft_split_kernel(int S, i
                                                                         const float2* __restrict__ W, float2* __restrict__ y,
                                                                         float2 alpha)
 {
-    constexpr int DY = 256, EXCH = 16 * 17;
+    constexpr int DY = 256, EXCH = 16 * 17, TILES = SPLIT_NT / 16;
     extern __shared__ float2 lds[];
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4, t = lane & 15;
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, t = lane & 15;
     float2* exch = lds + (4 * w + g) * EXCH;                      // the partials overlay these after the K loop
     long s;
     int ntile;
     decode_block_1d(S, N / SPLIT_NT, 256, true, s, ntile);
     const int n0 = ntile * SPLIT_NT;
-    const bool odd = t & 1;
     cpx tw[16];
     load_lane_twiddles<8>(t, tw);
 
-    floatx4_1d acc[4][4];
+    float4_v re[TILES][4], im[TILES][4];
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int i = 0; i < TILES; ++i)
 #pragma unroll
-        for (int a = 0; a < 4; ++a) acc[nt][a] = floatx4_1d{ 0.f, 0.f, 0.f, 0.f };
+        for (int a = 0; a < 4; ++a) re[i][a] = im[i][a] = float4_v{ 0.f, 0.f, 0.f, 0.f };
 
     // K is a multiple of 8 and a wave covers four consecutive channels: a wave is either fully inside K or idle
     const int k0 = 4 * w + g;
     const float2* src = x + ((long)k0 * S + s) * DY + t;
-    const float2* wsrc = W + k0 + (long)(n0 + (t >> 1)) * K;      // W[k][n = n0 + 8 nt + t / 2]
+    const float2* wsrc = W + k0 + (long)(n0 + t) * K;             // W[k][n = n0 + 16 i + t]
     auto issue = [&](cpx (&dst)[16], int kc) {                    // samples t + 16 i of channel kc + k0
         const float2* p = src + (long)kc * S * DY;
 #pragma unroll
@@ -451,38 +453,52 @@ __global__ __launch_bounds__(512) void fused_fft_mfma_ifft_split_kernel(int S, i
     };
     // the buffer is refilled as soon as the first pass has consumed it (a second buffer, two rounds ahead, was
     // measured slower: a round is bound by its arithmetic, not by the latency of its loads)
-    auto round = [&](cpx (&v)[16], int kc) {
-        float2 wv[4];
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) wv[nt] = wsrc[kc + (long)(8 * nt) * K];
-        cpx gg[16], out[4];
-        fwd_pass1(v, tw, gg);
-        if (kc + 32 + 4 * w < K) issue(v, kc + 32);
-        group_forward_finish<8>(gg, exch, t, out);
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) {
-            const float2 wa = make_float2(wv[nt].x * alpha.x - wv[nt].y * alpha.y, wv[nt].x * alpha.y + wv[nt].y * alpha.x);
-            const float ax = odd ? wa.y : wa.x, ay = odd ? wa.x : -wa.y;
-#pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                acc[nt][a] = __builtin_amdgcn_mfma_f32_16x16x4f32(ax, out[a].x, acc[nt][a], 0, 0, 0);
-                acc[nt][a] = __builtin_amdgcn_mfma_f32_16x16x4f32(ay, out[a].y, acc[nt][a], 0, 0, 0);
-            }
-        }
-    };
     cpx v[16];
     if (4 * w < K) issue(v, 0);
-    for (int kc = 0; kc + 4 * w < K; kc += 32) round(v, kc);
+    for (int kc = 0; kc + 4 * w < K; kc += 128) {
+        SplitOperand b[4];
+        float2 wv[TILES][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int kr = kc + 32 * j;
+            if (kr + 4 * w < K) {
+#pragma unroll
+                for (int i = 0; i < TILES; ++i) wv[i][j] = wsrc[kr + (long)(16 * i) * K];
+                cpx gg[16], out[4];
+                fwd_pass1(v, tw, gg);
+                if (kr + 32 + 4 * w < K) issue(v, kr + 32);
+                group_forward_finish<8>(gg, exch, t, out);
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    unsigned h, m, l;
+                    split_bf16_pair(out[a].x, out[a].y, h, m, l);
+                    b[a].h[j] = h; b[a].m[j] = m; b[a].l[j] = l;
+                }
+            } else {                                              // beyond K: zeros
+#pragma unroll
+                for (int i = 0; i < TILES; ++i) wv[i][j] = make_float2(0.f, 0.f);
+#pragma unroll
+                for (int a = 0; a < 4; ++a) b[a].h[j] = b[a].m[j] = b[a].l[j] = 0u;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < TILES; ++i) {
+            SplitOperand wre, wim;                                // rows (re, -im) and (im, re) of alpha W
+#pragma unroll
+            for (int j = 0; j < 4; ++j) split_weight_rows(wv[i][j], alpha, wre, wim, j);
+#pragma unroll
+            for (int a = 0; a < 4; ++a) mac_split_pair(wre, wim, b[a], re[i][a], im[i][a]);
+        }
+    }
     __syncthreads();                                              // every wave is done with its exchange regions
-    // D[row = 4 g + v][column = t] of tile (nt, a): channel n = 8 nt + 2 g + (v >> 1), re | im = v & 1, mode t + 16 a
+    // D[row = 4 g + q][column = t] of tile (i, a): output channel 16 i + 4 g + q, mode t + 16 a
     float2* sP = lds + (long)w * SPLIT_NT * SPLIT_PP;
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int i = 0; i < TILES; ++i)
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            sP[(8 * nt + 2 * g) * SPLIT_PP + t + 16 * a] = make_float2(acc[nt][a][0], acc[nt][a][1]);
-            sP[(8 * nt + 2 * g + 1) * SPLIT_PP + t + 16 * a] = make_float2(acc[nt][a][2], acc[nt][a][3]);
-        }
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sP[(16 * i + 4 * g + q) * SPLIT_PP + t + 16 * a] = make_float2(re[i][a][q], im[i][a][q]);
     __syncthreads();
     // lane group (w, g) owns output channel n = 4 w + g: sum of the eight partials, modes t + 16 a
     const int n = 4 * w + g;

@@ -216,17 +216,9 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
 #pragma unroll
             for (int i = 0; i < NTW; ++i) {
                 if constexpr (LATE) __builtin_amdgcn_sched_barrier(0);
-                SplitOperand wre, wim;
+                SplitOperand wre, wim;                          // rows (re, -im) and (im, re) of alpha W
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float2 w = wv[WSTEPS == 2 ? step : 0][i][j];
-                    unsigned h, m, l;
-                    split_bf16_pair(w.x * alpha.x - w.y * alpha.y, w.x * alpha.y + w.y * alpha.x, h, m, l);
-                    wre.h[j] = h ^ 0x80000000u; wre.m[j] = m ^ 0x80000000u; wre.l[j] = l ^ 0x80000000u;    // (re, -im)
-                    wim.h[j] = __builtin_amdgcn_alignbit(h, h, 16);                                        // (im, re)
-                    wim.m[j] = __builtin_amdgcn_alignbit(m, m, 16);
-                    wim.l[j] = __builtin_amdgcn_alignbit(l, l, 16);
-                }
+                for (int j = 0; j < 4; ++j) split_weight_rows(wv[WSTEPS == 2 ? step : 0][i][j], alpha, wre, wim, j);
                 if (WSTEPS == 1 && PAIR && step == 0 && 16 < kn && i == NTW - 1) load_w(1, wv[0], 0);
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
