@@ -91,13 +91,14 @@ def _dev_c64(t, name):
 
 def _same_device(*named):
     """every tensor is a contiguous complex64 GPU tensor, all on one device (checked before any pointer is taken)"""
-    dev = None
+    dev = -1
     for name, t in named:
         _dev_c64(t, name)
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise ValueError("%s is on %s, expected %s: all operands must live on one GPU" % (name, t.device, dev))
+        i = t.get_device()
+        if dev < 0:
+            dev = i
+        elif i != dev:
+            raise ValueError("%s is on %s, expected cuda:%d: all operands must live on one GPU" % (name, t.device, dev))
 
 
 def _need(cond, fmt, *args):
@@ -110,7 +111,9 @@ def _numel(t, name, n):
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of torch's current stream on the current device. The raw query: torch.cuda.current_stream() builds a Stream
+    object for it, 2.8 of the 8 us that a call of a small layer spent on the host."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _log2(v):
