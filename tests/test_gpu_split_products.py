@@ -35,6 +35,11 @@ def _bound(K):
     (576, 1000, 64, 1j),             # six builds per column block, a block with idle waves
     (65536 + 64, 72, 64, 0.0),       # more than one block of 256 columns per CU, a partly filled last one
     (524288 + 64, 72, 128, 0.0),     # 128-channel tiles, persistent walk, a partly filled last block
+    (4096, 64, 64, 0.0),             # tiles of 16 output channels
+    (8192, 200, 128, -1j),           # tiles of 32, the tile rebuilt, C read and written
+    (16384, 40, 128, 2.0),           # tiles of 64 in blocks of 128 columns, C read and written
+    (32768 + 64, 72, 128, 0.5),      # blocks of 256 columns, the same
+    (262144 + 64, 24, 128, 1 + 1j),  # tiles of 128, the same: C is read in two parts
     (262144 - 64, 32, 128, 0.0),     # N = 128 with 32 channels or fewer on a large grid
 ])
 def test_cgemm_edges(M, K, N, beta):

@@ -393,6 +393,8 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
 // Blocks are persistent over column blocks (XCD j takes the j-th eighth of them, so that an XCD keeps to one part of the
 // memory system); the strip of the next step - of the next column block after the last - is requested before the matrix
 // work of the current one, and nothing in the walk waits at a barrier, so loads, matrix work and stores of the waves overlap.
+// With beta the values of C are read 16 at a time before any is stored (M = 262,144, N = 128, K = 24: 198 -> 124 us, K = 64: 221 -> 154;
+// with a column block per block instead of the walk, so that nothing waits behind the strip of the next: 130, 175).
 //   Kw    = period of W along the contraction: channel k is weighted with W[k mod Kw + n Kw] (Kw = K: the plain product;
 //           Kw = K / R: the R parts of decimated images, see above, share the weights of their image's channel);
 //   Kp    = channels covered by one run over the tile (K, or Kw: the contraction then runs over the tile K / Kw times);
@@ -414,7 +416,6 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
     const bool resident = steps <= cap;                 // the tile is built once
     const bool eighths = (gridDim.x & 7) == 0 && (nblocks & 7) == 0;
     auto block_of = [&](long v) { return eighths ? (v & 7) * (nblocks >> 3) + (v >> 3) : v; };
-    const bool has_beta = beta.x != 0.f || beta.y != 0.f;
 
     // channels 8 kq ... 8 kq + 7 of step `step` of a run, of the lane's column. Branch free, so that the loads stay where
     // they are issued: lanes beyond the run (its last step may be short) read the first channels of the step again - the tile
@@ -436,9 +437,13 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
             const int k = GEMM_KSTEP * (s0 + s) + 8 * (l >> 4), n = n0 + 16 * t + (l & 15);
             SplitOperand re, im;
             float2 w[8];
-            const float2* src = W + (k % Kw) + (long)n * Kw;        // Kw is a multiple of 8
 #pragma unroll
-            for (int j = 0; j < 8; ++j) w[j] = k < Kp ? src[j] : make_float2(0.f, 0.f);
+            for (int j = 0; j < 8; ++j) w[j] = make_float2(0.f, 0.f);
+            if (k < Kp) {
+                const float2* src = W + (k % Kw) + (long)n * Kw;    // Kw is a multiple of 8
+#pragma unroll
+                for (int j = 0; j < 8; ++j) w[j] = src[j];
+            }
 #pragma unroll
             for (int j = 0; j < 8; ++j) w[j] = make_float2(w[j].x * alpha.x - w[j].y * alpha.y, w[j].x * alpha.y + w[j].y * alpha.x);
 #pragma unroll
@@ -455,66 +460,89 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
         }
     };
 
-    long v = blockIdx.x;                                // the grid is no larger than the number of column blocks
-    fetch(block_of(v), 0, 0, true);
-    if (resident) {
-        build(0, steps);
-        __syncthreads();
-    }
-    for (; v < nblocks; v += gridDim.x) {
-        const long mb = block_of(v);
-        const bool more = v + gridDim.x < nblocks;
-        const long nb = more ? block_of(v + gridDim.x) : mb;
-        float4_v re[NT], im[NT];
+    float4_v re[NT], im[NT];
+    auto clear = [&]() {
 #pragma unroll
         for (int t = 0; t < NT; ++t) re[t] = im[t] = float4_v{ 0.f, 0.f, 0.f, 0.f };
-        for (int run = 0; run < runs; ++run)
-            for (int step = 0; step < steps; ++step) {
-                if (!resident && step % cap == 0) {     // uniform over the block
-                    __syncthreads();
-                    build(step, steps - step < cap ? steps - step : cap);
-                    __syncthreads();
-                }
-                SplitOperand ar, ai;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    unsigned h, m, l;
-                    split_bf16_pair(bv[2 * j].x, bv[2 * j + 1].x, h, m, l);
-                    ar.h[j] = h; ar.m[j] = m; ar.l[j] = l;
-                    split_bf16_pair(bv[2 * j].y, bv[2 * j + 1].y, h, m, l);
-                    ai.h[j] = h; ai.m[j] = m; ai.l[j] = l;
-                }
-                asm volatile("" ::: "memory");          // operand reads of the tile stay inside the loop
-                const bool same = step + 1 < steps || run + 1 < runs;         // the next step belongs to this column block
-                fetch(same ? mb : nb, step + 1 < steps ? run : (same ? run + 1 : 0), step + 1 < steps ? step + 1 : 0, same || more);
-                __builtin_amdgcn_sched_barrier(0);
-                const uint4_v* frag = sW4 + (resident ? step : step % cap) * (NT * 384) + lane;
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    SplitOperand w{ frag[t * 384], frag[t * 384 + 64], frag[t * 384 + 128] };
-                    float4_v r = re[t], i = im[t];
-                    mac_split2(w, ar, ai, r, i);                        // Wr
-                    w = SplitOperand{ frag[t * 384 + 192], frag[t * 384 + 256], frag[t * 384 + 320] };
-                    i = mac_split(w, ar, i);                            // Wi
-                    w.h ^= 0x80008000u; w.m ^= 0x80008000u; w.l ^= 0x80008000u;
-                    r = mac_split(w, ai, r);                            // - Wi
-                    re[t] = r;
-                    im[t] = i;
-                }
-            }
-        if (mb * MBLOCK + wave * 16 < Mtot) {
-            // D[row = 4 kq + q][col] of tile t: output channel n0 + 16 t + 4 kq + q, the lane's column
-            float2* dst = C + mb * MBLOCK + lane_col + (long)(n0 + 4 * kq) * Mtot;
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    float2* p = dst + (long)(16 * t + q) * Mtot;
-                    float2 r = make_float2(re[t][q], im[t][q]);
-                    if (has_beta) r = cadd(r, cmul(*p, beta));          // variants A, B
-                    *p = r;
-                }
+    };
+    clear();
+    // one loop over column blocks, runs and steps: nested ones cost a copy of the strip at every edge between them
+    long v = blockIdx.x, mb = block_of(v);              // the grid is no larger than the number of column blocks
+    int run = 0, step = 0, slot = 0;                    // slot: the step's place in the tile
+    bool built = false;
+    fetch(mb, 0, 0, true);
+    while (true) {
+        if (slot == 0 && !(resident && built)) {        // uniform over the block
+            __syncthreads();
+            build(step, steps - step < cap ? steps - step : cap);
+            __syncthreads();
+            built = true;
         }
+        SplitOperand ar, ai;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            unsigned h, m, l;
+            split_bf16_pair(bv[2 * j].x, bv[2 * j + 1].x, h, m, l);
+            ar.h[j] = h; ar.m[j] = m; ar.l[j] = l;
+            split_bf16_pair(bv[2 * j].y, bv[2 * j + 1].y, h, m, l);
+            ai.h[j] = h; ai.m[j] = m; ai.l[j] = l;
+        }
+        asm volatile("" ::: "memory");                  // operand reads of the tile stay inside the loop
+        const bool run_ends = step + 1 == steps, last = run_ends && run + 1 == runs;
+        const bool more = v + gridDim.x < nblocks;
+        const int next_step = run_ends ? 0 : step + 1, next_run = last ? 0 : (run_ends ? run + 1 : run);
+        const long next_mb = last && more ? block_of(v + gridDim.x) : mb;
+        fetch(next_mb, next_run, next_step, !last || more);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint4_v* frag = sW4 + slot * (NT * 384) + lane;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            SplitOperand w{ frag[t * 384], frag[t * 384 + 64], frag[t * 384 + 128] };
+            float4_v r = re[t], i = im[t];
+            mac_split2(w, ar, ai, r, i);                            // Wr
+            w = SplitOperand{ frag[t * 384 + 192], frag[t * 384 + 256], frag[t * 384 + 320] };
+            i = mac_split(w, ar, i);                                // Wi
+            w.h ^= 0x80008000u; w.m ^= 0x80008000u; w.l ^= 0x80008000u;
+            r = mac_split(w, ai, r);                                // - Wi
+            re[t] = r;
+            im[t] = i;
+        }
+        if (last) {
+            if (mb * MBLOCK + wave * 16 < Mtot) {
+                // D[row = 4 kq + q][col] of tile t: output channel n0 + 16 t + 4 kq + q, the lane's column
+                float2* dst = C + mb * MBLOCK + lane_col + (long)(n0 + 4 * kq) * Mtot;
+                if (beta.x != 0.f || beta.y != 0.f) {               // variants A, B: C is read, up to 16 values at a time
+                    constexpr int AT_ONCE = NT < 4 ? NT : 4;
+#pragma unroll
+                    for (int t0 = 0; t0 < NT; t0 += AT_ONCE) {
+                        float2 c[AT_ONCE][4];
+#pragma unroll
+                        for (int t = 0; t < AT_ONCE; ++t)
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) c[t][q] = dst[(long)(16 * (t0 + t) + q) * Mtot];
+#pragma unroll
+                        for (int t = 0; t < AT_ONCE; ++t)
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) {
+                                c[t][q] = cmul(c[t][q], beta);
+                                re[t0 + t][q] += c[t][q].x;
+                                im[t0 + t][q] += c[t][q].y;
+                            }
+                    }
+                }
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) dst[(long)(16 * t + q) * Mtot] = make_float2(re[t][q], im[t][q]);
+            }
+            if (!more) return;
+            v += gridDim.x;
+            clear();
+        }
+        mb = next_mb;
+        run = next_run;
+        step = next_step;
+        slot = next_step == 0 || slot + 1 == cap ? 0 : slot + 1;
     }
 }
 
@@ -759,7 +787,10 @@ hipError_t launch_ifft2d_pad(int logDX, int logDY, const float2* spec, float2* y
 //  * K <= 16: fp32 matrix instructions (M = 262,144, N = 128, K = 16: 55 against 74 with a step of 32 channels); with
 //    several column blocks per CU the persistent kernel. K <= 32 as well for N >= 128 and 8 to 16 blocks of 256 columns x 64
 //    output channels per CU (M = 262,144, N = 128, K = 32: 77 against 88 us; from 16 on the 128-channel tile below is ahead).
-//  * otherwise the split kernel. At most half a block of 256 columns x 64 output channels per CU: blocks of 128 columns
+//  * otherwise the split kernel. Small products: blocks of 128 columns and the fewest output channels whose grid still fits one
+//    block per CU (K = 64, N = 64, tiles of 64 / 32 / 16 output channels: M = 64: 7.5 / 5.5 / 5.0; M = 8,192: 8.5 / 6.3 / 5.8; M = 16,384:
+//    9.1 / 6.9; N = 192, M = 4,096: 9.0 / 7.1).
+//    At most half a block of 256 columns x 64 output channels per CU: blocks of 128 columns
 //    (M = 16,384, N = 64, K = 64: fp32 18.6, 256 columns 14.0, 128 columns 11.1); also for N = 64 with one to two blocks per
 //    CU and more than 32 channels, where two blocks of 128 columns on a CU overlap each other's phases (M = 65,536, K = 64:
 //    22.7 / 21.5 / 19.6; M = 98,304: 36.2 / 26.9 / 24.2).
@@ -821,6 +852,11 @@ hipError_t launch_cgemm_modes(const float2* A, const float2* W, float2* C, long 
     using Tiles8 = std::integral_constant<int, 8>;
     using Columns128 = std::integral_constant<int, 512>;
     using Columns256 = std::integral_constant<int, 1024>;
+    using Tiles1 = std::integral_constant<int, 1>;
+    using Tiles2 = std::integral_constant<int, 2>;
+    const long strips = (Mtot + 127) / 128;
+    if (strips * (N / 16) <= cus) return launch_split(Tiles1{}, Columns128{}, 6, 2);
+    if (strips * (N / 32) <= cus) return launch_split(Tiles2{}, Columns128{}, 6, 2);
     if (2 * blocks <= cus || (N == 64 && K > 32 && blocks >= cus && blocks < 2 * cus)) return launch_split(Tiles4{}, Columns128{}, 6, 2);
     if (N % 128 == 0 && (Kw + GEMM_KSTEP - 1) / GEMM_KSTEP <= 3 && blocks >= 8 * cus) return launch_split(Tiles8{}, Columns128{}, 3, 1);
     return launch_split(Tiles4{}, Columns256{}, 6, 1);
