@@ -1,12 +1,10 @@
-// fp32 products on the bf16 matrix cores without loss of precision. A float is the exact sum of three bf16 values,
-//   x = h + m + l,   h = bf16(x), m = bf16(x - h), l = x - h - m      (round to nearest: |m| <= 2^-8 |x|, |l| <= 2^-16 |x|),
+// fp32 products on the bf16 matrix cores. A float is the exact sum of three bf16 values,
+//   x = h + m + l,   h = bf16(x), m = bf16(x - h), l = x - h - m      (round to nearest: |m| <= 2^-8 |x|, |l| <= 2^-17 |x|),
 // because a bf16 holds 8 of the 24 significant bits. A product is then formed from six of the nine partial products,
 //   x w ~ l h' + h l' + m m' + m h' + h m' + h h'
-// the three that are left out (m l', l m', l l') are below 2^-23 |x w| together, half the spacing of floats there. Sums
-// are fp32, as in v_mfma_f32_16x16x4_f32, but one instruction adds 32 channels instead of 4, so there are fewer roundings.
-// Range: the parts of values below 2^-109 (1.5e-33) reach the smallest bf16 number, 2^-133, so an operand is held to 2^-134
-// absolutely there (mode GEMM, K = 64: relative error 1.5e-7 at unit scale, 1.6e-7 at 1e-33, 3.8e-6 at 1e-35, 3.8e-5 at 1e-36; 1.5e-7 at 1e37);
-// magnitudes within 2^-9 of the largest float round up to infinity.
+// the three that are left out (m l', l m', l l') are at most 2^-24 |x w| together, the size of one fp32 rounding. Sums
+// are fp32, as in v_mfma_f32_16x16x4_f32, but one instruction adds 32 channels instead of 4, so there are fewer roundings: a sum of
+// K = 64 channels is off by 1.5e-7 of itself (2.1e-7 with the fp32 instructions), a single product by up to twice as much as there.
 // Six v_mfma_f32_16x16x32_bf16 (16 cycles each) do the work of eight v_mfma_f32_16x16x4_f32 (32 cycles each): 2.7 times the
 // rate of the fp32 matrix instructions for the same real product.
 #pragma once
@@ -29,6 +27,53 @@ __device__ __forceinline__ void split_bf16_pair(float a, float b, unsigned& h, u
     ra -= __builtin_bit_cast(float, m << 16);
     rb -= __builtin_bit_cast(float, m & 0xffff0000u);
     l = __builtin_bit_cast(unsigned, __builtin_convertvector((float2_v){ ra, rb }, bf16x2_t));
+}
+
+// Which operands the split holds: from 2^-110 (7.7e-34) on and up to 2^-9 below the largest float, and zero. Below 2^-110 the third part would need bits under the smallest bf16 number, 2^-133; infinities and
+// magnitudes within 2^-9 of the largest float leave a NaN in the remainder x - h. A wave whose operands include such values forms its
+// product again, with fp32 instructions, so that the results have fp32 precision and fp32 infinities over the whole range of floats:
+//   * small magnitudes are found in the operands: one minimum per two values; zeros, which are exact, are told apart only where the
+//     minimum is below the limit;
+//   * the others are found in the accumulators: each leaves a NaN or an infinity in every sum it takes part in.
+constexpr float kSplitSmallest = 0x1p-110f;
+__device__ __forceinline__ float smaller(float low, float a, float b)
+{
+    return __builtin_elementwise_minimum(__builtin_elementwise_minimum(low, __builtin_fabsf(a)), __builtin_fabsf(b));
+}
+__device__ __forceinline__ float smaller(float low, float2 a) { return smaller(low, a.x, a.y); }
+// is the condition true in any lane of the wave: uniform
+__device__ __forceinline__ bool any_lane(bool condition) { return __builtin_amdgcn_ballot_w64(condition) != 0; }
+// is one of the values small, but not zero, in any lane (a NaN among them hides the others, but not itself from the accumulators)
+template <int COUNT> __device__ __forceinline__ bool below_split_range(const float2 (&v)[COUNT])
+{
+    float low = 1.f;
+#pragma unroll
+    for (int j = 0; j < COUNT; ++j) low = smaller(low, v[j]);
+    if (__builtin_expect(!any_lane(low < kSplitSmallest), 1)) return false;
+    unsigned bits = ~0u;                                        // smallest 2 |bits| - 1: a zero wraps to the largest number
+#pragma unroll
+    for (int j = 0; j < COUNT; ++j) {
+        const unsigned a = 2u * __builtin_bit_cast(unsigned, v[j].x) - 1u, b = 2u * __builtin_bit_cast(unsigned, v[j].y) - 1u;
+        const unsigned u = a < b ? a : b;
+        bits = bits < u ? bits : u;
+    }
+    return any_lane(bits < 2u * __builtin_bit_cast(unsigned, kSplitSmallest) - 1u);
+}
+// the largest magnitude so far; NaN stays
+__device__ __forceinline__ float larger(float high, float4_v c)
+{
+    high = __builtin_elementwise_maximum(__builtin_elementwise_maximum(high, __builtin_fabsf(c[0])), __builtin_fabsf(c[1]));
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(high, __builtin_fabsf(c[2])), __builtin_fabsf(c[3]));
+}
+__device__ __forceinline__ bool not_finite(float a, float b) { return !(__builtin_elementwise_maximum(a, b) < __builtin_inff()); }
+
+// c += w a in fp32, four channels: one complex value of row (w) and column (a) lane % 16, channel lane / 16, per lane
+__device__ __forceinline__ void mac_fp32(float2 w, float2 a, float4_v& re, float4_v& im)
+{
+    re = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, a.x, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, a.y, im, 0, 0, 0);
+    re = __builtin_amdgcn_mfma_f32_16x16x4f32(-w.y, a.y, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, a.x, im, 0, 0, 0);
 }
 
 // the three parts of eight consecutive channels of one row or column: operands of v_mfma_f32_16x16x32_bf16

@@ -395,6 +395,8 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
 // work of the current one, and nothing in the walk waits at a barrier, so loads, matrix work and stores of the waves overlap.
 // With beta the values of C are read 16 at a time before any is stored (M = 262,144, N = 128, K = 24: 198 -> 124 us, K = 64: 221 -> 154;
 // with a column block per block instead of the walk, so that nothing waits behind the strip of the next: 130, 175).
+// Operands that the split does not hold (bf16_split.h) are found while they are split and in the accumulators, per wave and column
+// block; the wave then forms its product again with fp32 matrix instructions (two to four times the time of the column block).
 //   Kw    = period of W along the contraction: channel k is weighted with W[k mod Kw + n Kw] (Kw = K: the plain product;
 //           Kw = K / R: the R parts of decimated images, see above, share the weights of their image's channel);
 //   Kp    = channels covered by one run over the tile (K, or Kw: the contraction then runs over the tile K / Kw times);
@@ -409,6 +411,7 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
     float2 beta, long nblocks, int Kw, int Kp, int cap)
 {
     extern __shared__ uint4_v sW4[];
+    __shared__ unsigned sLow[THREADS / 64];             // per wave: it has built fragments with weights below the split's range
     constexpr int MBLOCK = THREADS / 4;                 // columns per block: 16 per wave
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 15, kq = lane >> 4;
     const int n0 = blockIdx.y * (16 * NT);
@@ -431,6 +434,7 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
         for (int j = 0; j < 8; ++j) bv[j] = (base + j * Mtot)[off];
     };
     // fragments of the steps s0 ... s0 + count - 1: entry (step, tile, kq, n mod 16) = eight consecutive channels of one n
+    bool low_weights = false;                           // once seen it holds for all column blocks: they share the weights
     auto build = [&](int s0, int count) {
         for (int e = tid; e < count * NT * 64; e += THREADS) {
             const int l = e & 63, t = (e >> 6) % NT, s = (e >> 6) / NT;
@@ -446,6 +450,7 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j) w[j] = make_float2(w[j].x * alpha.x - w[j].y * alpha.y, w[j].x * alpha.y + w[j].y * alpha.x);
+            low_weights |= below_split_range(w);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 unsigned h, m, lo;
@@ -458,6 +463,7 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
             dst[0] = re.h; dst[64] = re.m; dst[128] = re.l;
             dst[192] = im.h; dst[256] = im.m; dst[320] = im.l;
         }
+        if (lane == 0) sLow[wave] = low_weights;
     };
 
     float4_v re[NT], im[NT];
@@ -469,16 +475,19 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
     // one loop over column blocks, runs and steps: nested ones cost a copy of the strip at every edge between them
     long v = blockIdx.x, mb = block_of(v);              // the grid is no larger than the number of column blocks
     int run = 0, step = 0, slot = 0;                    // slot: the step's place in the tile
-    bool built = false;
+    bool built = false, low_column = false;             // low_column: small values among the wave's columns
+    unsigned low_tile = 0;
     fetch(mb, 0, 0, true);
     while (true) {
         if (slot == 0 && !(resident && built)) {        // uniform over the block
             __syncthreads();
             build(step, steps - step < cap ? steps - step : cap);
             __syncthreads();
+            low_tile |= sLow[lane & (THREADS / 64 - 1)];
             built = true;
         }
         SplitOperand ar, ai;
+        low_column |= below_split_range(bv);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             unsigned h, m, l;
@@ -509,6 +518,24 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
         }
         if (last) {
             if (mb * MBLOCK + wave * 16 < Mtot) {
+                float high[2] = { 0.f, 0.f };
+#pragma unroll
+                for (int t = 0; t < NT; ++t) { high[0] = larger(high[0], re[t]); high[1] = larger(high[1], im[t]); }
+                if (__builtin_expect(low_column | any_lane(low_tile != 0 | not_finite(high[0], high[1])), 0)) {
+                    // operands beyond the split: the product in fp32
+                    clear();
+                    const float2* a = A + mb * MBLOCK + lane_col;
+                    const float2* w = W + (long)(n0 + col) * Kw;
+#pragma unroll 1
+                    for (int k = kq; k < K; k += 4) {
+                        const float2 ak = a[k * Mtot];
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) {
+                            const float2 wk = w[k % Kw + (long)(16 * t) * Kw];
+                            mac_fp32(make_float2(wk.x * alpha.x - wk.y * alpha.y, wk.x * alpha.y + wk.y * alpha.x), ak, re[t], im[t]);
+                        }
+                    }
+                }
                 // D[row = 4 kq + q][col] of tile t: output channel n0 + 16 t + 4 kq + q, the lane's column
                 float2* dst = C + mb * MBLOCK + lane_col + (long)(n0 + 4 * kq) * Mtot;
                 if (beta.x != 0.f || beta.y != 0.f) {               // variants A, B: C is read, up to 16 values at a time
@@ -537,6 +564,7 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
             }
             if (!more) return;
             v += gridDim.x;
+            low_column = false;
             clear();
         }
         mb = next_mb;
