@@ -126,3 +126,102 @@ def test_cgemm_infinities_and_the_largest_floats(M, K, N, beta, value):
         fine = ~(inf | nan)
         scale = np.maximum(np.abs(ref[fine]), 0.01 * 0.01)
         assert np.max(np.abs(got[fine] - ref[fine]) / scale) < 2 * K * 2.0 ** -24 + 1e-5
+
+
+LAYERS = [                           # S, DY, K, N: the fused 1D kernel with 64 and 128 output channels per block
+    (260, 128, 40, 64), (513, 128, 104, 128),
+    (300, 256, 40, 64), (900, 256, 24, 64), (512, 256, 128, 128),
+    (260, 512, 40, 64), (520, 512, 104, 128),
+    (258, 1024, 40, 64), (256, 1024, 72, 128),
+]
+HALVES = [(9, 128, 40, 64), (513, 128, 40, 128), (9, 256, 72, 64), (400, 256, 40, 128), (9, 512, 40, 64), (400, 512, 40, 128),
+          (9, 1024, 40, 64), (390, 1024, 24, 128)]
+_TRANSFORMS = 2 * 16 ** 0.5 * 2.0 ** -24       # two transforms of eight real additions in a row per value
+
+
+def _layer_check(run, reference, x, W, scale, tol, channels_out):
+    """run(x, W) with some signal sets, then with some rows of W at `scale`: relative error of every signal set / output channel"""
+    S = x.shape[1]
+    sets = sorted({0, S // 2, S - 1})
+    idx = torch.tensor(sets, device="cuda")
+    xs = x.clone()
+    xs[:, idx[1:]] *= scale
+    y = run(xs, W)
+    assert not bool(torch.isnan(torch.view_as_real(y)).any())
+    pick = lambda a: a.index_select(1, idx).cpu().numpy()
+    ref = reference(pick(xs), W)
+    for i in range(len(sets)):
+        err = np.linalg.norm(pick(y)[:, i] - ref[:, i]) / np.linalg.norm(ref[:, i])
+        assert err < tol, ("signal set", sets[i], err)
+    Ws = W.copy()
+    Ws[1::3] *= np.float32(scale)
+    y = pick(run(x, Ws))
+    ref = reference(pick(x), Ws)
+    for n in range(channels_out):
+        err = np.linalg.norm(y[n] - ref[n]) / np.linalg.norm(ref[n])
+        assert err < tol, ("output channel", n, err)
+
+
+def _x(S, L, K):
+    gen = torch.Generator(device="cuda").manual_seed(S + L + K)
+    return torch.view_as_complex(torch.rand((K, S, L, 2), device="cuda", generator=gen) * 2 - 1)
+
+
+@pytest.mark.parametrize("scale", [1e-35, 1e-37, 1e20])
+@pytest.mark.parametrize("S,DY,K,N", LAYERS)
+def test_layer_1d_of_any_magnitude(S, DY, K, N, scale):
+    print("layer range", S, DY, K, N, scale, flush=True)
+    W = _complex(np.random.default_rng(S), N, K) / np.float32(np.sqrt(K))
+    run = lambda x, W: tf.layer_1d(x, _dev(W), alpha=0.5 - 0.75j)
+    _layer_check(run, lambda x, W: oracle.layer_1d(x, W, 0.5 - 0.75j), _x(S, DY, K), W, scale, _bound(K) + _TRANSFORMS, N)
+
+
+@pytest.mark.parametrize("scale", [1e-35, 1e-37, 1e20])
+@pytest.mark.parametrize("S,DY,K,N", HALVES)
+def test_halves_of_the_layer_of_any_magnitude(S, DY, K, N, scale):
+    print("halves range", S, DY, K, N, scale, flush=True)
+    W = _complex(np.random.default_rng(S), N, K) / np.float32(np.sqrt(K))
+
+    def forward(x, W):
+        C = torch.empty((N, S, 64), dtype=torch.complex64, device="cuda")
+        tf.fused_fft_cgemm(64 * S, N, K, x, _dev(W), C, 1.0, 0.0)
+        return C
+
+    def backward(A, W):
+        y = torch.empty((N, S, DY), dtype=torch.complex64, device="cuda")
+        tf.fused_cgemm_ifft(64 * S, N, K, A, _dev(W), y, 1.0)
+        return y
+
+    product = lambda A, W: oracle.cgemm(A.reshape(K, -1), W, 1.0).reshape(N, -1, 64)
+    _layer_check(forward, lambda x, W: product(oracle.fft_trunc_contig(x), W), _x(S, DY, K), W, scale, _bound(K) + _TRANSFORMS, N)
+    _layer_check(backward, lambda A, W: oracle.ifft_pad_contig(product(A, W), DY), _x(S, 64, K), W, scale, _bound(K) + _TRANSFORMS, N)
+
+
+@pytest.mark.parametrize("DY", [128, 256, 512, 1024])
+def test_halves_with_the_largest_floats(DY):
+    """values within a bf16 rounding of the largest float, whose products and transforms are in range again; infinities reach the
+    outputs that depend on them and no others"""
+    print("halves largest", DY, flush=True)
+    S, K, N = 3, 24, 64
+    rng = np.random.default_rng(DY)
+    A, W = _complex(rng, K, S, 64), _complex(rng, N, K) * np.float32(1e-4)
+    A[5, 1, 9] = 3.4e38 - 3.4028234e38j
+    y = torch.empty((N, S, DY), dtype=torch.complex64, device="cuda")
+    tf.fused_cgemm_ifft(64 * S, N, K, _dev(A), _dev(W), y, 1.0)
+    ref = oracle.ifft_pad_contig(oracle.cgemm(A.reshape(K, -1), W, 1.0).reshape(N, S, 64), DY)
+    y = y.cpu().numpy().astype(np.complex128)
+    for s in range(S):
+        assert np.linalg.norm(y[:, s] - ref[:, s]) / np.linalg.norm(ref[:, s]) < _bound(K) + _TRANSFORMS
+    x, W = _complex(rng, K, S, DY) * np.float32(1e-4), _complex(rng, N, K)
+    W[11, 7] = 3.4e38 + 1j
+    C = torch.empty((N, S, 64), dtype=torch.complex64, device="cuda")
+    tf.fused_fft_cgemm(64 * S, N, K, _dev(x), _dev(W), C, 1.0, 0.0)
+    ref = oracle.cgemm(oracle.fft_trunc_contig(x).reshape(K, -1), W, 1.0).reshape(N, S, 64)
+    C = C.cpu().numpy().astype(np.complex128)
+    for n in range(N):
+        assert np.linalg.norm(C[n] - ref[n]) / np.linalg.norm(ref[n]) < _bound(K) + _TRANSFORMS
+    W[11, 7] = np.inf
+    C = torch.empty((N, S, 64), dtype=torch.complex64, device="cuda")
+    tf.fused_fft_cgemm(64 * S, N, K, _dev(x), _dev(W), C, 1.0, 0.0)
+    bad = ~np.isfinite(C.cpu().numpy())
+    assert bad[11].all() and not np.delete(bad, 11, axis=0).any()

@@ -32,8 +32,8 @@ __device__ __forceinline__ void split_bf16_pair(float a, float b, unsigned& h, u
 // Which operands the split holds: from 2^-110 (7.7e-34) on and up to 2^-9 below the largest float, and zero. Below 2^-110 the third part would need bits under the smallest bf16 number, 2^-133; infinities and
 // magnitudes within 2^-9 of the largest float leave a NaN in the remainder x - h. A wave whose operands include such values forms its
 // product again, with fp32 instructions, so that the results have fp32 precision and fp32 infinities over the whole range of floats:
-//   * small magnitudes are found in the operands: one minimum per two values; zeros, which are exact, are told apart only where the
-//     minimum is below the limit;
+//   * small magnitudes are found in the operands, zeros, which are exact, aside (lower(): three instructions per two values; or one,
+//     smaller(), where zeros can be told apart later);
 //   * the others are found in the accumulators: each leaves a NaN or an infinity in every sum it takes part in.
 constexpr float kSplitSmallest = 0x1p-110f;
 __device__ __forceinline__ float smaller(float low, float a, float b)
@@ -41,6 +41,14 @@ __device__ __forceinline__ float smaller(float low, float a, float b)
     return __builtin_elementwise_minimum(__builtin_elementwise_minimum(low, __builtin_fabsf(a)), __builtin_fabsf(b));
 }
 __device__ __forceinline__ float smaller(float low, float2 a) { return smaller(low, a.x, a.y); }
+// smallest 2 |bits| - 1: a zero wraps to the largest number
+constexpr unsigned kSplitLow = (17u << 24) - 1;                  // of 2^-110
+__device__ __forceinline__ unsigned lower(unsigned low, float2 v)
+{
+    const unsigned a = 2u * __builtin_bit_cast(unsigned, v.x) - 1u, b = 2u * __builtin_bit_cast(unsigned, v.y) - 1u;
+    const unsigned u = a < b ? a : b;
+    return low < u ? low : u;
+}
 // is the condition true in any lane of the wave: uniform
 __device__ __forceinline__ bool any_lane(bool condition) { return __builtin_amdgcn_ballot_w64(condition) != 0; }
 // is one of the values small, but not zero, in any lane (a NaN among them hides the others, but not itself from the accumulators)
@@ -50,14 +58,10 @@ template <int COUNT> __device__ __forceinline__ bool below_split_range(const flo
 #pragma unroll
     for (int j = 0; j < COUNT; ++j) low = smaller(low, v[j]);
     if (__builtin_expect(!any_lane(low < kSplitSmallest), 1)) return false;
-    unsigned bits = ~0u;                                        // smallest 2 |bits| - 1: a zero wraps to the largest number
+    unsigned bits = ~0u;
 #pragma unroll
-    for (int j = 0; j < COUNT; ++j) {
-        const unsigned a = 2u * __builtin_bit_cast(unsigned, v[j].x) - 1u, b = 2u * __builtin_bit_cast(unsigned, v[j].y) - 1u;
-        const unsigned u = a < b ? a : b;
-        bits = bits < u ? bits : u;
-    }
-    return any_lane(bits < 2u * __builtin_bit_cast(unsigned, kSplitSmallest) - 1u);
+    for (int j = 0; j < COUNT; ++j) bits = lower(bits, v[j]);
+    return any_lane(bits < kSplitLow);
 }
 // the largest magnitude so far; NaN stays
 __device__ __forceinline__ float larger(float high, float4_v c)
@@ -80,12 +84,12 @@ __device__ __forceinline__ void mac_fp32(float2 w, float2 a, float4_v& re, float
 struct SplitOperand {
     uint4_v h, m, l;
 };
-// Element j of the two A operand rows of one complex weight times alpha, for a contraction over (re, im) pairs of the other
-// operand: (re, -im) gives the real part of the product, (im, re) the imaginary part.
-__device__ __forceinline__ void split_weight_rows(float2 w, float2 alpha, SplitOperand& real_row, SplitOperand& imag_row, int j)
+// Element j of the two A operand rows of one complex weight, for a contraction over (re, im) pairs of the other operand:
+// (re, -im) gives the real part of the product, (im, re) the imaginary part.
+__device__ __forceinline__ void split_weight_rows(float2 w, SplitOperand& real_row, SplitOperand& imag_row, int j)
 {
     unsigned h, m, l;
-    split_bf16_pair(w.x * alpha.x - w.y * alpha.y, w.x * alpha.y + w.y * alpha.x, h, m, l);
+    split_bf16_pair(w.x, w.y, h, m, l);
     real_row.h[j] = h ^ 0x80000000u; real_row.m[j] = m ^ 0x80000000u; real_row.l[j] = l ^ 0x80000000u;
     imag_row.h[j] = __builtin_amdgcn_alignbit(h, h, 16);
     imag_row.m[j] = __builtin_amdgcn_alignbit(m, m, 16);

@@ -486,7 +486,7 @@ __global__ __launch_bounds__(512) void fused_fft_mfma_ifft_split_kernel(int S, i
         for (int i = 0; i < TILES; ++i) {
             SplitOperand wre, wim;                                // rows (re, -im) and (im, re) of alpha W
 #pragma unroll
-            for (int j = 0; j < 4; ++j) split_weight_rows(wv[i][j], alpha, wre, wim, j);
+            for (int j = 0; j < 4; ++j) split_weight_rows(cmul(wv[i][j], alpha), wre, wim, j);
 #pragma unroll
             for (int a = 0; a < 4; ++a) mac_split_pair(wre, wim, b[a], re[i][a], im[i][a]);
         }

@@ -14,14 +14,18 @@
 //     its own 16-lane group (DY = 128: after one row rotation; DY = 512 / 1024: through the exchange region of the group, inside
 //     the wave). The product never passes a block barrier, nor does the backward phase.
 // What bounds it: the chain of phases of a wave (x, transform, product, backward, stores), hidden by blocks in other phases, up to
-// the rate of a mixed read and write stream (4.5 - 4.8 TB/s here; a copy of 2 GiB: 4.9). Hence the registers are held to three blocks per CU (NTW = 2: 158;
-// NTW = 1: 144) or four (NTW = 1: 116 - 124, the operand tile sharing the exchange regions, x requested after the second pass)
+// the rate of a mixed read and write stream (4.5 - 4.8 TB/s here; a copy of 2 GiB: 4.9). Hence, at lengths 128 / 256, the registers are
+// held to three blocks per CU (NTW = 2: 158 - 166; NTW = 1: 135) or four (NTW = 1: 123 - 126, the operand tile sharing the exchange
+// regions, x requested after the second pass), at 512 to two or three and at 1024 to two (the halves: up to four),
 // without spills: with spills the kernel is up to 70 % slower, because a reload waits for the x in flight.
 // Measured against the fp32 kernels it replaced (us, x and y from HBM): DY = 256, K = N = 128, S = 8192: 1135 -> 960;
 // K = N = 64, S = 4096: 247 -> 213; DY = 128, K = N = 64, S = 16384: 533 -> 447; K = N = 128, S = 8192: 735 -> 569; K = 40, N = 128,
 // S = 1000: 52 -> 41; DY = 512, K = N = 128, S = 2048: 652 -> 451; DY = 1024, K = N = 128, S = 1000: 601 -> 462. Halves against the SIMT kernel:
 // forward DY = 256, K = N = 64, S = 2048: 103 -> 77, K = N = 128: 341 -> 171; backward 112 -> 65, 298 -> 149; S = 64, K = N = 64: 22 -> 13 both. (Forward, DY = 1024,
-// K = 8, N = 64, S = 2048 is the one shape found slower: 47.8 -> 50.1.) Error against 64 bits: 2.4e-7 -> 2.0e-7 (K = 64), 3.2e-7 -> 2.7e-7 (K = 128).
+// K = 8, N = 64, S = 2048 is the one shape found slower: 47.8 -> 50.1.)
+// Error against 64 bits: 2.4e-7 -> 2.0e-7 (K = 64), 3.2e-7 -> 2.7e-7 (K = 128), the same from the smallest normal floats to the
+// largest: operands that the split does not hold (bf16_split.h) are noticed - small spectra and weights as they are split, the rest in
+// the accumulators - and product_fp32() stands in. Noticing costs 0 - 3 %, 1.2 % on average (the most: DY = 128, S = 4096, K = N = 128: 282 -> 292).
 #include "bf16_split.h"
 #include "group_fft.h"
 #include "kernels.h"
@@ -44,7 +48,8 @@ template <int LOGDY, bool ALIAS, bool FWD> struct GeoSplit {
     static constexpr int TILE_BYTES = (KC / 16) * STEP_BYTES;
     static constexpr int TILE_AT = ALIAS ? 0 : EXCH_BYTES;
     static constexpr int TW_AT = ALIAS ? EXCH_BYTES : EXCH_BYTES + TILE_BYTES;      // first-pass twiddles, then the powers w_L^e
-    static constexpr size_t LDS_BYTES = TW_AT + sizeof(float2) * (L * kTwLdsPitch + (L > 16 ? L : 0));
+    static constexpr int LOW_AT = TW_AT + (int)sizeof(float2) * (L * kTwLdsPitch + (L > 16 ? L : 0));   // a flag per wave
+    static constexpr size_t LDS_BYTES = LOW_AT + 4 * sizeof(unsigned);
     static_assert(!ALIAS || (TILE_BYTES <= EXCH_BYTES && CP == KC), "the operand tile must fit the exchange regions, one pass per round");
 };
 
@@ -55,6 +60,92 @@ template <int COUNT> TFNO_DEV void after(int& offset, const cpx (&g)[COUNT])
 {
 #pragma unroll
     for (int i = 0; i < COUNT; ++i) asm volatile("" : "+v"(offset) : "v"(g[i].x));
+}
+
+// First pass of two signals of 128 samples: v[0..7], v[8..15] are samples t + 16 i of each.
+TFNO_DEV void pair_first_pass(const cpx (&v)[16], const cpx* twrow, cpx (&gg)[16])
+{
+    cpx a8[8], b8[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) { a8[i] = v[i]; b8[i] = v[8 + i]; }
+    fft8<-1>(a8);
+    fft8<-1>(b8);
+    gg[0] = a8[0];
+    gg[8] = b8[0];
+#pragma unroll
+    for (int r = 1; r < 8; ++r) {
+        const cpx w = twrow[r];
+        gg[r] = cmul(a8[r], w);
+        gg[8 + r] = cmul(b8[r], w);
+    }
+}
+
+// The product of one wave in fp32, for operands that the split does not hold: the wave transforms all K channels by itself, as many at
+// a time as it has lane groups for, and takes its 16 NTW output channels from them four channels at a time. Several times as slow as
+// the loop that it stands in for. `region`: the exchange regions of the wave, free of other use.
+template <int LOGDY, int NTW, bool FWD>
+TFNO_DEV void product_fp32(long S, int K, long s, int nw, const float2* __restrict__ x, const float2* __restrict__ W, float2 alpha,
+                           const cpx* twrow, const cpx* powers, cpx* region, float4_v (&re)[NTW][4], float4_v (&im)[NTW][4])
+{
+    using G = GeoSplit<LOGDY, false, FWD>;
+    constexpr int DY = 1 << LOGDY, L = G::L, CHANNELS = !FWD ? 4 : (G::PAIR ? 8 : 64 / L);
+    const int lane = threadIdx.x & 63, group = lane / L, t = lane % L, kq = lane >> 4, col = lane & 15;
+    cpx* exch = region + group * G::EXCH;
+    const float2* w = W + (long)(nw + col) * K;
+#pragma unroll
+    for (int i = 0; i < NTW; ++i)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) re[i][a] = im[i][a] = float4_v{ 0.f, 0.f, 0.f, 0.f };
+#pragma unroll 1
+    for (int k = 0; k < K; k += CHANNELS) {
+        cpx b[4];
+        if constexpr (!FWD) {
+            const float2* p = x + (k + kq) * (64 * S) + s * 64 + col;
+#pragma unroll
+            for (int a = 0; a < 4; ++a) b[a] = p[16 * a];
+        } else {
+            const float2* p = x + ((long)(k + (G::PAIR ? 2 : 1) * group) * S + s) * DY + t;
+            cpx v[16], gg[16];
+            if constexpr (G::PAIR) {
+                cpx out[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) { v[i] = p[16 * i]; v[8 + i] = p[S * DY + 16 * i]; }
+                pair_first_pass(v, twrow, gg);
+                rows128_forward_finish(gg, exch, t, out);
+                wave_lds_fence();
+#pragma unroll
+                for (int a = 0; a < 8; ++a) exch[(t >> 3) * 64 + (t & 7) + 8 * a] = out[a];
+            } else {
+                cpx out[64 / L];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[i] = p[L * i];
+                fwd_pass1_lds(v, twrow, gg);
+                if constexpr (L > 16) wide_forward_finish<L, true>(gg, exch, powers, t, out);
+                else group_forward_finish<8>(gg, exch, t, out);
+                wave_lds_fence();
+#pragma unroll
+                for (int a = 0; a < 64 / L; ++a) exch[t + L * a] = out[a];
+            }
+            wave_lds_fence();
+        }
+#pragma unroll
+        for (int c0 = 0; c0 < CHANNELS; c0 += 4) {
+            // lane (kq, col): channel c of the round, modes col + 16 a; lanes without a channel multiply zeros
+            const int c = c0 + kq;
+            const bool live = CHANNELS >= 4 || c < CHANNELS;
+            if constexpr (FWD) {
+                const cpx* modes = region + (G::PAIR ? (c >> 1) * G::EXCH + (c & 1) * 64 : (live ? c : 0) * G::EXCH) + col;
+#pragma unroll
+                for (int a = 0; a < 4; ++a) b[a] = live ? modes[16 * a] : make_float2(0.f, 0.f);
+            }
+#pragma unroll
+            for (int i = 0; i < NTW; ++i) {
+                const float2 wk = live ? cmul(w[k + c + (long)(16 * i) * K], alpha) : make_float2(0.f, 0.f);
+#pragma unroll
+                for (int a = 0; a < 4; ++a) mac_fp32(wk, b[a], re[i][a], im[i][a]);
+            }
+        }
+    }
 }
 
 template <int LOGDY, int NTW, bool ALIAS, int BLOCKS, bool KEEP, bool FWD = true, bool INV = true>
@@ -80,6 +171,7 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
     char* tile = lds_split + G::TILE_AT;
     float2* twtab = reinterpret_cast<float2*>(lds_split + G::TW_AT);
     float2* powers = twtab + L * kTwLdsPitch;
+    unsigned* low_flags = reinterpret_cast<unsigned*>(lds_split + G::LOW_AT);
     fill_lds_twiddles<LOGDY, L>(twtab, tid, 256);
     if (LONG && tid < L) powers[tid] = kTwiddle1024[tid * (1024 / L)];
     const float2* twrow = twtab + t * kTwLdsPitch;
@@ -115,6 +207,7 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
         return tile + (c >> 4) * G::STEP_BYTES + a * 3072 + ((c >> 2) & 3) * 256 + column * 16 + (c & 3) * 4;
     };
 
+    bool low = false, low_weights = false;                      // of the wave: spectra too small for the split / such weights or zeros
     for (int kc = 0; kc < K; kc += KC) {
         const int kn = (K - kc) < KC ? (K - kc) : KC;           // a multiple of 8 (caller contract)
         constexpr int MODES = !FWD ? 4 : (PAIR ? 8 : 64 / L), WSTEPS = PAIR && NTW == 1 && BLOCKS < 4 ? 2 : 1;
@@ -143,19 +236,7 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
             } else if (busy) {
                 cpx gg[16];
                 if constexpr (PAIR) {
-                    cpx a8[8], b8[8];
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) { a8[i] = v[i]; b8[i] = v[8 + i]; }
-                    fft8<-1>(a8);
-                    fft8<-1>(b8);
-                    gg[0] = a8[0];
-                    gg[8] = b8[0];
-#pragma unroll
-                    for (int r = 1; r < 8; ++r) {
-                        const cpx w = twrow[r];
-                        gg[r] = cmul(a8[r], w);
-                        gg[8 + r] = cmul(b8[r], w);
-                    }
+                    pair_first_pass(v, twrow, gg);
                 } else {
                     fft16<-1>(v);
                     int row = 0;
@@ -194,6 +275,12 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
 #pragma unroll
                 for (int a = 0; a < MODES; ++a) out[a] = make_float2(0.f, 0.f);
             }
+            if (busy) {
+                unsigned bits = ~0u;
+#pragma unroll
+                for (int a = 0; a < MODES; ++a) bits = lower(bits, out[a]);
+                low |= any_lane(bits < kSplitLow);
+            }
             if (pass == 0) __syncthreads();                     // the operand tile of the last round is read / the exchanges are done
 #pragma unroll
             for (int a = 0; a < MODES; ++a) {
@@ -208,6 +295,7 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
                 *reinterpret_cast<unsigned*>(dst + 2048) = l;
             }
         }
+        if (kc + KC >= K && lane == 0) low_flags[wave] = low;
         __syncthreads();
 #pragma unroll
         for (int step = 0; step < KC / 16; ++step) {
@@ -217,8 +305,15 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
             for (int i = 0; i < NTW; ++i) {
                 if constexpr (LATE) __builtin_amdgcn_sched_barrier(0);
                 SplitOperand wre, wim;                          // rows (re, -im) and (im, re) of alpha W
+                float2 (&w4)[4] = wv[WSTEPS == 2 ? step : 0][i];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) split_weight_rows(wv[WSTEPS == 2 ? step : 0][i][j], alpha, wre, wim, j);
+                for (int j = 0; j < 4; ++j) w4[j] = cmul(w4[j], alpha);
+                float smallest = 1.f;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) smallest = smaller(smallest, w4[j]);
+                low_weights |= any_lane(smallest < kSplitSmallest);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) split_weight_rows(w4[j], wre, wim, j);
                 if (WSTEPS == 1 && PAIR && step == 0 && 16 < kn && i == NTW - 1) load_w(1, wv[0], 0);
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
@@ -230,6 +325,23 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
         }
         if constexpr (ALIAS) __syncthreads();                   // the operand tile is read: exchange regions again
     }
+
+    float high[2] = { 0.f, 0.f };
+#pragma unroll
+    for (int i = 0; i < NTW; ++i)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) { high[0] = larger(high[0], re[i][a]); high[1] = larger(high[1], im[i][a]); }
+    if (__builtin_expect(low_weights, 0)) {                     // which of the two
+        unsigned bits = ~0u;
+        const float2* w = W + (long)(nw + col) * K;
+#pragma unroll 1
+        for (int k = kq; k < K; k += 4)
+#pragma unroll
+            for (int i = 0; i < NTW; ++i) bits = lower(bits, cmul(w[k + (long)(16 * i) * K], alpha));
+        low_weights = any_lane(bits < kSplitLow);
+    }
+    if (__builtin_expect(low_weights | any_lane((low_flags[lane & 3] != 0) | not_finite(high[0], high[1])), 0))
+        product_fp32<LOGDY, NTW, FWD>(S, K, s, nw, x, W, alpha, twrow, powers, reinterpret_cast<float2*>(lds_split) + wave * (64 * 17), re, im);
 
     // D[row = 4 kq + q][col] of tile (i, a): output channel nw + 16 i + 4 kq + q, mode col + 16 a
 #pragma unroll
