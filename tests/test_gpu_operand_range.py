@@ -134,6 +134,7 @@ LAYERS = [                           # S, DY, K, N: the fused 1D kernel with 64 
     (260, 512, 40, 64), (520, 512, 104, 128),
     (258, 1024, 40, 64), (256, 1024, 72, 128),
 ]
+SMALL_GRIDS = [(3, 64, 64), (5, 136, 128), (9, 128, 192)]     # S, K, N at DY = 256: the channels split over the waves of a block
 HALVES = [(9, 128, 40, 64), (513, 128, 40, 128), (9, 256, 72, 64), (400, 256, 40, 128), (9, 512, 40, 64), (400, 512, 40, 128),
           (9, 1024, 40, 64), (390, 1024, 24, 128)]
 _TRANSFORMS = 2 * 16 ** 0.5 * 2.0 ** -24       # two transforms of eight real additions in a row per value
@@ -174,6 +175,17 @@ def test_layer_1d_of_any_magnitude(S, DY, K, N, scale):
     W = _complex(np.random.default_rng(S), N, K) / np.float32(np.sqrt(K))
     run = lambda x, W: tf.layer_1d(x, _dev(W), alpha=0.5 - 0.75j)
     _layer_check(run, lambda x, W: oracle.layer_1d(x, W, 0.5 - 0.75j), _x(S, DY, K), W, scale, _bound(K) + _TRANSFORMS, N)
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-35, 1e-37, 1e20])
+@pytest.mark.parametrize("S,K,N", SMALL_GRIDS)
+def test_small_grids_of_any_magnitude(S, K, N, scale, algo_1d):
+    print("small grid range", S, K, N, scale, flush=True)
+    algo_1d(6)
+    assert tf.query_1d_kernel(256, S, N, K) == 6
+    W = _complex(np.random.default_rng(S), N, K) / np.float32(np.sqrt(K))
+    run = lambda x, W: tf.layer_1d(x, _dev(W), alpha=0.5 - 0.75j)
+    _layer_check(run, lambda x, W: oracle.layer_1d(x, W, 0.5 - 0.75j), _x(S, 256, K), W, scale, _bound(K) + _TRANSFORMS, N)
 
 
 @pytest.mark.parametrize("scale", [1e-35, 1e-37, 1e20])

@@ -417,7 +417,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 // meet in LDS once (sP[w][n][m], pitch 72 complex: conflict-free b64 stores), every lane group sums the eight partials
 // of one output channel and runs its backward transform. The chain of latencies of an item is K / 32 rounds + K / 128 products +
 // one reduction + one backward pass, against three barriers and two tile builds per 32 channels in the kernel that
-// shares the spectra through LDS. S = 64, K = N = 128: 18.7 us with fp32 matrix instructions in every round, 17.2 now (K = 64: 13.4 / 13.5).
+// shares the spectra through LDS. S = 64, K = N = 128: 17.6 us
+// with fp32 matrix instructions in every round, 15.7 with the split, 16.2 with the search for operands that the split does not hold
+// (for which the wave's share of the product is formed in fp32 instead); K = 64: 13.1 / 13.1 / 13.4.
 constexpr int SPLIT_NT = 32, SPLIT_PP = 72;
 constexpr size_t SPLIT_LDS = sizeof(float2) * 8 * SPLIT_NT * SPLIT_PP;       // 147,456 B; covers the 32 exchange regions
 
@@ -455,6 +457,7 @@ __global__ __launch_bounds__(512) void fused_fft_mfma_ifft_split_kernel(int S, i
     // the buffer is refilled as soon as the first pass has consumed it (a second buffer, two rounds ahead, was
     // measured slower: a round is bound by its arithmetic, not by the latency of its loads)
     cpx v[16];
+    bool low = false;                                             // values too small for the split among the wave's operands
     if (4 * w < K) issue(v, 0);
     for (int kc = 0; kc + 4 * w < K; kc += 128) {
         SplitOperand b[4];
@@ -469,6 +472,10 @@ __global__ __launch_bounds__(512) void fused_fft_mfma_ifft_split_kernel(int S, i
                 fwd_pass1(v, tw, gg);
                 if (kr + 32 + 4 * w < K) issue(v, kr + 32);
                 group_forward_finish<8>(gg, exch, t, out);
+                unsigned bits = ~0u;
+#pragma unroll
+                for (int a = 0; a < 4; ++a) bits = lower(bits, out[a]);
+                low |= any_lane(bits < kSplitLow);
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
                     unsigned h, m, l;
@@ -486,9 +493,40 @@ __global__ __launch_bounds__(512) void fused_fft_mfma_ifft_split_kernel(int S, i
         for (int i = 0; i < TILES; ++i) {
             SplitOperand wre, wim;                                // rows (re, -im) and (im, re) of alpha W
 #pragma unroll
-            for (int j = 0; j < 4; ++j) split_weight_rows(cmul(wv[i][j], alpha), wre, wim, j);
+            for (int j = 0; j < 4; ++j) wv[i][j] = cmul(wv[i][j], alpha);
+            unsigned bits = ~0u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) bits = lower(bits, wv[i][j]);
+            low |= any_lane(bits < kSplitLow);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) split_weight_rows(wv[i][j], wre, wim, j);
 #pragma unroll
             for (int a = 0; a < 4; ++a) mac_split_pair(wre, wim, b[a], re[i][a], im[i][a]);
+        }
+    }
+    float high[2] = { 0.f, 0.f };
+#pragma unroll
+    for (int i = 0; i < TILES; ++i)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) { high[0] = larger(high[0], re[i][a]); high[1] = larger(high[1], im[i][a]); }
+    if (__builtin_expect(low | any_lane(not_finite(high[0], high[1])), 0)) {
+        // operands beyond the split: the wave's share of the product in fp32, one round of four channels at a time
+#pragma unroll
+        for (int i = 0; i < TILES; ++i)
+#pragma unroll
+            for (int a = 0; a < 4; ++a) re[i][a] = im[i][a] = float4_v{ 0.f, 0.f, 0.f, 0.f };
+#pragma unroll 1
+        for (int kr = 0; kr + 4 * w < K; kr += 32) {
+            cpx gg[16], out[4];
+            issue(v, kr);
+            fwd_pass1(v, tw, gg);
+            group_forward_finish<8>(gg, exch, t, out);
+#pragma unroll
+            for (int i = 0; i < TILES; ++i) {
+                const float2 wk = cmul(wsrc[kr + (long)(16 * i) * K], alpha);
+#pragma unroll
+                for (int a = 0; a < 4; ++a) mac_fp32(wk, out[a], re[i][a], im[i][a]);
+            }
         }
     }
     __syncthreads();                                              // every wave is done with its exchange regions
