@@ -450,7 +450,10 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j) w[j] = make_float2(w[j].x * alpha.x - w[j].y * alpha.y, w[j].x * alpha.y + w[j].y * alpha.x);
-            low_weights |= below_split_range(w);
+            unsigned bits = ~0u;                        // (zeros are common here: channels beyond Kp)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) bits = lower(bits, w[j]);
+            low_weights |= any_lane(bits < kSplitLow);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 unsigned h, m, lo;
@@ -480,7 +483,7 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
     fetch(mb, 0, 0, true);
     while (true) {
         if (slot == 0 && !(resident && built)) {        // uniform over the block
-            __syncthreads();
+            if (built) __syncthreads();                 // not before the first build: the last waves of a block start microseconds late
             build(step, steps - step < cap ? steps - step : cap);
             __syncthreads();
             low_tile |= sLow[lane & (THREADS / 64 - 1)];
@@ -816,7 +819,7 @@ hipError_t launch_ifft2d_pad(int logDX, int logDY, const float2* spec, float2* y
 //    several column blocks per CU the persistent kernel. K <= 32 as well for N >= 128 and 8 to 16 blocks of 256 columns x 64
 //    output channels per CU (M = 262,144, N = 128, K = 32: 77 against 88 us; from 16 on the 128-channel tile below is ahead).
 //  * otherwise the split kernel. Small products: blocks of 128 columns and the fewest output channels whose grid still fits one
-//    block per CU (K = 64, N = 64, tiles of 64 / 32 / 16 output channels: M = 64: 7.5 / 5.5 / 5.0; M = 8,192: 8.5 / 6.3 / 5.8; M = 16,384:
+//    block per CU (K = 64, N = 64, tiles of 64 / 32 / 16 output channels: M = 64: 7.5 / 5.5 / 4.7; M = 8,192: 8.5 / 6.3 / 5.5; M = 16,384:
 //    9.1 / 6.9; N = 192, M = 4,096: 9.0 / 7.1).
 //    At most half a block of 256 columns x 64 output channels per CU: blocks of 128 columns
 //    (M = 16,384, N = 64, K = 64: fp32 18.6, 256 columns 14.0, 128 columns 11.1); also for N = 64 with one to two blocks per
