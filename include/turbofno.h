@@ -165,7 +165,7 @@ int turbofno_layer_2d_noalloc(int bs, int DX, int DY, int K, int N, const void* 
  * output channels, 4 = as 2 with 32-channel output tiles, 5 = as 3, laid out for four blocks per compute unit (DY = 128 with
  * eight input channels: one wavefront per signal set and output tile), 6 = matrix cores, the K channels of an item split over
  * the waves of a block, 7 = matrix cores, the K channels of a signal set split over a cluster of blocks (see below), 8 = as 3
- * with 128 output channels per block where N allows and the size of the problem makes that the faster one (DY = 128 / 256).
+ * with 128 output channels per block where N is a multiple of 128.
  * A value a kernel is not built for falls back to the choice by size. Meant for tests and measurements; set returns
  * TURBOFNO_ERR_INVALID_ARG outside 0..TURBOFNO_1D_ALGO_MAX.
  */
@@ -218,10 +218,13 @@ int turbofno_set_exchange_wait_us(unsigned long long microseconds);
  *                             turbofno_set_1d_algo selector, in that selector's numbering (1 ... 8); 0 for arguments
  *                             the call would refuse. compute_units = 0 asks the current device (the only case that
  *                             touches the HIP runtime), any other value answers for a device of that many compute
- *                             units; exchange_attached says whether the stream has an exchange buffer.
+ *                             units; exchange_attached says whether the stream has an exchange buffer. Chosen by size, 8
+ *                             stands for blocks of 64 or of 128 output channels;
+ *   turbofno_query_1d_tile    output channels per block of that kernel (the clustered kernel: N); 0 as above.
  */
 int turbofno_query_2d_algo(int bs, int DX, int DY, int K, int N, int algo);
 int turbofno_query_1d_kernel(int logDY, long M, int N, int K, int compute_units, int exchange_attached);
+int turbofno_query_1d_tile(int logDY, long M, int N, int K, int compute_units, int exchange_attached);
 
 /* Explanation of the last non-zero return value on this thread ("" if none). Never NULL. */
 const char* turbofno_last_error_string(void);

@@ -83,3 +83,21 @@ def test_queries_answer_zero_for_arguments_the_calls_refuse():
     # an explicit algorithm is returned as it is
     assert tf.query_2d_algo(1, 256, 256, 16, 64, tf.ALGO_WHOLE_IMAGE) == tf.ALGO_WHOLE_IMAGE
     assert tf.query_2d_algo(1, 512, 1024, 16, 64, tf.ALGO_WHOLE_IMAGE) == tf.ALGO_WHOLE_IMAGE
+
+
+def test_output_channels_per_block(algo_1d):
+    assert tf.query_1d_tile(256, 1, 64, 8, CUS) == 32
+    assert tf.query_1d_tile(256, 64, 128, 128, CUS) == 32
+    assert tf.query_1d_tile(256, 64, 128, 128, CUS, exchange_attached=True) == 128
+    assert tf.query_1d_tile(256, 4096, 64, 64, CUS) == 64
+    assert tf.query_1d_tile(256, 8192, 128, 128, CUS) == 128
+    assert tf.query_1d_tile(256, 1000, 128, 16, CUS) == 64
+    assert tf.query_1d_tile(256, 4, 64, 12, CUS) == 0
+    for DY in (128, 256, 512, 1024):
+        for S in (1, 40, 2048):
+            for K in (8, 32, 128):
+                algo_1d(8)                      # whatever the size
+                assert tf.query_1d_tile(DY, S, 128, K, CUS) == 128 and tf.query_1d_tile(DY, S, 256, K, CUS) == 128
+                assert tf.query_1d_tile(DY, S, 64, K, CUS) == 64 and tf.query_1d_tile(DY, S, 192, K, CUS) == 64
+                algo_1d(3)
+                assert tf.query_1d_tile(DY, S, 128, K, CUS) == 64

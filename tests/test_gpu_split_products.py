@@ -140,6 +140,44 @@ def test_fused_1d_edges(S, DY, K, N):
 
 
 @pytest.mark.parametrize("S,DY,K,N", [
+    (1, 128, 8, 128), (11, 128, 72, 256), (2048, 128, 40, 256),      # S = 2048, 4096: XCD j walks the j-th eighth of the signal sets
+    (3, 256, 72, 256), (2048, 256, 32, 256), (13, 512, 24, 256), (1024, 512, 40, 128), (2, 1024, 8, 128), (130, 1024, 40, 256),
+])
+def test_blocks_of_128_output_channels(S, DY, K, N, algo_1d):
+    """forced by the selector at sizes where the rule takes other blocks: one and two blocks per signal set, both block orders"""
+    print("split 128 outputs", S, DY, K, N, flush=True)
+    algo_1d(8)
+    assert tf.query_1d_kernel(DY, S, N, K) == 8 and tf.query_1d_tile(DY, S, N, K) == 128
+    gen = torch.Generator(device="cuda").manual_seed(S + DY + K)
+    x = torch.view_as_complex(torch.rand((K, S, DY, 2), device="cuda", generator=gen) * 2 - 1)
+    W = _complex(np.random.default_rng(S), N, K) / np.float32(np.sqrt(K))
+    y = torch.full((N, S, DY), float("nan"), dtype=torch.complex64, device="cuda")
+    tf.layer_1d(x, _dev(W), y=y, alpha=0.5 - 0.75j)
+    torch.cuda.synchronize()
+    assert not bool(torch.isnan(torch.view_as_real(y)).any()), "rows of y left unwritten"
+    e = S // 8
+    idx = torch.tensor(sorted({0, S // 2, S - 1} | {p for p in (7, 8, e - 1, e, 7 * e) if 0 <= p < S}), device="cuda")
+    ref = oracle.layer_1d(x.index_select(1, idx).cpu().numpy(), W, 0.5 - 0.75j)
+    err = rel_l2(y.index_select(1, idx).cpu().numpy(), ref)
+    assert err < _bound(K) + 2 * 16 ** 0.5 * 2.0 ** -24, err
+
+
+@pytest.mark.parametrize("algo", [1, 3])
+@pytest.mark.parametrize("bs,DX,DY,K,N", [(1, 128, 256, 16, 128), (2, 256, 128, 40, 256), (1, 512, 256, 24, 128), (1, 256, 512, 40, 128),
+                                          (1, 1024, 512, 8, 128), (1, 512, 1024, 8, 128)])
+def test_blocks_of_128_output_channels_as_middle_stage(bs, DX, DY, K, N, algo, algo_1d):
+    """the same as the middle stage of a 2D layer of three kernels: plain stores"""
+    print("split 128 outputs middle", bs, DX, DY, K, N, algo, flush=True)
+    algo_1d(8)
+    rng = np.random.default_rng(DX + DY)
+    x, W = _complex(rng, K, bs, DX, DY), _complex(rng, N, K) / np.float32(np.sqrt(K))
+    y = tf.layer_2d(_dev(x), _dev(W), algo=algo, alpha=1 - 1j)
+    torch.cuda.synchronize()
+    ref = oracle.layer_2d(x, W, 1 - 1j)
+    assert rel_l2(y.cpu().numpy(), ref) < 1e-6 and max_rel(y.cpu().numpy(), ref) < 1e-5
+
+
+@pytest.mark.parametrize("S,DY,K,N", [
     (1, 128, 8, 64), (9, 128, 40, 192), (400, 128, 56, 128),        # rounds of 32 channels: one of eight, a last one of eight, of 24
     (1, 256, 8, 64), (9, 256, 40, 192), (400, 256, 72, 128),        # S = 400: blocks of 128 output channels
     (3, 512, 24, 64), (400, 512, 40, 128), (2, 1024, 8, 64), (390, 1024, 24, 128),

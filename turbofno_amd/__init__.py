@@ -27,6 +27,7 @@ from .api import (  # noqa: F401
     lib,
     library_path,
     query_1d_kernel,
+    query_1d_tile,
     query_2d_algo,
     set_1d_algo,
     set_exchange_wait_us,

@@ -67,6 +67,8 @@ def lib():
         L.turbofno_query_2d_algo.restype = i
         L.turbofno_query_1d_kernel.argtypes = [i, l, i, i, i, i]
         L.turbofno_query_1d_kernel.restype = i
+        L.turbofno_query_1d_tile.argtypes = [i, l, i, i, i, i]
+        L.turbofno_query_1d_tile.restype = i
         L.turbofno_last_error_string.restype = ctypes.c_char_p
         L.turbofno_abi_version.restype = i
         for name in ("turbofno_fused_fft_cgemm_ifft", "turbofno_fft_stride", "turbofno_ifft_stride",
@@ -177,6 +179,11 @@ def query_1d_kernel(DY, S, N, K, compute_units=256, exchange_attached=False):
     """The fused 1D kernel (numbering of set_1d_algo, 1 ... 8) for S signals per channel; 0 = refused. With an explicit
     compute_units this is pure arithmetic (no GPU needed)."""
     return int(lib().turbofno_query_1d_kernel(_log2(DY), MODES * S, N, K, int(compute_units), 1 if exchange_attached else 0))
+
+
+def query_1d_tile(DY, S, N, K, compute_units=256, exchange_attached=False):
+    """Output channels per block of the kernel that query_1d_kernel names; 0 = refused."""
+    return int(lib().turbofno_query_1d_tile(_log2(DY), MODES * S, N, K, int(compute_units), 1 if exchange_attached else 0))
 
 
 def fused_fft_cgemm_ifft(M, N, K, x, W, y, alpha=1.0 + 0j, beta=0j, C=None):

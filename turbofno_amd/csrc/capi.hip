@@ -162,6 +162,13 @@ int turbofno_query_1d_kernel(int logDY, long M, int N, int K, int compute_units,
     return tfno::pick_fused_1d_kernel(logDY, M / 64, N, K, algo_1d(), false, cus, exchange_attached != 0);
 }
 
+int turbofno_query_1d_tile(int logDY, long M, int N, int K, int compute_units, int exchange_attached)
+{
+    const int kernel = turbofno_query_1d_kernel(logDY, M, N, K, compute_units, exchange_attached);
+    if (kernel == 0) return 0;
+    return tfno::tile_of_fused_1d_kernel(kernel, logDY, M / 64, N, K, algo_1d(), compute_units > 0 ? compute_units : tfno::cu_count());
+}
+
 int turbofno_query_2d_algo(int bs, int DX, int DY, int K, int N, int algo)
 {
     if (bs <= 0 || K <= 0 || N <= 0 || K % 8 || N % 64) return 0;

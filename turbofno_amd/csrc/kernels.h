@@ -116,7 +116,10 @@ hipError_t exchange_attach(hipStream_t stream, void* buffer, size_t bytes);   //
 bool exchange_attached(hipStream_t stream);
 hipError_t exchange_gave_up(hipStream_t stream, unsigned* count);   // waits for the stream
 
-// Grids of about one block per CU and more, DY = 128 / 256 (layer1d_split.hip): one block per (signal set, 64 or, if `wide` and N
+// Output channels per block of the kernel that pick_fused_1d_kernel has named for the same sizes and selector.
+int tile_of_fused_1d_kernel(int kernel, int logDY, long S, int N, int K, int algo, long cus);
+
+// Grids of about one block per CU and more, every length (layer1d_split.hip): one block per (signal set, 64 or, if `wide` and N
 // allows, 128 output channels); `dense`: the variant for four blocks per CU.
 hipError_t launch_fused_split(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, bool wide,
                               bool dense, hipStream_t stream, int keep_y = 0);

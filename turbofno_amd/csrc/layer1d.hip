@@ -722,8 +722,9 @@ static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const
 // channels, 4 = as 2 with 32-channel output tiles, 5 = as 3 for large grids: four blocks per CU, or with eight channels of
 // length 128 one wavefront per (signal set, output tile), 6 = matrix cores, the eight waves of a block split the K channels of one
 // item (DY = 256), 7 = matrix cores, a cluster of blocks splits the K channels of one signal set (DY = 256, N = 64 / 128, small
-// grids), 8 = as 3 with 128 output channels per block where N allows (DY = 128, 256)
-// The return value uses the same numbers (1 ... 8). A selector value that a kernel is not built for falls back to the
+// grids), 8 = as 3 with 128 output channels per block where N allows
+// The return value uses the same numbers (1 ... 8); chosen by size, 8 stands for blocks of 64 or of 128 output channels
+// (tile_of_fused_1d_kernel). A selector value that a kernel is not built for falls back to the
 // choice by size.
 //
 // By size (measured on MI355X, us, kernel of the smaller grids against the split kernel):
@@ -793,15 +794,26 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y,
 // K = 96: 66 / 62, K = 40: 41.4 / 46.1; and where 128 fills one round of the CUs that 64 would need two for (S = 700, K = 64: 37.9 / 32.9).
 // DY = 512, S = 2048, K = 128: 502 / 451; S = 1000, K = 64: 153 / 165. DY = 1024 (two blocks per CU either way): S = 512, K = 64: 173 / 163;
 // S = 256, K = 32: 84 / 73, S = 512, K = 32: 134 / 140.
-static bool wide_tiles(int logDY, long S, int N, int K, long cus)
+static bool wide_tiles(int logDY, long S, int N, int K, int algo, long cus)
 {
     const long blocks = S * (N / 128), volume = (long)K * S;
     if (N % 128 != 0) return false;
+    if (algo == 8) return true;
     switch (logDY) {
     case 7: return (K >= 96 && blocks >= 2 * cus) || volume >= 160000 || (K >= 40 && blocks > 2 * cus && blocks <= 3 * cus);
     case 8: return volume >= 65536 && (K >= 64 || volume >= 160000);
     case 9: return (K >= 96 && blocks >= 2 * cus) || (K >= 40 && volume >= 80000);
     default: return K >= 64 ? blocks >= cus : blocks <= cus;
+    }
+}
+int tile_of_fused_1d_kernel(int kernel, int logDY, long S, int N, int K, int algo, long cus)
+{
+    switch (kernel) {
+    case kFused1dMfma512Tile32: return 32;
+    case kFused1dSplit: return SPLIT_NT;
+    case kFused1dCluster: return N;
+    case kFused1dWide: return wide_tiles(logDY, S, N, K, algo, cus) ? 128 : 64;
+    default: return 64;
     }
 }
 // Blocks of 64 output channels at DY = 256: registers and LDS for four per CU once there are more than three (S = 1000, K = N = 64:
@@ -826,7 +838,7 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
         if (logDY == 7 && K <= 8) return launch_fused_wave(S, N, K, x, W, y, alpha, stream, keep_y);
         return launch_fused_split(logDY, S, N, K, x, W, y, alpha, false, true, stream, keep_y);
     case kFused1dWide:
-        return launch_fused_split(logDY, S, N, K, x, W, y, alpha, wide_tiles(logDY, S, N, K, cus), dense_blocks(S, N, cus), stream, keep_y);
+        return launch_fused_split(logDY, S, N, K, x, W, y, alpha, wide_tiles(logDY, S, N, K, algo, cus), dense_blocks(S, N, cus), stream, keep_y);
     case kFused1dSplit: return keep_y ? launch_fused_split_k<true>(S, N, K, x, W, y, alpha, stream) : launch_fused_split_k<false>(S, N, K, x, W, y, alpha, stream);
     case kFused1dMfma512Tile32:
         return logDY == 8 ? launch_fused_mfma<8, 32>(S, N, K, x, W, y, alpha, stream, keep_y)
