@@ -118,6 +118,10 @@ def test_weights_with_a_period(bs, DX, DY, K, N):
     (258, 1024, 40, 64),             # DY = 1024: four passes per round, the last round with two
     (193, 1024, 8, 128),             # blocks of 128 channels, half a round
     (256, 1024, 72, 128),            # the same with a short last round
+    (512, 256, 24, 64),              # 1 and 2 MiB between channels: the waves of a block take every fourth output channel
+    (1024, 256, 72, 128),            # the same with blocks of 128 channels
+    (512, 512, 40, 192),
+    (512, 1024, 72, 64),             # 4 MiB: neighbouring channels again
 ])
 def test_fused_1d_edges(S, DY, K, N):
     """the fused 1D kernel with split products, chosen by size: every row of y written (y starts as NaN), the first, last and
@@ -181,6 +185,8 @@ def test_blocks_of_128_output_channels_as_middle_stage(bs, DX, DY, K, N, algo, a
     (1, 128, 8, 64), (9, 128, 40, 192), (400, 128, 56, 128),        # rounds of 32 channels: one of eight, a last one of eight, of 24
     (1, 256, 8, 64), (9, 256, 40, 192), (400, 256, 72, 128),        # S = 400: blocks of 128 output channels
     (3, 512, 24, 64), (400, 512, 40, 128), (2, 1024, 8, 64), (390, 1024, 24, 128),
+    (5, 512, 8, 192), (900, 1024, 8, 64),                           # eight channels: the SIMT kernel, both halves
+    (512, 256, 40, 64), (256, 512, 40, 128), (128, 1024, 24, 64),   # 1 MiB between channels: the waves of a block take every fourth one
 ])
 @pytest.mark.parametrize("beta", [0.0, -1 + 1j])
 def test_halves_of_the_layer(S, DY, K, N, beta):

@@ -21,8 +21,8 @@
 // Measured against the fp32 kernels it replaced (us, x and y from HBM): DY = 256, K = N = 128, S = 8192: 1135 -> 960;
 // K = N = 64, S = 4096: 247 -> 213; DY = 128, K = N = 64, S = 16384: 533 -> 447; K = N = 128, S = 8192: 735 -> 569; K = 40, N = 128,
 // S = 1000: 52 -> 41; DY = 512, K = N = 128, S = 2048: 652 -> 451; DY = 1024, K = N = 128, S = 1000: 601 -> 462. Halves against the SIMT kernel:
-// forward DY = 256, K = N = 64, S = 2048: 103 -> 77, K = N = 128: 341 -> 171; backward 112 -> 65, 298 -> 149; S = 64, K = N = 64: 22 -> 13 both. (Forward, DY = 1024,
-// K = 8, N = 64, S = 2048 is the one shape found slower: 47.8 -> 50.1.)
+// forward DY = 256, K = N = 64, S = 2048: 103 -> 77, K = N = 128: 341 -> 171; backward 112 -> 65, 298 -> 149; S = 64, K = N = 64: 22 -> 13 both; which
+// shapes stay with the SIMT kernel: launch_fused_fft_cgemm, launch_fused_cgemm_ifft.
 // Error against 64 bits: 2.4e-7 -> 2.0e-7 (K = 64), 3.2e-7 -> 2.7e-7 (K = 128), the same from the smallest normal floats to the
 // largest: operands that the split does not hold (bf16_split.h) are noticed - small spectra and weights as they are split, the rest in
 // the accumulators - and product_fp32() stands in. Noticing costs 0 - 3 %, 1.2 % on average (the most: DY = 128, S = 4096, K = N = 128: 282 -> 292).
@@ -84,14 +84,14 @@ TFNO_DEV void pair_first_pass(const cpx (&v)[16], const cpx* twrow, cpx (&gg)[16
 // a time as it has lane groups for, and takes its 16 NTW output channels from them four channels at a time. Several times as slow as
 // the loop that it stands in for. `region`: the exchange regions of the wave, free of other use.
 template <int LOGDY, int NTW, bool FWD>
-TFNO_DEV void product_fp32(long S, int K, long s, int nw, const float2* __restrict__ x, const float2* __restrict__ W, float2 alpha,
+TFNO_DEV void product_fp32(long S, int K, long s, int nw, int nstep, const float2* __restrict__ x, const float2* __restrict__ W, float2 alpha,
                            const cpx* twrow, const cpx* powers, cpx* region, float4_v (&re)[NTW][4], float4_v (&im)[NTW][4])
 {
     using G = GeoSplit<LOGDY, false, FWD>;
     constexpr int DY = 1 << LOGDY, L = G::L, CHANNELS = !FWD ? 4 : (G::PAIR ? 8 : 64 / L);
     const int lane = threadIdx.x & 63, group = lane / L, t = lane % L, kq = lane >> 4, col = lane & 15;
     cpx* exch = region + group * G::EXCH;
-    const float2* w = W + (long)(nw + col) * K;
+    const float2* w = W + (long)(nw + nstep * col) * K;
 #pragma unroll
     for (int i = 0; i < NTW; ++i)
 #pragma unroll
@@ -140,7 +140,7 @@ TFNO_DEV void product_fp32(long S, int K, long s, int nw, const float2* __restri
             }
 #pragma unroll
             for (int i = 0; i < NTW; ++i) {
-                const float2 wk = live ? cmul(w[k + c + (long)(16 * i) * K], alpha) : make_float2(0.f, 0.f);
+                const float2 wk = live ? cmul(w[k + c + (long)(16 * i * nstep) * K], alpha) : make_float2(0.f, 0.f);
 #pragma unroll
                 for (int a = 0; a < 4; ++a) mac_fp32(wk, b[a], re[i][a], im[i][a]);
             }
@@ -151,7 +151,7 @@ TFNO_DEV void product_fp32(long S, int K, long s, int nw, const float2* __restri
 template <int LOGDY, int NTW, bool ALIAS, int BLOCKS, bool KEEP, bool FWD = true, bool INV = true>
 __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S, int N, int K, const float2* __restrict__ x,
                                                                              const float2* __restrict__ W, float2* __restrict__ y,
-                                                                             float2 alpha, float2 beta)
+                                                                             float2 alpha, float2 beta, int wave_step)
 {
     using G = GeoSplit<LOGDY, ALIAS, FWD>;
     constexpr bool PAIR = G::PAIR, LONG = LOGDY >= 9;
@@ -165,7 +165,9 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
     long s;
     int ntile;
     decode_block_1d(S, N / (64 * NTW), DY, !KEEP, s, ntile);
-    const int nw = (ntile * 4 + wave) * (16 * NTW);             // first output channel of the wave
+    // output channels of the wave: nw, nw + nstep, ... (16 NTW of them)
+    const int nstep = INV && LOGDY >= 8 ? wave_step : 1;
+    const int nw = ntile * 64 * NTW + wave * (nstep == 1 ? 16 * NTW : 1);
     const long M = 64L * S;
     float2* exch = reinterpret_cast<float2*>(lds_split) + grp * G::EXCH;
     char* tile = lds_split + G::TILE_AT;
@@ -217,11 +219,11 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
         float2 wv[WSTEPS][NTW][4];
         auto load_w = [&](int step, float2 (&dst)[NTW][4], int offset) {
             const int k = 16 * step + 4 * kq;
-            const float2* p = W + (kc + (k < kn ? k : 0)) + (long)(nw + col) * K + offset;
+            const float2* p = W + (kc + (k < kn ? k : 0)) + (long)(nw + nstep * col) * K + offset;
 #pragma unroll
             for (int i = 0; i < NTW; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) dst[i][j] = p[(long)(16 * i) * K + j];
+                for (int j = 0; j < 4; ++j) dst[i][j] = p[(long)(16 * i * nstep) * K + j];
         };
 #pragma unroll
         for (int pass = 0; pass < KC / CP; ++pass) {
@@ -333,17 +335,17 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
         for (int a = 0; a < 4; ++a) { high[0] = larger(high[0], re[i][a]); high[1] = larger(high[1], im[i][a]); }
     if (__builtin_expect(low_weights, 0)) {                     // which of the two
         unsigned bits = ~0u;
-        const float2* w = W + (long)(nw + col) * K;
+        const float2* w = W + (long)(nw + nstep * col) * K;
 #pragma unroll 1
         for (int k = kq; k < K; k += 4)
 #pragma unroll
-            for (int i = 0; i < NTW; ++i) bits = lower(bits, cmul(w[k + (long)(16 * i) * K], alpha));
+            for (int i = 0; i < NTW; ++i) bits = lower(bits, cmul(w[k + (long)(16 * i * nstep) * K], alpha));
         low_weights = any_lane(bits < kSplitLow);
     }
     if (__builtin_expect(low_weights | any_lane((low_flags[lane & 3] != 0) | not_finite(high[0], high[1])), 0))
-        product_fp32<LOGDY, NTW, FWD>(S, K, s, nw, x, W, alpha, twrow, powers, reinterpret_cast<float2*>(lds_split) + wave * (64 * 17), re, im);
+        product_fp32<LOGDY, NTW, FWD>(S, K, s, nw, nstep, x, W, alpha, twrow, powers, reinterpret_cast<float2*>(lds_split) + wave * (64 * 17), re, im);
 
-    // D[row = 4 kq + q][col] of tile (i, a): output channel nw + 16 i + 4 kq + q, mode col + 16 a
+    // D[row = 4 kq + q][col] of tile (i, a): output channel nw + nstep (16 i + 4 kq + q), mode col + 16 a
 #pragma unroll
     for (int i = 0; i < NTW; ++i) {
         if constexpr (!INV) {
@@ -359,6 +361,7 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
         } else if constexpr (LONG) {
             // one output channel per L-lane group: the lanes that hold it store its 64 modes into the group's region
             constexpr int AT_ONCE = 64 / L;                     // channels per wave at a time
+            float2* first_row = y + ((long)(nw + nstep * 4 * (lane / L)) * S + s) * DY + t;
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll 1
@@ -372,18 +375,17 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
                     cpx e[16], yv[16];
                     wide_backward_inputs_of_stored<L, true>(powers, exch, t, e);
                     inv_pass2_lds(e, twrow, yv);
-                    const int n = nw + 16 * i + 4 * (AT_ONCE * h + lane / L) + q;
-                    store_row16<L, KEEP>(y + ((long)n * S + s) * DY + t, yv);
+                    store_row16<L, KEEP>(first_row + (long)(nstep * (16 * i + 4 * AT_ONCE * h + q)) * S * DY, yv);
                 }
         } else if constexpr (LOGDY == 8) {
-            float2* dst = y + ((long)(nw + 16 * i + 4 * kq) * S + s) * DY + t;
+            float2* dst = y + ((long)(nw + nstep * (16 * i + 4 * kq)) * S + s) * DY + t;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 cpx c[4], yv[16];
 #pragma unroll
                 for (int a = 0; a < 4; ++a) c[a] = make_float2(re[i][a][q], im[i][a][q]);
                 group_backward_lds<8>(c, twrow, exch, t, yv);
-                store_row16<16, KEEP>(dst + (long)q * S * DY, yv);
+                store_row16<16, KEEP>(dst + (long)(q * nstep) * S * DY, yv);
             }
         } else {
             float2* dst = y + ((long)(nw + 16 * i + 4 * kq) * S + s) * DY + t;
@@ -412,9 +414,16 @@ static hipError_t launch_split_k(long S, int N, int K, const float2* x, const fl
     using G = GeoSplit<LOGDY, ALIAS, FWD>;
     const long blocks = S * (N / (64 * NTW));
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+    // Channel strides of 1 or 2 MiB put all output channels of a signal set on the same memory channels: the four waves of a block then
+    // take every fourth channel each, so that the rows that are stored at one time lie one stride apart and not 16 (DY = 512, S = 256,
+    // N = 64, second half, K = 64: 23.5 -> 18.1 us, K = 8: 20.0 -> 15.2; whole layer DY = 256, S = 512, K = 64, N = 128: 44.9 -> 38.0).
+    // At other strides neighbouring rows are better kept in one wave (S = 300: 3 % slower; 4 MiB, DY = 1024, S = 512: 5 - 13 %), and so
+    // with 128 channels per block at DY = 512 (S = 512, K = N = 128: 101 / 112).
+    const long stride = S * (8L << LOGDY);
+    const bool step = (stride == (1L << 20) || stride == (2L << 20)) && !(LOGDY == 9 && NTW == 2);
     static_assert(G::LDS_BYTES <= 64 * 1024, "no attribute call needed below 64 KiB of dynamic LDS");
     hipLaunchKernelGGL((fused_fft_split_ifft_kernel<LOGDY, NTW, ALIAS, BLOCKS, KEEP, FWD, INV>), dim3((unsigned)blocks), dim3(256),
-                       G::LDS_BYTES, stream, (int)S, N, K, x, W, y, alpha, beta);
+                       G::LDS_BYTES, stream, (int)S, N, K, x, W, y, alpha, beta, step ? 4 : 1);
     return hipGetLastError();
 }
 // keep_y: plain instead of streaming stores of y, for a consumer that reads it at once (a template parameter of the kernels)
