@@ -17,10 +17,14 @@
 
 namespace tfno {
 
-template <int LOGDY, bool KEEP = false>
+// FUSE_FWD: the A operand is produced by forward transforms of x; otherwise it is read from the column-major matrix A[m + k M]
+//           (second half of the layer);
+// FUSE_INV: the product goes straight into zero-padded backward transforms; otherwise it is stored as
+//           C[m + n M] = alpha A W + beta C (first half).
+template <int LOGDY, bool FUSE_FWD, bool FUSE_INV, bool KEEP>
 __global__ __launch_bounds__(256) void fused_fft_cgemm_ifft_kernel(int S, int N, int K, const float2* __restrict__ x,
                                                                    const float2* __restrict__ W, float2* __restrict__ y,
-                                                                   float2 alpha)
+                                                                   float2 alpha, float2 beta)
 {
     using G = Geo1D<LOGDY>;
     constexpr int DY = G::DY, L = G::L, GROUPS = G::GROUPS, MM = G::MM, NN = G::NN;
@@ -35,6 +39,7 @@ __global__ __launch_bounds__(256) void fused_fft_cgemm_ifft_kernel(int S, int N,
     int ntile;
     decode_block_1d(S, N / 64, 1 << LOGDY, !KEEP, s, ntile);
     const int n0 = ntile * 64;
+    const long M = 64L * S;
     // signals of 128 samples are transformed in pairs by 16-lane groups (128-byte accesses): lane t16 of pair g/2 holds
     // samples t16 + 16 i of both signals, and ends up with the modes an 8-lane group would give lane (g, t)
     constexpr bool PAIR = LOGDY == 7;
@@ -51,27 +56,36 @@ __global__ __launch_bounds__(256) void fused_fft_cgemm_ifft_kernel(int S, int N,
         for (int b = 0; b < NN; ++b) acc[a][b] = make_float2(0.f, 0.f);
 
     for (int kc = 0; kc < K; kc += GROUPS) {
-        const int k = kc + g;
-        cpx out[MM];
-        if (k < K) {
-            cpx v[16];
-            if constexpr (PAIR) {
-                const float2* src = x + ((long)(kc + gpair) * S + s) * DY + t16;
+        if constexpr (FUSE_FWD) {
+            const int k = kc + g;
+            cpx out[MM];
+            if (k < K) {
+                cpx v[16];
+                if constexpr (PAIR) {
+                    const float2* src = x + ((long)(kc + gpair) * S + s) * DY + t16;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) { v[i] = src[16 * i]; v[8 + i] = src[(long)S * DY + 16 * i]; }
-                pair128_forward(v, tw, exch, t16, out);
+                    for (int i = 0; i < 8; ++i) { v[i] = src[16 * i]; v[8 + i] = src[(long)S * DY + 16 * i]; }
+                    pair128_forward(v, tw, exch, t16, out);
+                } else {
+                    const float2* src = x + ((long)k * S + s) * DY + t;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) v[i] = src[L * i];
+                    group_forward<LOGDY>(v, tw, exch, t, out);
+                }
             } else {
-                const float2* src = x + ((long)k * S + s) * DY + t;
 #pragma unroll
-                for (int i = 0; i < 16; ++i) v[i] = src[L * i];
-                group_forward<LOGDY>(v, tw, exch, t, out);
+                for (int a = 0; a < MM; ++a) out[a] = make_float2(0.f, 0.f);
             }
+#pragma unroll
+            for (int a = 0; a < MM; ++a) sA[g * G::SA_PITCH + (PAIR ? t + L * a : forward_mode_of_lane<LOGDY>(t, a))] = out[a];
         } else {
+            // A tile of the chunk: 64 contiguous rows (this block's signal) of GROUPS columns
 #pragma unroll
-            for (int a = 0; a < MM; ++a) out[a] = make_float2(0.f, 0.f);
+            for (int j = 0; j < (GROUPS * 64) / 256; ++j) {
+                const int mloc = (tid + 256 * j) % 64, kk = (tid + 256 * j) / 64;
+                sA[kk * G::SA_PITCH + mloc] = (kc + kk < K) ? x[s * 64 + mloc + (long)(kc + kk) * M] : make_float2(0.f, 0.f);
+            }
         }
-#pragma unroll
-        for (int a = 0; a < MM; ++a) sA[g * G::SA_PITCH + (PAIR ? t + L * a : forward_mode_of_lane<LOGDY>(t, a))] = out[a];
         // W chunk: GROUPS x 64 elements, consecutive threads read consecutive k (contiguous in memory)
 #pragma unroll
         for (int j = 0; j < (GROUPS * 64) / 256; ++j) {
@@ -100,17 +114,27 @@ __global__ __launch_bounds__(256) void fused_fft_cgemm_ifft_kernel(int S, int N,
 #pragma unroll
     for (int j = 0; j < NN; ++j) {
         const int n = n0 + g + GROUPS * j;
-        cpx c[MM], yv[16];
+        if constexpr (FUSE_INV) {
+            cpx c[MM], yv[16];
 #pragma unroll
-        for (int i = 0; i < MM; ++i) c[i] = cmul(acc[i][j], alpha);
-        if constexpr (PAIR) {
-            pair128_backward(c, tw, exch, t16, yv);
-            float2* dst = y + ((long)(n0 + gpair + GROUPS * j) * S + s) * DY + t16;
-            store_pair16<KEEP>(dst, (long)S * DY, yv);
+            for (int i = 0; i < MM; ++i) c[i] = cmul(acc[i][j], alpha);
+            if constexpr (PAIR) {
+                pair128_backward(c, tw, exch, t16, yv);
+                float2* dst = y + ((long)(n0 + gpair + GROUPS * j) * S + s) * DY + t16;
+                store_pair16<KEEP>(dst, (long)S * DY, yv);
+            } else {
+                group_backward<LOGDY>(c, tw, exch, t, yv);
+                float2* dst = y + ((long)n * S + s) * DY + t;
+                store_row16<L, KEEP>(dst, yv);
+            }
         } else {
-            group_backward<LOGDY>(c, tw, exch, t, yv);
-            float2* dst = y + ((long)n * S + s) * DY + t;
-            store_row16<L, KEEP>(dst, yv);
+            float2* dst = y + s * 64 + t + (long)n * M;          // C[m + n M], m = 64 s + t + L i
+#pragma unroll
+            for (int i = 0; i < MM; ++i) {
+                cpx r = cmul(acc[i][j], alpha);
+                if (beta.x != 0.f || beta.y != 0.f) r = cadd(r, cmul(dst[L * i], beta));
+                dst[L * i] = r;
+            }
         }
     }
 }
@@ -633,26 +657,30 @@ __global__ __launch_bounds__(256) void stride_DY_kernel(const float2* __restrict
 
 // keep_y: the output is read again at once (Y stage of the three-kernel 2D pipeline): plain instead of streaming stores,
 // as a template parameter of the kernels - a run-time branch around the stores cost the 1D layer up to 20 %
-template <int LOGDY, bool KEEP>
-static hipError_t launch_fused_1d_k(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, hipStream_t stream)
+template <int LOGDY, bool FUSE_FWD, bool FUSE_INV, bool KEEP>
+static hipError_t launch_fused_1d_k(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, float2 beta,
+                                    hipStream_t stream)
 {
     using G = Geo1D<LOGDY>;
     if (S * (N / 64) > 0x7fffffffL) return hipErrorInvalidValue;
     if constexpr (G::LDS_BYTES > 64 * 1024) {          // DY = 128: 32 channels per chunk, 70 KiB
         static std::atomic<unsigned long long> served;
-        if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(fused_fft_cgemm_ifft_kernel<LOGDY, KEEP>), G::LDS_BYTES, served);
+        if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(fused_fft_cgemm_ifft_kernel<LOGDY, FUSE_FWD, FUSE_INV, KEEP>),
+                                             G::LDS_BYTES, served);
             e != hipSuccess)
             return e;
     }
     dim3 grid((unsigned)(S * (N / 64)), 1, 1), block(256, 1, 1);
-    hipLaunchKernelGGL((fused_fft_cgemm_ifft_kernel<LOGDY, KEEP>), grid, block, G::LDS_BYTES, stream, (int)S, N, K, x, W, y, alpha);
+    hipLaunchKernelGGL((fused_fft_cgemm_ifft_kernel<LOGDY, FUSE_FWD, FUSE_INV, KEEP>), grid, block, G::LDS_BYTES, stream, (int)S, N, K, x, W,
+                       y, alpha, beta);
     return hipGetLastError();
 }
 template <int LOGDY>
 static hipError_t launch_fused_1d(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, hipStream_t stream, int keep_y)
 {
-    return keep_y ? launch_fused_1d_k<LOGDY, true>(S, N, K, x, W, y, alpha, stream)
-                  : launch_fused_1d_k<LOGDY, false>(S, N, K, x, W, y, alpha, stream);
+    const float2 beta = make_float2(0.f, 0.f);
+    return keep_y ? launch_fused_1d_k<LOGDY, true, true, true>(S, N, K, x, W, y, alpha, beta, stream)
+                  : launch_fused_1d_k<LOGDY, true, true, false>(S, N, K, x, W, y, alpha, beta, stream);
 }
 static hipError_t dispatch_fused_1d(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha,
                                     hipStream_t stream, int keep_y)
@@ -856,17 +884,30 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
     }
 }
 
+// The halves of the layer. Eight channels at lengths 512 / 1024: the SIMT kernel, where a round of 16 would be half padding (second
+// half, us, split / SIMT: DY = 512, S = 1 ... 128: 13.3 - 15.2 / 11.6 - 14.6, S = 1000: 58.5 / 54.8; DY = 1024, S = 1 ... 64: 22.6 / 19.5, but
+// with one block per CU, N = 64, S = 256: 24.5 / 26.8; with 16 channels they are 6 % apart at most. First half, with blocks of 64 output
+// channels: DY = 512, S = 4096: 54.2 / 50.8, DY = 1024, N = 64: S = 2048: 49.4 / 46.4, S = 700: 20.2 / 21.7). Otherwise the split kernel: halves, geometric mean of 1232 shapes against the SIMT kernel 0.66.
 hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C,
                                   float2 alpha, float2 beta, hipStream_t stream)
 {
     // blocks of 128 output channels from one and a half per CU (N = 128, K = 64, DY = 256: S = 700 42.6 -> 34.4 us, S = 256 19.0 -> 19.9)
-    const bool wide = N % 128 == 0 && 2 * S * (N / 128) >= 3L * cu_count();
+    const long cus = cu_count(), items = S * (N / 64);
+    const bool wide = N % 128 == 0 && 2 * S * (N / 128) >= 3 * cus;
+    if (K <= 8 && !wide) {
+        if (logDY == 9) return launch_fused_1d_k<9, true, false, false>(S, N, K, x, W, C, alpha, beta, stream);
+        if (logDY == 10 && N % 128 != 0 && items > 3 * cus && items <= 8 * cus) return launch_fused_1d_k<10, true, false, false>(S, N, K, x, W, C, alpha, beta, stream);
+    }
     return launch_split_forward(logDY, S, N, K, x, W, C, alpha, beta, wide, stream);
 }
 
 hipError_t launch_fused_cgemm_ifft(int logDY, long S, int N, int K, const float2* A, const float2* W, float2* y,
                                    float2 alpha, hipStream_t stream)
 {
+    const float2 beta = make_float2(0.f, 0.f);
+    const long cus = cu_count(), items = S * (N / 64);
+    if (K <= 8 && logDY == 9) return launch_fused_1d_k<9, false, true, false>(S, N, K, A, W, y, alpha, beta, stream);
+    if (K <= 8 && logDY == 10 && (4 * items < 3 * cus || items > cus)) return launch_fused_1d_k<10, false, true, false>(S, N, K, A, W, y, alpha, beta, stream);
     return launch_split_backward(logDY, S, N, K, A, W, y, alpha, stream);
 }
 
