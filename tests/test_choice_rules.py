@@ -101,3 +101,16 @@ def test_output_channels_per_block(algo_1d):
                 assert tf.query_1d_tile(DY, S, 64, K, CUS) == 64 and tf.query_1d_tile(DY, S, 192, K, CUS) == 64
                 algo_1d(3)
                 assert tf.query_1d_tile(DY, S, 128, K, CUS) == 64
+
+
+def test_1d_kernels_where_the_last_round_or_the_last_blocks_are_nearly_empty():
+    assert tf.query_1d_kernel(128, 256, 64, 16, CUS) == 8           # one block of 64 output channels per CU
+    assert tf.query_1d_kernel(128, 128, 128, 40, CUS) == 2          # eight of 32 channels in the last round
+    assert tf.query_1d_kernel(128, 128, 128, 64, CUS) == 3
+    assert tf.query_1d_kernel(1024, 600, 64, 40, CUS) == 1          # two to three blocks per CU, of which two fit at a time
+    assert tf.query_1d_kernel(1024, 512, 64, 40, CUS) == 3
+    assert tf.query_1d_kernel(1024, 1000, 64, 40, CUS) == 3
+    assert tf.query_1d_kernel(1024, 512, 192, 48, CUS) == 1
+    assert tf.query_1d_kernel(1024, 512, 192, 64, CUS) == 3
+    assert tf.query_1d_tile(256, 400, 128, 32, CUS) == 128          # 800 blocks of 64 channels, 768 at a time
+    assert tf.query_1d_tile(256, 512, 128, 32, CUS) == 64

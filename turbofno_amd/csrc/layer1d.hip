@@ -760,12 +760,17 @@ static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const
 //    every K, even K = 8 where most of a chunk is padding;
 //  * about one block of 64 output channels per CU and more, lengths 128 / 256: the split kernel (layer1d_split.hip). DY = 128 with
 //    32 channels or more from three quarters of the CUs on (N = 64: S = 200, K = 64: 13.8 / 12.2, S = 128: 10.9 / 11.8; N = 128:
-//    S = 100, K = 64: 13.5 / 12.1), DY = 256 from seven eighths on (N = 64: S = 256, K = 32: 14.7 / 13.2, S = 128, K = 64: 13.5 / 16.9),
+//    S = 100, K = 64: 13.5 / 12.1), unless every CU has a block, N = 128 and less than half of the last round of 32 channels is used (S = 128,
+//    K = 40: 10.9 / 11.5, K = 64: 13.2 / 13.1; S = 120, K = 40: 10.8 / 10.2); with 16 channels or more and one block per CU (N = 64, S = 256, K = 16: 8.9 / 7.7); DY = 256 from seven eighths on (N = 64: S = 256, K = 32: 14.7 / 13.2, S = 128, K = 64: 13.5 / 16.9),
 //    with N = 128 from three quarters on (S = 128, K = 64: 19.1 / 17.9; S = 64: 14.0 / 16.9);
 //  * lengths 512 / 1024, more than one block per CU: the split kernel from the number of channels on where it is ahead of the SIMT
 //    kernel, which has less to do per channel (DY = 512, S = 2048, N = 64: K = 24 127 / 120, K = 40 185 / 170, K = 128 358 / 305; S = 512:
 //    K = 16 38 / 42, K = 40 52 / 51; N = 128, S = 1000: K = 32 144 / 123, K = 128 327 / 244; DY = 1024, N = 64: S = 2048, K = 32 325 / 318, S = 512,
-//    K = 16 68 / 68; N = 128, S = 1000: K = 32 246 / 257, K = 64 389 / 349). On small grids the 512-thread kernel (S = 128, K = 64, DY = 512:
+//    K = 16 68 / 68; N = 128, S = 1000: K = 32 246 / 257, K = 64 389 / 349). DY = 1024 with N no multiple of 128: the split kernel fits two
+//    blocks on a CU, the SIMT kernel three, so below 64 channels the latter is ahead where rounds of two per CU would be at most three
+//    quarters full (N = 64: S = 600: K = 32 98 / 102, K = 40 107 / 114, K = 64 159 / 143; S = 512, K = 40: 88 / 80; N = 192, K = 40: S = 200:
+//    104 / 113, S = 300: 147 / 139) and on large grids of three blocks or more per signal set (N = 192, S = 600: K = 40 242 / 259,
+//    K = 64 341 / 319). On small grids the 512-thread kernel (S = 128, K = 64, DY = 512:
 //    25.9 / 28.9).
 int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y, long cus, bool exchange_attached)
 {
@@ -775,10 +780,10 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y,
     if (algo == 5 && !long_signal && built) return kFused1dDense;
     if (algo == 0 && !long_signal && built) {
         const long blocks = N % 128 == 0 ? S * (N / 128) : items;
+        if (logDY == 7 && N % 128 != 0 && K >= 16 && blocks >= cus && blocks <= (K >= 128 ? 4 : 2) * cus) return kFused1dWide;
         if (blocks > cus) {
             if (N % 128 == 0 && K >= 16) return kFused1dWide;           // 128 or 64 output channels per block: wide_tiles()
             // blocks of 64 output channels, a few per CU
-            if (logDY == 7 && N % 128 != 0 && K >= 16 && blocks <= (K >= 128 ? 4 : 2) * cus) return kFused1dWide;
             if (logDY == 8 && N % 128 != 0 && K >= 128 && blocks <= 4 * cus) return kFused1dWide;
         }
         // DY = 128: several items per SIMD
@@ -794,12 +799,15 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y,
     if (algo == 8) algo = 0;
     // not quite one block per CU
     if (algo == 0 && logDY == 7 && K >= 16 && N % 128 == 0 && 2 * items >= 3 * cus && items <= 2 * cus) return kFused1dWide;
-    if (algo == 0 && logDY == 7 && K >= 32 && 4 * items >= 3 * cus && items <= cus) return kFused1dMfma256;
+    const bool short_round = N % 128 == 0 && K % 32 > 0 && K % 32 < 16 && items == cus;
+    if (algo == 0 && logDY == 7 && K >= 32 && !short_round && 4 * items >= 3 * cus && items <= cus) return kFused1dMfma256;
     if (algo == 0 && logDY == 8 && (N % 128 == 0 ? 4 * items >= 3 * cus : 8 * items >= 7 * cus) && items <= cus) return kFused1dMfma256;
     // lengths 512 / 1024, more than one block per CU
     if (algo == 0 && long_signal && built && items > cus) {
         if (N % 128 == 0 && K >= (logDY == 9 ? 32 : 64)) return kFused1dWide;
-        if (N % 128 != 0 && K >= (logDY == 9 ? 40 : 32)) return kFused1dMfma256;
+        const long rounds = (items + 2 * cus - 1) / (2 * cus);
+        const bool simt_fits_better = logDY == 10 && K < 64 && rounds > 1 && (2 * items <= 3 * rounds * cus || (N > 64 && items > 5 * cus));
+        if (N % 128 != 0 && K >= (logDY == 9 ? 40 : 32) && !simt_fits_better) return kFused1dMfma256;
         const long blocks = N % 128 == 0 ? S * (N / 128) : 0;
         if (logDY == 10 && 4 * blocks >= 3 * cus && blocks <= cus) return kFused1dWide;
     }
@@ -818,7 +826,8 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y,
 // Split kernel, N a multiple of 128: blocks of 128 output channels transform every input once per 128 outputs, blocks of 64 twice as
 // often (the second time from L2), but they are finer and four fit a CU instead of three. 128 pays where the repeated transforms or reads
 // are many (us, 64 / 128): DY = 256, S = 8192, K = 128: 1180 / 960; S = 4096, K = 40: 336 / 296, K = 32: 218 / 222; S = 1000, K = 96: 94 / 89,
-// K = 64: 77 / 78; S = 333, K = 128: 46.6 / 50.9. DY = 128, S = 8192, K = 128: 654 / 569; S = 3000, K = 64: 138 / 123, K = 32: 92 / 101; S = 1000,
+// K = 64: 77 / 78; S = 333, K = 128: 46.6 / 50.9; just above three blocks of 64 per CU, which are two rounds of them (S = 400: K = 32: 31.8 / 28.4,
+// K = 128: 58.5 / 50.7; S = 448: 30.2 / 29.9, 59.8 / 54.1). DY = 128, S = 8192, K = 128: 654 / 569; S = 3000, K = 64: 138 / 123, K = 32: 92 / 101; S = 1000,
 // K = 96: 66 / 62, K = 40: 41.4 / 46.1; and where 128 fills one round of the CUs that 64 would need two for (S = 700, K = 64: 37.9 / 32.9).
 // DY = 512, S = 2048, K = 128: 502 / 451; S = 1000, K = 64: 153 / 165. DY = 1024 (two blocks per CU either way): S = 512, K = 64: 173 / 163;
 // S = 256, K = 32: 84 / 73, S = 512, K = 32: 134 / 140.
@@ -829,7 +838,7 @@ static bool wide_tiles(int logDY, long S, int N, int K, int algo, long cus)
     if (algo == 8) return true;
     switch (logDY) {
     case 7: return (K >= 96 && blocks >= 2 * cus) || volume >= 160000 || (K >= 40 && blocks > 2 * cus && blocks <= 3 * cus);
-    case 8: return volume >= 65536 && (K >= 64 || volume >= 160000);
+    case 8: return (volume >= 65536 && (K >= 64 || volume >= 160000)) || (K >= 16 && 2 * blocks > 3 * cus && 4 * blocks <= 7 * cus);
     case 9: return (K >= 96 && blocks >= 2 * cus) || (K >= 40 && volume >= 80000);
     default: return K >= 64 ? blocks >= cus : blocks <= cus;
     }
