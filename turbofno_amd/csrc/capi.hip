@@ -159,7 +159,7 @@ int turbofno_query_1d_kernel(int logDY, long M, int N, int K, int compute_units,
 {
     if (check_gemm_dims(M, N, K) || !length_built(logDY)) return 0;
     const long cus = compute_units > 0 ? compute_units : tfno::cu_count();
-    return tfno::pick_fused_1d_kernel(logDY, M / 64, N, K, algo_1d(), false, cus, exchange_attached != 0);
+    return tfno::pick_fused_1d_kernel(logDY, M / 64, N, K, algo_1d(), cus, exchange_attached != 0);
 }
 
 int turbofno_query_1d_tile(int logDY, long M, int N, int K, int compute_units, int exchange_attached)

@@ -100,9 +100,9 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
 // The kernel that call runs (the selector values 1 ... 8), from the sizes alone.
 enum {
     kFused1dSimt = 1, kFused1dMfma512 = 2, kFused1dMfma256 = 3, kFused1dMfma512Tile32 = 4, kFused1dDense = 5,
-    kFused1dSplit = 6, kFused1dCluster = 7, kFused1dWide = 8
+    kFused1dSplitK = 6, kFused1dCluster = 7, kFused1dWide = 8
 };
-int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y, long cus, bool exchange_attached);
+int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, long cus, bool exchange_attached);
 
 // Cluster variant of the fused 1D layer (layer1d_cluster.hip): cluster size for a problem on `cus` compute units (0 = not
 // applicable), the launch (hipErrorNotReady when no exchange buffer is attached to the stream), the bound of its

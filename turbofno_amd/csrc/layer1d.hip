@@ -719,7 +719,7 @@ static hipError_t launch_fused_mfma(long S, int N, int K, const float2* x, const
 
 // keep_y as for the other kernels: as the middle stage of one 256 x 256 image, K = 64, N = 128, the layer takes 37.1 us, 40.6 with streaming stores
 template <bool KEEP>
-static hipError_t launch_fused_split_k(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, hipStream_t stream)
+static hipError_t launch_fused_split_channels(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, hipStream_t stream)
 {
     static std::atomic<unsigned long long> served;
     if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(fused_fft_mfma_ifft_split_kernel<KEEP>), SPLIT_LDS, served);
@@ -751,6 +751,8 @@ static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const
 // length 128 one wavefront per (signal set, output tile), 6 = matrix cores, the eight waves of a block split the K channels of one
 // item (DY = 256), 7 = matrix cores, a cluster of blocks splits the K channels of one signal set (DY = 256, N = 64 / 128, small
 // grids), 8 = as 3 with 128 output channels per block where N allows
+// The same rule holds where y is read again at once (middle stage of a 2D layer): the lines were drawn with x and y streamed, and of
+// 3166 2D layers in three stages, lengths 128 to 1024, none lost against a rule that treated that case apart.
 // The return value uses the same numbers (1 ... 8); chosen by size, 8 stands for blocks of 64 or of 128 output channels
 // (tile_of_fused_1d_kernel). A selector value that a kernel is not built for falls back to the
 // choice by size.
@@ -772,7 +774,7 @@ static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const
 //    104 / 113, S = 300: 147 / 139) and on large grids of three blocks or more per signal set (N = 192, S = 600: K = 40 242 / 259,
 //    K = 64 341 / 319). On small grids the 512-thread kernel (S = 128, K = 64, DY = 512:
 //    25.9 / 28.9).
-int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y, long cus, bool exchange_attached)
+int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, long cus, bool exchange_attached)
 {
     const bool built = logDY >= 7 && logDY <= 10;
     const bool long_signal = logDY >= 9;            // 512 / 1024
@@ -815,7 +817,7 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y,
     if (pick == 0) pick = (built && items <= cus) ? 2 : (long_signal ? 1 : 3);
     // small grids, 64 channels or more: eight waves split the K channels of one item (10-16 % ahead of the kernel that
     // shares the spectra through LDS; level at K = 32)
-    if (logDY == 8 && (algo == 6 || (algo == 0 && K >= 64 && S * (N / SPLIT_NT) <= cus))) return kFused1dSplit;
+    if (logDY == 8 && (algo == 6 || (algo == 0 && K >= 64 && S * (N / SPLIT_NT) <= cus))) return kFused1dSplitK;
     // few blocks: tiles of 32 output channels put twice as many CUs to work (each block still transforms all K inputs)
     if (pick == 2 && (logDY == 7 || logDY == 8) && (algo == 4 || (algo == 0 && S * (N / 32) <= cus))) return kFused1dMfma512Tile32;
     if (pick == 2 && built) return kFused1dMfma512;
@@ -823,7 +825,7 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y,
     return kFused1dSimt;
 }
 
-// Split kernel, N a multiple of 128: blocks of 128 output channels transform every input once per 128 outputs, blocks of 64 twice as
+// Split kernel (layer1d_split.hip), N a multiple of 128: blocks of 128 output channels transform every input once per 128 outputs, blocks of 64 twice as
 // often (the second time from L2), but they are finer and four fit a CU instead of three. 128 pays where the repeated transforms or reads
 // are many (us, 64 / 128): DY = 256, S = 8192, K = 128: 1180 / 960; S = 4096, K = 40: 336 / 296, K = 32: 218 / 222; S = 1000, K = 96: 94 / 89,
 // K = 64: 77 / 78; S = 333, K = 128: 46.6 / 50.9; just above three blocks of 64 per CU, which are two rounds of them (S = 400: K = 32: 31.8 / 28.4,
@@ -833,13 +835,13 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, bool keep_y,
 // S = 256, K = 32: 84 / 73, S = 512, K = 32: 134 / 140.
 static bool wide_tiles(int logDY, long S, int N, int K, int algo, long cus)
 {
-    const long blocks = S * (N / 128), volume = (long)K * S;
+    const long blocks = S * (N / 128), volume = (long)K * S / cus;       // forward transforms per CU
     if (N % 128 != 0) return false;
     if (algo == 8) return true;
     switch (logDY) {
-    case 7: return (K >= 96 && blocks >= 2 * cus) || volume >= 160000 || (K >= 40 && blocks > 2 * cus && blocks <= 3 * cus);
-    case 8: return (volume >= 65536 && (K >= 64 || volume >= 160000)) || (K >= 16 && 2 * blocks > 3 * cus && 4 * blocks <= 7 * cus);
-    case 9: return (K >= 96 && blocks >= 2 * cus) || (K >= 40 && volume >= 80000);
+    case 7: return (K >= 96 && blocks >= 2 * cus) || volume >= 625 || (K >= 40 && blocks > 2 * cus && blocks <= 3 * cus);
+    case 8: return (volume >= 256 && (K >= 64 || volume >= 625)) || (K >= 16 && 2 * blocks > 3 * cus && 4 * blocks <= 7 * cus);
+    case 9: return (K >= 96 && blocks >= 2 * cus) || (K >= 40 && volume >= 312);
     default: return K >= 64 ? blocks >= cus : blocks <= cus;
     }
 }
@@ -847,7 +849,7 @@ int tile_of_fused_1d_kernel(int kernel, int logDY, long S, int N, int K, int alg
 {
     switch (kernel) {
     case kFused1dMfma512Tile32: return 32;
-    case kFused1dSplit: return SPLIT_NT;
+    case kFused1dSplitK: return SPLIT_NT;
     case kFused1dCluster: return N;
     case kFused1dWide: return wide_tiles(logDY, S, N, K, algo, cus) ? 128 : 64;
     default: return 64;
@@ -864,11 +866,11 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
     // caches instead of streaming it past them; the clustered kernel ignores it
     const int keep_y = y_is_reread ? 1 : 0;
     const long cus = cu_count();
-    int kernel = pick_fused_1d_kernel(logDY, S, N, K, algo, y_is_reread, cus, exchange_attached(stream));
+    int kernel = pick_fused_1d_kernel(logDY, S, N, K, algo, cus, exchange_attached(stream));
     if (kernel == kFused1dCluster) {
         const hipError_t e = launch_fused_cluster(S, N, K, cluster_size_1d(logDY, S, N, K, cus), x, W, y, alpha, stream);
         if (e != hipErrorNotReady) return e;
-        kernel = pick_fused_1d_kernel(logDY, S, N, K, algo, y_is_reread, cus, false);    // detached in between
+        kernel = pick_fused_1d_kernel(logDY, S, N, K, algo, cus, false);    // detached in between
     }
     switch (kernel) {
     case kFused1dDense:
@@ -876,7 +878,7 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
         return launch_fused_split(logDY, S, N, K, x, W, y, alpha, false, true, stream, keep_y);
     case kFused1dWide:
         return launch_fused_split(logDY, S, N, K, x, W, y, alpha, wide_tiles(logDY, S, N, K, algo, cus), dense_blocks(S, N, cus), stream, keep_y);
-    case kFused1dSplit: return keep_y ? launch_fused_split_k<true>(S, N, K, x, W, y, alpha, stream) : launch_fused_split_k<false>(S, N, K, x, W, y, alpha, stream);
+    case kFused1dSplitK: return keep_y ? launch_fused_split_channels<true>(S, N, K, x, W, y, alpha, stream) : launch_fused_split_channels<false>(S, N, K, x, W, y, alpha, stream);
     case kFused1dMfma512Tile32:
         return logDY == 8 ? launch_fused_mfma<8, 32>(S, N, K, x, W, y, alpha, stream, keep_y)
                           : launch_fused_mfma<7, 32>(S, N, K, x, W, y, alpha, stream, keep_y);
