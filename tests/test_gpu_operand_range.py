@@ -18,7 +18,8 @@ def _dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
-# fp32 sums of 2 K products each: (2 K)^0.5 roundings of 2^-24 as a random walk, doubled
+# fp32 sums of 2 K products each: (2 K)^0.5 roundings of 2^-24 as a random walk, doubled (single rows and columns: not the cap that the
+# tests of whole results have)
 def _bound(K):
     return 2.0 * (2 * K) ** 0.5 * 2.0 ** -24
 
