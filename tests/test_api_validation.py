@@ -94,3 +94,15 @@ def test_noalloc_refuses_oversized_problem_without_gpu():
     # bs=32, 256 x 256, K=N=64: 128 MiB of intermediates, the static scratch holds 64 MiB; refused before any GPU call
     rc = L.turbofno_layer_2d_noalloc(32, 256, 256, 64, 64, 1, 1, 1, 1.0, 0.0, 2, None)
     assert rc == 3 and b"static scratch" in L.turbofno_last_error_string()
+
+
+def test_stream_handle_without_the_raw_query(monkeypatch):
+    """a torch that lacks the private query: the handle comes from the public stream object"""
+    import types
+    from turbofno_amd import api
+    monkeypatch.setattr(api, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=1234))
+    assert api._stream() == 1234
+    monkeypatch.setattr(api, "_raw_stream", lambda device: 5678 + device)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    assert api._stream() == 5678

@@ -180,6 +180,19 @@ def test_weights_with_a_period(bs, DX, DY, K, N):
     assert rel_l2(y.cpu().numpy(), ref) < 1e-6 and max_rel(y.cpu().numpy(), ref) < 1e-5
 
 
+@pytest.mark.parametrize("M", [64, 4096, 65536 + 64])
+def test_mode_gemm_in_place(M):
+    """64 output channels over the 64 input channels"""
+    print("split cgemm in place", M, flush=True)
+    rng = np.random.default_rng(M)
+    A, W = _complex(rng, 64, M), _complex(rng, 64, 64)
+    C = _dev(A)
+    for _ in range(3):
+        C.copy_(torch.from_numpy(A))
+        tf.cgemm(M, 64, 64, C, _dev(W), C, 1.0, 0.0)
+        assert rel_l2(C.cpu().numpy(), oracle.cgemm(A, W, 1.0)) < _bound(64)
+
+
 # of the shapes below, those with 128 output channels per block
 WIDE = {(512, 256, 128, 128), (912, 256, 72, 128), (513, 128, 104, 128), (1100, 128, 96, 256), (520, 512, 104, 128), (193, 1024, 8, 128),
         (256, 1024, 72, 128), (1024, 256, 72, 128)}

@@ -885,7 +885,8 @@ hipError_t launch_cgemm_modes(const float2* A, const float2* W, float2* C, long 
     using Columns256 = std::integral_constant<int, 1024>;
     using Tiles1 = std::integral_constant<int, 1>;
     using Tiles2 = std::integral_constant<int, 2>;
-    const long strips = (Mtot + 127) / 128;
+    // (64 output channels in place of the 64 input channels: one block has to hold all of a strip's outputs)
+    const long strips = A == C ? cus : (Mtot + 127) / 128;
     if (strips * (N / 16) <= cus) return launch_split(Tiles1{}, Columns128{}, 6, 2);
     if (strips * (N / 32) <= cus) return launch_split(Tiles2{}, Columns128{}, 6, 2);
     if (2 * blocks <= cus || (N == 64 && K > 32 && blocks >= cus && blocks < 2 * cus)) return launch_split(Tiles4{}, Columns128{}, 6, 2);
