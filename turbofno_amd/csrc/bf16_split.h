@@ -32,8 +32,8 @@ __device__ __forceinline__ void split_bf16_pair(float a, float b, unsigned& h, u
 // Which operands the split holds: from 2^-110 (7.7e-34) on and up to 2^-9 below the largest float, and zero. Below 2^-110 the third part would need bits under the smallest bf16 number, 2^-133; infinities and
 // magnitudes within 2^-9 of the largest float leave a NaN in the remainder x - h. A wave whose operands include such values forms its
 // product again, with fp32 instructions, so that the results have fp32 precision and fp32 infinities over the whole range of floats:
-//   * small magnitudes are found in the operands, zeros, which are exact, aside (lower(): three instructions per two values; or one,
-//     smaller(), where zeros can be told apart later);
+//   * small magnitudes are found in the operands, zeros, which are exact, aside: lower(), three instructions per two values, or where a
+//     branch costs nothing below_split_range(), one per two values as long as there are no zeros;
 //   * the others are found in the accumulators: each leaves a NaN or an infinity in every sum it takes part in.
 constexpr float kSplitSmallest = 0x1p-110f;
 __device__ __forceinline__ float smaller(float low, float a, float b)

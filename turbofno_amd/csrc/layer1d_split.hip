@@ -209,7 +209,7 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
         return tile + (c >> 4) * G::STEP_BYTES + a * 3072 + ((c >> 2) & 3) * 256 + column * 16 + (c & 3) * 4;
     };
 
-    bool low = false, low_weights = false;                      // of the wave: spectra too small for the split / such weights or zeros
+    bool low = false, low_weights = false;                      // spectra / weights of the wave that are too small for the split
     for (int kc = 0; kc < K; kc += KC) {
         const int kn = (K - kc) < KC ? (K - kc) : KC;           // a multiple of 8 (caller contract)
         constexpr int MODES = !FWD ? 4 : (PAIR ? 8 : 64 / L), WSTEPS = PAIR && NTW == 1 && BLOCKS < 4 ? 2 : 1;
@@ -310,10 +310,10 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
                 float2 (&w4)[4] = wv[WSTEPS == 2 ? step : 0][i];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) w4[j] = cmul(w4[j], alpha);
-                float smallest = 1.f;
+                unsigned bits = ~0u;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) smallest = smaller(smallest, w4[j]);
-                low_weights |= any_lane(smallest < kSplitSmallest);
+                for (int j = 0; j < 4; ++j) bits = lower(bits, w4[j]);
+                low_weights |= any_lane(bits < kSplitLow);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) split_weight_rows(w4[j], wre, wim, j);
                 if (WSTEPS == 1 && PAIR && step == 0 && 16 < kn && i == NTW - 1) load_w(1, wv[0], 0);
@@ -333,15 +333,6 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
     for (int i = 0; i < NTW; ++i)
 #pragma unroll
         for (int a = 0; a < 4; ++a) { high[0] = larger(high[0], re[i][a]); high[1] = larger(high[1], im[i][a]); }
-    if (__builtin_expect(low_weights, 0)) {                     // which of the two
-        unsigned bits = ~0u;
-        const float2* w = W + (long)(nw + nstep * col) * K;
-#pragma unroll 1
-        for (int k = kq; k < K; k += 4)
-#pragma unroll
-            for (int i = 0; i < NTW; ++i) bits = lower(bits, cmul(w[k + (long)(16 * i * nstep) * K], alpha));
-        low_weights = any_lane(bits < kSplitLow);
-    }
     if (__builtin_expect(low_weights | any_lane((low_flags[lane & 3] != 0) | not_finite(high[0], high[1])), 0))
         product_fp32<LOGDY, NTW, FWD>(S, K, s, nw, nstep, x, W, alpha, twrow, powers, reinterpret_cast<float2*>(lds_split) + wave * (64 * 17), re, im);
 
