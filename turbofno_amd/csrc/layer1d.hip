@@ -895,9 +895,10 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
     }
 }
 
-// The halves of the layer. Eight channels at lengths 512 / 1024: the SIMT kernel, where a round of 16 would be half padding (second
+// The halves of the layer. Few channels at lengths 512 / 1024: the SIMT kernel; with eight a round of 16 would be half padding (second
 // half, us, split / SIMT: DY = 512, S = 1 ... 128: 13.3 - 15.2 / 11.6 - 14.6, S = 1000: 58.5 / 54.8; DY = 1024, S = 1 ... 64: 22.6 / 19.5, but
-// with one block per CU, N = 64, S = 256: 24.5 / 26.8; with 16 channels they are 6 % apart at most. First half, with blocks of 64 output
+// with one block per CU, N = 64, S = 256: 24.5 / 26.8; with 16 channels only DY = 1024 on small grids: S = 1 ... 128: 23.3 - 24.7 /
+// 21.5 - 23.4. First half, with blocks of 64 output
 // channels: DY = 512, S = 4096: 54.2 / 50.8, DY = 1024, N = 64: S = 2048: 49.4 / 46.4, S = 700: 20.2 / 21.7). Otherwise the split kernel: halves, geometric mean of 1232 shapes against the SIMT kernel 0.66.
 hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C,
                                   float2 alpha, float2 beta, hipStream_t stream)
@@ -918,7 +919,7 @@ hipError_t launch_fused_cgemm_ifft(int logDY, long S, int N, int K, const float2
     const float2 beta = make_float2(0.f, 0.f);
     const long cus = cu_count(), items = S * (N / 64);
     if (K <= 8 && logDY == 9) return launch_fused_1d_k<9, false, true, false>(S, N, K, A, W, y, alpha, beta, stream);
-    if (K <= 8 && logDY == 10 && (4 * items < 3 * cus || items > cus)) return launch_fused_1d_k<10, false, true, false>(S, N, K, A, W, y, alpha, beta, stream);
+    if (logDY == 10 && (4 * items < 3 * cus ? K <= 16 : K <= 8 && items > cus)) return launch_fused_1d_k<10, false, true, false>(S, N, K, A, W, y, alpha, beta, stream);
     return launch_split_backward(logDY, S, N, K, A, W, y, alpha, stream);
 }
 
