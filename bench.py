@@ -258,7 +258,7 @@ def main():
         "metric": "fused FFT-CGEMM-iFFT ms/layer, 2D bs=%d 256x256 K=N=64" % bs,
         "value": round(ms, 4), "unit": "ms/layer", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": round(ms, 4), "higher_is_better": False, "scaling": "weak", "vs_baseline": None,
-        "dtype": "complex64 (fp32 arithmetic)", "data": "synthetic",
+        "dtype": "complex64 (fp32; matrix products from exact three-part bf16 splits of fp32 operands)", "data": "synthetic",
         "config": {"workload": "2D layer bs=%d 256x256 K=64 N=64, 64x64 modes, Gaussian random field input" % bs,
                    "algo": ("auto -> " if args.algo == 0 else "") + {1: "three-kernel", 2: "whole-image", 3: "three-kernel, rows first"}[algo]},
         "settle": {"ms": args.settle_ms, "steps": settle_steps},

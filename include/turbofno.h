@@ -20,6 +20,10 @@
  *     exp(-2 pi i jm/D), backward transforms exp(+2 pi i jm/D) and are UNNORMALISED.
  *   - Layouts: x[K][S][DY] (signal (k,s) at (k*S+s)*DY), W[k + n*K], y[N][S][DY]; in 2D
  *     x[K][bs][DX][DY], y[N][bs][DX][DY].
+ *   - Precision: operands, sums and results are fp32 over the whole range of floats, infinities and NaN included. Products of
+ *     most sizes are formed from bf16 parts of their operands on the matrix cores; where a spectrum or weight (times alpha) that is
+ *     not zero lies below 2^-110 or within 2^-9 of the largest float, is infinite or NaN, that part of the product is formed with
+ *     fp32 instructions instead, and takes two to three times as long.
  */
 #ifndef TURBOFNO_H
 #define TURBOFNO_H
@@ -109,7 +113,7 @@ int turbofno_layer_2d(int bs, int DX, int DY, int K, int N, const void* x, const
  * not care. Requires DX in {128, 256} and DY in {128, 256, 512, 1024} (the layer handles longer DX as interleaved
  * parts, which have no stand-alone meaning).
  *   turbofno_cgemm : C[m + n*M] = alpha * sum_k A[m + k*M] * B[k + n*K] + beta * C[m + n*M] (column major,
- *   lda = M, ldb = K, ldc = M) on the fp32 matrix cores. Replaces the reference's cgemm kernel
+ *   lda = M, ldb = K, ldc = M) on the matrix cores. Replaces the reference's cgemm kernel
  *   (fusion_variants/1D_A_exp_fft+cgemm+ifft/cgemm.cuh:4, launch 1D_A.../fused.cu:199), same argument order
  *   (M, N, K, A, B, C, alpha, beta). C is read only when beta != 0. Requires M % 64 == 0, M < 2^27,
  *   N % 64 == 0, K % 8 == 0.

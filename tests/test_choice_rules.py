@@ -2,8 +2,9 @@
 integer arithmetic when the number of compute units is passed in). A change of a rule that moves a configuration onto
 another kernel has to show up here, next to the GPU parity test that covers that kernel:
   1D kernels (numbering of turbofno_set_1d_algo): 1 SIMT, 2 / 3 matrix cores with 512- / 256-thread blocks, 4 matrix
-  cores with 32-channel output tiles, 5 one wavefront per item, 6 K split over the waves of a block, 7 K split over a
-  cluster of blocks (only with an exchange buffer attached), 8 tiles of 128 output channels;
+  cores with 32-channel output tiles, 5 as 3 for four blocks per CU (one wavefront per item for eight channels of length
+  128), 6 K split over the waves of a block, 7 K split over a cluster of blocks (only with an exchange buffer attached),
+  8 as 3 with 64 or 128 output channels per block;
   2D algorithms: 1 three kernels (X axis first), 2 whole image, 3 three kernels (rows first).
 GPU parity of each: tests/test_gpu_parity.py (every selector forced), tests/test_gpu_fullsize.py (the configurations at
 full size), tests/test_gpu_cluster.py (7), tests/test_gpu_large_grids.py."""

@@ -31,7 +31,7 @@ def _check(got, ref, tol, what):
     (40003, 128, 8, 128, 0),         # 80,006 blocks, S odd: exercises the tail of the block decode
     (33001, 256, 8, 128, 0),         # 66,002 blocks at DY = 256
     (66000, 128, 16, 64, 1),         # SIMT kernel, 66,000 blocks
-    (33000, 256, 32, 128, 3),        # 256-thread matrix-core kernel, 66,000 blocks
+    (33000, 256, 32, 128, 3),        # 256-thread split-product kernel, 66,000 blocks
 ])
 def test_layer_1d_beyond_65536_blocks(S, DY, K, N, algo, tol, algo_1d):
     print("large grid layer_1d", S, DY, K, N, algo, flush=True)
@@ -52,11 +52,11 @@ def test_layer_1d_beyond_65536_blocks(S, DY, K, N, algo, tol, algo_1d):
 
 @pytest.mark.parametrize("S,DY,K,N,algo", [
     (2048, 256, 8, 128, 0),          # 4 MiB between the rows of a signal set, two output tiles per set
-    (4096, 256, 16, 64, 3),          # 8 MiB, 256-thread matrix-core kernel
-    (4096, 128, 16, 64, 5),          # 4 MiB, one wavefront per item
+    (4096, 256, 16, 64, 3),          # 8 MiB, 256-thread split-product kernel
+    (4096, 128, 16, 64, 5),          # 4 MiB, four blocks per CU
     (1024, 512, 8, 128, 0),          # 4 MiB at length 512
     (512, 1024, 8, 64, 1),           # 4 MiB at length 1024, SIMT kernel
-    (2048, 256, 32, 256, 8),         # wide tiles, two per signal set
+    (2048, 256, 32, 256, 8),         # blocks of 128 channels, two per signal set
     (2048, 256, 64, 64, 6),          # eight waves split the channels of an item, two 32-channel tiles per signal set
     (2048, 256, 64, 128, 2),         # 512-thread matrix-core kernel
     (8192, 256, 8, 64, 0),           # 16 MiB: the largest stride that takes this block order
@@ -87,9 +87,9 @@ def test_layer_1d_channel_strides_that_are_multiples_of_4MiB(S, DY, K, N, algo, 
     (262144, 40, 64, 0.0),           # four per CU
     (65536, 64, 128, 0.0),           # two n tiles share the CUs: 128 blocks per n tile, two column blocks each
     (65536 + 64, 48, 192, 0.0),      # three n tiles, a partly filled last column block
-    (262144, 104, 128, 0.0),         # more than 64 channels, eight column blocks per CU: the whole W tile in LDS, chunks of 32
+    (262144, 104, 128, 0.0),         # more than 64 channels, eight column blocks per CU: four steps, the whole W tile in LDS
     (524288 + 128, 72, 64, 0.0),     # the same with one n tile and a partly filled last column block
-    (262144, 40, 64, 0.25 - 0.5j),   # C read and written (beta): the kernel with one column block per block
+    (262144, 40, 64, 0.25 - 0.5j),   # C read and written (beta)
 ])
 def test_cgemm_with_several_column_blocks_per_cu(M, K, N, beta, tol):
     """the mode GEMM as persistent blocks that walk the column blocks: every column written (C starts as NaN when beta

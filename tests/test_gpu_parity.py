@@ -85,13 +85,13 @@ def test_layer_1d_random_shapes(seed, tol, algo_1d):
 
 
 @pytest.mark.parametrize("bs,DY,K,N", [
-    (1030, 128, 16, 64),             # DY=128: from two items per CU on for K <= 16
-    (600, 128, 40, 128),             # DY=128, 1200 items, K = 5 rounds of 8 channels
-    (2100, 256, 8, 64),              # DY=256: from eight items per CU on
-    (1040, 256, 72, 128),            # DY=256, 2080 items, two N tiles, K = 18 rounds of 4 channels
+    (1030, 128, 16, 64),             # DY=128: half a round of 32 channels
+    (600, 128, 40, 128),             # DY=128, 1200 items, the last round with eight channels
+    (2100, 256, 8, 64),              # DY=256: half a round of 16 channels
+    (1040, 256, 72, 128),            # DY=256, 2080 items, the last of five rounds with eight channels
 ])
 def test_layer_1d_large_grids(bs, DY, K, N, tol):
-    """grids large enough for the size rule to pick the one-wavefront-per-item kernel (on a 256-CU device)"""
+    """grids of several blocks per CU (on a 256-CU device)"""
     print("case layer_1d large grid", bs, DY, K, N, flush=True)
     x, W = workloads.uniform_1d(3 + bs + DY + K, bs, DY, K, N)
     y = tf.layer_1d(dev(x), dev(W), alpha=1 - 1j)
@@ -314,9 +314,9 @@ SIZE_RULE_SHAPES = [
     (1, 128, 8, 64, 4), (40, 256, 24, 128, 4),        # at most one 32-channel tile per CU: 512 threads, tiles of 32
     (200, 128, 16, 64, 2), (200, 256, 40, 64, 2),     # up to one 64-channel item per CU: 512 threads
     (300, 256, 32, 64, 3), (700, 256, 8, 64, 3),      # several items per CU: 256 threads
-    (300, 128, 32, 64, 8), (800, 128, 64, 128, 8),    # DY = 128: wide tiles
-    (1000, 256, 16, 128, 8), (300, 256, 128, 64, 8),   # DY = 256: tiles of 128 channels / 128 input channels
-    (1100, 128, 24, 64, 5), (600, 128, 8, 64, 5),     # DY = 128, several items per SIMD: one wavefront per item
+    (300, 128, 32, 64, 8), (800, 128, 64, 128, 8),    # DY = 128: a few blocks of 64 channels per CU / N = 128
+    (1000, 256, 16, 128, 8), (300, 256, 128, 64, 8),   # DY = 256: the same
+    (1100, 128, 24, 64, 5), (600, 128, 8, 64, 5),     # DY = 128, several items per SIMD: four blocks per CU / one wavefront per item
     (64, 256, 64, 128, 6), (100, 256, 96, 64, 6),     # small grids, 64 channels or more: K split over the waves of a block
     (100, 512, 16, 64, 2), (300, 512, 16, 64, 1), (300, 1024, 64, 64, 3),   # the long lengths
 ]

@@ -10,7 +10,7 @@
 //   fft2d_trunc    image (k,b): DX row FFTs along Y (coalesced rows, 64 modes kept, held in registers),
 //                  redistribution through LDS, 64 column FFTs along X (64 modes kept)
 //                  -> spec[k][b][4096]                          reads 8 DX DY bytes, writes 32 KiB
-//   cgemm_modes    C[n][b][m] = alpha * sum_k W[k][n] spec[k][b][m] on the fp32 matrix cores
+//   cgemm_modes    C[n][b][m] = alpha * sum_k W[k][n] spec[k][b][m] on the matrix cores
 //   ifft2d_pad     exact mirror -> y[n][b][DX][DY]              reads 32 KiB, writes 8 DX DY bytes
 //
 // so x is read once and y written once; padded / discarded modes are never touched in memory.
