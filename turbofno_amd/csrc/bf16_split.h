@@ -29,11 +29,12 @@ __device__ __forceinline__ void split_bf16_pair(float a, float b, unsigned& h, u
     l = __builtin_bit_cast(unsigned, __builtin_convertvector((float2_v){ ra, rb }, bf16x2_t));
 }
 
-// Which operands the split holds: from 2^-110 (7.7e-34) on and up to 2^-9 below the largest float, and zero. Below 2^-110 the third part would need bits under the smallest bf16 number, 2^-133; infinities and
-// magnitudes within 2^-9 of the largest float leave a NaN in the remainder x - h. A wave whose operands include such values forms its
-// product again, with fp32 instructions, so that the results have fp32 precision and fp32 infinities over the whole range of floats:
-//   * small magnitudes are found in the operands, zeros, which are exact, aside: lower(), three instructions per two values, or where a
-//     branch costs nothing below_split_range(), one per two values as long as there are no zeros;
+// Which operands the split holds: zero, and magnitudes from 2^-110 (7.7e-34) to 2^-9 below the largest float. Below 2^-110 the third
+// part would need bits under the smallest bf16 number, 2^-133; infinities and the top of the range leave a NaN in the remainder x - h.
+// A wave whose operands include such values forms its product again, with fp32 instructions, so that the results have fp32 precision
+// and fp32 infinities over the whole range of floats:
+//   * small magnitudes are found in the operands: below_split_range(), one minimum per two values, and a second look that tells zeros
+//     apart, which are exact; or, where zeros are common, lower(), three instructions per two values without a branch;
 //   * the others are found in the accumulators: each leaves a NaN or an infinity in every sum it takes part in.
 constexpr float kSplitSmallest = 0x1p-110f;
 __device__ __forceinline__ float smaller(float low, float a, float b)

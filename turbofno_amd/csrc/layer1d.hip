@@ -442,8 +442,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 // of one output channel and runs its backward transform. The chain of latencies of an item is K / 32 rounds + K / 128 products +
 // one reduction + one backward pass, against three barriers and two tile builds per 32 channels in the kernel that
 // shares the spectra through LDS. S = 64, K = N = 128: 17.6 us
-// with fp32 matrix instructions in every round, 15.7 with the split, 16.2 with the search for operands that the split does not hold
-// (for which the wave's share of the product is formed in fp32 instead); K = 64: 13.1 / 13.1 / 13.4.
+// with fp32 matrix instructions in every round, 15.7 with the split, 16.0 with the search for operands that the split does not hold
+// (for which the wave's share of the product is formed in fp32 instead); K = 64: 13.1 / 13.1 / 13.2.
 constexpr int SPLIT_NT = 32, SPLIT_PP = 72;
 constexpr size_t SPLIT_LDS = sizeof(float2) * 8 * SPLIT_NT * SPLIT_PP;       // 147,456 B; covers the 32 exchange regions
 
@@ -496,10 +496,7 @@ __global__ __launch_bounds__(512) void fused_fft_mfma_ifft_split_kernel(int S, i
                 fwd_pass1(v, tw, gg);
                 if (kr + 32 + 4 * w < K) issue(v, kr + 32);
                 group_forward_finish<8>(gg, exch, t, out);
-                unsigned bits = ~0u;
-#pragma unroll
-                for (int a = 0; a < 4; ++a) bits = lower(bits, out[a]);
-                low |= any_lane(bits < kSplitLow);
+                low |= below_split_range(out);
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
                     unsigned h, m, l;
@@ -518,7 +515,7 @@ __global__ __launch_bounds__(512) void fused_fft_mfma_ifft_split_kernel(int S, i
             SplitOperand wre, wim;                                // rows (re, -im) and (im, re) of alpha W
 #pragma unroll
             for (int j = 0; j < 4; ++j) wv[i][j] = cmul(wv[i][j], alpha);
-            unsigned bits = ~0u;
+            unsigned bits = ~0u;                                  // (zeros are common here: channels beyond K)
 #pragma unroll
             for (int j = 0; j < 4; ++j) bits = lower(bits, wv[i][j]);
             low |= any_lane(bits < kSplitLow);

@@ -25,7 +25,7 @@
 // shapes stay with the SIMT kernel: launch_fused_fft_cgemm, launch_fused_cgemm_ifft.
 // Error against 64 bits: 2.4e-7 -> 2.0e-7 (K = 64), 3.2e-7 -> 2.7e-7 (K = 128), the same from the smallest normal floats to the
 // largest: operands that the split does not hold (bf16_split.h) are noticed - small spectra and weights as they are split, the rest in
-// the accumulators - and product_fp32() stands in. Noticing costs 0 - 3 %, 1.2 % on average (the most: DY = 128, S = 4096, K = N = 128: 282 -> 292).
+// the accumulators - and product_fp32() stands in. Noticing costs 0 - 2 % (the most: DY = 128, S = 4096, K = N = 128: 295 -> 301), up to 4 % of the halves on small grids.
 #include "bf16_split.h"
 #include "group_fft.h"
 #include "kernels.h"
@@ -277,12 +277,7 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
 #pragma unroll
                 for (int a = 0; a < MODES; ++a) out[a] = make_float2(0.f, 0.f);
             }
-            if (busy) {
-                unsigned bits = ~0u;
-#pragma unroll
-                for (int a = 0; a < MODES; ++a) bits = lower(bits, out[a]);
-                low |= any_lane(bits < kSplitLow);
-            }
+            if (busy) low |= below_split_range(out);
             if (pass == 0) __syncthreads();                     // the operand tile of the last round is read / the exchanges are done
 #pragma unroll
             for (int a = 0; a < MODES; ++a) {
