@@ -165,8 +165,8 @@ int turbofno_layer_2d_noalloc(int bs, int DX, int DY, int K, int N, const void* 
 /*
  * Process-wide choice of the fused 1D kernel behind turbofno_fused_fft_cgemm_ifft / turbofno_layer_1d and the Y stage
  * of the three-kernel 2D path (their reference-shaped signatures have no room for a selector): 0 = by problem size
- * (default), 1 = SIMT contraction, 2 = matrix cores with 512-thread blocks, 3 = matrix cores with 256-thread blocks of 64
- * output channels, 4 = as 2 with 32-channel output tiles, 5 = as 3, laid out for four blocks per compute unit (DY = 128 with
+ * (default), 1 = SIMT contraction, 2 = matrix cores with 512-thread blocks of 64 output channels, 3 = matrix cores with
+ * 256-thread blocks of 64 output channels, 4 = as 2 with 32-channel output tiles (DY = 128 / 256), 5 = as 3, laid out for four blocks per compute unit (DY = 128 with
  * eight input channels: one wavefront per signal set and output tile), 6 = matrix cores, the K channels of an item split over
  * the waves of a block, 7 = matrix cores, the K channels of a signal set split over a cluster of blocks (see below), 8 = as 3
  * with 128 output channels per block where N is a multiple of 128.
@@ -222,8 +222,9 @@ int turbofno_set_exchange_wait_us(unsigned long long microseconds);
  *                             turbofno_set_1d_algo selector, in that selector's numbering (1 ... 8); 0 for arguments
  *                             the call would refuse. compute_units = 0 asks the current device (the only case that
  *                             touches the HIP runtime), any other value answers for a device of that many compute
- *                             units; exchange_attached says whether the stream has an exchange buffer. Chosen by size, 8
- *                             stands for blocks of 64 or of 128 output channels;
+ *                             units; exchange_attached says whether the stream has an exchange buffer. Chosen by size, 2
+ *                             and 4 stand for blocks of 16, 32 or 64 output channels, 6 for such blocks too where they
+ *                             are ahead of the K split, 8 for blocks of 64 or of 128;
  *   turbofno_query_1d_tile    output channels per block of that kernel (the clustered kernel: N); 0 as above.
  */
 int turbofno_query_2d_algo(int bs, int DX, int DY, int K, int N, int algo);

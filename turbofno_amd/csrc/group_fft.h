@@ -21,11 +21,16 @@ template <int LOGDY> struct Geo1D {
 
 // Lengths 512 / 1024: a group of L = 32 / 64 lanes owns one signal, lane t holds samples t + L i. The scheme of the wide_*
 // codelets (inner 16-point transforms over the lanes tt = a + A b, A = L / 16, then a sum over a), with the lanes and the
-// two exchanges laid out for the LDS banks (64 banks of 4 bytes, 32 lanes of 8 bytes per cycle):
+// two exchanges laid out for the LDS banks (8 bytes per lane: a read takes 32 lanes per cycle over 64 banks of 4 bytes, a write 16 lanes
+// over 32 banks):
 //   second-pass lane t = 16 a + r computes inner_a[c] of bin r, then finishes the modes r + 16 (a + A j) = t + L j: the
 //     natural order, L consecutive modes per slot j;
 //   first exchange: the A rows a + A b of one b side by side, [b][a][16 bins] with a pitch of 16 A + 1: the read of one b
-//     covers 32 consecutive elements per half wavefront, the write of one bin is conflict-free for L = 32 (2-way for 64);
+//     covers 32 consecutive elements per half wavefront. Left at that, the write of one bin meets the same banks from the A parts of a
+//     row, two (L = 32) or four ways (64: 16 cycles instead of 4). SPREAD: the bins of part a at k ^ (16 / A) a, without conflicts, for
+//     A write addresses instead of one: the 1D kernels at L = 64 (small grids, DY = 1024, K = 128, S = 16: 44.3 -> 38.7 us; first half, S =
+//     256, K = 32: 21.0 -> 19.7) and the one for small grids at L = 32 (22.3 -> 21.6); not the image kernels, which have no registers left for the
+//     addresses (16 images of 512 x 512: 588 -> 597 us);
 //   second exchange: [c][16 a' + r] with a pitch of L + 16: writes are consecutive, and the lanes a and a + 1 of a half
 //     wavefront, which read the rows c = a + A j and c + 1, land 16 elements apart modulo 32.
 // The powers w_L^e, e < L, come from the constant table, or (FROM_ARRAY) from an array of L values that the caller keeps
@@ -36,21 +41,34 @@ template <int L, bool FROM_ARRAY> TFNO_DEV cpx wide_pow(const cpx* powers, int e
     if constexpr (FROM_ARRAY) return powers[e];
     else return kTwiddle1024[(e * (1024 / L)) & 1023];
 }
-template <int L, bool FROM_ARRAY>
+template <int L, bool FROM_ARRAY, bool SPREAD = false>
 TFNO_DEV void wide_forward_finish(const cpx (&g)[16], cpx* exch, const cpx* powers, int t, cpx (&out)[64 / L])
 {
     constexpr int A = L / 16, MM = 64 / L, P1 = 16 * A + 1, PS = L + 16;
     static_assert(16 * P1 <= L * 17 && 4 * PS <= L * 17, "both exchanges fit the group's region");
     const int r = t % 16, a = t / 16;
     wave_lds_fence();
+    constexpr int H = 16 / A;                        // SPREAD: bin k of part a sits at k ^ (H a)
+    if constexpr (SPREAD) {
+        const int ta = t % A;
+        cpx* row = exch + (t / A) * P1 + ta * 16;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) exch[(t / A) * P1 + (t % A) * 16 + k] = g[k];
+        for (int h = 0; h < A; ++h) {
+            cpx* part = row + H * (h ^ ta);
+#pragma unroll
+            for (int k = 0; k < H; ++k) part[k] = g[H * h + k];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) exch[(t / A) * P1 + (t % A) * 16 + k] = g[k];
+    }
     wave_lds_fence();
     cpx inner[4];
     {
         cpx u[16];
+        const cpx* column = exch + (SPREAD ? t ^ (H * a) : t);
 #pragma unroll
-        for (int b = 0; b < 16; ++b) u[b] = exch[b * P1 + t];      // lane tt = a + A b, bin r
+        for (int b = 0; b < 16; ++b) u[b] = column[b * P1];        // lane tt = a + A b, bin r
         dft16_first4<-1>(u, inner);
     }
     wave_lds_fence();                                // every lane of the group has read the first exchange
@@ -113,7 +131,7 @@ TFNO_DEV void group_forward_finish(const cpx (&g)[16], cpx* exch, int t, cpx (&o
 {
     constexpr int L = Geo1D<LOGDY>::L;
     if constexpr (L >= 32) {
-        wide_forward_finish<L, false>(g, exch, nullptr, t, out);
+        wide_forward_finish<L, false, L == 64>(g, exch, nullptr, t, out);
         return;
     }
     wave_lds_fence();
@@ -256,7 +274,7 @@ TFNO_DEV void rows128_backward(const cpx (&c)[8], const TW& twrow, cpx* exch, in
 template <int L>
 TFNO_DEV void wide_rows_forward_finish(const cpx (&g)[16], cpx* exch, const cpx* wsm, int t, cpx (&out)[64 / L])
 {
-    wide_forward_finish<L, true>(g, exch, wsm, t, out);
+    wide_forward_finish<L, true, false>(g, exch, wsm, t, out);
 }
 // c[mm] = mode t + L mm of the row. On return y[i] = sample t + L i.
 template <int L>
@@ -265,6 +283,24 @@ TFNO_DEV void wide_rows_backward(const cpx (&c)[64 / L], const cpx* twrow, const
     cpx e[16];
     wide_backward_inputs<L, true>(c, wsm, exch, t, e);
     inv_pass2_lds(e, twrow, y);
+}
+
+// First pass of two signals of 128 samples: v[0..7], v[8..15] are samples t + 16 i of each.
+TFNO_DEV void pair128_first_pass(const cpx (&v)[16], const cpx* twrow, cpx (&gg)[16])
+{
+    cpx a8[8], b8[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) { a8[i] = v[i]; b8[i] = v[8 + i]; }
+    fft8<-1>(a8);
+    fft8<-1>(b8);
+    gg[0] = a8[0];
+    gg[8] = b8[0];
+#pragma unroll
+    for (int r = 1; r < 8; ++r) {
+        const cpx w = twrow[r];
+        gg[r] = cmul(a8[r], w);
+        gg[8 + r] = cmul(b8[r], w);
+    }
 }
 
 // The same pairing for the 1D kernels, with the twiddles in registers (tw[r] = w_128^(t r), t < 16): a 16-lane group

@@ -5,15 +5,6 @@
 
 namespace tfno {
 
-// LDS layout of a real-expanded W' tile for v_mfma_f32_16x16x4_f32 (the block-per-item matrix-core
-// 1D kernels): float index  (k/4)*kWGroup + ((k&3)>>1)*kWHalf + n'*4 + (k&1)*2 + c  holds W'[n' = 2n + c'][2k + c],
-// {Wr, -Wi} for c' = 0 and {Wi, Wr} for c' = 1. An operand read (16 n' x 4 channels) takes 256 contiguous bytes per
-// half wavefront: conflict free. The strides are 512 + 4 and 1024 + 8 floats so that the tile BUILD, whose lanes run
-// along k (the contiguous direction of W in memory), spreads a half wavefront over all 64 banks as well; with the
-// unpadded strides every lane of such a store fell on the same two banks.
-constexpr int kWHalf = 516;
-constexpr int kWGroup = 1032;
-
 #ifdef __HIPCC__
 // Block -> (signal set s, output tile) for the fused 1D kernels. Consecutive workgroups go to different XCDs (eight L2s),
 // and every output tile of a signal set re-reads the same K input rows: the tiles of one s are therefore given block
@@ -128,6 +119,14 @@ hipError_t launch_fused_split(int logDY, long S, int N, int K, const float2* x, 
 hipError_t launch_split_forward(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C, float2 alpha, float2 beta,
                                 bool wide, hipStream_t stream);
 hipError_t launch_split_backward(int logDY, long S, int N, int K, const float2* A, const float2* W, float2* y, float2 alpha, hipStream_t stream);
+
+// Small grids, every length (layer1d_small.hip): one 512-thread block per (signal set, nt output channels), nt = 16, 32, 64; the layer and its halves.
+hipError_t launch_fused_small(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, int nt,
+                              hipStream_t stream, int keep_y = 0);
+hipError_t launch_small_forward(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C, float2 alpha, float2 beta,
+                                int nt, hipStream_t stream);
+hipError_t launch_small_backward(int logDY, long S, int N, int K, const float2* A, const float2* W, float2* y, float2 alpha, int nt,
+                                 hipStream_t stream);
 
 // Halves of the fused kernel (variants B and C) and the stand-alone contiguous transforms (variant A).
 hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C,

@@ -139,178 +139,7 @@ __global__ __launch_bounds__(256) void fused_fft_cgemm_ifft_kernel(int S, int N,
     }
 }
 
-// Fused 1D layer with the contraction on the fp32 matrix cores, for channel counts where the GEMM dominates the
-// arithmetic (K >= one chunk). Same operands, grid (S, N/64) and block-traverses-K schedule as the kernel above;
-// 512 threads = 8 waves:
-//   * a chunk is KC = 512/L channels (32 for DY=256, 64 for DY=128): every L-lane group transforms one channel and
-//     leaves its 64 modes in sA[k][m]; two chunks of loads are in flight per group (a buffer is refilled as soon as the
-//     first pass has consumed it), so they travel under the exchanges, the W tile builds and the matrix work;
-//   * C'[n'][m] += W'[n'][k'] A'[k'][m] is the 4-real form of the complex product on v_mfma_f32_16x16x4_f32:
-//     n' = (n, re|im) 128 rows, m 64 columns = 8 x 4 tiles, four per wave (one m tile, four n' tiles), so one read of
-//     A from LDS feeds eight matrix instructions. W' (alpha folded in) uses the conflict-free LDS order kWGroup / kWHalf;
-//     sA has a pitch of 80 complex so that the two k rows a half wave reads fall on disjoint banks;
-//   * the product goes through LDS once (sC, pitch 72) to reach the lane groups that run the zero-padded backward
-//     transforms and store y.
-// sA aliases the exchange regions of the lane groups (the transforms of a chunk are complete before sA is written),
-// sC aliases the W' tile.
 typedef float floatx4_1d __attribute__((ext_vector_type(4)));
-
-// NT_ = output channels per block: 64, or 32 to spread a small grid over twice as many CUs (DY = 128 / 256).
-template <int LOGDY, int NT_ = 64> struct GeoMfma1D {
-    static constexpr int L = Geo1D<LOGDY>::L, MM = 64 / L;
-    static constexpr int THREADS = 512;                       // one block per CU
-    static constexpr int NT = NT_;
-    static constexpr int NTW = (NT / 2) / (THREADS / 64);     // 16x16 tiles per wave: one m tile x NTW n' tiles
-    static constexpr int KC = THREADS / L;                    // channels per chunk = lane groups per block
-    static constexpr int PA = 80, PC = 72;                    // pitches (complex) of sA and sC
-    static constexpr int EXCH = L * 17;
-    static constexpr int REGION0 = KC * EXCH > KC * PA ? KC * EXCH : KC * PA;              // exchange | sA
-    static constexpr int WTILE = (KC / 4) * kWGroup / 2;                                   // W' tile in complex units
-    static constexpr int REGION1 = WTILE > NT * PC ? WTILE : NT * PC;                      // W' | sC   (complex)
-    static_assert(NT == 64 || NT == 32, "tiles of 64 or 32 output channels");
-    static constexpr int PASSES = (NT + KC - 1) / KC;         // backward passes; the last may use only NT % KC lane groups
-    static constexpr int DEPTH = 2;                           // chunks of loads in flight per lane group
-    static constexpr size_t LDS_BYTES = sizeof(float2) * (size_t)(REGION0 + REGION1);
-};
-
-template <int LOGDY, int NT, bool KEEP = false>
-__global__ __launch_bounds__(512, 1) void fused_fft_mfma_ifft_kernel(int S, int N, int K, const float2* __restrict__ x,
-                                                                      const float2* __restrict__ W, float2* __restrict__ y,
-                                                                      float2 alpha)
-{
-    using G = GeoMfma1D<LOGDY, NT>;
-    constexpr int NTW = G::NTW;
-    constexpr int DY = 1 << LOGDY, L = G::L, MM = G::MM, KC = G::KC, PA = G::PA, PC = G::PC;
-    extern __shared__ float2 lds[];
-    float2* sA = lds;                                          // [KC][PA]; aliases the exchange regions
-    float* sW = reinterpret_cast<float*>(lds + G::REGION0);    // W' tile, layout of kWGroup / kWHalf
-    float2* sC = lds + G::REGION0;                             // [64][PC]; aliases sW after the K loop
-
-    const int tid = threadIdx.x;
-    const int g = tid / L, t = tid % L;                        // transform role: lane group = channel of the chunk
-    const int wave = tid >> 6, lane = tid & 63, col = lane & 15, kq = lane >> 4;   // matrix role
-    const int mt = wave & 3, nt0 = (wave >> 2) * NTW;          // m tile, first of the wave's NTW n' tiles
-    long s;
-    int ntile;
-    decode_block_1d(S, N / NT, 1 << LOGDY, !KEEP, s, ntile);
-    const int n0 = ntile * NT;
-    // DY = 128: signals are transformed in pairs by 16-lane groups (see the SIMT kernel)
-    constexpr bool PAIR = LOGDY == 7;
-    const int t16 = tid % 16, gpair = (tid / 16) * 2;
-    float2* exch = PAIR ? lds + (tid / 16) * (2 * G::EXCH) : lds + g * G::EXCH;
-
-    cpx tw[16];
-    load_lane_twiddles<LOGDY>(PAIR ? t16 : t, tw);
-
-    floatx4_1d acc[NTW];
-#pragma unroll
-    for (int i = 0; i < NTW; ++i) acc[i] = floatx4_1d{ 0.f, 0.f, 0.f, 0.f };
-
-    // loads of this lane group's channel(s) of the chunk that starts at channel kc
-    auto issue = [&](cpx (&dst)[16], int kc) {
-        if constexpr (PAIR) {
-            const float2* src = x + ((long)(kc + gpair) * S + s) * DY + t16;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) { dst[i] = src[16 * i]; dst[8 + i] = src[(long)S * DY + 16 * i]; }
-        } else {
-            const float2* src = x + ((long)(kc + g) * S + s) * DY + t;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) dst[i] = src[L * i];
-        }
-    };
-    // two chunks of loads in flight per lane group: buffer b receives chunk c + 2 as soon as chunk c has left it
-    cpx v0[16], v1[16];
-    if (g < K) issue(v0, 0);
-    if (G::DEPTH == 2 && KC + g < K) issue(v1, KC);
-
-    auto chunk = [&](cpx (&v)[16], int kc) {
-        const int kn = (K - kc) < KC ? (K - kc) : KC;          // multiple of 8 (caller contract)
-        // W chunk: lanes run along k, the contiguous direction of W[k + n*K]
-        constexpr int WPT = KC * NT / G::THREADS;
-        float2 wv[WPT];
-#pragma unroll
-        for (int u = 0; u < WPT; ++u) {
-            const int idx = tid + u * G::THREADS;
-            const int k = idx % KC, n = idx / KC;
-            wv[u] = (k < kn) ? W[(kc + k) + (long)(n0 + n) * K] : make_float2(0.f, 0.f);
-        }
-        cpx out[MM];
-        if (g < kn) {
-            if constexpr (PAIR) {
-                cpx w[16];
-#pragma unroll
-                for (int i = 0; i < 16; ++i) w[i] = v[i];
-                if (kc + G::DEPTH * KC + g < K) issue(v, kc + G::DEPTH * KC);
-                pair128_forward(w, tw, exch, t16, out);
-            } else {
-                cpx gg[16];
-                fwd_pass1(v, tw, gg);
-                if (kc + G::DEPTH * KC + g < K) issue(v, kc + G::DEPTH * KC);    // the chunk DEPTH chunks ahead
-                group_forward_finish<LOGDY>(gg, exch, t, out);
-            }
-        }
-        __syncthreads();                                       // all exchanges done: sA may overwrite them
-        if (g < kn) {
-#pragma unroll
-            for (int a = 0; a < MM; ++a) sA[g * PA + (PAIR ? t + L * a : forward_mode_of_lane<LOGDY>(t, a))] = out[a];
-        }
-#pragma unroll
-        for (int u = 0; u < WPT; ++u) {
-            const int idx = tid + u * G::THREADS;
-            const int k = idx % KC, n = idx / KC;
-            const float2 w = make_float2(wv[u].x * alpha.x - wv[u].y * alpha.y, wv[u].x * alpha.y + wv[u].y * alpha.x);
-            float* dstw = &sW[(k >> 2) * kWGroup + ((k & 3) >> 1) * kWHalf + (2 * n) * 4 + (k & 1) * 2];
-            *reinterpret_cast<float2*>(dstw) = make_float2(w.x, -w.y);
-            *reinterpret_cast<float2*>(dstw + 4) = make_float2(w.y, w.x);
-        }
-        __syncthreads();
-        const float2* arow = sA + kq * PA + mt * 16 + col;
-        const float* wrow = sW + (kq >> 1) * kWHalf + (nt0 * 16 + col) * 4 + (kq & 1) * 2;
-        for (int kg = 0; kg < kn / 4; ++kg) {
-            const float2 b = arow[kg * 4 * PA];
-#pragma unroll
-            for (int i = 0; i < NTW; ++i) {
-                const float2 a = *reinterpret_cast<const float2*>(wrow + kg * kWGroup + i * 64);
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, acc[i], 0, 0, 0);
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, acc[i], 0, 0, 0);
-            }
-        }
-        __syncthreads();                                       // sA / sW are free again (next chunk, or sC below)
-    };
-    for (int kc = 0; kc < K; kc += G::DEPTH * KC) {
-        chunk(v0, kc);
-        if (G::DEPTH == 2 && kc + KC < K) chunk(v1, kc + KC);
-    }
-
-    // D[row = 4 kq + v][col] of tile i: n' = 16 (nt0 + i) + 4 kq + v = 2 n + c'  ->  n = 8 (nt0 + i) + 2 kq + (v >> 1)
-#pragma unroll
-    for (int i = 0; i < NTW; ++i) {
-        const int n = 8 * (nt0 + i) + 2 * kq;
-        sC[n * PC + mt * 16 + col] = make_float2(acc[i][0], acc[i][1]);
-        sC[(n + 1) * PC + mt * 16 + col] = make_float2(acc[i][2], acc[i][3]);
-    }
-    __syncthreads();
-    cpx c[G::PASSES][MM];
-#pragma unroll
-    for (int pass = 0; pass < G::PASSES; ++pass)
-#pragma unroll
-        for (int a = 0; a < MM; ++a) c[pass][a] = (g + KC * pass < NT) ? sC[(g + KC * pass) * PC + t + L * a] : make_float2(0.f, 0.f);
-#pragma unroll
-    for (int pass = 0; pass < G::PASSES; ++pass) {
-        const int n = g + KC * pass;
-        if (n >= NT) break;                                    // whole waves (NT and KC are multiples of 32 channels)
-        cpx yv[16];
-        if constexpr (PAIR) {
-            pair128_backward(c[pass], tw, exch, t16, yv);
-            float2* dst = y + ((long)(n0 + gpair + KC * pass) * S + s) * DY + t16;
-            store_pair16<KEEP>(dst, (long)S * DY, yv);
-        } else {
-            group_backward<LOGDY>(c[pass], tw, exch, t, yv);
-            float2* dst = y + ((long)(n0 + n) * S + s) * DY + t;
-            store_row16<L, KEEP>(dst, yv);
-        }
-    }
-}
 
 // Fused 1D layer for DY = 128 and eight input channels: ONE WAVEFRONT per (signal set, 64 output channels), no block barrier
 // and no staging of operands through LDS. The register layouts of the transforms and of v_mfma_f32_16x16x4_f32 coincide:
@@ -432,7 +261,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     }
 }
 
-// Fused 1D layer for small grids (every block has a CU to itself), DY = 256: the eight waves of a block share ONE
+// Fused 1D layer for grids of more than half a block of 32 output channels per CU and at most one, DY = 256, 112 channels or more (fewer
+// blocks or channels: layer1d_small.hip): the eight waves of a block share ONE
 // item (signal set, 32 output channels) and split its K input channels: wave w transforms channels 32 r + 4 w + g in round r,
 // g = 16-lane group. Four rounds give a lane four channels of its modes t + 16 a: with real and imaginary part the eight
 // consecutive values of the contraction that a lane holds of the B operand of v_mfma_f32_16x16x32_bf16, so a wave multiplies its
@@ -440,9 +270,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 // output channels x 4 m tiles). The K loop has no barrier and stages nothing through LDS. The eight partial products
 // meet in LDS once (sP[w][n][m], pitch 72 complex: conflict-free b64 stores), every lane group sums the eight partials
 // of one output channel and runs its backward transform. The chain of latencies of an item is K / 32 rounds + K / 128 products +
-// one reduction + one backward pass, against three barriers and two tile builds per 32 channels in the kernel that
-// shares the spectra through LDS. S = 64, K = N = 128: 17.6 us
-// with fp32 matrix instructions in every round, 15.7 with the split, 16.0 with the search for operands that the split does not hold
+// one reduction + one backward pass. S = 64, K = N = 128: 17.6 us with fp32 matrix instructions in every round, 15.7 with the split, 16.0 with the search for operands that the split does not hold
 // (for which the wave's share of the product is formed in fp32 instead); K = 64: 13.1 / 13.1 / 13.2.
 constexpr int SPLIT_NT = 32, SPLIT_PP = 72;
 constexpr size_t SPLIT_LDS = sizeof(float2) * 8 * SPLIT_NT * SPLIT_PP;       // 147,456 B; covers the 32 exchange regions
@@ -691,29 +519,6 @@ static hipError_t dispatch_fused_1d(int logDY, long S, int N, int K, const float
     }
 }
 
-template <int LOGDY, int NT, bool KEEP>
-static hipError_t launch_fused_mfma_k(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha,
-                                      hipStream_t stream)
-{
-    using G = GeoMfma1D<LOGDY, NT>;
-    static std::atomic<unsigned long long> served;
-    if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(fused_fft_mfma_ifft_kernel<LOGDY, NT, KEEP>),
-                                         G::LDS_BYTES, served);
-        e != hipSuccess)
-        return e;
-    if (S * (N / NT) > 0x7fffffffL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((fused_fft_mfma_ifft_kernel<LOGDY, NT, KEEP>), dim3((unsigned)(S * (N / NT))), dim3(G::THREADS),
-                       G::LDS_BYTES, stream, (int)S, N, K, x, W, y, alpha);
-    return hipGetLastError();
-}
-template <int LOGDY, int NT = 64>
-static hipError_t launch_fused_mfma(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha,
-                                    hipStream_t stream, int keep_y = 0)
-{
-    return keep_y ? launch_fused_mfma_k<LOGDY, NT, true>(S, N, K, x, W, y, alpha, stream)
-                  : launch_fused_mfma_k<LOGDY, NT, false>(S, N, K, x, W, y, alpha, stream);
-}
-
 // keep_y as for the other kernels: as the middle stage of one 256 x 256 image, K = 64, N = 128, the layer takes 37.1 us, 40.6 with streaming stores
 template <bool KEEP>
 static hipError_t launch_fused_split_channels(long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, hipStream_t stream)
@@ -743,25 +548,30 @@ static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const
 
 // Which fused 1D kernel runs for a problem: pure arithmetic on the sizes, the selector `algo`, the number of compute
 // units and whether the stream has an exchange buffer attached (no device call), so that callers and tests can ask.
-// algo: 0 = by size, 1 = SIMT kernel, 2 = matrix cores with 512-thread blocks, 3 = matrix cores with 256-thread blocks of 64 output
-// channels, 4 = as 2 with 32-channel output tiles, 5 = as 3 for large grids: four blocks per CU, or with eight channels of
-// length 128 one wavefront per (signal set, output tile), 6 = matrix cores, the eight waves of a block split the K channels of one
-// item (DY = 256), 7 = matrix cores, a cluster of blocks splits the K channels of one signal set (DY = 256, N = 64 / 128, small
-// grids), 8 = as 3 with 128 output channels per block where N allows
+// algo: 0 = by size, 1 = SIMT kernel, 2 = matrix cores with 512-thread blocks of 64 output channels (layer1d_small.hip), 3 = matrix cores
+// with 256-thread blocks of 64 output channels (layer1d_split.hip), 4 = as 2 with 32 output channels, 5 = as 3 for large grids: four
+// blocks per CU, or with eight channels of length 128 one wavefront per (signal set, output tile), 6 = matrix cores, the eight waves of
+// a block split the K channels of one item (DY = 256), 7 = matrix cores, a cluster of blocks splits the K channels of one signal set
+// (DY = 256, N = 64 / 128, small grids), 8 = as 3 with 128 output channels per block where N allows
 // The same rule holds where y is read again at once (middle stage of a 2D layer): the lines were drawn with x and y streamed, and of
 // 3166 2D layers in three stages, lengths 128 to 1024, none lost against a rule that treated that case apart.
-// The return value uses the same numbers (1 ... 8); chosen by size, 8 stands for blocks of 64 or of 128 output channels
-// (tile_of_fused_1d_kernel). A selector value that a kernel is not built for falls back to the
-// choice by size.
+// The return value uses the same numbers (1 ... 8); chosen by size, 2 and 4 stand for blocks of 16, 32 or 64 output channels of the
+// small-grid kernel, 6 for that kernel or the K split, 8 for blocks of 64 or of 128 output channels (tile_of_fused_1d_kernel). A selector
+// value that a kernel is not built for falls back to the choice by size.
 //
-// By size (measured on MI355X, us, kernel of the smaller grids against the split kernel):
-//  * while every block has a CU to itself: matrix cores, 8 waves per block - the shortest chain of latencies for
-//    every K, even K = 8 where most of a chunk is padding;
-//  * about one block of 64 output channels per CU and more, lengths 128 / 256: the split kernel (layer1d_split.hip). DY = 128 with
-//    32 channels or more from three quarters of the CUs on (N = 64: S = 200, K = 64: 13.8 / 12.2, S = 128: 10.9 / 11.8; N = 128:
-//    S = 100, K = 64: 13.5 / 12.1), unless every CU has a block, N = 128 and less than half of the last round of 32 channels is used (S = 128,
-//    K = 40: 10.9 / 11.5, K = 64: 13.2 / 13.1; S = 120, K = 40: 10.8 / 10.2); with 16 channels or more and one block per CU (N = 64, S = 256, K = 16: 8.9 / 7.7); DY = 256 from seven eighths on (N = 64: S = 256, K = 32: 14.7 / 13.2, S = 128, K = 64: 13.5 / 16.9),
-//    with N = 128 from three quarters on (S = 128, K = 64: 19.1 / 17.9; S = 64: 14.0 / 16.9);
+// By size (measured on MI355X, us):
+//  * while every block of 64 output channels has a CU to itself, every length: the small-grid kernel, with the fewest output channels per
+//    block that still give every block a CU (small_tile). Against the best of the other kernels here (the split kernel, and for long
+//    signals the SIMT kernel): N = 64, DY = 128: S = 160, K = 32: 7.8 / 9.3, S = 256, K = 128: 17.7 / 19.3; DY = 256: S = 128, K = 64: 11.3 / 16.9,
+//    S = 256, K = 64: 15.3 / 17.4; DY = 512, S = 128, K = 64: 18.7 / 28.9. Exceptions, all with nearly a block of 64 channels per CU, whose lines lie where the
+//    other kernel is level: the split kernel for DY = 256 with up to 16 channels (S = 256, K = 16: 10.5 / 9.9; N = 128, S = 128, K = 8: 10.2 / 10.4), and for
+//    DY = 128 with 49 to 64 channels, of which the small-grid kernel leaves a sixth to a round of its own (N = 64, S = 200, K = 64: 11.6 / 11.5,
+//    S = 256: 12.2 / 11.9; N = 128, S = 100: 11.6 / 11.5), and with 32 or 40 channels and N no multiple of 128 (S = 256, K = 32: 9.0 / 8.8, S = 200: 8.3 / 8.5),
+//    16 to 40 channels with exactly one block per CU (S = 256, K = 16: 8.2 / 8.1);
+//  * DY = 256, 64 channels or more, blocks of 32 output channels at most one per CU: reported as 6, run by the small-grid kernel (S = 64: N = 128, K = 64:
+//    12.0 / 13.6 for the K split, K = 96: 15.0 / 15.9; S = 1: K = 64: 8.6 / 10.9), from 112 channels on with more than half of the CUs by
+//    the K split, whose rounds have no barrier (S = 64, N = 128, K = 128: 17.6 / 17.1; S = 128, N = 64: 16.8 / 16.4);
+//  * more than one block of 64 output channels per CU, lengths 128 / 256: the split kernel;
 //  * lengths 512 / 1024, more than one block per CU: the split kernel from the number of channels on where it is ahead of the SIMT
 //    kernel, which has less to do per channel (DY = 512, S = 2048, N = 64: K = 24 127 / 120, K = 40 185 / 170, K = 128 358 / 305; S = 512:
 //    K = 16 38 / 42, K = 40 52 / 51; N = 128, S = 1000: K = 32 144 / 123, K = 128 327 / 244; DY = 1024, N = 64: S = 2048, K = 32 325 / 318, S = 512,
@@ -769,8 +579,7 @@ static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const
 //    blocks on a CU, the SIMT kernel three, so below 64 channels the latter is ahead where rounds of two per CU would be at most three
 //    quarters full (N = 64: S = 600: K = 32 98 / 102, K = 40 107 / 114, K = 64 159 / 143; S = 512, K = 40: 88 / 80; N = 192, K = 40: S = 200:
 //    104 / 113, S = 300: 147 / 139) and on large grids of three blocks or more per signal set (N = 192, S = 600: K = 40 242 / 259,
-//    K = 64 341 / 319). On small grids the 512-thread kernel (S = 128, K = 64, DY = 512:
-//    25.9 / 28.9).
+//    K = 64 341 / 319).
 int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, long cus, bool exchange_attached)
 {
     const bool built = logDY >= 7 && logDY <= 10;
@@ -779,7 +588,8 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, long cus, bo
     if (algo == 5 && !long_signal && built) return kFused1dDense;
     if (algo == 0 && !long_signal && built) {
         const long blocks = N % 128 == 0 ? S * (N / 128) : items;
-        if (logDY == 7 && N % 128 != 0 && K >= 16 && blocks >= cus && blocks <= (K >= 128 ? 4 : 2) * cus) return kFused1dWide;
+        if (logDY == 7 && N % 128 != 0 && K >= 16 && (blocks > cus || (blocks == cus && K <= 40)) && blocks <= (K >= 128 ? 4 : 2) * cus)
+            return kFused1dWide;
         if (blocks > cus) {
             if (N % 128 == 0 && K >= 16) return kFused1dWide;           // 128 or 64 output channels per block: wide_tiles()
             // blocks of 64 output channels, a few per CU
@@ -796,11 +606,12 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, long cus, bo
     }
     if (algo == 8 && built) return kFused1dWide;
     if (algo == 8) algo = 0;
+    if (algo == 0 && logDY == 7 && K >= 16 && N % 128 == 0 && items > cus && items <= 2 * cus) return kFused1dWide;
     // not quite one block per CU
-    if (algo == 0 && logDY == 7 && K >= 16 && N % 128 == 0 && 2 * items >= 3 * cus && items <= 2 * cus) return kFused1dWide;
-    const bool short_round = N % 128 == 0 && K % 32 > 0 && K % 32 < 16 && items == cus;
-    if (algo == 0 && logDY == 7 && K >= 32 && !short_round && 4 * items >= 3 * cus && items <= cus) return kFused1dMfma256;
-    if (algo == 0 && logDY == 8 && (N % 128 == 0 ? 4 * items >= 3 * cus : 8 * items >= 7 * cus) && items <= cus) return kFused1dMfma256;
+    if (algo == 0 && items <= cus) {
+        if (logDY == 7 && 4 * items >= 3 * cus && ((K > 48 && K <= 64) || (N % 128 != 0 && K >= 32 && K <= 40))) return kFused1dMfma256;
+        if (logDY == 8 && 8 * items >= 7 * cus && K <= 16) return kFused1dMfma256;
+    }
     // lengths 512 / 1024, more than one block per CU
     if (algo == 0 && long_signal && built && items > cus) {
         if (N % 128 == 0 && K >= (logDY == 9 ? 32 : 64)) return kFused1dWide;
@@ -812,10 +623,7 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, long cus, bo
     }
     int pick = algo == 4 ? 2 : algo;
     if (pick == 0) pick = (built && items <= cus) ? 2 : (long_signal ? 1 : 3);
-    // small grids, 64 channels or more: eight waves split the K channels of one item (10-16 % ahead of the kernel that
-    // shares the spectra through LDS; level at K = 32)
     if (logDY == 8 && (algo == 6 || (algo == 0 && K >= 64 && S * (N / SPLIT_NT) <= cus))) return kFused1dSplitK;
-    // few blocks: tiles of 32 output channels put twice as many CUs to work (each block still transforms all K inputs)
     if (pick == 2 && (logDY == 7 || logDY == 8) && (algo == 4 || (algo == 0 && S * (N / 32) <= cus))) return kFused1dMfma512Tile32;
     if (pick == 2 && built) return kFused1dMfma512;
     if (pick == 3 && built) return kFused1dMfma256;
@@ -842,11 +650,22 @@ static bool wide_tiles(int logDY, long S, int N, int K, int algo, long cus)
     default: return K >= 64 ? blocks >= cus : blocks <= cus;
     }
 }
+// Output channels per block of the small-grid kernel: the fewest that leave every block a CU to itself. The blocks of a signal set repeat
+// each other's forward transforms, but they run side by side, and each has fewer backward transforms to do one after the other (us, 16 / 32 / 64
+// channels, N = 64: S = 1, K = 32: DY = 128 5.3 / 5.9 / 7.0, DY = 1024 13.8 / 18.0 / 23.5; S = 64, K = 8: DY = 512 8.3 / 8.6 / 12.4; S = 100: 12.9 / 8.5 / 9.4 at
+// DY = 256, K = 24). DY = 256 with eight channels keeps at least 32 (S = 1: 5.3 / 5.9): the size that turbofno_query_1d_tile has always named there.
+static int small_tile(int logDY, long S, int N, int K, long cus)
+{
+    if (S * (N / 16) <= cus && !(logDY == 8 && K <= 8)) return 16;
+    return S * (N / 32) <= cus ? 32 : 64;
+}
+static bool splits_channels_over_waves(long S, int N, int K, int algo, long cus) { return algo == 6 || (K >= 112 && 2 * S * (N / SPLIT_NT) > cus); }
 int tile_of_fused_1d_kernel(int kernel, int logDY, long S, int N, int K, int algo, long cus)
 {
     switch (kernel) {
-    case kFused1dMfma512Tile32: return 32;
-    case kFused1dSplitK: return SPLIT_NT;
+    case kFused1dMfma512: return algo == 2 ? 64 : small_tile(logDY, S, N, K, cus);
+    case kFused1dMfma512Tile32: return algo == 4 ? 32 : small_tile(logDY, S, N, K, cus);
+    case kFused1dSplitK: return splits_channels_over_waves(S, N, K, algo, cus) ? SPLIT_NT : small_tile(logDY, S, N, K, cus);
     case kFused1dCluster: return N;
     case kFused1dWide: return wide_tiles(logDY, S, N, K, algo, cus) ? 128 : 64;
     default: return 64;
@@ -875,33 +694,42 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
         return launch_fused_split(logDY, S, N, K, x, W, y, alpha, false, true, stream, keep_y);
     case kFused1dWide:
         return launch_fused_split(logDY, S, N, K, x, W, y, alpha, wide_tiles(logDY, S, N, K, algo, cus), dense_blocks(S, N, cus), stream, keep_y);
-    case kFused1dSplitK: return keep_y ? launch_fused_split_channels<true>(S, N, K, x, W, y, alpha, stream) : launch_fused_split_channels<false>(S, N, K, x, W, y, alpha, stream);
+    case kFused1dSplitK:
+        if (splits_channels_over_waves(S, N, K, algo, cus))
+            return keep_y ? launch_fused_split_channels<true>(S, N, K, x, W, y, alpha, stream) : launch_fused_split_channels<false>(S, N, K, x, W, y, alpha, stream);
+        [[fallthrough]];
     case kFused1dMfma512Tile32:
-        return logDY == 8 ? launch_fused_mfma<8, 32>(S, N, K, x, W, y, alpha, stream, keep_y)
-                          : launch_fused_mfma<7, 32>(S, N, K, x, W, y, alpha, stream, keep_y);
-    case kFused1dMfma512:
-        switch (logDY) {
-        case 7: return launch_fused_mfma<7>(S, N, K, x, W, y, alpha, stream, keep_y);
-        case 8: return launch_fused_mfma<8>(S, N, K, x, W, y, alpha, stream, keep_y);
-        case 9: return launch_fused_mfma<9>(S, N, K, x, W, y, alpha, stream, keep_y);
-        default: return launch_fused_mfma<10>(S, N, K, x, W, y, alpha, stream, keep_y);
-        }
+    case kFused1dMfma512: {
+        // y in the place of x: one block per signal set, so that nobody reads what another block has overwritten
+        const bool in_place = x < y + (long)N * S * (1L << logDY) && y < x + (long)K * S * (1L << logDY);
+        const int tile = in_place ? 64 : tile_of_fused_1d_kernel(kernel, logDY, S, N, K, algo, cus);
+        return launch_fused_small(logDY, S, N, K, x, W, y, alpha, tile, stream, keep_y);
+    }
     case kFused1dMfma256:
         return launch_fused_split(logDY, S, N, K, x, W, y, alpha, false, logDY <= 8 && dense_blocks(S, N, cus), stream, keep_y);
     default: return dispatch_fused_1d(logDY, S, N, K, x, W, y, alpha, stream, keep_y);
     }
 }
 
-// The halves of the layer. Few channels at lengths 512 / 1024: the SIMT kernel; with eight a round of 16 would be half padding (second
-// half, us, split / SIMT: DY = 512, S = 1 ... 128: 13.3 - 15.2 / 11.6 - 14.6, S = 1000: 58.5 / 54.8; DY = 1024, S = 1 ... 64: 22.6 / 19.5, but
-// with one block per CU, N = 64, S = 256: 24.5 / 26.8; with 16 channels only DY = 1024 on small grids: S = 1 ... 128: 23.3 - 24.7 /
-// 21.5 - 23.4. First half, with blocks of 64 output
-// channels: DY = 512, S = 4096: 54.2 / 50.8, DY = 1024, N = 64: S = 2048: 49.4 / 46.4, S = 700: 20.2 / 21.7). Otherwise the split kernel: halves, geometric mean of 1232 shapes against the SIMT kernel 0.66.
+// The halves of the layer. While every block of 64 output channels has a CU to itself: the small-grid kernel (us, split kernel / small-grid
+// kernel with 16, 32 or 64 output channels). First half: the fewest output channels pay from 32 input channels on and up to half of the CUs
+// (DY = 256, N = 64, K = 128: S = 1: 20.3 / 11.3, 12.5, 15.1, S = 64: 21.5 / 12.9, 13.5, 16.0; DY = 1024, K = 128, S = 64: 65.8 / 39.4, 36.7, 37.8; DY = 256, K = 8, S = 1:
+// 4.4 / 3.8, 4.0, 4.2); a block of 64 on every CU: DY = 128, K = 64, S = 256: 10.4 / 10.2, DY = 1024, K = 32: 21.0 / 16.1. Second half: DY = 256, K = 32, S = 1: 8.4 / 4.5, 5.3, 7.1;
+// DY = 1024, K = 8, S = 1: 19.4 / 6.3, 9.6, 15.8, S = 64: 21.1 / 9.2, 11.1, 17.3, S = 200: 25.7 / 22.4 with 64; but a block of 64 on every CU: DY = 256, N = 64, K = 8: 8.7 / 9.1 (N = 128:
+// 9.4 / 9.1), DY = 512: 14.8 / 15.4, DY = 1024: 26.8 / 28.1.
+// Larger grids: the SIMT kernel with few channels at lengths 512 / 1024; with eight a round of 16 would be half padding (second
+// half, us, split / SIMT: DY = 512, S = 1000: 58.5 / 54.8. First half, with blocks of 64 output
+// channels: DY = 512, S = 4096: 54.2 / 50.8, DY = 1024, N = 64: S = 2048: 49.4 / 46.4, S = 700: 20.2 / 21.7). Otherwise the split kernel: halves,
+// geometric mean of 1232 shapes against the SIMT kernel 0.66.
 hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C,
                                   float2 alpha, float2 beta, hipStream_t stream)
 {
-    // blocks of 128 output channels from one and a half per CU (N = 128, K = 64, DY = 256: S = 700 42.6 -> 34.4 us, S = 256 19.0 -> 19.9)
     const long cus = cu_count(), items = S * (N / 64);
+    if (items <= cus) {
+        const int tile = K >= 32 && 2 * S * (N / 16) <= cus ? 16 : (S * (N / 32) <= cus ? 32 : 64);
+        return launch_small_forward(logDY, S, N, K, x, W, C, alpha, beta, tile, stream);
+    }
+    // blocks of 128 output channels from one and a half per CU (N = 128, K = 64, DY = 256: S = 700 42.6 -> 34.4 us, S = 256 19.0 -> 19.9)
     const bool wide = N % 128 == 0 && 2 * S * (N / 128) >= 3 * cus;
     if (K <= 8 && !wide) {
         if (logDY == 9) return launch_fused_1d_k<9, true, false, false>(S, N, K, x, W, C, alpha, beta, stream);
@@ -915,8 +743,13 @@ hipError_t launch_fused_cgemm_ifft(int logDY, long S, int N, int K, const float2
 {
     const float2 beta = make_float2(0.f, 0.f);
     const long cus = cu_count(), items = S * (N / 64);
-    if (K <= 8 && logDY == 9) return launch_fused_1d_k<9, false, true, false>(S, N, K, A, W, y, alpha, beta, stream);
-    if (logDY == 10 && (4 * items < 3 * cus ? K <= 16 : K <= 8 && items > cus)) return launch_fused_1d_k<10, false, true, false>(S, N, K, A, W, y, alpha, beta, stream);
+    if (items <= cus && (logDY == 7 || (logDY == 8 && N % 128 == 0) || 8 * items <= 7 * cus)) {
+        const int tile = S * (N / 16) <= cus ? 16 : (S * (N / 32) <= cus ? 32 : 64);
+        return launch_small_backward(logDY, S, N, K, A, W, y, alpha, tile, stream);
+    }
+    if (K <= 8 && (logDY == 9 || (logDY == 10 && items > cus)))
+        return logDY == 9 ? launch_fused_1d_k<9, false, true, false>(S, N, K, A, W, y, alpha, beta, stream)
+                          : launch_fused_1d_k<10, false, true, false>(S, N, K, A, W, y, alpha, beta, stream);
     return launch_split_backward(logDY, S, N, K, A, W, y, alpha, stream);
 }
 

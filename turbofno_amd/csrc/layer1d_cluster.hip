@@ -7,7 +7,7 @@
 // repetition is the critical path. Here member q of a cluster
 //   1. transforms channels [q K/P, (q+1) K/P) of the signal set (32 at a time, one per 16-lane group),
 //   2. multiplies them with the matching rows of W for ALL N output channels on v_mfma_f32_16x16x4_f32
-//      (spectra and the real-expanded W' tile staged through LDS as in fused_fft_mfma_ifft_kernel),
+//      (spectra and the real-expanded W' tile staged through LDS),
 //   3. publishes the partial products of the output channels it does not own to the other members through device
 //      memory, keeps its own N/P channels in LDS,
 //   4. waits (bounded) until all P members have published, adds the P-1 foreign partials to its own, runs the

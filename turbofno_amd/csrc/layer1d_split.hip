@@ -62,24 +62,6 @@ template <int COUNT> TFNO_DEV void after(int& offset, const cpx (&g)[COUNT])
     for (int i = 0; i < COUNT; ++i) asm volatile("" : "+v"(offset) : "v"(g[i].x));
 }
 
-// First pass of two signals of 128 samples: v[0..7], v[8..15] are samples t + 16 i of each.
-TFNO_DEV void pair_first_pass(const cpx (&v)[16], const cpx* twrow, cpx (&gg)[16])
-{
-    cpx a8[8], b8[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) { a8[i] = v[i]; b8[i] = v[8 + i]; }
-    fft8<-1>(a8);
-    fft8<-1>(b8);
-    gg[0] = a8[0];
-    gg[8] = b8[0];
-#pragma unroll
-    for (int r = 1; r < 8; ++r) {
-        const cpx w = twrow[r];
-        gg[r] = cmul(a8[r], w);
-        gg[8 + r] = cmul(b8[r], w);
-    }
-}
-
 // The product of one wave in fp32, for operands that the split does not hold: the wave transforms all K channels by itself, as many at
 // a time as it has lane groups for, and takes its 16 NTW output channels from them four channels at a time. Several times as slow as
 // the loop that it stands in for. `region`: the exchange regions of the wave, free of other use.
@@ -110,7 +92,7 @@ TFNO_DEV void product_fp32(long S, int K, long s, int nw, int nstep, const float
                 cpx out[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) { v[i] = p[16 * i]; v[8 + i] = p[S * DY + 16 * i]; }
-                pair_first_pass(v, twrow, gg);
+                pair128_first_pass(v, twrow, gg);
                 rows128_forward_finish(gg, exch, t, out);
                 wave_lds_fence();
 #pragma unroll
@@ -120,7 +102,7 @@ TFNO_DEV void product_fp32(long S, int K, long s, int nw, int nstep, const float
 #pragma unroll
                 for (int i = 0; i < 16; ++i) v[i] = p[L * i];
                 fwd_pass1_lds(v, twrow, gg);
-                if constexpr (L > 16) wide_forward_finish<L, true>(gg, exch, powers, t, out);
+                if constexpr (L > 16) wide_forward_finish<L, true, L == 64>(gg, exch, powers, t, out);
                 else group_forward_finish<8>(gg, exch, t, out);
                 wave_lds_fence();
 #pragma unroll
@@ -238,7 +220,7 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
             } else if (busy) {
                 cpx gg[16];
                 if constexpr (PAIR) {
-                    pair_first_pass(v, twrow, gg);
+                    pair128_first_pass(v, twrow, gg);
                 } else {
                     fft16<-1>(v);
                     int row = 0;
@@ -261,7 +243,7 @@ __global__ __launch_bounds__(256, BLOCKS) void fused_fft_split_ifft_kernel(int S
                 }
                 if constexpr (!LATE) issue(kc + (pass + 1) * CP, later);
                 if constexpr (PAIR) rows128_forward_finish(gg, exch, t, out);
-                else if constexpr (LONG) wide_forward_finish<L, true>(gg, exch, powers, t, out);
+                else if constexpr (LONG) wide_forward_finish<L, true, L == 64>(gg, exch, powers, t, out);
                 else group_forward_finish<8>(gg, exch, t, out);
                 if constexpr (LATE) {
                     later = 0;
