@@ -389,7 +389,8 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
 // Rows of a tile are 16 output channels n, columns 16 consecutive m, contraction in steps of 32 channels (eight per lane
 // of a quarter wavefront). A wave owns 16 m and all 16 NT output channels of its block: an element of A is loaded and split
 // once per block, and its parts meet NT fragments of W read from LDS. The W tile holds the parts of alpha W as fragments
-// in lane order, 6 x 1 KiB per (step, 16 channels): an operand is one conflict-free 16-byte read.
+// in lane order, 6 x 1 KiB per (step, 16 channels): an operand is one conflict-free 16-byte read. With HALVES a step is two of 16 channels whose
+// (re, im) pairs share one instruction, so that a last step of at most 16 channels costs half (see launch_cgemm_modes).
 // Blocks are persistent over column blocks (XCD j takes the j-th eighth of them, so that an XCD keeps to one part of the
 // memory system); the strip of the next step - of the next column block after the last - is requested before the matrix
 // work of the current one, and nothing in the walk waits at a barrier, so loads, matrix work and stores of the waves overlap.
@@ -405,7 +406,7 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
 constexpr int GEMM_KSTEP = 32;
 constexpr size_t kSplitStepBytes = 6 * 1024;            // LDS of one step of 16 output channels
 
-template <int NT, int THREADS>
+template <int NT, int THREADS, bool HALVES>
 __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_split_kernel(
     const float2* __restrict__ A, const float2* __restrict__ W, float2* __restrict__ C, long Mtot, int K, float2 alpha,
     float2 beta, long nblocks, int Kw, int Kp, int cap)
@@ -424,47 +425,64 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
     // they are issued: lanes beyond the run (its last step may be short) read the first channels of the step again - the tile
     // holds zeros there - and waves beyond the last column read the first strip (nothing is stored from it). `live` is false
     // after the last step of the block: every lane then reads one line.
-    const unsigned lane_row = (unsigned)(8 * kq * Mtot), lane_col = wave * 16 + col;
+    // HALVES: channels 4 kq ... 4 kq + 3 of both halves of the step.
+    constexpr int PER_LANE = HALVES ? 4 : 8;            // consecutive channels of a lane
+    const unsigned lane_row = (unsigned)(PER_LANE * kq * Mtot), lane_col = wave * 16 + col;
     float2 bv[8];
     auto fetch = [&](long mb, int run, int step, bool live) {
         const bool column = mb * MBLOCK + wave * 16 < Mtot;       // Mtot is a multiple of 16; Kp of 8
         const float2* base = A + (column ? mb * MBLOCK : 0) + (long)(run * Kp + GEMM_KSTEP * step) * Mtot;    // uniform
-        const unsigned off = live ? (column ? lane_col : (unsigned)col) + (GEMM_KSTEP * step + 8 * kq < Kp ? lane_row : 0u) : 0u;
+        const int left = Kp - GEMM_KSTEP * step - PER_LANE * kq;  // channels of the step from the lane's first on
+        const unsigned first = live ? (column ? lane_col : (unsigned)col) : 0u;
+        if constexpr (HALVES) {
+            const unsigned off = live && left > 0 ? first + lane_row : first, row = live && left > 0 ? (unsigned)Mtot : 0u;
+            const bool second = live && left > 16;
+            const float2* upper = base + (second ? 16 * Mtot + (long)(first + lane_row) : (long)first);
+            const unsigned upper_row = second ? (unsigned)Mtot : 0u;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) bv[j] = (base + j * Mtot)[off];
+            for (int j = 0; j < 4; ++j) { bv[j] = base[off + j * row]; bv[4 + j] = upper[j * upper_row]; }
+        } else {
+            const unsigned off = first + (live && left > 0 ? lane_row : 0u);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) bv[j] = (base + j * Mtot)[off];
+        }
     };
-    // fragments of the steps s0 ... s0 + count - 1: entry (step, tile, kq, n mod 16) = eight consecutive channels of one n
+    // fragments of the steps s0 ... s0 + count - 1: entry (step, tile, kq, n mod 16) = eight consecutive channels of one n, real and imaginary
+    // parts apart. HALVES: entry (half step, tile, kq, n mod 16) = four consecutive channels as (re, im) pairs
     bool low_weights = false;                           // once seen it holds for all column blocks: they share the weights
     auto build = [&](int s0, int count) {
-        for (int e = tid; e < count * NT * 64; e += THREADS) {
+        for (int e = tid; e < (HALVES ? 2 : 1) * count * NT * 64; e += THREADS) {
             const int l = e & 63, t = (e >> 6) % NT, s = (e >> 6) / NT;
-            const int k = GEMM_KSTEP * (s0 + s) + 8 * (l >> 4), n = n0 + 16 * t + (l & 15);
-            SplitOperand re, im;
-            float2 w[8];
+            const int k = GEMM_KSTEP * s0 + (HALVES ? 16 : GEMM_KSTEP) * s + PER_LANE * (l >> 4), n = n0 + 16 * t + (l & 15);
+            float2 w[PER_LANE];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) w[j] = make_float2(0.f, 0.f);
+            for (int j = 0; j < PER_LANE; ++j) w[j] = make_float2(0.f, 0.f);
             if (k < Kp) {
                 const float2* src = W + (k % Kw) + (long)n * Kw;    // Kw is a multiple of 8
 #pragma unroll
-                for (int j = 0; j < 8; ++j) w[j] = src[j];
+                for (int j = 0; j < PER_LANE; ++j) w[j] = src[j];
             }
 #pragma unroll
-            for (int j = 0; j < 8; ++j) w[j] = make_float2(w[j].x * alpha.x - w[j].y * alpha.y, w[j].x * alpha.y + w[j].y * alpha.x);
+            for (int j = 0; j < PER_LANE; ++j) w[j] = make_float2(w[j].x * alpha.x - w[j].y * alpha.y, w[j].x * alpha.y + w[j].y * alpha.x);
             unsigned bits = ~0u;                        // (zeros are common here: channels beyond Kp)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) bits = lower(bits, w[j]);
+            for (int j = 0; j < PER_LANE; ++j) bits = lower(bits, w[j]);
             low_weights |= any_lane(bits < kSplitLow);
+            SplitOperand re, im;                        // HALVES: re holds the pairs
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 unsigned h, m, lo;
-                split_bf16_pair(w[2 * j].x, w[2 * j + 1].x, h, m, lo);
+                if constexpr (HALVES) split_bf16_pair(w[j].x, w[j].y, h, m, lo);
+                else split_bf16_pair(w[2 * j].x, w[2 * j + 1].x, h, m, lo);
                 re.h[j] = h; re.m[j] = m; re.l[j] = lo;
-                split_bf16_pair(w[2 * j].y, w[2 * j + 1].y, h, m, lo);
-                im.h[j] = h; im.m[j] = m; im.l[j] = lo;
+                if constexpr (!HALVES) {
+                    split_bf16_pair(w[2 * j].y, w[2 * j + 1].y, h, m, lo);
+                    im.h[j] = h; im.m[j] = m; im.l[j] = lo;
+                }
             }
-            uint4_v* dst = sW4 + (e >> 6) * 384 + l;
+            uint4_v* dst = sW4 + (e >> 6) * (HALVES ? 192 : 384) + l;
             dst[0] = re.h; dst[64] = re.m; dst[128] = re.l;
-            dst[192] = im.h; dst[256] = im.m; dst[320] = im.l;
+            if constexpr (!HALVES) { dst[192] = im.h; dst[256] = im.m; dst[320] = im.l; }
         }
         if (lane == 0) sLow[wave] = low_weights;
     };
@@ -489,16 +507,19 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
             low_tile |= sLow[lane & (THREADS / 64 - 1)];
             built = true;
         }
-        SplitOperand ar, ai;
+        SplitOperand ar, ai;                            // HALVES: the (re, im) pairs of the two halves
         low_column |= below_split_range(bv);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             unsigned h, m, l;
-            split_bf16_pair(bv[2 * j].x, bv[2 * j + 1].x, h, m, l);
+            if constexpr (HALVES) split_bf16_pair(bv[j].x, bv[j].y, h, m, l);
+            else split_bf16_pair(bv[2 * j].x, bv[2 * j + 1].x, h, m, l);
             ar.h[j] = h; ar.m[j] = m; ar.l[j] = l;
-            split_bf16_pair(bv[2 * j].y, bv[2 * j + 1].y, h, m, l);
+            if constexpr (HALVES) split_bf16_pair(bv[4 + j].x, bv[4 + j].y, h, m, l);
+            else split_bf16_pair(bv[2 * j].y, bv[2 * j + 1].y, h, m, l);
             ai.h[j] = h; ai.m[j] = m; ai.l[j] = l;
         }
+        const bool both = GEMM_KSTEP * step + 16 < Kp;  // HALVES: the second half has channels; uniform
         asm volatile("" ::: "memory");                  // operand reads of the tile stay inside the loop
         const bool run_ends = step + 1 == steps, last = run_ends && run + 1 == runs;
         const bool more = v + gridDim.x < nblocks;
@@ -507,17 +528,39 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
         fetch(next_mb, next_run, next_step, !last || more);
         __builtin_amdgcn_sched_barrier(0);
         const uint4_v* frag = sW4 + slot * (NT * 384) + lane;
+        if constexpr (HALVES) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            SplitOperand w{ frag[t * 384], frag[t * 384 + 64], frag[t * 384 + 128] };
-            float4_v r = re[t], i = im[t];
-            mac_split2(w, ar, ai, r, i);                            // Wr
-            w = SplitOperand{ frag[t * 384 + 192], frag[t * 384 + 256], frag[t * 384 + 320] };
-            i = mac_split(w, ar, i);                                // Wi
-            w.h ^= 0x80008000u; w.m ^= 0x80008000u; w.l ^= 0x80008000u;
-            r = mac_split(w, ai, r);                                // - Wi
-            re[t] = r;
-            im[t] = i;
+            for (int u = 0; u < 2; ++u) {
+                if (u == 1 && !both) break;
+                const SplitOperand& a = u == 0 ? ar : ai;
+                SplitOperand for_re, for_im;            // (re, -im) and (im, re): with (re, im) of a weight the real and the imaginary part
+                for_re.h = a.h ^ 0x80000000u; for_re.m = a.m ^ 0x80000000u; for_re.l = a.l ^ 0x80000000u;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    for_im.h[j] = __builtin_amdgcn_alignbit(a.h[j], a.h[j], 16);
+                    for_im.m[j] = __builtin_amdgcn_alignbit(a.m[j], a.m[j], 16);
+                    for_im.l[j] = __builtin_amdgcn_alignbit(a.l[j], a.l[j], 16);
+                }
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const uint4_v* f = frag + (u * NT + t) * 192;
+                    const SplitOperand w{ f[0], f[64], f[128] };
+                    mac_split2(w, for_re, for_im, re[t], im[t]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                SplitOperand w{ frag[t * 384], frag[t * 384 + 64], frag[t * 384 + 128] };
+                float4_v r = re[t], i = im[t];
+                mac_split2(w, ar, ai, r, i);                            // Wr
+                w = SplitOperand{ frag[t * 384 + 192], frag[t * 384 + 256], frag[t * 384 + 320] };
+                i = mac_split(w, ar, i);                                // Wi
+                w.h ^= 0x80008000u; w.m ^= 0x80008000u; w.l ^= 0x80008000u;
+                r = mac_split(w, ai, r);                                // - Wi
+                re[t] = r;
+                im[t] = i;
+            }
         }
         if (last) {
             if (mb * MBLOCK + wave * 16 < Mtot) {
@@ -577,8 +620,7 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
     }
 }
 
-// Few channels (K <= 16; K <= 32 in one range of sizes, see launch_cgemm_modes): a step of 32 channels would be mostly
-// padding. fp32 matrix instructions over groups of four channels instead, three real products per complex one:
+// Few channels on some large products (K <= 16; K <= 32 in one range of sizes, see launch_cgemm_modes): fp32 matrix instructions over groups of four channels instead, three real products per complex one:
 //   P1 = c (a + b),  P2 = (d - c) a,  P3 = (c + d) b   =>   re = P1 - P3,  im = P1 + P2      (alpha W = c + i d, A = a + i b)
 // A block is 16 waves; wave w owns the 16-m strip w and 64 output channels; the strip sits in NG float2 registers per
 // lane, all loads in flight while the W'' tile is built, and every n tile is stored as soon as it is complete.
@@ -815,9 +857,12 @@ hipError_t launch_ifft2d_pad(int logDX, int logDY, const float2* spec, float2* y
 
 // Which kernel (times for the stand-alone product on operands that come from HBM, in us, column of the kernel before /
 // this one):
-//  * K <= 16: fp32 matrix instructions (M = 262,144, N = 128, K = 16: 55 against 74 with a step of 32 channels); with
-//    several column blocks per CU the persistent kernel. K <= 32 as well for N >= 128 and 8 to 16 blocks of 256 columns x 64
-//    output channels per CU (M = 262,144, N = 128, K = 32: 77 against 88 us; from 16 on the 128-channel tile below is ahead).
+//  * K <= 16: the split kernel (half a step) up to five blocks of 256 columns x 64 output channels per CU for N = 64 and multiples of 128, two for
+//    others, and for multiples of 128 from sixteen on (fp32 / split: K = 16, M = 4,096, N = 64, with beta: 9.5 / 7.4; M = 98,304: N = 64 16.0 / 13.1, N = 128
+//    23.1 / 20.5; M = 163,840, N = 128: 35.6 / 32.0; M = 524,288, N = 128: 157 / 136). Between, fp32 matrix instructions, with
+//    several column blocks per CU the persistent kernel (M = 262,144: N = 128 55.3 / 64.7, N = 192 78.8 / 114; M = 524,288, N = 64: 75.8 / 77.7; M =
+//    65,536, N = 192: 23.0 / 23.7). K <= 32 as well for N >= 128 and 8 to 16 such blocks
+//    per CU (M = 262,144, N = 128, K = 32: 77 against 88 us; from 16 on the 128-channel tile below is ahead).
 //  * otherwise the split kernel. Small products: blocks of 128 columns and the fewest output channels whose grid still fits one
 //    block per CU (K = 64, N = 64, tiles of 64 / 32 / 16 output channels: M = 64: 7.5 / 5.5 / 4.7; M = 8,192: 8.5 / 6.3 / 5.5; M = 16,384:
 //    9.1 / 6.9; N = 192, M = 4,096: 9.0 / 7.1).
@@ -846,27 +891,30 @@ hipError_t launch_cgemm_modes(const float2* A, const float2* W, float2* C, long 
                            stream, A, W, C, Mtot, N, K, alpha, columns, Kw);
         return hipGetLastError();
     };
+    const bool split_ahead = N % 128 == 0 || N == 64 ? blocks <= 5 * cus || (no_beta && N % 128 == 0 && blocks >= 16 * cus) : blocks <= 2 * cus;
+    const bool few = K <= 16 && !split_ahead;
     // Persistent not with beta: reading C back inside the walk waits for the strip requested just before it
     // (K = 32, M = 262,144: 79 against 74 us).
-    if (K <= 16 && no_beta && columns >= 2 * cus) return launch_persistent(std::integral_constant<int, 4>{});
+    if (few && no_beta && columns >= 2 * cus) return launch_persistent(std::integral_constant<int, 4>{});
     if (K > 16 && K <= 32 && no_beta && N >= 128 && blocks >= 8 * cus && blocks < 16 * cus)
         return launch_persistent(std::integral_constant<int, 8>{});
-    if (K <= 16) {
+    if (few) {
         hipLaunchKernelGGL((cgemm_modes3m_kernel<4>), dim3((unsigned)columns, (unsigned)(N / 64), 1), dim3(GEMM_THREADS), 0, stream, A,
                            W, C, Mtot, N, K, alpha, beta, Kw);
         return hipGetLastError();
     }
 
     // cap: steps of 32 channels that the tile can hold; per_cu: blocks per CU
-    auto launch_split = [&](auto nt_const, auto threads_const, int cap, int per_cu) -> hipError_t {
+    auto launch_split_as = [&](auto nt_const, auto threads_const, auto halves_const, int cap, int per_cu) -> hipError_t {
         constexpr int NT = decltype(nt_const)::value, THREADS = decltype(threads_const)::value;
+        constexpr bool HALVES = decltype(halves_const)::value;
         // one run over the tile covers one period of the weights where that wastes no part of a step, or else all K
         // channels, if the tile can hold them
         const bool periods = Kw % GEMM_KSTEP == 0 || (K + GEMM_KSTEP - 1) / GEMM_KSTEP > cap;
         const int Kp = periods ? Kw : K, steps = (Kp + GEMM_KSTEP - 1) / GEMM_KSTEP;
         const size_t lds_bytes = kSplitStepBytes * NT * (steps < cap ? steps : cap);
         static std::atomic<unsigned long long> served;
-        if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(cgemm_modes_split_kernel<NT, THREADS>), kSplitStepBytes * NT * cap, served);
+        if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(cgemm_modes_split_kernel<NT, THREADS, HALVES>), kSplitStepBytes * NT * cap, served);
             e != hipSuccess)
             return e;
         const long nblocks = (Mtot + THREADS / 4 - 1) / (THREADS / 4), tiles = N / (16 * NT);
@@ -875,9 +923,18 @@ hipError_t launch_cgemm_modes(const float2* A, const float2* W, float2* C, long 
         if (g >= 8) g -= g % 8;
         if (g < 1) g = 1;
         if (g > nblocks) g = nblocks;
-        hipLaunchKernelGGL((cgemm_modes_split_kernel<NT, THREADS>), dim3((unsigned)g, (unsigned)tiles, 1), dim3(THREADS), lds_bytes, stream,
+        hipLaunchKernelGGL((cgemm_modes_split_kernel<NT, THREADS, HALVES>), dim3((unsigned)g, (unsigned)tiles, 1), dim3(THREADS), lds_bytes, stream,
                            A, W, C, Mtot, K, alpha, beta, nblocks, Kw, Kp, cap);
         return hipGetLastError();
+    };
+    // A last step of at most 16 channels: steps in halves, the empty one skipped (us, whole steps / halves: M = 163,840, N = 128: K = 40 52.4 / 47.4,
+    // K = 72 75.2 / 70.2, K = 104 102.2 / 98.3; M = 65,536, N = 64: 14.6 / 14.2, 19.3 / 18.7, 23.7 / 23.3). Not where it is not needed (K = 64, M = 163,840, N = 128: 56.5 / 58.1),
+    // and on small products, whose tiles of 16 or 32 outputs have more per column to rearrange, up to 48 channels (M = 4,096, N = 64: K = 40 5.0 / 4.9, K = 72
+    // 5.9 / 5.9, K = 104 6.9 / 7.1); nor beyond 128 (K = 200, M = 65,536, N = 64: 42.2 / 43.4).
+    auto launch_split = [&](auto nt, auto threads, int cap, int per_cu) {
+        const int last = Kw % GEMM_KSTEP;
+        if (last > 0 && last <= GEMM_KSTEP / 2 && Kw <= (decltype(nt)::value >= 4 ? 128 : 48)) return launch_split_as(nt, threads, std::true_type{}, cap, per_cu);
+        return launch_split_as(nt, threads, std::false_type{}, cap, per_cu);
     };
     using Tiles4 = std::integral_constant<int, 4>;
     using Tiles8 = std::integral_constant<int, 8>;
