@@ -90,9 +90,9 @@ int turbofno_layer_1d(int bs, int dimX, int DY, int K, int N, const void* x, con
  * (fusion_variants/2D_D_exp_fused_fft_cgemm_ifft/fused_trunc_2D.cu:133-172). The reference keeps its
  * intermediates t1/t2 in buffers owned by main(); here the caller passes `workspace` of at least
  * turbofno_layer_2d_workspace_bytes(...) bytes (256-byte aligned). x is not modified.
- * algo: TURBOFNO_2D_AUTO picks by size (lengths up to 256: WHOLE_IMAGE from a batch of 8, and from a batch of 4 when
- * there are enough images; THREE_KERNEL below; longer axes: WHOLE_IMAGE from 0.6 to 4.5 GiB of input and output,
- * depending on the lengths, else ROWS_FIRST or THREE_KERNEL); the workspace query with the same arguments,
+ * algo: TURBOFNO_2D_AUTO picks by size (lengths up to 256: WHOLE_IMAGE from a batch of 8, and from smaller ones when
+ * there are enough images or channels; mostly THREE_KERNEL below; longer axes: WHOLE_IMAGE from 0.6 to 4.5 GiB of input and
+ * output, depending on the lengths, and earlier with many channels, else ROWS_FIRST or THREE_KERNEL); the workspace query with the same arguments,
  * and turbofno_query_2d_algo, make the same
  * choice. Every algorithm takes every pair of lengths in {128, 256, 512, 1024} (WHOLE_IMAGE handles images of 512 or
  * 1024 rows as two or four interleaved parts of 256 rows that the contraction sums over). ROWS_FIRST is the three-stage structure with the axes exchanged

@@ -50,15 +50,50 @@ int check_gemm_dims(long M, int N, int K)
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// Many input channels for the number of images: the three-stage paths run their middle stage at the rate of its transforms and products, in
+// blocks that repeat the forward transforms, while the whole-image path has the mode GEMM and two image kernels with one block per image (or part
+// of one). It is ahead at smaller sizes the more channels there are, provided the rounds of 256 blocks of its two kernels are reasonably full: 264
+// images are two rounds. Measured on MI355X, three stages (the better order) / whole image, us:
+//   128 x 128: bs = 12, K = 64, N = 64: 71.4 / 63.9; bs = 6, K = 88, N = 64: 1.06 the other way, N = 128: 0.99
+//   128 x 256: bs = 3, K = 64, N = 64: 41.9 / 38.4; bs = 6, K = 112: 87 / 81 (108 for the order that was taken); bs = 2, K = 64, N = 64: 1.03 the other way, K = 136 (272 images): 44.6 / 46.0
+//   256 x 128: bs = 12, K = 64, N = 64: 114 / 102; bs = 10, K = 64: 1.04 the other way
+//   256 x 256: bs = 2, K = 112, N = 64: 56.5 / 53.0; bs = 4, K = 112: 102 / 91; bs = 3, K = 88 (264 images): 1.08 the other way
+//   256 x 512: bs = 2, K = 112, N = 64: 95 / 85, bs = 4, K = 72 (288 images): 138 / 145; 512 x 256: bs = 3, K = 112: 145 / 128, bs = 2, K = 104: 83 / 88, bs = 3, K = 48 (288 parts): 1.17 the other way
+//   512 x 512: bs = 1, K = 112, N = 64: 101 / 86, bs = 2, K = 48, N = 64: level; 1024 x 256: bs = 3, K = 112: 260 / 240; 1024 x 512: bs = 1, K = 112: 186 / 170;
+//   1024 x 1024: bs = 1, K = 112: 317 / 302
+// The intermediates of the whole-image path are the smaller ones at all of these lengths.
+bool whole_image_ahead_by_channels(int bs, int lx, int ly, int K, int N)
+{
+    const long parts = lx > 1 ? 1L << (lx - 1) : 1, forward = parts * K * bs, backward = parts * N * bs;
+    const long rounds = (forward + 255) / 256 + (backward + 255) / 256;
+    auto filled = [&](long percent) { return 100 * (forward + backward) >= percent * 256 * rounds; };
+    switch (4 * lx + ly) {                              // log2 DX - 7, log2 DY - 7
+    case 0: return forward >= (N >= 128 ? 430 : 600);
+    case 1: return forward >= (N >= 128 ? 120 : 144) && (forward <= 256 || forward >= 300 || filled(58));
+    case 4: return forward >= 760;
+    case 5: return forward >= (N >= 128 ? 160 : 240) && filled(74);
+    case 6: return forward >= 200 && (forward <= 256 || forward >= 350) && filled(68);
+    case 9: return forward >= 440 && filled(82);
+    case 10: return forward >= 190 && filled(68) && (K >= 96 || N >= 128);
+    case 13: return forward >= 890;
+    case 14: return (forward >= 440 && K >= 96) || forward >= 900;
+    case 15: return forward >= 440 && K >= 96;
+    default: return false;
+    }
+}
+
 // AUTO: the whole-image path runs one persistent block per image and moves 2/3 of the bytes of the three-kernel path,
 // which in turn spreads an image over many blocks and gets three short launches through sooner when there are few
 // images. Measured on MI355X (256 CUs; 160 shapes, both paths back to back): from a batch of 8 the whole-image path is
 // ahead (by up to 2x at bs = 16) but for two groups of shapes (below); with a batch of 4 to 7 it is ahead for 256 x 256
-// images once (K + N) * bs reaches 768 images in and out, and for 128 x 256 images with N >= 128; below a batch of 4 the
-// three-kernel path is 12-100 % ahead everywhere.
+// images once (K + N) * bs reaches 768 images in and out, and for 128 x 256 images with N >= 128; with many channels earlier (above). Otherwise
+// three stages, X axis first; whole rows of 128 x 256 images first while the grids are smallest, because their intermediates are half as large (bs = 1, K =
+// 40, N = 64: 22.9 / 20.3, K = 88: 1.06 the other way; bs = 2, K = 16: 26.7 / 24.7, N = 128: 36.3 / 36.1).
 int pick_algo(int bs, int DX, int DY, int K, int N, int algo)
 {
     if (algo != TURBOFNO_2D_AUTO) return algo;
+    if (length_built(log2_exact(DX)) && length_built(log2_exact(DY)) && whole_image_ahead_by_channels(bs, log2_exact(DX) - 7, log2_exact(DY) - 7, K, N))
+        return TURBOFNO_2D_WHOLE_IMAGE;
     if (DX > 256 || DY > 256) {
         // Long axes on the whole-image kernels (512 / 1024 rows as interleaved parts of 256, rows of 512 / 1024 with 32 /
         // 64 lanes each): x and y move once and nothing but 64 x 64 modes in between, against intermediates of 1/8 (length
@@ -76,10 +111,18 @@ int pick_algo(int bs, int DX, int DY, int K, int N, int algo)
         // otherwise three stages. The axis that is transformed first is the one whose
         // truncation shrinks the intermediates most, i.e. the longer one (DY = 4 DX: half the time of the other order;
         // DX = 4 DY: the reverse). Square images: whole rows first (9-18 % ahead) unless the grid is small.
+        // The smallest problems with DX of 256 or 512 are sooner through with the X axis first, whose kernels have more and smaller blocks (rows first / X
+        // axis first: 256 x 512, bs = 1: K = 16, N = 64 34.8 / 32.7, N = 128 51.5 / 45.7, K = 112 31 / 33; 256 x 1024, K = 16: 51.8 / 49.3, K = 32: 56.2 / 59.6; 512 x 1024, K
+        // = 16: 85.4 / 79.0). Its intermediates are larger there, at most 60 MiB below these limits.
+        const long mib = ((long)K + N) * bs * DX * DY >> 17;
+        if ((DX == 256 && DY == 512 && mib <= 240 && K <= 64) || (DX == 256 && DY == 1024 && mib <= 240 && K <= 16) ||
+            (DX == 512 && DY == 1024 && mib <= 320 && K <= 32))
+            return TURBOFNO_2D_THREE_KERNEL;
         if (DY != DX) return DY > DX ? TURBOFNO_2D_ROWS_FIRST : TURBOFNO_2D_THREE_KERNEL;
         return (DY >= 1024 || (long)K * bs >= 128) ? TURBOFNO_2D_ROWS_FIRST : TURBOFNO_2D_THREE_KERNEL;
     }
     if (bs >= 16) return TURBOFNO_2D_WHOLE_IMAGE;
+    if (DX == 128 && DY == 256 && ((bs == 1 && K <= 64) || (bs == 2 && N == 64 && K <= 24))) return TURBOFNO_2D_ROWS_FIRST;
     if (bs < 4) return TURBOFNO_2D_THREE_KERNEL;
     const bool big = DX == 256 && DY == 256;
     if (bs >= 8) {
