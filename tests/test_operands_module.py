@@ -1,0 +1,97 @@
+"""The compiled operand checks of the binding (csrc/operands.cpp) against the checks in Python: what one takes the other takes with the same
+result, what one refuses the other refuses with the same error."""
+import numpy as np
+import pytest
+import torch
+
+import turbofno_amd as tf
+from turbofno_amd import api
+
+needs_module = pytest.mark.skipif(api._operands is None, reason="extension not built")
+
+
+def _c64(*shape, device):
+    return torch.zeros(shape, dtype=torch.complex64, device=device)
+
+
+def _forms(device):
+    """(name, call): every call site of the module, with operands right and wrong in one respect each"""
+    z = lambda *s: _c64(*s, device=device)
+    K, S, D, N = 8, 2, 128, 64
+    x, W, y = z(K, S, D), z(N, K), z(N, S, D)
+    x2, y2 = z(K, 1, 128, 128), z(N, 1, 128, 128)
+    ws = torch.zeros(tf.layer_2d_workspace_bytes(1, 128, 128, K, N), dtype=torch.uint8, device=device)
+    wide = z(K, S, 2 * D)
+    one = [
+        ("plain", (x, W, y), {}), ("parameter", (torch.nn.Parameter(x), W, y), {}), ("view", (wide.view(-1)[:K * S * D].view(K, S, D), W, y), {}),
+        ("offset by one value", (wide.view(-1)[1:1 + K * S * D].view(K, S, D), W, y), {}), ("strided", (wide[:, :, ::2], W, y), {}),
+        ("transposed W", (x, z(K, N).t(), y), {}), ("double", (x.to(torch.complex128), W, y), {}), ("real", (x.real.contiguous(), W, y), {}),
+        ("two dimensions", (x.view(K, S * D), W, y), {}), ("W of other K", (x, z(N, K + 8), y), {}), ("y of other N", (x, W, z(2 * N, S, D)), {}),
+        ("K no multiple of 8", (z(4, S, D), z(N, 4), y), {}), ("length not built", (z(K, S, 200), W, z(N, S, 200)), {}), ("array", (np.zeros((K, S, D), np.complex64), W, y), {}),
+        ("alpha real", (x, W, y), dict(alpha=2)), ("alpha text", (x, W, y), dict(alpha="1+2j")), ("alpha wrong", (x, W, y), dict(alpha="one")), ("alpha none", (x, W, y), dict(alpha=None)),
+        ("dimX", (x, W, y), dict(dimX=2)), ("dimX no divisor", (x, W, y), dict(dimX=3)), ("dimX zero", (x, W, y), dict(dimX=0)), ("dimX numpy", (x, W, y), dict(dimX=np.int64(2))),
+        ("no y", (x, W), {}), ("no signals", (z(K, 0, D), W, z(N, 0, D)), {}), ("conjugate view", (x.conj(), W, y), {}),
+    ]
+    two = [
+        ("plain", (x2, W, y2), dict(workspace=ws)), ("small workspace", (x2, W, y2), dict(workspace=ws[:-256])), ("no workspace", (x2, W, y2), {}),
+        ("float workspace", (x2, W, y2), dict(workspace=ws.float())), ("misaligned workspace", (x2, W, y2), dict(workspace=ws[8:])),
+        ("strided workspace", (x2, W, y2), dict(workspace=ws[::2])), ("algo 9", (x2, W, y2), dict(workspace=ws, algo=9)), ("algo -1", (x2, W, y2), dict(workspace=ws, algo=-1)),
+        ("y transposed", (x2, W, y2.transpose(2, 3)), dict(workspace=ws)), ("W of other K", (x2, z(N, 16), y2), dict(workspace=ws)),
+    ]
+    M = 64 * S
+    A, C = z(K, M), z(N, M)
+    rest = [
+        ("cgemm", lambda: tf.cgemm(M, N, K, A, W, C)), ("cgemm sizes", lambda: tf.cgemm(M, N, K + 8, A, W, C)), ("cgemm strided", lambda: tf.cgemm(M // 2, N, K, A[:, ::2], W, C)),
+        ("cgemm float size", lambda: tf.cgemm(float(M), N, K, A, W, C)),
+        ("fused", lambda: tf.fused_fft_cgemm_ifft(M, N, K, x, W, y)), ("fused sizes", lambda: tf.fused_fft_cgemm_ifft(2 * M, N, K, x, W, y)),
+        ("first half", lambda: tf.fused_fft_cgemm(M, N, K, x, W, C)), ("second half", lambda: tf.fused_cgemm_ifft(M, N, K, A, W, y)),
+        ("second half sizes", lambda: tf.fused_cgemm_ifft(M, N, K, A, W, y[:, :1])), ("forward", lambda: tf.fft_stride_DY(x, z(K * S, 64), 8, K * S)),
+        ("forward sizes", lambda: tf.fft_stride_DY(x, z(K * S, 32), 8, K * S)), ("backward", lambda: tf.ifft_stride_DY(z(K * S, 64), x, 8, K * S)),
+        ("X axis", lambda: tf.fft_stride(x2, z(K, 64, 128), 8, 128, 128 * K)), ("X axis back", lambda: tf.ifft_stride(z(K, 64, 128), x2, 8, 128, 128 * K)),
+        ("X axis sizes", lambda: tf.fft_stride(x2, z(K, 64, 64), 8, 128, 128 * K)),
+    ]
+    forms = [("1d " + n, (lambda a=a, k=k: tf.layer_1d(*a, **k))) for n, a, k in one] + [("2d " + n, (lambda a=a, k=k: tf.layer_2d(*a, **k))) for n, a, k in two]
+    return forms + rest
+
+
+def _outcome(call):
+    try:
+        return "returned", tuple(call().shape)
+    except Exception as e:
+        return type(e), str(e)
+
+
+def _compare(device, monkeypatch):
+    for name, call in _forms(device):
+        print("form", name, flush=True)
+        with_module = _outcome(call)
+        with monkeypatch.context() as m:
+            m.setattr(api, "_operands", None)
+            without = _outcome(call)
+        assert with_module == without, name
+
+
+@needs_module
+def test_same_refusals_without_a_gpu(monkeypatch):
+    _compare("cpu", monkeypatch)
+
+
+@needs_module
+@pytest.mark.gpu
+def test_same_results_and_refusals(monkeypatch):
+    """zeros in: every call either runs (the kernels accept the form) or raises before a launch"""
+    _compare("cuda", monkeypatch)
+    torch.cuda.synchronize()
+
+
+@needs_module
+@pytest.mark.gpu
+def test_module_takes_the_plain_call():
+    """the short way is the one that runs: status 0, the operands' own addresses, None or -1 for what is left to Python"""
+    x, W, y = _c64(8, 2, 128, device="cuda"), _c64(64, 8, device="cuda"), _c64(64, 2, 128, device="cuda")
+    tf.lib()
+    assert api._operands.layer_1d(api._LAYER_1D, x, W, y, 1 + 0j, 1, api._stream()) == 0
+    assert api._operands.layer_1d(api._LAYER_1D, x.cpu(), W, y, 1 + 0j, 1, api._stream()) == -1
+    assert api._operands.operands(x, x.numel(), y, y.numel()) == (x.data_ptr(), y.data_ptr())
+    assert api._operands.operands(x, x.numel() + 1) is None
+    torch.cuda.synchronize()

@@ -10,9 +10,15 @@ import os
 
 import torch
 
+try:
+    from . import _operands             # operand checks without a trip through Python per attribute (csrc/operands.cpp)
+except ImportError:                     # not built, or built for another torch: the checks below do the same
+    _operands = None
+
 MODES = 64
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB = None
+_LAYER_1D = _LAYER_2D = None            # addresses of the two layer entry points
 
 
 class TurboFNOError(RuntimeError):
@@ -27,7 +33,7 @@ def library_path():
 
 def lib():
     """Loads libturbofno.so; raises (no fallback) when it has not been built."""
-    global _LIB
+    global _LIB, _LAYER_1D, _LAYER_2D
     if _LIB is None:
         path = library_path()
         if not os.path.exists(path):
@@ -76,6 +82,8 @@ def lib():
                      "turbofno_cgemm", "turbofno_fft_stride_DY", "turbofno_ifft_stride_DY", "turbofno_fused_fft_cgemm",
                      "turbofno_fused_cgemm_ifft", "turbofno_layer_2d_noalloc", "turbofno_set_1d_algo"):
             getattr(L, name).restype = i
+        _LAYER_1D = ctypes.cast(L.turbofno_layer_1d, vp).value
+        _LAYER_2D = ctypes.cast(L.turbofno_layer_2d, vp).value
         _LIB = L
     return _LIB
 
@@ -110,6 +118,19 @@ def _need(cond, fmt, *args):
 
 def _numel(t, name, n):
     _need(t.numel() == n, "%s holds %d elements, the call needs exactly %d", name, t.numel(), n)
+
+
+def _addresses(names, *args):
+    """args: tensor, elements, tensor, elements, ... -> their addresses: contiguous complex64 GPU tensors of exactly those sizes, all on one device"""
+    if _operands is not None:
+        found = _operands.operands(*args)
+        if found is not None:
+            return found
+    tensors = args[::2]
+    for name, t, n in zip(names, tensors, args[1::2]):
+        _numel(t, name, n)
+    _same_device(*zip(names, tensors))
+    return tuple(t.data_ptr() for t in tensors)
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
@@ -197,13 +218,9 @@ def fused_fft_cgemm_ifft(M, N, K, x, W, y, alpha=1.0 + 0j, beta=0j, C=None):
     DY = x.shape[-1]
     _need(M > 0 and M % MODES == 0, "M=%d must be a positive multiple of %d", M, MODES)
     S = M // MODES
-    _numel(x, "x", K * S * DY)
-    _numel(W, "W", K * N)
-    _numel(y, "y", N * S * DY)
-    _same_device(("x", x), ("W", W), ("y", y))
+    px, pW, py = _addresses(("x", "W", "y"), x, K * S * DY, W, K * N, y, N * S * DY)
     a, b = complex(alpha), complex(beta)
-    _check(lib().turbofno_fused_fft_cgemm_ifft(_log2(DY), M, N, K, x.data_ptr(), W.data_ptr(),
-                                               None if C is None else _dev_c64(C, "C"), y.data_ptr(),
+    _check(lib().turbofno_fused_fft_cgemm_ifft(_log2(DY), M, N, K, px, pW, None if C is None else _dev_c64(C, "C"), py,
                                                a.real, a.imag, b.real, b.imag, _stream()))
     return y
 
@@ -217,10 +234,8 @@ def fft_stride(inp, out, threadblock_bs, DY, total, dimX=MODES):
     """X-axis truncated forward transform: in[total/DY][DX][DY] -> out[total/DY][dimX][DY]."""
     DX = inp.shape[-2]
     nsig = _stride_args(inp, out, DY, total, dimX, DX)
-    _numel(inp, "in", nsig * DX * DY)
-    _numel(out, "out", nsig * dimX * DY)
-    _same_device(("in", inp), ("out", out))
-    _check(lib().turbofno_fft_stride(_log2(DX), inp.data_ptr(), out.data_ptr(), threadblock_bs, DY,
+    src, dst = _addresses(("in", "out"), inp, nsig * DX * DY, out, nsig * dimX * DY)
+    _check(lib().turbofno_fft_stride(_log2(DX), src, dst, threadblock_bs, DY,
                                      total, dimX, _stream()))
     return out
 
@@ -229,16 +244,20 @@ def ifft_stride(inp, out, threadblock_bs, DY, total, dimX=MODES):
     """X-axis zero-padded backward transform: in[total/DY][dimX][DY] -> out[total/DY][DX][DY]."""
     DX = out.shape[-2]
     nsig = _stride_args(inp, out, DY, total, dimX, DX)
-    _numel(inp, "in", nsig * dimX * DY)
-    _numel(out, "out", nsig * DX * DY)
-    _same_device(("in", inp), ("out", out))
-    _check(lib().turbofno_ifft_stride(_log2(DX), inp.data_ptr(), out.data_ptr(), threadblock_bs, DY,
+    src, dst = _addresses(("in", "out"), inp, nsig * dimX * DY, out, nsig * DX * DY)
+    _check(lib().turbofno_ifft_stride(_log2(DX), src, dst, threadblock_bs, DY,
                                       total, dimX, _stream()))
     return out
 
 
 def layer_1d(x, W, y=None, alpha=1.0 + 0j, dimX=1):
     """x: [K][bs*dimX][DY], W: [N][K] (element W[k + n*K]) -> y: [N][bs*dimX][DY]."""
+    if _operands is not None and y is not None and getattr(x, "is_cuda", False):
+        lib()
+        rc = _operands.layer_1d(_LAYER_1D, x, W, y, alpha, dimX, _stream())
+        if rc >= 0:
+            _check(rc)
+            return y
     _need(x.dim() == 3 and W.dim() == 2, "x must be [K][S][DY] and W [N][K]")
     K, S, DY = x.shape
     N = W.shape[0]
@@ -274,6 +293,12 @@ def layer_2d(x, W, y=None, alpha=1.0 + 0j, workspace=None, algo=0):
     """x: [K][bs][DX][DY], W: [N][K] -> y: [N][bs][DX][DY]. `workspace`: uint8 GPU tensor (allocated
     here when omitted; pass one to keep allocation out of a timed loop). algo: 0 by size, 1 three kernels with the X
     axis first, 2 one block per image, 3 three kernels with whole rows first."""
+    if _operands is not None and y is not None and workspace is not None and getattr(x, "is_cuda", False):
+        lib()
+        rc = _operands.layer_2d(_LAYER_2D, x, W, y, alpha, workspace, algo, _stream())
+        if rc >= 0:
+            _check(rc)
+            return y
     K, bs, DX, DY, N, y = _layer_2d_operands(x, W, y)
     need = layer_2d_workspace_bytes(bs, DX, DY, K, N, algo)
     if workspace is None:
@@ -325,32 +350,25 @@ def ifft2d_pad(spec, y):
 
 def cgemm(M, N, K, A, B, C, alpha=1.0 + 0j, beta=0j):
     """C[m + n*M] = alpha * sum_k A[m + k*M] B[k + n*K] + beta * C  (A: [K][M], B: [N][K], C: [N][M] as tensors)."""
-    _numel(A, "A", M * K)
-    _numel(B, "B", K * N)
-    _numel(C, "C", M * N)
-    _same_device(("A", A), ("B", B), ("C", C))
+    pA, pB, pC = _addresses(("A", "B", "C"), A, M * K, B, K * N, C, M * N)
     a, b = complex(alpha), complex(beta)
-    _check(lib().turbofno_cgemm(M, N, K, A.data_ptr(), B.data_ptr(), C.data_ptr(), a.real, a.imag,
+    _check(lib().turbofno_cgemm(M, N, K, pA, pB, pC, a.real, a.imag,
                                 b.real, b.imag, _stream()))
     return C
 
 
 def fft_stride_DY(inp, out, threadblock_bs, total):
     """Contiguous truncated forward transform: in[total][DY] -> out[total][64]."""
-    _numel(inp, "in", total * inp.shape[-1])
-    _numel(out, "out", total * MODES)
-    _same_device(("in", inp), ("out", out))
-    _check(lib().turbofno_fft_stride_DY(_log2(inp.shape[-1]), inp.data_ptr(), out.data_ptr(),
+    src, dst = _addresses(("in", "out"), inp, total * inp.shape[-1], out, total * MODES)
+    _check(lib().turbofno_fft_stride_DY(_log2(inp.shape[-1]), src, dst,
                                         threadblock_bs, total, _stream()))
     return out
 
 
 def ifft_stride_DY(inp, out, threadblock_bs, total):
     """Contiguous zero-padded backward transform: in[total][64] -> out[total][DY]."""
-    _numel(inp, "in", total * MODES)
-    _numel(out, "out", total * out.shape[-1])
-    _same_device(("in", inp), ("out", out))
-    _check(lib().turbofno_ifft_stride_DY(_log2(out.shape[-1]), inp.data_ptr(), out.data_ptr(),
+    src, dst = _addresses(("in", "out"), inp, total * MODES, out, total * out.shape[-1])
+    _check(lib().turbofno_ifft_stride_DY(_log2(out.shape[-1]), src, dst,
                                          threadblock_bs, total, _stream()))
     return out
 
@@ -358,24 +376,16 @@ def ifft_stride_DY(inp, out, threadblock_bs, total):
 def fused_fft_cgemm(M, N, K, x, W, C, alpha=1.0 + 0j, beta=0j):
     """Variant B's first kernel: C[N][M] = alpha * FFT_trunc(x) W + beta C, x: [K][S][DY]."""
     _need(M > 0 and M % MODES == 0, "M=%d must be a positive multiple of %d", M, MODES)
-    _numel(x, "x", K * (M // MODES) * x.shape[-1])
-    _numel(W, "W", K * N)
-    _numel(C, "C", M * N)
-    _same_device(("x", x), ("W", W), ("C", C))
+    px, pW, pC = _addresses(("x", "W", "C"), x, K * (M // MODES) * x.shape[-1], W, K * N, C, M * N)
     a, b = complex(alpha), complex(beta)
-    _check(lib().turbofno_fused_fft_cgemm(_log2(x.shape[-1]), M, N, K, x.data_ptr(), W.data_ptr(),
-                                          C.data_ptr(), a.real, a.imag, b.real, b.imag, _stream()))
+    _check(lib().turbofno_fused_fft_cgemm(_log2(x.shape[-1]), M, N, K, px, pW, pC, a.real, a.imag, b.real, b.imag, _stream()))
     return C
 
 
 def fused_cgemm_ifft(M, N, K, A, W, y, alpha=1.0 + 0j):
     """Variant C's second kernel: y[N][S][DY] = iFFT_pad(alpha * A W), A: [K][M]."""
     _need(M > 0 and M % MODES == 0, "M=%d must be a positive multiple of %d", M, MODES)
-    _numel(A, "A", M * K)
-    _numel(W, "W", K * N)
-    _numel(y, "y", N * (M // MODES) * y.shape[-1])
-    _same_device(("A", A), ("W", W), ("y", y))
+    pA, pW, py = _addresses(("A", "W", "y"), A, M * K, W, K * N, y, N * (M // MODES) * y.shape[-1])
     a = complex(alpha)
-    _check(lib().turbofno_fused_cgemm_ifft(_log2(y.shape[-1]), M, N, K, A.data_ptr(), W.data_ptr(), None,
-                                           y.data_ptr(), a.real, a.imag, 0.0, 0.0, _stream()))
+    _check(lib().turbofno_fused_cgemm_ifft(_log2(y.shape[-1]), M, N, K, pA, pW, None, py, a.real, a.imag, 0.0, 0.0, _stream()))
     return y
