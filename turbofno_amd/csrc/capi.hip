@@ -87,8 +87,8 @@ bool whole_image_ahead_by_channels(int bs, int lx, int ly, int K, int N)
 // images. Measured on MI355X (256 CUs; 160 shapes, both paths back to back): from a batch of 8 the whole-image path is
 // ahead (by up to 2x at bs = 16) but for two groups of shapes (below); with a batch of 4 to 7 it is ahead for 256 x 256
 // images once (K + N) * bs reaches 768 images in and out, and for 128 x 256 images with N >= 128; with many channels earlier (above). Otherwise
-// three stages, X axis first; whole rows of 128 x 256 images first while the grids are smallest, because their intermediates are half as large (bs = 1, K =
-// 40, N = 64: 22.9 / 20.3, K = 88: 1.06 the other way; bs = 2, K = 16: 26.7 / 24.7, N = 128: 36.3 / 36.1).
+// three stages, X axis first; whole rows of 128 x 256 images first while the grids are smallest, because their intermediates are half as large (rows first / X
+// axis first, N = 64: bs = 1: K = 32 0.91, K = 64 0.85; bs = 2: K = 16 0.88, K = 32 1.01; bs = 3: K = 8 0.89, K = 16 1.00).
 int pick_algo(int bs, int DX, int DY, int K, int N, int algo)
 {
     if (algo != TURBOFNO_2D_AUTO) return algo;
@@ -111,18 +111,17 @@ int pick_algo(int bs, int DX, int DY, int K, int N, int algo)
         // otherwise three stages. The axis that is transformed first is the one whose
         // truncation shrinks the intermediates most, i.e. the longer one (DY = 4 DX: half the time of the other order;
         // DX = 4 DY: the reverse). Square images: whole rows first (9-18 % ahead) unless the grid is small.
-        // The smallest problems with DX of 256 or 512 are sooner through with the X axis first, whose kernels have more and smaller blocks (rows first / X
-        // axis first: 256 x 512, bs = 1: K = 16, N = 64 34.8 / 32.7, N = 128 51.5 / 45.7, K = 112 31 / 33; 256 x 1024, K = 16: 51.8 / 49.3, K = 32: 56.2 / 59.6; 512 x 1024, K
-        // = 16: 85.4 / 79.0). Its intermediates are larger there, at most 60 MiB below these limits.
+        // The smallest problems with DX of 256 or 512 are sooner through with the X axis first (rows first / X axis first: 256 x 512, bs = 1: K = 16, N = 64 1.05,
+        // N = 128 1.10, K = 64 1.00; bs = 2, K = 8, N = 64 1.11; bs = 3, K = 32 1.01; 512 x 1024, bs = 1: K = 8, N = 64 1.05, K = 16 1.02, N = 128 1.00; 256 x 1024, K = 8: 0.96). Its
+        // intermediates are larger there, at most 60 MiB below these limits.
         const long mib = ((long)K + N) * bs * DX * DY >> 17;
-        if ((DX == 256 && DY == 512 && mib <= 240 && K <= 64) || (DX == 256 && DY == 1024 && mib <= 240 && K <= 16) ||
-            (DX == 512 && DY == 1024 && mib <= 320 && K <= 32))
+        if ((DX == 256 && DY == 512 && mib <= 240 && K <= 64) || (DX == 512 && DY == 1024 && mib <= 320 && K <= 16))
             return TURBOFNO_2D_THREE_KERNEL;
         if (DY != DX) return DY > DX ? TURBOFNO_2D_ROWS_FIRST : TURBOFNO_2D_THREE_KERNEL;
         return (DY >= 1024 || (long)K * bs >= 128) ? TURBOFNO_2D_ROWS_FIRST : TURBOFNO_2D_THREE_KERNEL;
     }
     if (bs >= 16) return TURBOFNO_2D_WHOLE_IMAGE;
-    if (DX == 128 && DY == 256 && ((bs == 1 && K <= 64) || (bs == 2 && N == 64 && K <= 24))) return TURBOFNO_2D_ROWS_FIRST;
+    if (DX == 128 && DY == 256 && ((bs == 1 && K <= 64) || (bs == 2 && K <= (N == 64 ? 24 : 16)) || (bs == 3 && K <= 8))) return TURBOFNO_2D_ROWS_FIRST;
     if (bs < 4) return TURBOFNO_2D_THREE_KERNEL;
     const bool big = DX == 256 && DY == 256;
     if (bs >= 8) {

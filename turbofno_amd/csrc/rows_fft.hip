@@ -15,23 +15,24 @@
 
 namespace tfno {
 
-template <int LOGDY> struct GeoRows {
+template <int LOGDY, int ROWS_> struct GeoRows {
     using G = Geo1D<LOGDY>;
-    static constexpr int BATCHES = LOGDY == 7 ? 1 : LOGDY == 8 ? 2 : LOGDY == 9 ? 4 : 8;   // rows are transformed GROUPS at a time
-    static constexpr int ROWS = BATCHES * G::GROUPS;                  // rows of the image per block: 32 at every length
+    static constexpr int ROWS = ROWS_;                                // rows of the image per block
+    static constexpr int BATCHES = ROWS / G::GROUPS;                  // rows are transformed GROUPS at a time
+    static_assert(BATCHES >= 1, "a block has no more lane groups than rows");
     static constexpr int PT = ROWS + 1;                               // pitch (complex) of the tile [64][ROWS]
     static constexpr size_t LDS_BYTES = sizeof(float2) * (size_t)(G::GROUPS * G::EXCH + 64 * PT);
 };
 
 // The forward kernel is persistent: a block walks the row blocks blockIdx.x, + gridDim.x, ... and requests the first rows
 // of its next row block while it still works on the current one (x is streamed past the caches: it is read once).
-template <int LOGDY>
+template <int LOGDY, int ROWS>
 __global__ __launch_bounds__(256) void fft_rows_trunc_kernel(const float2* __restrict__ in, float2* __restrict__ out, int DX,
                                                             long nblocks)
 {
     using G = Geo1D<LOGDY>;
-    using R = GeoRows<LOGDY>;
-    constexpr int DY = G::DY, L = G::L, GROUPS = G::GROUPS, MM = G::MM, ROWS = R::ROWS, PT = R::PT;
+    using R = GeoRows<LOGDY, ROWS>;
+    constexpr int DY = G::DY, L = G::L, GROUPS = G::GROUPS, MM = G::MM, PT = R::PT;
     extern __shared__ float2 lds[];
     const int tid = threadIdx.x, g = tid / L, t = tid % L;
     float2* exch = lds + g * G::EXCH;
@@ -70,12 +71,12 @@ __global__ __launch_bounds__(256) void fft_rows_trunc_kernel(const float2* __res
 
 // One block per row block, not persistent: a persistent version with the next tile requested ahead was 8-17 % slower
 // (its blocks drift into lockstep and the stores arrive in bursts; the hardware's own block scheduling keeps them apart).
-template <int LOGDY>
+template <int LOGDY, int ROWS>
 __global__ __launch_bounds__(256) void ifft_rows_pad_kernel(const float2* __restrict__ in, float2* __restrict__ out, int DX)
 {
     using G = Geo1D<LOGDY>;
-    using R = GeoRows<LOGDY>;
-    constexpr int DY = G::DY, L = G::L, GROUPS = G::GROUPS, MM = G::MM, ROWS = R::ROWS, PT = R::PT;
+    using R = GeoRows<LOGDY, ROWS>;
+    constexpr int DY = G::DY, L = G::L, GROUPS = G::GROUPS, MM = G::MM, PT = R::PT;
     extern __shared__ float2 lds[];
     const int tid = threadIdx.x, g = tid / L, t = tid % L;
     float2* exch = lds + g * G::EXCH;
@@ -100,23 +101,45 @@ __global__ __launch_bounds__(256) void ifft_rows_pad_kernel(const float2* __rest
     }
 }
 
-template <int LOGDY, bool INVERSE>
-static hipError_t launch_rows_t(const float2* in, float2* out, int DX, long nimg, hipStream_t stream)
+template <int LOGDY, bool INVERSE, int ROWS>
+static hipError_t launch_rows_k(const float2* in, float2* out, int DX, long nimg, hipStream_t stream)
 {
-    using R = GeoRows<LOGDY>;
+    using R = GeoRows<LOGDY, ROWS>;
     static_assert(R::LDS_BYTES <= 64 * 1024, "fits the default dynamic LDS limit");
-    if (DX % R::ROWS) return hipErrorInvalidValue;
-    const long blocks = nimg * (DX / R::ROWS);
+    if (DX % ROWS) return hipErrorInvalidValue;
+    const long blocks = nimg * (DX / ROWS);
     if (blocks <= 0 || blocks > 0x7fffffffL) return hipErrorInvalidValue;
     if constexpr (INVERSE) {
-        hipLaunchKernelGGL((ifft_rows_pad_kernel<LOGDY>), dim3((unsigned)blocks), dim3(256), R::LDS_BYTES, stream, in, out, DX);
+        hipLaunchKernelGGL((ifft_rows_pad_kernel<LOGDY, ROWS>), dim3((unsigned)blocks), dim3(256), R::LDS_BYTES, stream, in, out, DX);
     } else {
         // as many blocks as the CUs hold at once (LDS: 43-52 KiB per block)
         const long resident = (long)cu_count() * (long)((160 * 1024) / R::LDS_BYTES);
-        hipLaunchKernelGGL((fft_rows_trunc_kernel<LOGDY>), dim3((unsigned)(blocks < resident ? blocks : resident)), dim3(256),
+        hipLaunchKernelGGL((fft_rows_trunc_kernel<LOGDY, ROWS>), dim3((unsigned)(blocks < resident ? blocks : resident)), dim3(256),
                            R::LDS_BYTES, stream, in, out, DX, blocks);
     }
     return hipGetLastError();
+}
+// Rows per block: 32, whose transposed accesses are two cache lines long; fewer on small grids, so that more blocks (and CUs) share the rows and
+// each has fewer batches one after the other. The limits are rows of the call per CU. Whole layers of one image, rows first, 32 rows / the rule (us):
+// 128 x 256, K = 8, N = 64 19.6 / 17.7 (4 and 32 rows per CU), 128 x 512 24.7 / 21.3, 128 x 1024 34.6 / 28.7; two of 256 x 1024, K = 8: 80 / 75. Beyond them: DY =
+// 256, backward with 64 rows per CU 24.3 / 25.9, 256: 55.7 / 60.9; DY = 512, backward, 64: 34.1 / 34.9, forward with 8 rows per block, 32: 38.8 / 38.9;
+// DY = 1024, backward, 256: 147.8 / 149.8.
+template <int LOGDY, bool INVERSE> struct RowsPerBlock {
+    static constexpr int EIGHT_TO = LOGDY == 10 ? (INVERSE ? 128 : 64) : LOGDY == 9 && !INVERSE ? 16 : 0;
+    static constexpr int SIXTEEN_TO = LOGDY == 10 ? (INVERSE ? 0 : 128) : LOGDY == 9 ? (INVERSE ? 32 : 64) : LOGDY == 8 ? 32 : 0;
+};
+template <int LOGDY, bool INVERSE>
+static hipError_t launch_rows_t(const float2* in, float2* out, int DX, long nimg, hipStream_t stream)
+{
+    using Limit = RowsPerBlock<LOGDY, INVERSE>;
+    const long rows = nimg * DX, cus = cu_count();
+    if constexpr (Limit::EIGHT_TO > 0) {
+        if (rows <= Limit::EIGHT_TO * cus) return launch_rows_k<LOGDY, INVERSE, 8>(in, out, DX, nimg, stream);
+    }
+    if constexpr (Limit::SIXTEEN_TO > 0) {
+        if (rows <= Limit::SIXTEEN_TO * cus) return launch_rows_k<LOGDY, INVERSE, 16>(in, out, DX, nimg, stream);
+    }
+    return launch_rows_k<LOGDY, INVERSE, 32>(in, out, DX, nimg, stream);
 }
 
 template <bool INVERSE>
