@@ -26,7 +26,6 @@
 namespace tfno {
 
 namespace {
-constexpr int TPITCH = 66;                       // row pitch (complex) of the DX x 64 redistribution tile
 constexpr int EXCH_ELEMS = 1024 * 17;            // exchange regions of all lane groups of a 1024-thread block
 
 // Geometry of the whole-image kernels for a DX x DY image (DX rows of DY contiguous samples).
@@ -44,7 +43,7 @@ template <int LOGX, int LOGY> struct Geo2D {
     static constexpr int MMY = PAIRED ? 8 : 64 / LY;          // modes per lane after one row pass
     static constexpr int MMX = 64 / LX;                       // modes per lane after the column pass
     static constexpr int COLT = 64 * LX;                      // threads that take part in the column pass
-    static constexpr int TILE = DX * TPITCH;
+    static constexpr int TILE = DX * 68;                      // the largest pitch of TileMap
     static constexpr int LDS_MAIN = EXCH_ELEMS > TILE ? EXCH_ELEMS : TILE;   // exchange regions alias the tile
     // after them: first-pass twiddles of the rows (one table row per lane of a group) and of the columns, and for rows
     // of 512 / 1024 the powers w_LY^e, e < LY, of the second pass
@@ -52,32 +51,45 @@ template <int LOGX, int LOGY> struct Geo2D {
     static constexpr size_t LDS_BYTES = sizeof(float2) * (size_t)(LDS_MAIN + TWY_ELEMS + kTwLdsSize + WSM_ELEMS);
     static_assert(LOGY >= 7 && LOGY <= 10, "rows of 128 to 1024");
     static_assert(ITY >= 1 && COLT <= 1024 && GY * LY * 17 <= EXCH_ELEMS, "unsupported image shape");
-    // element offset of the lane's i-th sample from its first one
+    // element offset of the lane's i-th sample from its first one; pair: rows between the two of a paired group
     // (logr: the rows of the image lie 2^logr rows of the array apart, see the decimated images below)
-    static __device__ __forceinline__ constexpr int sample_off(int i, int logr = 0)
+    static __device__ __forceinline__ constexpr int sample_off(int i, int pair, int logr = 0)
     {
-        return PAIRED ? (i & 7) * 16 + (i >> 3) * ((4 * DY) << logr) : LY * i;
+        return PAIRED ? (i & 7) * 16 + (i >> 3) * ((pair * DY) << logr) : LY * i;
     }
     // column of the redistribution tile (mode along Y) that lane t of a row group holds in slot mm
     static __device__ __forceinline__ constexpr int tile_col(int t, int mm) { return PAIRED ? (t & 7) + 8 * mm : t + LY * mm; }
 };
 
-// First row (within one pass) of lane group g. The two groups that share an LDS cycle (one half wavefront) must
-// hit disjoint banks of the pitch-66 tile, i.e. sit 8 rows apart (4 rows = 16 banks).
-//   rows of 256: one row per group; groups 2j, 2j+1 get rows 8 apart.
-//   rows of 128: group g owns rows a and a + 4 (lanes 0-7 / 8-15 finish one each: 16 banks apart), a enumerating the
-//   rows with bit 2 clear; groups 2j, 2j+1 again 8 rows apart.
-//   rows of 512 / 1024: one row per group, a group is at least half a wavefront: any order.
-template <bool PAIRED, bool WIDE = false> __device__ __forceinline__ int first_row_in_pass(int g)
-{
-    const int jh = g & 1, rest = g >> 1;
-    if constexpr (WIDE) return g;
-    else if constexpr (!PAIRED) return jh * 8 + (rest % 8) + (rest / 8) * 16;
-    else {
-        const int s = jh * 4 + (rest % 4) + (rest / 4) * 8;    // pair index, partner groups 4 apart
-        return (s & 3) + 8 * (s >> 2);
+// The redistribution tile [DX][64] and which rows the lane groups take, laid out for the LDS banks: an 8-byte read serves 32 lanes per cycle
+// over 64 banks (element numbers modulo 32 differ), an 8-byte write 16 lanes over 32 banks (modulo 16).
+//   forward: rows are written (16 lanes: 16 modes of a row, or 8 modes of each row of a pair, which have to lie 8 elements apart modulo 16) and
+//     columns are read (32 lanes: LX rows of 2 or 4 columns): a pitch of 2 modulo 32 for 16 rows, of 4 modulo 32 for 8 rows;
+//   backward: columns are written (16 lanes: LX rows of 1 or 2 columns): an odd pitch for 16 rows, 2 modulo 16 for 8; rows are read (32 lanes: two
+//     groups, whose rows have to lie 16 elements apart modulo 32, and 8 for the rows of a pair).
+// One pitch of 66 for all cases put the writes of the backward kernel of 256 rows and the reads of the forward kernel of 128 rows on the same banks two by
+// two (us per layer, before / now: 16 images of 256 x 256, K = N = 64: 211.6 / 204.8; 36 images, K = 56: 444.9 / 425.4; 40 of 128 x 128, K = 72: 194.2 / 189.9; 16 of
+// 512 x 128: 237.9 / 233.1). Backward kernels of decimated images other than 512 x 128 keep 66 and its order of the rows, which lie 2 or 4 rows apart
+// in memory there (8 images of 1024 x 256: 312 / 331 with 65).
+//   PAIR:    rows of 128: group g owns the rows a and a + PAIR (lanes 0-7 / 8-15 finish one each), a enumerating the rows in question;
+//   PARTNER: rows between the first rows of the groups 2j and 2j + 1. Rows of 512 / 1024: a group is at least half a wavefront: any order.
+template <int LOGX, int LOGY, int LOGR, bool FORWARD> struct TileMap {
+    static constexpr bool ODD = !FORWARD && LOGX == 8 && (LOGR == 0 || (LOGR == 1 && LOGY == 7));
+    static constexpr int PITCH = ODD ? 65 : FORWARD && LOGX == 7 ? 68 : 66;
+    static constexpr int PAIR = ODD ? 8 : FORWARD && LOGX == 7 ? 2 : 4;
+    static constexpr int PARTNER = ODD ? 16 : 8;
+    // first row (within one pass) of lane group g
+    template <bool PAIRED, bool WIDE> static __device__ __forceinline__ int first_row(int g)
+    {
+        const int jh = g & 1, rest = g >> 1;
+        if constexpr (WIDE) return g;
+        else if constexpr (!PAIRED) return jh * PARTNER + rest % PARTNER + (rest / PARTNER) * (2 * PARTNER);
+        else {
+            const int s = jh * PAIR + rest % PAIR + (rest / PAIR) * (2 * PAIR);    // pair index
+            return s % PAIR + (s / PAIR) * (2 * PAIR);
+        }
     }
-}
+};
 
 // Decimated images (LOGR > 0): an image of R DX x DY, R = 2^LOGR, too long along X for one block, is handled as R parts
 // of DX x DY: part r holds the rows R j + r. Its transform along X splits exactly (one radix-R decimation in time step):
@@ -124,8 +136,8 @@ template <int LOGD> __device__ __forceinline__ void fill_decimation_twiddles(flo
 // Forward image kernel: truncated 2D transform of one DX x DY image per block iteration.
 // 1024 threads = 16 waves per CU (4 per SIMD: the arithmetic is issue bound, so full occupancy matters more
 // than registers). A block is persistent over images (img = blockIdx.x, += gridDim.x). Pass 1 transforms the
-// rows (along Y) with LY-lane groups and keeps the 64 retained modes of every row in registers; a pitch-66
-// LDS tile redistributes them; pass 2 transforms the 64 columns (along X) with LX-lane groups.
+// rows (along Y) with LY-lane groups and keeps the 64 retained modes of every row in registers; an
+// LDS tile (TileMap) redistributes them; pass 2 transforms the 64 columns (along X) with LX-lane groups.
 // Each group keeps ONE row in flight: the loads of its next row are issued as soon as the first radix-4
 // stage has consumed the row registers, so they travel while the rest of the transform runs, across the
 // column pass and across image boundaries. Inter-pass twiddles live in LDS to stay within 128 VGPRs.
@@ -135,6 +147,7 @@ __global__ __launch_bounds__(1024) void fft2d_trunc_kernel(const float2* __restr
                                                            int nimg, int nfull)
 {
     using G = Geo2D<LOGX, LOGY>;
+    using T2 = TileMap<LOGX, LOGY, LOGR, true>;
     constexpr int DY = G::DY, LX = G::LX, LY = G::LY, ITY = G::ITY, MMY = G::MMY, MMX = G::MMX;
     extern __shared__ float2 lds[];
     const int tid = threadIdx.x;
@@ -154,9 +167,9 @@ __global__ __launch_bounds__(1024) void fft2d_trunc_kernel(const float2* __restr
     if constexpr (LOGR > 0) fill_decimation_twiddles<LOGX + LOGR>(twsub, tid, 1024);
     __syncthreads();
 
-    const int row0 = first_row_in_pass<G::PAIRED, G::WIDE>(gy);
+    const int row0 = T2::template first_row<G::PAIRED, G::WIDE>(gy);
     // row the lane finishes after the exchange, and its first mode (paired rows: lanes 8-15 take the second row)
-    const int trow = G::PAIRED ? row0 + 4 * (ty >> 3) : row0;
+    const int trow = G::PAIRED ? row0 + T2::PAIR * (ty >> 3) : row0;
     // scalar base + 32-bit lane offset keeps the load addresses out of the vector registers
     const unsigned lane_off = (unsigned)(((row0 * DY) << LOGR) + ty);
     // x is streamed exactly once: non-temporal loads keep it from evicting the 64x64 spectra, which the
@@ -164,7 +177,7 @@ __global__ __launch_bounds__(1024) void fft2d_trunc_kernel(const float2* __restr
     auto issue = [&](cpx (&dst)[16], long array_row, int it, unsigned off) {
         const float2* base = x + (array_row + ((G::RPP * it) << LOGR)) * (long)DY;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) dst[i] = load_streaming(&base[off + (unsigned)G::sample_off(i, LOGR)]);
+        for (int i = 0; i < 16; ++i) dst[i] = load_streaming(&base[off + (unsigned)G::sample_off(i, T2::PAIR, LOGR)]);
     };
 
     long img = blockIdx.x;
@@ -219,13 +232,13 @@ __global__ __launch_bounds__(1024) void fft2d_trunc_kernel(const float2* __restr
         for (int it = 0; it < ITY; ++it)
 #pragma unroll
             for (int mm = 0; mm < MMY; ++mm)
-                lds[(trow + G::RPP * it) * TPITCH + G::tile_col(ty, mm)] = T[it][mm];
+                lds[(trow + G::RPP * it) * T2::PITCH + G::tile_col(ty, mm)] = T[it][mm];
         __syncthreads();
         // pass 2: columns (along X); group gx owns column q = gx, lane tx holds rows tx + LX i
         cpx c[16];
         if (tid < G::COLT) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) c[i] = lds[(tx + LX * i) * TPITCH + gx];
+            for (int i = 0; i < 16; ++i) c[i] = lds[(tx + LX * i) * T2::PITCH + gx];
         }
         __syncthreads();
         if (tid < G::COLT) {
@@ -270,6 +283,7 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
                                                           int nimg, int even_share, int nfull)
 {
     using G = Geo2D<LOGX, LOGY>;
+    using T2 = TileMap<LOGX, LOGY, LOGR, false>;
     constexpr int DY = G::DY, LX = G::LX, LY = G::LY, ITY = G::ITY, MMY = G::MMY, MMX = G::MMX;
     extern __shared__ float2 lds[];
     const int tid = threadIdx.x;
@@ -289,8 +303,8 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
     if constexpr (LOGR > 0) fill_decimation_twiddles<LOGX + LOGR>(twsub, tid, 1024);
     __syncthreads();
 
-    const int row0 = first_row_in_pass<G::PAIRED, G::WIDE>(gy);
-    const int trow = G::PAIRED ? row0 + 4 * (ty >> 3) : row0;      // row whose modes the lane takes from the tile
+    const int row0 = T2::template first_row<G::PAIRED, G::WIDE>(gy);
+    const int trow = G::PAIRED ? row0 + T2::PAIR * (ty >> 3) : row0;      // row whose modes the lane takes from the tile
     const unsigned lane_off = (unsigned)(((row0 * DY) << LOGR) + ty);
     const bool col_thread = tid < G::COLT;
     // part r of a decimated image is transformed from the spectrum of the whole image
@@ -348,7 +362,7 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
         __syncthreads();
         if (col_thread) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) lds[(tx + LX * i) * TPITCH + gx] = u[i];
+            for (int i = 0; i < 16; ++i) lds[(tx + LX * i) * T2::PITCH + gx] = u[i];
             // next image's spectrum (for the last image: a harmless re-read of its own 32 KiB)
             const float2* src = spectrum_of(pre);
 #pragma unroll
@@ -360,7 +374,7 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
         for (int it = 0; it < ITY; ++it)
 #pragma unroll
             for (int mm = 0; mm < MMY; ++mm)
-                cc[it][mm] = lds[(trow + G::RPP * it) * TPITCH + G::tile_col(ty, mm)];
+                cc[it][mm] = lds[(trow + G::RPP * it) * T2::PITCH + G::tile_col(ty, mm)];
         __syncthreads();
         // pass 2: rows (q -> y), coalesced row stores.
         // y is written once and not re-read by this layer: non-temporal stores stop half a gigabyte of
@@ -375,7 +389,7 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
             // uniform base + lane offset + immediates
             float2* dst = y + (first_array_row<LOGX, LOGR, PART_MAJOR>(img, nfull) + ((G::RPP * it) << LOGR)) * (long)DY;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) store_streaming(dst + lane_off + G::sample_off(i, LOGR), yv[i]);
+            for (int i = 0; i < 16; ++i) store_streaming(dst + lane_off + G::sample_off(i, T2::PAIR, LOGR), yv[i]);
         }
     }
 }
