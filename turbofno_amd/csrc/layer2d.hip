@@ -446,9 +446,9 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
     auto fetch = [&](long mb, int run, int step, bool live) {
         const bool column = mb * MBLOCK + wave * 16 < Mtot;       // Mtot is a multiple of 16; Kp of 8
         const float2* base = A + (column ? mb * MBLOCK : 0) + (long)(run * Kp + GEMM_KSTEP * step) * Mtot;    // uniform
-        const int left = Kp - GEMM_KSTEP * step - PER_LANE * kq;  // channels of the step from the lane's first on
-        const unsigned first = live ? (column ? lane_col : (unsigned)col) : 0u;
         if constexpr (HALVES) {
+            const int left = Kp - GEMM_KSTEP * step - PER_LANE * kq;      // channels of the step from the lane's first on
+            const unsigned first = live ? (column ? lane_col : (unsigned)col) : 0u;
             const unsigned off = live && left > 0 ? first + lane_row : first, row = live && left > 0 ? (unsigned)Mtot : 0u;
             const bool second = live && left > 16;
             const float2* upper = base + (second ? 16 * Mtot + (long)(first + lane_row) : (long)first);
@@ -456,7 +456,7 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
 #pragma unroll
             for (int j = 0; j < 4; ++j) { bv[j] = base[off + j * row]; bv[4 + j] = upper[j * upper_row]; }
         } else {
-            const unsigned off = first + (live && left > 0 ? lane_row : 0u);
+            const unsigned off = live ? (column ? lane_col : (unsigned)col) + (GEMM_KSTEP * step + 8 * kq < Kp ? lane_row : 0u) : 0u;
 #pragma unroll
             for (int j = 0; j < 8; ++j) bv[j] = (base + j * Mtot)[off];
         }
