@@ -29,8 +29,9 @@ template <int LOGDY> struct Geo1D {
 //     covers 32 consecutive elements per half wavefront. Left at that, the write of one bin meets the same banks from the A parts of a
 //     row, two (L = 32) or four ways (64: 16 cycles instead of 4). SPREAD: the bins of part a at k ^ (16 / A) a, without conflicts, for
 //     A write addresses instead of one: the 1D kernels at L = 64 (small grids, DY = 1024, K = 128, S = 16: 44.3 -> 38.7 us; first half, S =
-//     256, K = 32: 21.0 -> 19.7) and the one for small grids at L = 32 (22.3 -> 21.6); not the image kernels, which have no registers left for the
-//     addresses (16 images of 512 x 512: 588 -> 597 us);
+//     256, K = 32: 21.0 -> 19.7) and the one for small grids at L = 32 (22.3 -> 21.6); not where there are no registers for the addresses: the image
+//     kernels (16 images of 512 x 512: 588 -> 597 us) and the SIMT first half, which they take from 125 registers to 129, from four blocks
+//     on a CU to three (DY = 1024, K = 8, N = 64: S = 1000 25.3 -> 29.4 us);
 //   second exchange: [c][16 a' + r] with a pitch of L + 16: writes are consecutive, and the lanes a and a + 1 of a half
 //     wavefront, which read the rows c = a + A j and c + 1, land 16 elements apart modulo 32.
 // The powers w_L^e, e < L, come from the constant table, or (FROM_ARRAY) from an array of L values that the caller keeps
@@ -126,12 +127,12 @@ template <int LOGDY> TFNO_DEV constexpr int forward_mode_of_lane(int t, int mm)
 // second half of the forward transform: exchange of the twiddled first-pass results g[] inside the
 // L-lane group, then the pruned L-point DFT. On return lane `t` holds mode forward_mode_of_lane<LOGDY>(t, mm) =
 // t + L*mm in out[mm].
-template <int LOGDY>
+template <int LOGDY, bool SPREAD = Geo1D<LOGDY>::L == 64>
 TFNO_DEV void group_forward_finish(const cpx (&g)[16], cpx* exch, int t, cpx (&out)[Geo1D<LOGDY>::MM])
 {
     constexpr int L = Geo1D<LOGDY>::L;
     if constexpr (L >= 32) {
-        wide_forward_finish<L, false, L == 64>(g, exch, nullptr, t, out);
+        wide_forward_finish<L, false, SPREAD>(g, exch, nullptr, t, out);
         return;
     }
     wave_lds_fence();
@@ -156,12 +157,12 @@ TFNO_DEV void group_forward_finish(const cpx (&g)[16], cpx* exch, int t, cpx (&o
 
 // forward transform of one signal by one L-lane group; lane t holds samples t + L*i in v[].
 // On return lane `t` holds mode forward_mode_of_lane<LOGDY>(t, mm) in out[mm].
-template <int LOGDY>
+template <int LOGDY, bool SPREAD = Geo1D<LOGDY>::L == 64>
 TFNO_DEV void group_forward(cpx (&v)[16], const cpx (&tw)[16], cpx* exch, int t, cpx (&out)[Geo1D<LOGDY>::MM])
 {
     cpx g[16];
     fwd_pass1(v, tw, g);
-    group_forward_finish<LOGDY>(g, exch, t, out);
+    group_forward_finish<LOGDY, SPREAD>(g, exch, t, out);
 }
 
 // zero-padded backward transform; lane t holds modes m = t + L*mm in c[]; returns samples t + L*i in y[].

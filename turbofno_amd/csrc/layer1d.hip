@@ -70,7 +70,7 @@ __global__ __launch_bounds__(256) void fused_fft_cgemm_ifft_kernel(int S, int N,
                     const float2* src = x + ((long)k * S + s) * DY + t;
 #pragma unroll
                     for (int i = 0; i < 16; ++i) v[i] = src[L * i];
-                    group_forward<LOGDY>(v, tw, exch, t, out);
+                    group_forward<LOGDY, LOGDY == 10 && FUSE_INV>(v, tw, exch, t, out);    // SPREAD: not without the registers for it
                 }
             } else {
 #pragma unroll
