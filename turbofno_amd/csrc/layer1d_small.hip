@@ -347,7 +347,9 @@ __global__ __launch_bounds__(512, 1) void fused_fft_small_ifft_kernel(int S, int
             if constexpr (LONG) {
                 cpx e[16];
                 wide_backward_inputs<L, true>(c, powers, exch, t, e);
-                inv_pass2_lds(e, twrow, yv);
+                // twiddles from registers, for up to eight transforms in a row (DY = 1024, K = 8, N = 64, S = 129: 19.0 us with those
+                // in LDS, 16.8; DY = 512, S = 144: 12.4 / 11.1; second half, K = 32, S = 130: DY = 1024 18.6 / 16.0, DY = 512 12.3 / 11.0)
+                inv_pass2(e, tw, yv);
             } else {
                 group_backward_lds<8>(c, twrow, exch, t, yv);
             }
