@@ -223,8 +223,7 @@ int turbofno_set_exchange_wait_us(unsigned long long microseconds);
  *                             the call would refuse. compute_units = 0 asks the current device (the only case that
  *                             touches the HIP runtime), any other value answers for a device of that many compute
  *                             units; exchange_attached says whether the stream has an exchange buffer. Chosen by size, 2
- *                             and 4 stand for blocks of 16, 32 or 64 output channels, 6 for such blocks too where they
- *                             are ahead of the K split, 8 for blocks of 64 or of 128;
+ *                             and 4 stand for blocks of 16, 32 or 64 output channels, 8 for blocks of 64 or of 128;
  *   turbofno_query_1d_tile    output channels per block of that kernel (the clustered kernel: N); 0 as above.
  */
 int turbofno_query_2d_algo(int bs, int DX, int DY, int K, int N, int algo);

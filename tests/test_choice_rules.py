@@ -27,9 +27,24 @@ def test_1d_kernels_of_configuration_2():
 
 
 def test_1d_kernels_of_configuration_3():
-    for K in (64, 128):
+    for K, without in ((64, 4), (128, 6)):
         assert tf.query_1d_kernel(256, 64, 128, K, CUS, exchange_attached=True) == 7
-        assert tf.query_1d_kernel(256, 64, 128, K, CUS, exchange_attached=False) == 6
+        assert tf.query_1d_kernel(256, 64, 128, K, CUS, exchange_attached=False) == without
+
+
+def test_1d_k_split_is_named_where_it_runs():
+    """112 channels or more, blocks of 32 output channels for more than half of the CUs and at most one each; the query names the
+    small-grid kernel, and its tile, everywhere else"""
+    for N in (64, 128, 192, 256):
+        most = CUS // (N // 32)
+        for K in (112, 128, 136):
+            assert tf.query_1d_kernel(256, most, N, K, CUS) == 6 and tf.query_1d_tile(256, most, N, K, CUS) == 32, (N, K)
+            assert tf.query_1d_kernel(256, most // 2 + 1, N, K, CUS) == 6, (N, K)
+            assert tf.query_1d_kernel(256, most // 2, N, K, CUS) == 4 and tf.query_1d_tile(256, most // 2, N, K, CUS) == 16, (N, K)
+            assert tf.query_1d_kernel(256, most + 1, N, K, CUS) == 2, (N, K)
+        for K in (64, 72, 80, 88, 96):
+            assert tf.query_1d_kernel(256, most, N, K, CUS) == 4, (N, K)
+    assert tf.query_1d_kernel(256, 1, 64, 64, CUS) == 4 and tf.query_1d_tile(256, 1, 64, 64, CUS) == 16
 
 
 def test_2d_algorithms_of_configurations_4_and_5():

@@ -317,7 +317,8 @@ SIZE_RULE_SHAPES = [
     (300, 128, 32, 64, 8), (800, 128, 64, 128, 8),    # DY = 128: a few blocks of 64 channels per CU / N = 128
     (1000, 256, 16, 128, 8), (300, 256, 128, 64, 8),   # DY = 256: the same
     (1100, 128, 24, 64, 5), (600, 128, 8, 64, 5),     # DY = 128, several items per SIMD: four blocks per CU / one wavefront per item
-    (64, 256, 64, 128, 6), (100, 256, 96, 64, 6),     # small grids, 64 channels or more: K split over the waves of a block
+    (64, 256, 64, 128, 4), (100, 256, 96, 64, 4),     # small grids, 64 channels or more
+    (64, 256, 128, 128, 6), (100, 256, 120, 64, 6),   # the same from 112 on: K split over the waves of a block
     (100, 512, 16, 64, 2), (300, 512, 16, 64, 1), (300, 1024, 64, 64, 3),   # the long lengths
 ]
 

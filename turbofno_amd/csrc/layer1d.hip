@@ -556,7 +556,7 @@ static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const
 // The same rule holds where y is read again at once (middle stage of a 2D layer): the lines were drawn with x and y streamed, and of
 // 3166 2D layers in three stages, lengths 128 to 1024, none lost against a rule that treated that case apart.
 // The return value uses the same numbers (1 ... 8); chosen by size, 2 and 4 stand for blocks of 16, 32 or 64 output channels of the
-// small-grid kernel, 6 for that kernel or the K split, 8 for blocks of 64 or of 128 output channels (tile_of_fused_1d_kernel). A selector
+// small-grid kernel, 8 for blocks of 64 or of 128 output channels (tile_of_fused_1d_kernel). A selector
 // value that a kernel is not built for falls back to the choice by size.
 //
 // By size (measured on MI355X, us):
@@ -568,9 +568,9 @@ static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const
 //    DY = 128 with 49 to 64 channels, of which the small-grid kernel leaves a sixth to a round of its own (N = 64, S = 200, K = 64: 11.6 / 11.5,
 //    S = 256: 12.2 / 11.9; N = 128, S = 100: 11.6 / 11.5), and with 32 or 40 channels and N no multiple of 128 (S = 256, K = 32: 9.0 / 8.8, S = 200: 8.3 / 8.5),
 //    16 to 40 channels with exactly one block per CU (S = 256, K = 16: 8.2 / 8.1);
-//  * DY = 256, 64 channels or more, blocks of 32 output channels at most one per CU: reported as 6, run by the small-grid kernel (S = 64: N = 128, K = 64:
-//    12.0 / 13.6 for the K split, K = 96: 15.0 / 15.9; S = 1: K = 64: 8.6 / 10.9), from 112 channels on with more than half of the CUs by
-//    the K split, whose rounds have no barrier (S = 64, N = 128, K = 128: 17.6 / 17.1; S = 128, N = 64: 16.8 / 16.4);
+//  * DY = 256, 112 channels or more, blocks of 32 output channels for more than half of the CUs and at most one each: the K split, whose
+//    rounds have no barrier (small-grid kernel / K split: S = 64, N = 128, K = 128: 17.6 / 17.1; S = 128, N = 64: 16.8 / 16.4). Not with fewer
+//    channels or blocks (S = 64, N = 128: K = 64 12.0 / 13.6, K = 96: 15.0 / 15.9; S = 1: K = 64: 8.6 / 10.9);
 //  * more than one block of 64 output channels per CU, lengths 128 / 256: the split kernel;
 //  * lengths 512 / 1024, more than one block per CU: the split kernel from the number of channels on where it is ahead of the SIMT
 //    kernel, which has less to do per channel (DY = 512, S = 2048, N = 64: K = 24 127 / 120, K = 40 185 / 170, K = 128 358 / 305; S = 512:
@@ -623,7 +623,8 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, long cus, bo
     }
     int pick = algo == 4 ? 2 : algo;
     if (pick == 0) pick = (built && items <= cus) ? 2 : (long_signal ? 1 : 3);
-    if (logDY == 8 && (algo == 6 || (algo == 0 && K >= 64 && S * (N / SPLIT_NT) <= cus))) return kFused1dSplitK;
+    const long split_blocks = S * (N / SPLIT_NT);
+    if (logDY == 8 && (algo == 6 || (algo == 0 && K >= 112 && 2 * split_blocks > cus && split_blocks <= cus))) return kFused1dSplitK;
     if (pick == 2 && (logDY == 7 || logDY == 8) && (algo == 4 || (algo == 0 && S * (N / 32) <= cus))) return kFused1dMfma512Tile32;
     if (pick == 2 && built) return kFused1dMfma512;
     if (pick == 3 && built) return kFused1dMfma256;
@@ -659,13 +660,12 @@ static int small_tile(int logDY, long S, int N, int K, long cus)
     if (S * (N / 16) <= cus && !(logDY == 8 && K <= 8)) return 16;
     return S * (N / 32) <= cus ? 32 : 64;
 }
-static bool splits_channels_over_waves(long S, int N, int K, int algo, long cus) { return algo == 6 || (K >= 112 && 2 * S * (N / SPLIT_NT) > cus); }
 int tile_of_fused_1d_kernel(int kernel, int logDY, long S, int N, int K, int algo, long cus)
 {
     switch (kernel) {
     case kFused1dMfma512: return algo == 2 ? 64 : small_tile(logDY, S, N, K, cus);
     case kFused1dMfma512Tile32: return algo == 4 ? 32 : small_tile(logDY, S, N, K, cus);
-    case kFused1dSplitK: return splits_channels_over_waves(S, N, K, algo, cus) ? SPLIT_NT : small_tile(logDY, S, N, K, cus);
+    case kFused1dSplitK: return SPLIT_NT;
     case kFused1dCluster: return N;
     case kFused1dWide: return wide_tiles(logDY, S, N, K, algo, cus) ? 128 : 64;
     default: return 64;
@@ -695,9 +695,7 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
     case kFused1dWide:
         return launch_fused_split(logDY, S, N, K, x, W, y, alpha, wide_tiles(logDY, S, N, K, algo, cus), dense_blocks(S, N, cus), stream, keep_y);
     case kFused1dSplitK:
-        if (splits_channels_over_waves(S, N, K, algo, cus))
-            return keep_y ? launch_fused_split_channels<true>(S, N, K, x, W, y, alpha, stream) : launch_fused_split_channels<false>(S, N, K, x, W, y, alpha, stream);
-        [[fallthrough]];
+        return keep_y ? launch_fused_split_channels<true>(S, N, K, x, W, y, alpha, stream) : launch_fused_split_channels<false>(S, N, K, x, W, y, alpha, stream);
     case kFused1dMfma512Tile32:
     case kFused1dMfma512: {
         // y in the place of x: one block per signal set, so that nobody reads what another block has overwritten
