@@ -33,11 +33,11 @@ def test_1d_kernels_of_configuration_3():
 
 
 def test_1d_k_split_is_named_where_it_runs():
-    """112 channels or more, blocks of 32 output channels for more than half of the CUs and at most one each; the query names the
+    """more than 96 channels, blocks of 32 output channels for more than half of the CUs and at most one each; the query names the
     small-grid kernel, and its tile, everywhere else"""
     for N in (64, 128, 192, 256):
         most = CUS // (N // 32)
-        for K in (112, 128, 136):
+        for K in (104, 112, 128, 136):
             assert tf.query_1d_kernel(256, most, N, K, CUS) == 6 and tf.query_1d_tile(256, most, N, K, CUS) == 32, (N, K)
             assert tf.query_1d_kernel(256, most // 2 + 1, N, K, CUS) == 6, (N, K)
             assert tf.query_1d_kernel(256, most // 2, N, K, CUS) == 4 and tf.query_1d_tile(256, most // 2, N, K, CUS) == 16, (N, K)

@@ -261,7 +261,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     }
 }
 
-// Fused 1D layer for grids of more than half a block of 32 output channels per CU and at most one, DY = 256, 112 channels or more (fewer
+// Fused 1D layer for grids of more than half a block of 32 output channels per CU and at most one, DY = 256, more than 96 channels (fewer
 // blocks or channels: layer1d_small.hip): the eight waves of a block share ONE
 // item (signal set, 32 output channels) and split its K input channels: wave w transforms channels 32 r + 4 w + g in round r,
 // g = 16-lane group. Four rounds give a lane four channels of its modes t + 16 a: with real and imaginary part the eight
@@ -568,9 +568,10 @@ static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const
 //    DY = 128 with 49 to 64 channels, of which the small-grid kernel leaves a sixth to a round of its own (N = 64, S = 200, K = 64: 11.6 / 11.5,
 //    S = 256: 12.2 / 11.9; N = 128, S = 100: 11.6 / 11.5), and with 32 or 40 channels and N no multiple of 128 (S = 256, K = 32: 9.0 / 8.8, S = 200: 8.3 / 8.5),
 //    16 to 40 channels with exactly one block per CU (S = 256, K = 16: 8.2 / 8.1);
-//  * DY = 256, 112 channels or more, blocks of 32 output channels for more than half of the CUs and at most one each: the K split, whose
-//    rounds have no barrier (small-grid kernel / K split: S = 64, N = 128, K = 128: 17.6 / 17.1; S = 128, N = 64: 16.8 / 16.4). Not with fewer
-//    channels or blocks (S = 64, N = 128: K = 64 12.0 / 13.6, K = 96: 15.0 / 15.9; S = 1: K = 64: 8.6 / 10.9);
+//  * DY = 256, more than 96 channels (a fourth round), blocks of 32 output channels for more than half of the CUs and at most one each: the
+//    K split, whose rounds have no barrier (small-grid kernel / K split: S = 64, N = 128: K = 104 15.8 / 15.2, K = 128: 17.6 / 17.1; S = 100,
+//    N = 64, K = 104: 14.5 / 13.9). Not with fewer channels or blocks (S = 64, N = 128: K = 64 11.7 / 13.2, K = 96: 14.6 / 15.3; S = 60, N = 64,
+//    K = 104: 13.0 / 13.5);
 //  * more than one block of 64 output channels per CU, lengths 128 / 256: the split kernel;
 //  * lengths 512 / 1024, more than one block per CU: the split kernel from the number of channels on where it is ahead of the SIMT
 //    kernel, which has less to do per channel (DY = 512, S = 2048, N = 64: K = 24 127 / 120, K = 40 185 / 170, K = 128 358 / 305; S = 512:
@@ -624,7 +625,7 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, long cus, bo
     int pick = algo == 4 ? 2 : algo;
     if (pick == 0) pick = (built && items <= cus) ? 2 : (long_signal ? 1 : 3);
     const long split_blocks = S * (N / SPLIT_NT);
-    if (logDY == 8 && (algo == 6 || (algo == 0 && K >= 112 && 2 * split_blocks > cus && split_blocks <= cus))) return kFused1dSplitK;
+    if (logDY == 8 && (algo == 6 || (algo == 0 && K > 96 && 2 * split_blocks > cus && split_blocks <= cus))) return kFused1dSplitK;
     if (pick == 2 && (logDY == 7 || logDY == 8) && (algo == 4 || (algo == 0 && S * (N / 32) <= cus))) return kFused1dMfma512Tile32;
     if (pick == 2 && built) return kFused1dMfma512;
     if (pick == 3 && built) return kFused1dMfma256;
