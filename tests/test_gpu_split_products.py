@@ -283,6 +283,7 @@ def test_blocks_of_128_output_channels_as_middle_stage(bs, DX, DY, K, N, algo, a
 @pytest.mark.parametrize("S,DY,K,N", [
     (1, 128, 8, 64), (9, 128, 40, 192), (400, 128, 56, 128),        # rounds of 32 channels: one of eight, a last one of eight, of 24
     (1, 256, 8, 64), (9, 256, 40, 192), (400, 256, 72, 128),        # S = 400: blocks of 128 output channels
+    (160, 128, 56, 64),                                              # first half with a short round, less than one block per CU
     (3, 512, 24, 64), (400, 512, 40, 128), (2, 1024, 8, 64), (390, 1024, 24, 128),
     (5, 512, 8, 192), (900, 1024, 8, 64), (3, 1024, 16, 128),       # few channels: the SIMT kernel, both halves or the second
     (512, 256, 40, 64), (256, 512, 40, 128), (128, 1024, 24, 64),   # 1 MiB between channels: the waves of a block take every fourth one

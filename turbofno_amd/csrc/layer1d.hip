@@ -713,7 +713,8 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
 // The halves of the layer. While every block of 64 output channels has a CU to itself: the small-grid kernel (us, split kernel / small-grid
 // kernel with 16, 32 or 64 output channels). First half: the fewest output channels pay from 32 input channels on and up to half of the CUs
 // (DY = 256, N = 64, K = 128: S = 1: 20.3 / 11.3, 12.5, 15.1, S = 64: 21.5 / 12.9, 13.5, 16.0; DY = 1024, K = 128, S = 64: 65.8 / 39.4, 36.7, 37.8; DY = 256, K = 8, S = 1:
-// 4.4 / 3.8, 4.0, 4.2); a block of 64 on every CU: DY = 128, K = 64, S = 256: 10.4 / 10.2, DY = 1024, K = 32: 21.0 / 16.1. Second half: DY = 256, K = 32, S = 1: 8.4 / 4.5, 5.3, 7.1;
+// 4.4 / 3.8, 4.0, 4.2); a block of 64 on every CU: DY = 128, K = 64, S = 256: 10.4 / 10.2, DY = 1024, K = 32: 21.0 / 16.1. Not with 49 to 64 channels
+// of length 128 in blocks of 64 outputs, whose rounds hold 48 (S = 200: K = 48 8.8 / 7.6, K = 56 9.5 / 9.8, K = 64 9.8 / 9.9, K = 72 11.8 / 10.5). Second half: DY = 256, K = 32, S = 1: 8.4 / 4.5, 5.3, 7.1;
 // DY = 1024, K = 8, S = 1: 19.4 / 6.3, 9.6, 15.8, S = 64: 21.1 / 9.2, 11.1, 17.3, S = 200: 25.7 / 22.4 with 64; but a block of 64 on every CU: DY = 256, N = 64, K = 8: 8.7 / 9.1 (N = 128:
 // 9.4 / 9.1), DY = 512: 14.8 / 15.4, DY = 1024: 26.8 / 28.1.
 // Larger grids: the SIMT kernel with few channels at lengths 512 / 1024; with eight a round of 16 would be half padding (second
@@ -724,7 +725,8 @@ hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2*
                                   float2 alpha, float2 beta, hipStream_t stream)
 {
     const long cus = cu_count(), items = S * (N / 64);
-    if (items <= cus) {
+    const bool short_round = logDY == 7 && K > 48 && K <= 64 && 2 * items > cus && items < cus;
+    if (items <= cus && !short_round) {
         const int tile = K >= 32 && 2 * S * (N / 16) <= cus ? 16 : (S * (N / 32) <= cus ? 32 : 64);
         return launch_small_forward(logDY, S, N, K, x, W, C, alpha, beta, tile, stream);
     }
