@@ -8,6 +8,9 @@ another kernel has to show up here, next to the GPU parity test that covers that
   2D algorithms: 1 three kernels (X axis first), 2 whole image, 3 three kernels (rows first).
 GPU parity of each: tests/test_gpu_parity.py (every selector forced), tests/test_gpu_fullsize.py (the configurations at
 full size), tests/test_gpu_cluster.py (7), tests/test_gpu_large_grids.py."""
+import os
+import subprocess
+
 import turbofno_amd as tf
 
 CUS = 256       # MI355X
@@ -130,3 +133,24 @@ def test_1d_kernels_where_the_last_round_or_the_last_blocks_are_nearly_empty():
     assert tf.query_1d_kernel(1024, 512, 192, 64, CUS) == 3
     assert tf.query_1d_tile(256, 400, 128, 32, CUS) == 128          # 800 blocks of 64 channels, 768 at a time
     assert tf.query_1d_tile(256, 512, 128, 32, CUS) == 64
+
+
+def test_mode_gemm_steps(tmp_path):
+    """half steps follow the run that is walked, not the period of the weights: with R parts per image a run mostly covers all R of them"""
+    exe = str(tmp_path / "gemm_steps_check")
+    source = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host", "gemm_steps_check.cpp")
+    subprocess.run(["g++", "-O1", "-std=c++17", source, "-o", exe], check=True)
+    wide, narrow, small = (4, 1024, 6), (4, 512, 6), (1, 512, 6)
+    cases = [   # parts, channels per part, kernel -> channels per run, half steps
+        (1, 8, wide, 8, 1), (1, 16, wide, 16, 1), (1, 24, wide, 24, 0), (1, 32, wide, 32, 0), (1, 72, wide, 72, 1), (1, 64, wide, 64, 0),
+        (1, 72, (8, 512, 3), 72, 1), (1, 96, (8, 512, 3), 96, 0),
+        (2, 16, wide, 32, 0), (2, 48, wide, 96, 0), (2, 80, wide, 160, 0),          # full steps although the period ends in a short one
+        (4, 8, wide, 32, 0), (4, 16, wide, 64, 0), (4, 40, wide, 160, 0), (4, 48, wide, 192, 0),
+        (2, 24, wide, 48, 1), (2, 56, wide, 112, 1), (2, 88, wide, 176, 1),         # the other way round
+        (2, 104, wide, 104, 1), (4, 72, wide, 72, 1), (4, 56, wide, 56, 0), (2, 32, wide, 32, 0),   # more than the tile holds, whole periods: run by run
+        (1, 48, small, 48, 1), (1, 72, small, 72, 0), (2, 24, small, 48, 1), (2, 40, small, 80, 0), (4, 72, small, 72, 0),
+        (1, 112, narrow, 112, 1), (1, 136, narrow, 136, 0), (1, 136, wide, 136, 1), (1, 200, wide, 200, 0), (2, 72, narrow, 144, 0), (2, 72, wide, 144, 1),
+    ]
+    lines = "".join("%d %d %d %d %d\n" % ((r * k, k) + kernel) for r, k, kernel, _, _ in cases)
+    out = subprocess.run([exe], input=lines, check=True, capture_output=True, text=True).stdout.splitlines()
+    assert [tuple(map(int, ln.split())) for ln in out] == [c[3:] for c in cases]

@@ -167,10 +167,12 @@ def test_small_grids_with_many_channels(S, K, N, algo_1d):
 
 
 @pytest.mark.parametrize("bs,DX,DY,K,N", [(2, 512, 128, 8, 64), (1, 512, 256, 40, 64), (1, 1024, 128, 24, 128), (1, 1024, 128, 104, 64),
-                                          (1, 512, 128, 64, 64), (1, 512, 128, 200, 64)])
+                                          (1, 512, 128, 64, 64), (1, 512, 128, 200, 64), (1, 512, 128, 16, 64), (2, 512, 128, 24, 128), (1, 1024, 128, 40, 64),
+                                          (5, 512, 128, 72, 128)])
 def test_weights_with_a_period(bs, DX, DY, K, N):
     """whole images in 2 / 4 interleaved parts: the contraction runs over the parts with the weights of their channel, as one
-    run over all parts (K = 8, 24, 40) or as one run per part (K = 64, 104; K = 200 with a tile that is rebuilt)"""
+    run over all parts (K = 8, 24, 40) or as one run per part (K = 64, 104; K = 200 with a tile that is rebuilt); K = 16, 40 and 24, 72: a run
+    whose last step is full and short where that of a part is not"""
     print("split period", bs, DX, DY, K, N, flush=True)
     rng = np.random.default_rng(DX + K)
     x, W = _complex(rng, K, bs, DX, DY), _complex(rng, N, K) / np.float32(np.sqrt(K))

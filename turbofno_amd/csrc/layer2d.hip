@@ -19,6 +19,7 @@
 // lanes coincide, every access is contiguous per wavefront) and the GEMM is oblivious to it.
 #include "bf16_split.h"
 #include "group_fft.h"
+#include "gemm_steps.h"
 #include "kernels.h"
 #include <string>
 #include <type_traits>
@@ -404,7 +405,7 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
 // of a quarter wavefront). A wave owns 16 m and all 16 NT output channels of its block: an element of A is loaded and split
 // once per block, and its parts meet NT fragments of W read from LDS. The W tile holds the parts of alpha W as fragments
 // in lane order, 6 x 1 KiB per (step, 16 channels): an operand is one conflict-free 16-byte read. With HALVES a step is two of 16 channels whose
-// (re, im) pairs share one instruction, so that a last step of at most 16 channels costs half (see launch_cgemm_modes).
+// (re, im) pairs share one instruction, so that a last step of at most 16 channels costs half (gemm_steps.h).
 // Blocks are persistent over column blocks (XCD j takes the j-th eighth of them, so that an XCD keeps to one part of the
 // memory system); the strip of the next step - of the next column block after the last - is requested before the matrix
 // work of the current one, and nothing in the walk waits at a barrier, so loads, matrix work and stores of the waves overlap.
@@ -417,7 +418,6 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
 //   Kp    = channels covered by one run over the tile (K, or Kw: the contraction then runs over the tile K / Kw times);
 //   cap   = steps that the tile can hold; with more steps in a run the tile is rebuilt as the contraction proceeds.
 // ---------------------------------------------------------------------------------------------
-constexpr int GEMM_KSTEP = 32;
 constexpr size_t kSplitStepBytes = 6 * 1024;            // LDS of one step of 16 output channels
 
 template <int NT, int THREADS, bool HALVES>
@@ -919,13 +919,10 @@ hipError_t launch_cgemm_modes(const float2* A, const float2* W, float2* C, long 
     }
 
     // cap: steps of 32 channels that the tile can hold; per_cu: blocks per CU
-    auto launch_split_as = [&](auto nt_const, auto threads_const, auto halves_const, int cap, int per_cu) -> hipError_t {
+    auto launch_split_as = [&](auto nt_const, auto threads_const, auto halves_const, int Kp, int cap, int per_cu) -> hipError_t {
         constexpr int NT = decltype(nt_const)::value, THREADS = decltype(threads_const)::value;
         constexpr bool HALVES = decltype(halves_const)::value;
-        // one run over the tile covers one period of the weights where that wastes no part of a step, or else all K
-        // channels, if the tile can hold them
-        const bool periods = Kw % GEMM_KSTEP == 0 || (K + GEMM_KSTEP - 1) / GEMM_KSTEP > cap;
-        const int Kp = periods ? Kw : K, steps = (Kp + GEMM_KSTEP - 1) / GEMM_KSTEP;
+        const int steps = (Kp + GEMM_KSTEP - 1) / GEMM_KSTEP;
         const size_t lds_bytes = kSplitStepBytes * NT * (steps < cap ? steps : cap);
         static std::atomic<unsigned long long> served;
         if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(cgemm_modes_split_kernel<NT, THREADS, HALVES>), kSplitStepBytes * NT * cap, served);
@@ -941,14 +938,10 @@ hipError_t launch_cgemm_modes(const float2* A, const float2* W, float2* C, long 
                            A, W, C, Mtot, K, alpha, beta, nblocks, Kw, Kp, cap);
         return hipGetLastError();
     };
-    // A last step of at most 16 channels: steps in halves, the empty one skipped (us, whole steps / halves: M = 163,840, N = 128: K = 40 52.4 / 47.4,
-    // K = 72 75.2 / 70.2, K = 104 102.2 / 98.3; M = 65,536, N = 64: 14.6 / 14.2, 19.3 / 18.7, 23.7 / 23.3). Not where it is not needed (K = 64, M = 163,840, N = 128: 56.5 / 58.1),
-    // and on small products, whose tiles of 16 or 32 outputs have more per column to rearrange, up to 48 channels (M = 4,096, N = 64: K = 40 5.0 / 4.9, K = 72
-    // 5.9 / 5.9, K = 104 6.9 / 7.1); nor beyond 128 (K = 200, M = 65,536, N = 64: 42.2 / 43.4).
     auto launch_split = [&](auto nt, auto threads, int cap, int per_cu) {
-        const int last = Kw % GEMM_KSTEP;
-        if (last > 0 && last <= GEMM_KSTEP / 2 && Kw <= (decltype(nt)::value >= 4 ? 128 : 48)) return launch_split_as(nt, threads, std::true_type{}, cap, per_cu);
-        return launch_split_as(nt, threads, std::false_type{}, cap, per_cu);
+        const GemmWalk walk = gemm_walk(K, Kw, decltype(nt)::value, decltype(threads)::value, cap);
+        return walk.halves ? launch_split_as(nt, threads, std::true_type{}, walk.run, cap, per_cu)
+                           : launch_split_as(nt, threads, std::false_type{}, walk.run, cap, per_cu);
     };
     using Tiles4 = std::integral_constant<int, 4>;
     using Tiles8 = std::integral_constant<int, 8>;
