@@ -105,7 +105,8 @@ def test_queries_answer_zero_for_arguments_the_calls_refuse():
 
 
 def test_output_channels_per_block(algo_1d):
-    assert tf.query_1d_tile(256, 1, 64, 8, CUS) == 32
+    assert tf.query_1d_tile(256, 1, 64, 8, CUS) == 16 and tf.query_1d_tile(256, 64, 64, 8, CUS) == 16
+    assert tf.query_1d_tile(256, 65, 64, 8, CUS) == 32 and tf.query_1d_tile(256, 129, 64, 8, CUS) == 64
     assert tf.query_1d_tile(256, 64, 128, 128, CUS) == 32
     assert tf.query_1d_tile(256, 64, 128, 128, CUS, exchange_attached=True) == 128
     assert tf.query_1d_tile(256, 4096, 64, 64, CUS) == 64

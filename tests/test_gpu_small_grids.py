@@ -20,12 +20,11 @@ SHAPES = [(1, 8, 64), (9, 40, 64), (3, 72, 128), (5, 136, 192)]
 @pytest.mark.parametrize("S,K,N", SHAPES)
 @pytest.mark.parametrize("tile", [64, 32, 16])
 def test_small_grid_edges(tile, S, K, N, DY, algo_1d):
-    """selector 2: blocks of 64 output channels, 4: of 32 (DY = 128 / 256, else by size); by size: of 16 (eight channels at
-    DY = 256: 32). Every row of y written (y starts as NaN)."""
+    """selector 2: blocks of 64 output channels, 4: of 32 (DY = 128 / 256, else by size); by size: of 16. Every row of y written (y starts as NaN)."""
     print("small grid", tile, S, K, N, DY, flush=True)
     algo_1d({64: 2, 32: 4, 16: 0}[tile])
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
-        expect = 64 if tile == 64 else 32 if (tile == 32 and DY <= 256) or (DY == 256 and K == 8) else 16
+        expect = 64 if tile == 64 else 32 if tile == 32 and DY <= 256 else 16
         assert tf.query_1d_tile(DY, S, N, K, compute_units=0) == expect
     x, W = _x(S, DY, K), _complex(np.random.default_rng(S), N, K) / np.float32(np.sqrt(K))
     y = torch.full((N, S, DY), float("nan"), dtype=torch.complex64, device="cuda")

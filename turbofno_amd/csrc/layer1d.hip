@@ -655,17 +655,17 @@ static bool wide_tiles(int logDY, long S, int N, int K, int algo, long cus)
 // Output channels per block of the small-grid kernel: the fewest that leave every block a CU to itself. The blocks of a signal set repeat
 // each other's forward transforms, but they run side by side, and each has fewer backward transforms to do one after the other (us, 16 / 32 / 64
 // channels, N = 64: S = 1, K = 32: DY = 128 5.3 / 5.9 / 7.0, DY = 1024 13.8 / 18.0 / 23.5; S = 64, K = 8: DY = 512 8.3 / 8.6 / 12.4; S = 100: 12.9 / 8.5 / 9.4 at
-// DY = 256, K = 24). DY = 256 with eight channels keeps at least 32 (S = 1: 5.3 / 5.9): the size that turbofno_query_1d_tile has always named there.
-static int small_tile(int logDY, long S, int N, int K, long cus)
+// DY = 256, K = 24; DY = 256, K = 8: S = 1 5.3 / 5.9, S = 64 6.1 / 6.6).
+static int small_tile(long S, int N, long cus)
 {
-    if (S * (N / 16) <= cus && !(logDY == 8 && K <= 8)) return 16;
+    if (S * (N / 16) <= cus) return 16;
     return S * (N / 32) <= cus ? 32 : 64;
 }
 int tile_of_fused_1d_kernel(int kernel, int logDY, long S, int N, int K, int algo, long cus)
 {
     switch (kernel) {
-    case kFused1dMfma512: return algo == 2 ? 64 : small_tile(logDY, S, N, K, cus);
-    case kFused1dMfma512Tile32: return algo == 4 ? 32 : small_tile(logDY, S, N, K, cus);
+    case kFused1dMfma512: return algo == 2 ? 64 : small_tile(S, N, cus);
+    case kFused1dMfma512Tile32: return algo == 4 ? 32 : small_tile(S, N, cus);
     case kFused1dSplitK: return SPLIT_NT;
     case kFused1dCluster: return N;
     case kFused1dWide: return wide_tiles(logDY, S, N, K, algo, cus) ? 128 : 64;
