@@ -20,6 +20,9 @@
  *     exp(-2 pi i jm/D), backward transforms exp(+2 pi i jm/D) and are UNNORMALISED.
  *   - Layouts: x[K][S][DY] (signal (k,s) at (k*S+s)*DY), W[k + n*K], y[N][S][DY]; in 2D
  *     x[K][bs][DX][DY], y[N][bs][DX][DY].
+ *   - Results must not overlap inputs. With 64 output channels two calls also run in place, because the block that reads a signal's
+ *     channels then writes all of its outputs: turbofno_cgemm with C == A; turbofno_fused_fft_cgemm_ifft and turbofno_layer_1d
+ *     with y == x, as long as no value is outside the range that "Precision" names.
  *   - Precision: operands, sums and results are fp32 over the whole range of floats, infinities and NaN included. Products of
  *     most sizes are formed from bf16 parts of their operands on the matrix cores; where a spectrum or weight (times alpha) that is
  *     not zero lies below 2^-110 or within 2^-9 of the largest float, is infinite or NaN, that part of the product is formed with

@@ -46,14 +46,22 @@ def test_small_grids_of_any_magnitude(algo, S, DY, K, N, scale, algo_1d):
     _layer_check(run, lambda x, W: oracle.layer_1d(x, W, 0.5 - 0.75j), _x(S, DY, K), W, scale, tol, N)
 
 
-@pytest.mark.parametrize("DY", [512, 1024])
-def test_y_in_the_place_of_x(DY):
-    """one block per signal set, whatever the size would choose: nothing of x is overwritten before it is read"""
-    S, K, N = 20, 64, 64
-    print("small grid in place", DY, flush=True)
+@pytest.mark.parametrize("DY", [128, 256, 512, 1024])
+@pytest.mark.parametrize("S,K,attach", [(20, 64, False), (100, 128, False), (20, 64, True), (300, 40, False)])
+def test_y_in_the_place_of_x(S, K, attach, DY):
+    """64 output channels: one block per signal set, whatever the size would choose (tiles of 16 or 32, the K split, a cluster):
+    nothing of x is overwritten before it is read"""
+    N = 64
+    print("small grid in place", S, K, attach, DY, flush=True)
     x, W = _x(S, DY, K), _complex(np.random.default_rng(S), N, K) / np.float32(np.sqrt(K))
     ref = oracle.layer_1d(x.cpu().numpy(), W, 1.0)
-    for _ in range(3):
-        y = x.clone()
-        tf.layer_1d(y, _dev(W), y=y)
-        assert rel_l2(y.cpu().numpy(), ref) < _bound(K, 2)
+    buffer = tf.ExchangeBuffer() if attach else None
+    try:
+        for _ in range(3):
+            y = torch.zeros((max(K, N), S, DY), dtype=torch.complex64, device="cuda")
+            y[:K] = x
+            tf.layer_1d(y[:K], _dev(W), y=y[:N])
+            assert rel_l2(y[:N].cpu().numpy(), ref) < _bound(K, 2)
+    finally:
+        if buffer is not None:
+            buffer.close()

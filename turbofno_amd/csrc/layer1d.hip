@@ -676,6 +676,8 @@ int tile_of_fused_1d_kernel(int kernel, int logDY, long S, int N, int K, int alg
 // 49.9 / 46.2 us); with two per CU the larger register budget is ahead (S = 512, K = 96: 37.4 / 39.3).
 static bool dense_blocks(long S, int N, long cus) { return S * (N / 64) > 3 * cus; }
 
+static bool overlap(const float2* a, long na, const float2* b, long nb) { return a < b + nb && b < a + na; }
+
 hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* y,
                                        float2 alpha, int algo, hipStream_t stream, bool y_is_reread)
 {
@@ -683,12 +685,16 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
     // caches instead of streaming it past them; the clustered kernel ignores it
     const int keep_y = y_is_reread ? 1 : 0;
     const long cus = cu_count();
-    int kernel = pick_fused_1d_kernel(logDY, S, N, K, algo, cus, exchange_attached(stream));
+    // y in the place of x with 64 output channels: one block per signal set, which reads its rows of x before it writes them. (With more the
+    // blocks of a signal set would race; the members of a cluster may read x again after others have written.)
+    const bool in_place = N == 64 && overlap(x, (long)K * S << logDY, y, (long)N * S << logDY);
+    int kernel = pick_fused_1d_kernel(logDY, S, N, K, algo, cus, !in_place && exchange_attached(stream));
     if (kernel == kFused1dCluster) {
         const hipError_t e = launch_fused_cluster(S, N, K, cluster_size_1d(logDY, S, N, K, cus), x, W, y, alpha, stream);
         if (e != hipErrorNotReady) return e;
         kernel = pick_fused_1d_kernel(logDY, S, N, K, algo, cus, false);    // detached in between
     }
+    if (in_place && kernel == kFused1dSplitK) kernel = kFused1dMfma512;
     switch (kernel) {
     case kFused1dDense:
         if (logDY == 7 && K <= 8) return launch_fused_wave(S, N, K, x, W, y, alpha, stream, keep_y);
@@ -699,8 +705,6 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
         return keep_y ? launch_fused_split_channels<true>(S, N, K, x, W, y, alpha, stream) : launch_fused_split_channels<false>(S, N, K, x, W, y, alpha, stream);
     case kFused1dMfma512Tile32:
     case kFused1dMfma512: {
-        // y in the place of x: one block per signal set, so that nobody reads what another block has overwritten
-        const bool in_place = x < y + (long)N * S * (1L << logDY) && y < x + (long)K * S * (1L << logDY);
         const int tile = in_place ? 64 : tile_of_fused_1d_kernel(kernel, logDY, S, N, K, algo, cus);
         return launch_fused_small(logDY, S, N, K, x, W, y, alpha, tile, stream, keep_y);
     }
