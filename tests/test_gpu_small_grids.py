@@ -65,3 +65,24 @@ def test_y_in_the_place_of_x(S, K, attach, DY):
     finally:
         if buffer is not None:
             buffer.close()
+
+
+@pytest.mark.parametrize("DY", [128, 256, 512, 1024])
+def test_halves_of_one_signal_in_place(DY):
+    """one signal, 64 output channels: C over x and y over A, read by one block before it writes"""
+    N = K = 64
+    print("halves in place", DY, flush=True)
+    x, W = _x(1, DY, K), _complex(np.random.default_rng(DY), N, K) / np.float32(np.sqrt(K))
+    spectra = oracle.fft_trunc_contig(x.cpu().numpy()).reshape(K, 64)
+    first = oracle.cgemm(spectra, W, 1.0)
+    second = oracle.ifft_pad_contig(oracle.cgemm(first.astype(np.complex64), W, 1.0).reshape(N, 1, 64), DY)
+    for _ in range(3):
+        buf = x.clone()
+        C = buf.view(-1)[:N * 64].view(N, 64)
+        tf.fused_fft_cgemm(64, N, K, buf, _dev(W), C)
+        assert rel_l2(C.cpu().numpy(), first) < _bound(K, 1)
+        buf = torch.zeros((N, 1, DY), dtype=torch.complex64, device="cuda")
+        A = buf.view(-1)[:K * 64].view(K, 64)
+        A.copy_(torch.from_numpy(first.astype(np.complex64)))
+        tf.fused_cgemm_ifft(64, N, K, A, _dev(W), buf)
+        assert rel_l2(buf.cpu().numpy(), second) < _bound(K, 1)

@@ -731,7 +731,9 @@ hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2*
     const long cus = cu_count(), items = S * (N / 64);
     const bool short_round = logDY == 7 && K > 48 && K <= 64 && 2 * items > cus && items < cus;
     if (items <= cus && !short_round) {
-        const int tile = K >= 32 && 2 * S * (N / 16) <= cus ? 16 : (S * (N / 32) <= cus ? 32 : 64);
+        // C over x (one signal, 64 output channels): one block, which reads before it writes
+        const bool shared = overlap(x, (long)K * S << logDY, C, 64L * S * N);
+        const int tile = shared ? 64 : K >= 32 && 2 * S * (N / 16) <= cus ? 16 : (S * (N / 32) <= cus ? 32 : 64);
         return launch_small_forward(logDY, S, N, K, x, W, C, alpha, beta, tile, stream);
     }
     // blocks of 128 output channels from one and a half per CU (N = 128, K = 64, DY = 256: S = 700 42.6 -> 34.4 us, S = 256 19.0 -> 19.9)
@@ -749,7 +751,8 @@ hipError_t launch_fused_cgemm_ifft(int logDY, long S, int N, int K, const float2
     const float2 beta = make_float2(0.f, 0.f);
     const long cus = cu_count(), items = S * (N / 64);
     if (items <= cus && (logDY == 7 || (logDY == 8 && N % 128 == 0) || 8 * items <= 7 * cus)) {
-        const int tile = S * (N / 16) <= cus ? 16 : (S * (N / 32) <= cus ? 32 : 64);
+        const bool shared = overlap(A, 64L * S * K, y, (long)N * S << logDY);   // y over A, likewise
+        const int tile = shared ? 64 : S * (N / 16) <= cus ? 16 : (S * (N / 32) <= cus ? 32 : 64);
         return launch_small_backward(logDY, S, N, K, A, W, y, alpha, tile, stream);
     }
     if (K <= 8 && (logDY == 9 || (logDY == 10 && items > cus)))
