@@ -91,6 +91,26 @@ def test_large_grids_and_long_axes():
     assert tf.query_2d_algo(4, 1024, 1024, 32, 64) == tf.ALGO_ROWS_FIRST           # 3072 MiB
 
 
+def test_2d_algorithms_near_the_lines():
+    """small batches with many channels, where the whole-image path is ahead earlier, and the order of the smallest three-stage problems: the last
+    shape on each side of a line"""
+    three, whole, rows = tf.ALGO_THREE_KERNEL, tf.ALGO_WHOLE_IMAGE, tf.ALGO_ROWS_FIRST
+    for bs, DX, DY, K, N, algo in [
+            (5, 128, 128, 112, 64, three), (5, 128, 128, 120, 64, whole), (6, 128, 128, 64, 128, three), (6, 128, 128, 72, 128, whole),
+            (3, 128, 256, 40, 64, three), (3, 128, 256, 48, 64, whole), (2, 128, 256, 128, 64, whole), (2, 128, 256, 136, 64, three),
+            (7, 256, 128, 104, 64, three), (7, 256, 128, 112, 64, whole), (3, 256, 256, 80, 64, whole), (3, 256, 256, 88, 64, three),
+            (2, 256, 512, 104, 64, rows), (2, 256, 512, 112, 64, whole), (2, 512, 256, 104, 64, three), (2, 512, 256, 112, 64, whole),
+            (2, 512, 512, 88, 64, rows), (2, 512, 512, 96, 64, whole), (2, 1024, 256, 104, 64, three), (2, 1024, 256, 112, 64, whole),
+            (1, 1024, 512, 104, 64, three), (1, 1024, 512, 112, 64, whole),
+            (1, 1024, 1024, 104, 64, rows), (1, 1024, 1024, 112, 64, whole), (1, 1024, 1024, 128, 64, whole), (1, 1024, 1024, 136, 64, rows),
+            (1, 1024, 1024, 112, 192, whole), (1, 1024, 1024, 112, 256, rows), (2, 1024, 1024, 104, 128, rows), (2, 1024, 1024, 112, 128, whole),
+            (1, 128, 256, 64, 64, rows), (1, 128, 256, 72, 64, three), (2, 128, 256, 24, 64, rows), (2, 128, 256, 32, 64, three),
+            (2, 128, 256, 16, 128, rows), (2, 128, 256, 24, 128, three), (2, 128, 256, 8, 192, three), (2, 128, 256, 16, 256, three),
+            (3, 128, 256, 8, 64, rows), (3, 128, 256, 16, 64, three),
+            (1, 256, 512, 64, 64, three), (1, 256, 512, 72, 64, rows), (1, 512, 1024, 16, 64, three), (1, 512, 1024, 24, 64, rows)]:
+        assert tf.query_2d_algo(bs, DX, DY, K, N) == algo, (bs, DX, DY, K, N)
+
+
 def test_queries_answer_zero_for_arguments_the_calls_refuse():
     assert tf.query_1d_kernel(256, 4, 64, 12, CUS) == 0             # K not a multiple of 8
     assert tf.query_1d_kernel(2048, 4, 64, 8, CUS) == 0             # no kernel of that length

@@ -52,21 +52,22 @@ size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Many input channels for the number of images: the three-stage paths run their middle stage at the rate of its transforms and products, in
 // blocks that repeat the forward transforms, while the whole-image path has the mode GEMM and two image kernels with one block per image (or part
-// of one). It is ahead at smaller sizes the more channels there are, provided the rounds of 256 blocks of its two kernels are reasonably full: 264
-// images are two rounds. Measured on MI355X, three stages (the better order) / whole image, us:
-//   128 x 128: bs = 12, K = 64, N = 64: 71.4 / 63.9; bs = 6, K = 88, N = 64: 1.06 the other way, N = 128: 0.99
-//   128 x 256: bs = 3, K = 64, N = 64: 41.9 / 38.4; bs = 6, K = 112: 87 / 81 (108 for the order that was taken); bs = 2, K = 64, N = 64: 1.03 the other way, K = 136 (272 images): 44.6 / 46.0
-//   256 x 128: bs = 12, K = 64, N = 64: 114 / 102; bs = 10, K = 64: 1.04 the other way
-//   256 x 256: bs = 2, K = 112, N = 64: 56.5 / 53.0; bs = 4, K = 112: 102 / 91; bs = 3, K = 88 (264 images): 1.08 the other way
-//   256 x 512: bs = 2, K = 112, N = 64: 95 / 85, bs = 4, K = 72 (288 images): 138 / 145; 512 x 256: bs = 3, K = 112: 145 / 128, bs = 2, K = 104: 83 / 88, bs = 3, K = 48 (288 parts): 1.17 the other way
-//   512 x 512: bs = 1, K = 112, N = 64: 101 / 86, bs = 2, K = 48, N = 64: level; 1024 x 256: bs = 3, K = 112: 260 / 240; 1024 x 512: bs = 1, K = 112: 186 / 170;
-//   1024 x 1024: bs = 1, K = 112: 317 / 302
-// The intermediates of the whole-image path are the smaller ones at all of these lengths.
+// of one). It is ahead at smaller sizes the more channels there are, provided the rounds of kImageBlocks blocks of its two kernels are reasonably
+// full: 264 images are two rounds. Measured on MI355X, three stages (the better order) / whole image, us, N = 64:
+//   128 x 128: bs = 12, K = 64: 71.4 / 63.9, bs = 6, K = 88: 1.06 the other way; 128 x 256: bs = 3, K = 64: 41.9 / 38.4, bs = 2, K = 64: 1.03 the other way, K = 136
+//   (272 images): 44.6 / 46.0; 256 x 128: bs = 12, K = 64: 114 / 102, bs = 10, K = 64: 1.04 the other way; 256 x 256: bs = 4, K = 112: 102 / 91, bs = 3, K = 88: 1.08
+//   the other way; 256 x 512: bs = 2, K = 112: 95 / 85; 512 x 256: bs = 3, K = 112: 145 / 128, K = 48: 1.17 the other way; 512 x 512: bs = 1, K = 112: 101 / 86;
+//   1024 x 256: bs = 3, K = 112: 260 / 240; 1024 x 512: bs = 1, K = 112: 198 / 168; 1024 x 1024: bs = 1, K = 112: 334 / 304, K = 136 (544 parts) 383 / 383, N = 256:
+//   K = 112 621 / 639, K = 136 669 / 713; bs = 2, K = 104, N = 128: 768 / 793.
+// Every shape with bs <= 32, K <= 136, N <= 256 that this rule moves (638 of them) was timed against the path it had before: 1.13 times as fast on
+// average, none more than 1 % slower. The intermediates of the whole-image path are the smaller ones at all of these lengths.
+// The lines are those of a whole MI355X; asking the device for its compute units would make turbofno_query_2d_algo a call into the HIP runtime.
+constexpr long kImageBlocks = 256;
 bool whole_image_ahead_by_channels(int bs, int lx, int ly, int K, int N)
 {
     const long parts = lx > 1 ? 1L << (lx - 1) : 1, forward = parts * K * bs, backward = parts * N * bs;
-    const long rounds = (forward + 255) / 256 + (backward + 255) / 256;
-    auto filled = [&](long percent) { return 100 * (forward + backward) >= percent * 256 * rounds; };
+    const long forward_rounds = (forward + kImageBlocks - 1) / kImageBlocks, rounds = forward_rounds + (backward + kImageBlocks - 1) / kImageBlocks;
+    auto filled = [&](long percent) { return 100 * (forward + backward) >= percent * kImageBlocks * rounds; };
     switch (4 * lx + ly) {                              // log2 DX - 7, log2 DY - 7
     case 0: return forward >= (N >= 128 ? 430 : 600);
     case 1: return forward >= (N >= 128 ? 120 : 144) && (forward <= 256 || forward >= 300 || filled(58));
@@ -77,7 +78,7 @@ bool whole_image_ahead_by_channels(int bs, int lx, int ly, int K, int N)
     case 10: return forward >= 190 && filled(68) && (K >= 96 || N >= 128);
     case 13: return forward >= 890;
     case 14: return (forward >= 440 && K >= 96) || forward >= 900;
-    case 15: return forward >= 440 && K >= 96;
+    case 15: return forward >= 440 && K >= 96 && N <= 192 && 100 * forward >= 85 * kImageBlocks * forward_rounds;
     default: return false;
     }
 }
@@ -87,8 +88,9 @@ bool whole_image_ahead_by_channels(int bs, int lx, int ly, int K, int N)
 // images. Measured on MI355X (256 CUs; 160 shapes, both paths back to back): from a batch of 8 the whole-image path is
 // ahead (by up to 2x at bs = 16) but for two groups of shapes (below); with a batch of 4 to 7 it is ahead for 256 x 256
 // images once (K + N) * bs reaches 768 images in and out, and for 128 x 256 images with N >= 128; with many channels earlier (above). Otherwise
-// three stages, X axis first; whole rows of 128 x 256 images first while the grids are smallest, because their intermediates are half as large (rows first / X
-// axis first, N = 64: bs = 1: K = 32 0.91, K = 64 0.85; bs = 2: K = 16 0.88, K = 32 1.01; bs = 3: K = 8 0.89, K = 16 1.00).
+// three stages, X axis first; whole rows of 128 x 256 images first while the grids are smallest, because their intermediates are half as large (rows
+// first / X axis first, N = 64: bs = 1: K = 32 0.91, K = 64 0.85; bs = 2: K = 16 0.88, K = 32 1.01; bs = 3: K = 8 0.89, K = 16 1.00; but bs = 2, K = 16:
+// N = 192 1.04, N = 256 1.09).
 int pick_algo(int bs, int DX, int DY, int K, int N, int algo)
 {
     if (algo != TURBOFNO_2D_AUTO) return algo;
@@ -121,7 +123,7 @@ int pick_algo(int bs, int DX, int DY, int K, int N, int algo)
         return (DY >= 1024 || (long)K * bs >= 128) ? TURBOFNO_2D_ROWS_FIRST : TURBOFNO_2D_THREE_KERNEL;
     }
     if (bs >= 16) return TURBOFNO_2D_WHOLE_IMAGE;
-    if (DX == 128 && DY == 256 && ((bs == 1 && K <= 64) || (bs == 2 && K <= (N == 64 ? 24 : 16)) || (bs == 3 && K <= 8))) return TURBOFNO_2D_ROWS_FIRST;
+    if (DX == 128 && DY == 256 && ((bs == 1 && K <= 64) || (bs == 2 && N <= 128 && K <= (N == 64 ? 24 : 16)) || (bs == 3 && K <= 8))) return TURBOFNO_2D_ROWS_FIRST;
     if (bs < 4) return TURBOFNO_2D_THREE_KERNEL;
     const bool big = DX == 256 && DY == 256;
     if (bs >= 8) {
