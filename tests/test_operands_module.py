@@ -1,5 +1,8 @@
 """The compiled operand checks of the binding (csrc/operands.cpp) against the checks in Python: what one takes the other takes with the same
 result, what one refuses the other refuses with the same error."""
+import sysconfig
+import types
+
 import numpy as np
 import pytest
 import torch
@@ -69,6 +72,21 @@ def _compare(device, monkeypatch):
             m.setattr(api, "_operands", None)
             without = _outcome(call)
         assert with_module == without, name
+
+
+def test_a_module_of_another_torch_is_left_alone():
+    """it would read tensors at the offsets of another build's headers"""
+    here = "torch %s, %s" % (torch.__version__, sysconfig.get_config_var("SOABI"))
+    module = types.SimpleNamespace(built_for=here)
+    assert api._of_this_torch(module) is module
+    for other in ("torch 2.9.0, " + sysconfig.get_config_var("SOABI"), "torch %s, cpython-311-x86_64-linux-gnu" % torch.__version__, "", None):
+        assert api._of_this_torch(types.SimpleNamespace(built_for=other)) is None, other
+    assert api._of_this_torch(types.SimpleNamespace()) is None         # built before the module named its torch
+
+
+@needs_module
+def test_the_built_module_names_its_torch():
+    assert api._operands.built_for == "torch %s, %s" % (torch.__version__, sysconfig.get_config_var("SOABI"))
 
 
 @needs_module

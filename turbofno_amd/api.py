@@ -7,12 +7,21 @@ complex64 tensors resident on the GPU; every call is asynchronous on torch's cur
 """
 import ctypes
 import os
+import sysconfig
 
 import torch
 
+
+def _of_this_torch(module):
+    """the compiled module if it was built with this torch for this Python, else None: it reads tensors at the offsets of the headers it was built with"""
+    wanted = "torch %s, %s" % (torch.__version__, sysconfig.get_config_var("SOABI"))
+    return module if getattr(module, "built_for", None) == wanted else None
+
+
 try:
     from . import _operands             # operand checks without a trip through Python per attribute (csrc/operands.cpp)
-except ImportError:                     # not built, or built for another torch: the checks below do the same
+    _operands = _of_this_torch(_operands)
+except ImportError:                     # not built: the checks below do the same
     _operands = None
 
 MODES = 64

@@ -153,4 +153,13 @@ PyModuleDef module = { PyModuleDef_HEAD_INIT, "_operands", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__operands(void) { return PyModule_Create(&module); }
+// BUILT_FOR: torch and Python of the headers, "torch <version>, <SOABI>"; the binding leaves the module alone under any other
+PyMODINIT_FUNC PyInit__operands(void)
+{
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "built_for", BUILT_FOR) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}
