@@ -23,6 +23,13 @@ const at::Tensor* gpu_tensor(PyObject* o, at::ScalarType type, int& device)
     return t.get_device() == device ? &t : nullptr;
 }
 
+// The interpreter's lock is given back while a launch waits for room in the queue (the caller's frame holds the operands), and taken again
+// however the call ends
+struct WithoutLock {
+    PyThreadState* held = PyEval_SaveThread();
+    ~WithoutLock() { PyEval_RestoreThread(held); }
+};
+
 bool fits_int(int64_t v) { return v >= 0 && v <= INT_MAX; }
 
 // alpha as anything with a complex value; false leaves the question to Python
@@ -97,10 +104,8 @@ PyObject* layer_1d(PyObject*, PyObject* const* args, Py_ssize_t count)
                 if (W->size(1) == K && y->size(0) == N && y->size(1) == S && y->size(2) == DY && dimX > 0 && S % dimX == 0 && fits_int(K) && fits_int(S) &&
                     fits_int(DY) && fits_int(N) && fits_int(dimX)) {
                     void *px = x->data_ptr(), *pW = W->data_ptr(), *py = y->data_ptr();
-                    // a launch may wait for room in the queue: not with the interpreter's lock (the caller's frame holds the operands)
-                    Py_BEGIN_ALLOW_THREADS
+                    const WithoutLock unlocked;
                     rc = call((int)(S / dimX), (int)dimX, (int)DY, (int)K, (int)N, px, pW, py, re, im, stream);
-                    Py_END_ALLOW_THREADS
                 }
             }
         } catch (...) {
@@ -131,9 +136,8 @@ PyObject* layer_2d(PyObject*, PyObject* const* args, Py_ssize_t count)
                     fits_int(DX) && fits_int(DY) && fits_int(N)) {
                     void *px = x->data_ptr(), *pW = W->data_ptr(), *py = y->data_ptr(), *pws = ws->data_ptr();
                     const size_t bytes = (size_t)ws->numel();
-                    Py_BEGIN_ALLOW_THREADS
+                    const WithoutLock unlocked;
                     rc = call((int)bs, (int)DX, (int)DY, (int)K, (int)N, px, pW, py, re, im, pws, bytes, (int)algo, stream);
-                    Py_END_ALLOW_THREADS
                 }
             }
         } catch (...) {
