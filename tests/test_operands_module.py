@@ -1,5 +1,5 @@
-"""The compiled operand checks of the binding (csrc/operands.cpp) against the checks in Python: what one takes the other takes with the same
-result, what one refuses the other refuses with the same error."""
+"""The compiled operand checks of the binding (csrc/operands.cpp) against the checks in Python: what one takes the other takes, with the same
+values, what one refuses the other refuses with the same error."""
 import sysconfig
 import types
 
@@ -96,7 +96,7 @@ def test_same_refusals_without_a_gpu(monkeypatch):
 
 @needs_module
 @pytest.mark.gpu
-def test_same_results_and_refusals(monkeypatch):
+def test_same_forms_taken_and_refused(monkeypatch):
     """zeros in: every call either runs (the kernels accept the form) or raises before a launch"""
     _compare("cuda", monkeypatch)
     torch.cuda.synchronize()
@@ -113,3 +113,45 @@ def test_module_takes_the_plain_call():
     assert api._operands.operands(x, x.numel(), y, y.numel()) == (x.data_ptr(), y.data_ptr())
     assert api._operands.operands(x, x.numel() + 1) is None
     torch.cuda.synchronize()
+
+
+def _random(*shape):
+    gen = torch.Generator(device="cuda").manual_seed(len(shape) + shape[0])
+    return torch.view_as_complex(torch.rand(shape + (2,), device="cuda", generator=gen) * 2 - 1)
+
+
+def _values(call, y):
+    y.fill_(float("nan"))
+    call()
+    return torch.view_as_real(y).clone()
+
+
+@needs_module
+@pytest.mark.gpu
+def test_same_values_either_way(monkeypatch):
+    """the same launch with the same arguments: alpha's parts, dimX, the algorithm and the workspace, bit for bit"""
+    alpha, K, N = 0.5 - 0.75j, 16, 64
+    W = _random(N, K)
+    x, y = _random(K, 6, 256), torch.empty((N, 6, 256), dtype=torch.complex64, device="cuda")
+    calls = [("layer_1d dimX=%d" % d, lambda d=d: tf.layer_1d(x, W, y=y, alpha=alpha, dimX=d), y) for d in (1, 2)]
+    x2, y2 = _random(K, 2, 128, 256), torch.empty((N, 2, 128, 256), dtype=torch.complex64, device="cuda")
+    for algo in (0, 1, 2, 3):
+        ws = torch.zeros(tf.layer_2d_workspace_bytes(2, 128, 256, K, N, algo), dtype=torch.uint8, device="cuda")
+        calls.append(("layer_2d algo=%d" % algo, lambda algo=algo, ws=ws: tf.layer_2d(x2, W, y=y2, alpha=alpha, workspace=ws, algo=algo), y2))
+    M = 64 * 6
+    A, C = _random(K, M), torch.empty((N, M), dtype=torch.complex64, device="cuda")
+    calls += [("cgemm", lambda: tf.cgemm(M, N, K, A, W, C, alpha), C), ("fused", lambda: tf.fused_fft_cgemm_ifft(M, N, K, x, W, y, alpha), y),
+              ("first half", lambda: tf.fused_fft_cgemm(M, N, K, x, W, C, alpha), C), ("second half", lambda: tf.fused_cgemm_ifft(M, N, K, A, W, y, alpha), y)]
+    results = {}
+    for name, call, out in calls:
+        print("values", name, flush=True)
+        short = _values(call, out)
+        with monkeypatch.context() as m:
+            m.setattr(api, "_operands", None)
+            long = _values(call, out)
+        assert not bool(torch.isnan(short).any()), name
+        assert torch.equal(short, long), name
+        results[name] = short
+    # the algorithms round differently: a call that ran another one would show
+    layers = [results["layer_2d algo=%d" % a] for a in (1, 2, 3)]
+    assert not torch.equal(layers[0], layers[1]) and not torch.equal(layers[1], layers[2]) and not torch.equal(layers[0], layers[2])
