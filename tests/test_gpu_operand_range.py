@@ -138,7 +138,8 @@ LAYERS = [                           # S, DY, K, N: the fused 1D kernel with 64 
 ]
 SMALL_GRIDS = [(3, 64, 64), (5, 136, 128), (9, 128, 192)]     # S, K, N at DY = 256: the channels split over the waves of a block
 HALVES = [(9, 128, 40, 64), (513, 128, 40, 128), (9, 256, 72, 64), (400, 256, 40, 128), (9, 512, 40, 64), (400, 512, 40, 128),
-          (9, 1024, 40, 64), (390, 1024, 24, 128), (256, 512, 24, 64), (128, 1024, 8, 128)]
+          (9, 1024, 40, 64), (390, 1024, 24, 128), (256, 512, 24, 64), (128, 1024, 8, 128),
+          (300, 512, 8, 64)]                     # the SIMT kernel
 _TRANSFORMS = 2 * 16 ** 0.5 * 2.0 ** -24       # two transforms of eight real additions in a row per value
 
 

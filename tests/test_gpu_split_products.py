@@ -287,7 +287,7 @@ def test_blocks_of_128_output_channels_as_middle_stage(bs, DX, DY, K, N, algo, a
     (1, 256, 8, 64), (9, 256, 40, 192), (400, 256, 72, 128),        # S = 400: blocks of 128 output channels
     (160, 128, 56, 64),                                              # first half with a short round, less than one block per CU
     (3, 512, 24, 64), (400, 512, 40, 128), (2, 1024, 8, 64), (390, 1024, 24, 128),
-    (5, 512, 8, 192), (900, 1024, 8, 64), (3, 1024, 16, 128),       # few channels: the SIMT kernel, both halves or the second
+    (5, 512, 8, 192), (900, 1024, 8, 64), (3, 1024, 16, 128),       # few channels; the second: first half by the SIMT kernel
     (512, 256, 40, 64), (256, 512, 40, 128), (128, 1024, 24, 64),   # 1 MiB between channels: the waves of a block take every fourth one
 ])
 @pytest.mark.parametrize("beta", [0.0, -1 + 1j])
@@ -315,3 +315,37 @@ def test_halves_of_the_layer(S, DY, K, N, beta):
     assert rel_l2(pick(C), ref) < _bound(K, 1)
     ref = oracle.ifft_pad_contig(oracle.cgemm(pick(C).reshape(N, -1), W2, 1 - 1j).reshape(N, -1, 64), DY)
     assert rel_l2(pick(y), ref) < _bound(N, 1)
+
+
+@pytest.mark.parametrize("S,DY,N", [
+    (300, 512, 64), (900, 1024, 64),     # both halves by the SIMT kernel (first half at 1024: three to eight blocks per CU)
+    (300, 1024, 64),                     # the second
+    (240, 512, 64),                      # the second, between seven eighths of a block and a block per CU
+    (150, 512, 192),                     # both, three blocks per signal set
+])
+@pytest.mark.parametrize("beta", [0.0, -1 + 1j])
+def test_halves_with_eight_channels_on_larger_grids(S, DY, N, beta):
+    """the SIMT kernel, which sums in fp32 without splits: every value of C and y written, the halves apart from each other"""
+    K = 8
+    print("SIMT halves", S, DY, N, beta, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(S + DY)
+    rng = np.random.default_rng(S + N)
+    x = torch.view_as_complex(torch.rand((K, S, DY, 2), device="cuda", generator=gen) * 2 - 1)
+    A = torch.view_as_complex(torch.rand((K, S, 64, 2), device="cuda", generator=gen) * 2 - 1)
+    W = _complex(rng, N, K) / np.float32(np.sqrt(K))
+    C0 = torch.full((N, S, 64), float("nan"), dtype=torch.complex64, device="cuda") if beta == 0.0 else \
+        torch.view_as_complex(torch.rand((N, S, 64, 2), device="cuda", generator=gen) * 2 - 1)
+    C, y = C0.clone(), torch.full((N, S, DY), float("nan"), dtype=torch.complex64, device="cuda")
+    tf.fused_fft_cgemm(64 * S, N, K, x, _dev(W), C, 0.5 - 0.75j, beta)
+    tf.fused_cgemm_ifft(64 * S, N, K, A, _dev(W), y, 1 - 1j)
+    torch.cuda.synchronize()
+    assert not bool(torch.isnan(torch.view_as_real(C)).any()), "values of C left unwritten"
+    assert not bool(torch.isnan(torch.view_as_real(y)).any()), "rows of y left unwritten"
+    idx = torch.tensor(sorted({0, 7, S // 2, S - 9, S - 1}), device="cuda")
+    pick = lambda a: a.index_select(1, idx).cpu().numpy()
+    ref = oracle.cgemm(oracle.fft_trunc_contig(pick(x)).reshape(K, -1), W, 0.5 - 0.75j).reshape(N, -1, 64)
+    if beta != 0.0:
+        ref = ref + beta * pick(C0).astype(np.complex128)
+    assert rel_l2(pick(C), ref) < _bound(K, 1)
+    ref = oracle.ifft_pad_contig(oracle.cgemm(pick(A).reshape(K, -1), W, 1 - 1j).reshape(N, -1, 64), DY)
+    assert rel_l2(pick(y), ref) < _bound(K, 1)
