@@ -156,6 +156,19 @@ def test_1d_kernels_where_the_last_round_or_the_last_blocks_are_nearly_empty():
     assert tf.query_1d_tile(256, 512, 128, 32, CUS) == 64
 
 
+def test_1d_kernels_with_nearly_a_block_per_cu():
+    """where the small-grid kernel (2) gives way to the kernels that it was measured against: the last shape on each side of a line"""
+    for N in (64, 128, 256):
+        tiles = N // 64
+        for K, last in ((8, 208), (16, 192)):           # DY = 256: the split kernel
+            assert tf.query_1d_kernel(256, last // tiles, N, K, CUS) == 2, (N, K)
+            assert tf.query_1d_kernel(256, last // tiles + 1, N, K, CUS) == 3, (N, K)
+        assert tf.query_1d_kernel(256, CUS // tiles, N, 24, CUS) == 2
+        # DY = 1024: the SIMT kernel, which takes what is left over as well
+        assert tf.query_1d_kernel(1024, 192 // tiles - 1, N, 8, CUS) == 2 and tf.query_1d_kernel(1024, 192 // tiles, N, 8, CUS) == 1
+        assert tf.query_1d_kernel(1024, CUS // tiles, N, 16, CUS) == 2
+
+
 def test_mode_gemm_steps(tmp_path):
     """half steps follow the run that is walked, not the period of the weights: with R parts per image a run mostly covers all R of them"""
     exe = str(tmp_path / "gemm_steps_check")
