@@ -720,9 +720,12 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
 // kernel with 16, 32 or 64 output channels). First half: the fewest output channels pay from 32 input channels on and up to half of the CUs
 // (DY = 256, N = 64, K = 128: S = 1: 20.3 / 11.3, 12.5, 15.1, S = 64: 21.5 / 12.9, 13.5, 16.0; DY = 1024, K = 128, S = 64: 65.8 / 39.4, 36.7, 37.8; DY = 256, K = 8, S = 1:
 // 4.4 / 3.8, 4.0, 4.2); a block of 64 on every CU: DY = 128, K = 64, S = 256: 10.4 / 10.2, DY = 1024, K = 32: 21.0 / 16.1. Not with 49 to 64 channels
-// of length 128 in blocks of 64 outputs, whose rounds hold 48 (S = 200: K = 48 8.8 / 7.6, K = 56 9.5 / 9.8, K = 64 9.8 / 9.9, K = 72 11.8 / 10.5). Second half: DY = 256, K = 32, S = 1: 8.4 / 4.5, 5.3, 7.1;
+// of length 128 in blocks of 64 outputs, whose rounds hold 48 (S = 200: K = 48 8.8 / 7.6, K = 56 9.5 / 9.8, K = 64 9.8 / 9.9, K = 72 11.8 / 10.5; S = 128,
+// N = 128, K = 56: 9.8 / 10.1). Second half: DY = 256, K = 32, S = 1: 8.4 / 4.5, 5.3, 7.1;
 // DY = 1024, K = 8, S = 1: 19.4 / 6.3, 9.6, 15.8, S = 64: 21.1 / 9.2, 11.1, 17.3, S = 200: 25.7 / 22.4 with 64; but a block of 64 on every CU: DY = 256, N = 64, K = 8: 8.7 / 9.1 (N = 128:
-// 9.4 / 9.1), DY = 512: 14.8 / 15.4, DY = 1024: 26.8 / 28.1.
+// 9.4 / 9.1), DY = 512: 14.8 / 15.4, DY = 1024: 26.8 / 28.1. Few channels and more than 64 outputs: up to three quarters of the CUs (DY = 256, K = 16:
+// S = 50, N = 256 level, S = 54 8.8 / 9.1; DY = 512, K = 8 (SIMT kernel): S = 62, N = 192 0.98, S = 70 12.8 / 13.4); DY = 1024 with more than 128
+// outputs up to 13 of 16 (N = 256, K = 48: S = 52 0.98, S = 56 27.3 / 28.8).
 // Larger grids: the SIMT kernel with few channels at lengths 512 / 1024; with eight a round of 16 would be half padding (second
 // half, us, split / SIMT: DY = 512, S = 1000: 58.5 / 54.8. First half, with blocks of 64 output
 // channels: DY = 512, S = 4096: 54.2 / 50.8, DY = 1024, N = 64: S = 2048: 49.4 / 46.4, S = 700: 20.2 / 21.7). Otherwise the split kernel: halves,
@@ -731,7 +734,7 @@ hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2*
                                   float2 alpha, float2 beta, hipStream_t stream)
 {
     const long cus = cu_count(), items = S * (N / 64);
-    const bool short_round = logDY == 7 && K > 48 && K <= 64 && 2 * items > cus && items < cus;
+    const bool short_round = logDY == 7 && K > 48 && K <= 64 && 2 * items > cus && (items < cus || N % 128 == 0);
     if (items <= cus && !short_round) {
         // C over x (one signal, 64 output channels): one block, which reads before it writes
         const bool shared = overlap(x, (long)K * S << logDY, C, 64L * S * N);
@@ -747,12 +750,20 @@ hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2*
     return launch_split_forward(logDY, S, N, K, x, W, C, alpha, beta, wide, stream);
 }
 
+static bool small_second_half(int logDY, long items, int N, int K, long cus)
+{
+    if (items > cus || logDY == 7) return items <= cus;
+    if (N > 64 && ((logDY == 8 && K <= 16) || (logDY == 9 && K <= 8))) return 4 * items <= 3 * cus;
+    if (logDY == 8 && N % 128 == 0) return true;
+    if (logDY == 10 && N > 128) return 16 * items <= 13 * cus;
+    return 8 * items <= 7 * cus;
+}
 hipError_t launch_fused_cgemm_ifft(int logDY, long S, int N, int K, const float2* A, const float2* W, float2* y,
                                    float2 alpha, hipStream_t stream)
 {
     const float2 beta = make_float2(0.f, 0.f);
     const long cus = cu_count(), items = S * (N / 64);
-    if (items <= cus && (logDY == 7 || (logDY == 8 && N % 128 == 0) || 8 * items <= 7 * cus)) {
+    if (small_second_half(logDY, items, N, K, cus)) {
         const bool shared = overlap(A, 64L * S * K, y, (long)N * S << logDY);   // y over A, likewise
         const int tile = shared ? 64 : S * (N / 16) <= cus ? 16 : (S * (N / 32) <= cus ? 32 : 64);
         return launch_small_backward(logDY, S, N, K, A, W, y, alpha, tile, stream);
