@@ -725,7 +725,7 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
 // DY = 1024, K = 8, S = 1: 19.4 / 6.3, 9.6, 15.8, S = 64: 21.1 / 9.2, 11.1, 17.3, S = 200: 25.7 / 22.4 with 64; but a block of 64 on every CU: DY = 256, N = 64, K = 8: 8.7 / 9.1 (N = 128:
 // 9.4 / 9.1), DY = 512: 14.8 / 15.4, DY = 1024: 26.8 / 28.1. Few channels and more than 64 outputs: up to three quarters of the CUs (DY = 256, K = 16:
 // S = 50, N = 256 level, S = 54 8.8 / 9.1; DY = 512, K = 8 (SIMT kernel): S = 62, N = 192 0.98, S = 70 12.8 / 13.4); DY = 1024 with more than 128
-// outputs up to 13 of 16 (N = 256, K = 48: S = 52 0.98, S = 56 27.3 / 28.8).
+// outputs up to 13 of 16 (N = 256, K = 48: S = 52 0.98, S = 56 27.3 / 28.8), and so DY = 512, K = 8, N = 64 (S = 222: 12.9 / 13.4).
 // Larger grids: the SIMT kernel with few channels at lengths 512 / 1024; with eight a round of 16 would be half padding (second
 // half, us, split / SIMT: DY = 512, S = 1000: 58.5 / 54.8. First half, with blocks of 64 output
 // channels: DY = 512, S = 4096: 54.2 / 50.8, DY = 1024, N = 64: S = 2048: 49.4 / 46.4, S = 700: 20.2 / 21.7). Otherwise the split kernel: halves,
@@ -755,7 +755,7 @@ static bool small_second_half(int logDY, long items, int N, int K, long cus)
     if (items > cus || logDY == 7) return items <= cus;
     if (N > 64 && ((logDY == 8 && K <= 16) || (logDY == 9 && K <= 8))) return 4 * items <= 3 * cus;
     if (logDY == 8 && N % 128 == 0) return true;
-    if (logDY == 10 && N > 128) return 16 * items <= 13 * cus;
+    if ((logDY == 10 && N > 128) || (logDY == 9 && K <= 8)) return 16 * items <= 13 * cus;
     return 8 * items <= 7 * cus;
 }
 hipError_t launch_fused_cgemm_ifft(int logDY, long S, int N, int K, const float2* A, const float2* W, float2* y,
