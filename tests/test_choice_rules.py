@@ -165,7 +165,7 @@ def test_1d_kernels_with_nearly_a_block_per_cu():
             assert tf.query_1d_kernel(256, last // tiles + 1, N, K, CUS) == 3, (N, K)
         assert tf.query_1d_kernel(256, CUS // tiles, N, 24, CUS) == 2
         # DY = 1024: the SIMT kernel, which takes what is left over as well
-        assert tf.query_1d_kernel(1024, 192 // tiles - 1, N, 8, CUS) == 2 and tf.query_1d_kernel(1024, 192 // tiles, N, 8, CUS) == 1
+        assert tf.query_1d_kernel(1024, 192 // tiles, N, 8, CUS) == 2 and tf.query_1d_kernel(1024, 192 // tiles + 1, N, 8, CUS) == 1
         assert tf.query_1d_kernel(1024, CUS // tiles, N, 16, CUS) == 2
 
 

@@ -567,8 +567,8 @@ static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const
 //    other kernel is level: the split kernel for DY = 256 with up to 16 channels (S = 256, K = 16: 10.5 / 9.9; N = 256: S = 52, K = 16 9.8 / 9.4, S = 54, K = 8 9.7 / 9.5), and for
 //    DY = 128 with 49 to 64 channels, of which the small-grid kernel leaves a sixth to a round of its own (N = 64, S = 200, K = 64: 11.6 / 11.5,
 //    S = 256: 12.2 / 11.9; N = 128, S = 100: 11.6 / 11.5), and with 32 or 40 channels and N no multiple of 128 (S = 256, K = 32: 9.0 / 8.8, S = 200: 8.3 / 8.5),
-//    16 to 40 channels with exactly one block per CU (S = 256, K = 16: 8.2 / 8.1); the SIMT kernel for DY = 1024 with eight channels from three
-//    quarters of the CUs on (S = 200: 24.4 / 23.9, S = 245 28.5 / 27.3);
+//    16 to 40 channels with exactly one block per CU (S = 256, K = 16: 8.2 / 8.1); the SIMT kernel for DY = 1024 with eight channels on more than
+//    three quarters of the CUs (S = 200: 24.4 / 23.9, S = 245 28.5 / 27.3; as middle stage of three images with S = 192 the small-grid kernel is 4 us ahead);
 //  * DY = 256, more than 96 channels (a fourth round), blocks of 32 output channels for more than half of the CUs and at most one each: the
 //    K split, whose rounds have no barrier (small-grid kernel / K split: S = 64, N = 128: K = 104 15.8 / 15.2, K = 128: 17.6 / 17.1; S = 100,
 //    N = 64, K = 104: 14.5 / 13.9). Not with fewer channels or blocks (S = 64, N = 128: K = 64 11.7 / 13.2, K = 96: 14.6 / 15.3; S = 60, N = 64,
@@ -613,7 +613,7 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, long cus, bo
     if (algo == 0 && items <= cus) {
         if (logDY == 7 && 4 * items >= 3 * cus && ((K > 48 && K <= 64) || (N % 128 != 0 && K >= 32 && K <= 40))) return kFused1dMfma256;
         if (logDY == 8 && K <= 16 && (K <= 8 ? 16 * items > 13 * cus : 4 * items > 3 * cus)) return kFused1dMfma256;
-        if (logDY == 10 && 4 * items >= 3 * cus && K <= 8) return kFused1dSimt;
+        if (logDY == 10 && 4 * items > 3 * cus && K <= 8) return kFused1dSimt;
     }
     // lengths 512 / 1024, more than one block per CU
     if (algo == 0 && long_signal && built && items > cus) {
