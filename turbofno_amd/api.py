@@ -13,7 +13,8 @@ import torch
 
 
 def _of_this_torch(module):
-    """the compiled module if it was built with this torch for this Python, else None: it reads tensors at the offsets of the headers it was built with"""
+    """the compiled module if it was built with this torch for this Python, else None: it reads tensors at the offsets of the
+    headers it was built with"""
     wanted = "torch %s, %s" % (torch.__version__, sysconfig.get_config_var("SOABI"))
     return module if getattr(module, "built_for", None) == wanted else None
 

@@ -50,18 +50,20 @@ int check_gemm_dims(long M, int N, int K)
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-// Many input channels for the number of images: the three-stage paths run their middle stage at the rate of its transforms and products, in
-// blocks that repeat the forward transforms, while the whole-image path has the mode GEMM and two image kernels with one block per image (or part
-// of one). It is ahead at smaller sizes the more channels there are, provided the rounds of kImageBlocks blocks of its two kernels are reasonably
-// full: 264 images are two rounds. Measured on MI355X, three stages (the better order) / whole image, us, N = 64:
-//   128 x 128: bs = 12, K = 64: 71.4 / 63.9, bs = 6, K = 88: 1.06 the other way; 128 x 256: bs = 3, K = 64: 41.9 / 38.4, bs = 2, K = 64: 1.03 the other way, K = 136
-//   (272 images): 44.6 / 46.0; 256 x 128: bs = 12, K = 64: 114 / 102, bs = 10, K = 64: 1.04 the other way; 256 x 256: bs = 4, K = 112: 102 / 91, bs = 3, K = 88: 1.08
-//   the other way; 256 x 512: bs = 2, K = 112: 95 / 85; 512 x 256: bs = 3, K = 112: 145 / 128, K = 48: 1.17 the other way; 512 x 512: bs = 1, K = 112: 101 / 86;
-//   1024 x 256: bs = 3, K = 112: 260 / 240; 1024 x 512: bs = 1, K = 112: 198 / 168; 1024 x 1024: bs = 1, K = 112: 334 / 304, K = 136 (544 parts) 383 / 383, N = 256:
-//   K = 112 621 / 639, K = 136 669 / 713; bs = 2, K = 104, N = 128: 768 / 793.
-// Every shape with bs <= 32, K <= 136, N <= 256 that this rule moves (638 of them) was timed against the path it had before: 1.13 times as fast on
-// average, none more than 1 % slower. The intermediates of the whole-image path are the smaller ones at all of these lengths.
-// The lines are those of a whole MI355X; asking the device for its compute units would make turbofno_query_2d_algo a call into the HIP runtime.
+// Many input channels for the number of images: the three-stage paths run their middle stage at the rate of its transforms and
+// products, in blocks that repeat the forward transforms, while the whole-image path has the mode GEMM and two image kernels with
+// one block per image (or part of one). It is ahead at smaller sizes the more channels there are, provided the rounds of
+// kImageBlocks blocks of its two kernels are reasonably full: 264 images are two rounds. Measured on MI355X, N = 64, three stages
+// (the better order) / whole image, us:
+//   128 x 128: bs = 12, K = 64 71.4 / 63.9; 128 x 256: bs = 3, K = 64 41.9 / 38.4, bs = 2, K = 136 (272 images) 44.6 / 46.0;
+//   256 x 128: bs = 12, K = 64 114 / 102; 256 x 256: bs = 4, K = 112 102 / 91; 256 x 512: bs = 2, K = 112 95 / 85;
+//   512 x 256: bs = 3, K = 112 145 / 128; 512 x 512: bs = 1, K = 112 101 / 86; 1024 x 256: bs = 3, K = 112 260 / 240;
+//   1024 x 512: bs = 1, K = 112 198 / 168; 1024 x 1024: bs = 1: K = 112 334 / 304, K = 136 (544 parts) 383 / 383, N = 256, K = 112
+//   621 / 639; bs = 2, K = 104, N = 128 768 / 793.
+// Every shape with bs <= 32, K <= 136, N <= 256 that this rule moves (638 of them) was timed against the path it had before: 1.13
+// times as fast on average, none more than 1 % slower. The intermediates of the whole-image path are the smaller ones.
+// The lines are those of a whole MI355X; asking the device for its compute units would make turbofno_query_2d_algo a call into the
+// HIP runtime.
 constexpr long kImageBlocks = 256;
 bool whole_image_ahead_by_channels(int bs, int lx, int ly, int K, int N)
 {
@@ -87,14 +89,15 @@ bool whole_image_ahead_by_channels(int bs, int lx, int ly, int K, int N)
 // which in turn spreads an image over many blocks and gets three short launches through sooner when there are few
 // images. Measured on MI355X (256 CUs; 160 shapes, both paths back to back): from a batch of 8 the whole-image path is
 // ahead (by up to 2x at bs = 16) but for two groups of shapes (below); with a batch of 4 to 7 it is ahead for 256 x 256
-// images once (K + N) * bs reaches 768 images in and out, and for 128 x 256 images with N >= 128; with many channels earlier (above). Otherwise
-// three stages, X axis first; whole rows of 128 x 256 images first while the grids are smallest, because their intermediates are half as large (rows
-// first / X axis first, N = 64: bs = 1: K = 32 0.91, K = 64 0.85; bs = 2: K = 16 0.88, K = 32 1.01; bs = 3: K = 8 0.89, K = 16 1.00; but bs = 2, K = 16:
-// N = 192 1.04, N = 256 1.09).
+// images once (K + N) * bs reaches 768 images in and out, and for 128 x 256 images with N >= 128; with many channels earlier
+// (above). Otherwise three stages, X axis first; whole rows of 128 x 256 images first while the grids are smallest, because their
+// intermediates are half as large (rows first / X axis first, N = 64: bs = 1, K = 64 0.85; bs = 2: K = 16 0.88, K = 32 1.01; bs = 3:
+// K = 8 0.89, K = 16 1.00; but bs = 2, K = 16: N = 192 1.04, N = 256 1.09).
 int pick_algo(int bs, int DX, int DY, int K, int N, int algo)
 {
     if (algo != TURBOFNO_2D_AUTO) return algo;
-    if (length_built(log2_exact(DX)) && length_built(log2_exact(DY)) && whole_image_ahead_by_channels(bs, log2_exact(DX) - 7, log2_exact(DY) - 7, K, N))
+    if (length_built(log2_exact(DX)) && length_built(log2_exact(DY)) &&
+        whole_image_ahead_by_channels(bs, log2_exact(DX) - 7, log2_exact(DY) - 7, K, N))
         return TURBOFNO_2D_WHOLE_IMAGE;
     if (DX > 256 || DY > 256) {
         // Long axes on the whole-image kernels (512 / 1024 rows as interleaved parts of 256, rows of 512 / 1024 with 32 /
@@ -113,9 +116,9 @@ int pick_algo(int bs, int DX, int DY, int K, int N, int algo)
         // otherwise three stages. The axis that is transformed first is the one whose
         // truncation shrinks the intermediates most, i.e. the longer one (DY = 4 DX: half the time of the other order;
         // DX = 4 DY: the reverse). Square images: whole rows first (9-18 % ahead) unless the grid is small.
-        // The smallest problems with DX of 256 or 512 are sooner through with the X axis first (rows first / X axis first: 256 x 512, bs = 1: K = 16, N = 64 1.05,
-        // N = 128 1.10, K = 64 1.00; bs = 2, K = 8, N = 64 1.11; bs = 3, K = 32 1.01; 512 x 1024, bs = 1: K = 8, N = 64 1.05, K = 16 1.02, N = 128 1.00; 256 x 1024, K = 8: 0.96). Its
-        // intermediates are larger there, at most 60 MiB below these limits.
+        // The smallest problems with DX of 256 or 512 are sooner through with the X axis first (rows first / X axis first, N = 64:
+        // 256 x 512: bs = 1: K = 16 1.05, K = 64 1.00; bs = 2, K = 8 1.11; bs = 3, K = 32 1.01; 512 x 1024, bs = 1: K = 8 1.05, K = 16 1.02; but
+        // 256 x 1024, K = 8: 0.96). Its intermediates are larger there, at most 60 MiB below these limits.
         const long mib = ((long)K + N) * bs * DX * DY >> 17;
         if ((DX == 256 && DY == 512 && mib <= 240 && K <= 64) || (DX == 512 && DY == 1024 && mib <= 320 && K <= 16))
             return TURBOFNO_2D_THREE_KERNEL;
@@ -123,7 +126,8 @@ int pick_algo(int bs, int DX, int DY, int K, int N, int algo)
         return (DY >= 1024 || (long)K * bs >= 128) ? TURBOFNO_2D_ROWS_FIRST : TURBOFNO_2D_THREE_KERNEL;
     }
     if (bs >= 16) return TURBOFNO_2D_WHOLE_IMAGE;
-    if (DX == 128 && DY == 256 && ((bs == 1 && K <= 64) || (bs == 2 && N <= 128 && K <= (N == 64 ? 24 : 16)) || (bs == 3 && K <= 8))) return TURBOFNO_2D_ROWS_FIRST;
+    if (DX == 128 && DY == 256 && ((bs == 1 && K <= 64) || (bs == 2 && N <= 128 && K <= (N == 64 ? 24 : 16)) || (bs == 3 && K <= 8)))
+        return TURBOFNO_2D_ROWS_FIRST;
     if (bs < 4) return TURBOFNO_2D_THREE_KERNEL;
     const bool big = DX == 256 && DY == 256;
     if (bs >= 8) {

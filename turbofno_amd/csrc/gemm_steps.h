@@ -11,14 +11,14 @@ struct GemmWalk {
     bool halves;      // steps in halves of 16 channels, an empty second half skipped
 };
 
-// K: all channels; Kw: period of the weights; nt: tiles of 16 output channels per block; threads per block; cap: steps that the tile can hold.
-// One run covers one period of the weights where that wastes no part of a step, or else all K channels, if the tile can hold them.
-// Half steps where the last step of a run holds at most 16 channels (us, whole steps / halves: M = 163,840, N = 128: K = 40 52.4 / 47.4, K = 104
-// 102.2 / 98.3, K = 176 153.8 / 146.7; two parts, M = 65,536, N = 128: K = 2 x 24 25.1 / 22.7, K = 2 x 72 52.6 / 50.6), and not where it
-// is full or nearly so (M = 163,840, N = 128, K = 64: 56.5 / 58.1; four parts, M = 4,096, N = 64, K = 4 x 40: 8.0 / 8.7). Longest run that gains:
-// 48 channels with tiles of 16 or 32 outputs, which have more per column to rearrange (M = 4,096, N = 64: K = 2 x 40 6.2 / 6.3, K = 2 x 56 7.1 / 7.3);
-// 128 with 64 outputs in blocks of 512 threads (M = 65,536, N = 64: K = 112 25.9 / 25.7, K = 136 29.8 / 30.6); else whatever the tile
-// holds (beyond that: M = 163,840, N = 128, K = 200 192.5 / 194.9).
+// K: all channels; Kw: period of the weights; nt: tiles of 16 output channels per block; threads per block; cap: steps that the tile
+// can hold. One run covers one period of the weights where that wastes no part of a step, or else all K channels, if the tile can
+// hold them. Half steps where the last step of a run holds at most 16 channels (us, whole steps / halves: M = 163,840, N = 128: K =
+// 40 52.4 / 47.4, K = 104 102.2 / 98.3, K = 176 153.8 / 146.7; two parts of 24, M = 65,536, N = 128 25.1 / 22.7), and not where it is
+// full or nearly so (M = 163,840, N = 128, K = 64 56.5 / 58.1; four parts of 40, M = 4,096, N = 64 8.0 / 8.7). Longest run that gains:
+//   48 channels with tiles of 16 or 32 outputs, which have more per column to rearrange (M = 4,096, N = 64: two parts of 56 7.1 / 7.3);
+//   128 with 64 outputs in blocks of 512 threads (M = 65,536, N = 64: K = 112 25.9 / 25.7, K = 136 29.8 / 30.6);
+//   else whatever the tile holds (beyond that: M = 163,840, N = 128, K = 200 192.5 / 194.9).
 inline GemmWalk gemm_walk(int K, int Kw, int nt, int threads, int cap)
 {
     const bool periods = Kw % GEMM_KSTEP == 0 || (K + GEMM_KSTEP - 1) / GEMM_KSTEP > cap;

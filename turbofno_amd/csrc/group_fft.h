@@ -21,17 +21,17 @@ template <int LOGDY> struct Geo1D {
 
 // Lengths 512 / 1024: a group of L = 32 / 64 lanes owns one signal, lane t holds samples t + L i. The scheme of the wide_*
 // codelets (inner 16-point transforms over the lanes tt = a + A b, A = L / 16, then a sum over a), with the lanes and the
-// two exchanges laid out for the LDS banks (8 bytes per lane: a read takes 32 lanes per cycle over 64 banks of 4 bytes, a write 16 lanes
-// over 32 banks):
+// two exchanges laid out for the LDS banks (8 bytes per lane: a read takes 32 lanes per cycle over 64 banks of 4 bytes, a write 16
+// lanes over 32 banks):
 //   second-pass lane t = 16 a + r computes inner_a[c] of bin r, then finishes the modes r + 16 (a + A j) = t + L j: the
 //     natural order, L consecutive modes per slot j;
 //   first exchange: the A rows a + A b of one b side by side, [b][a][16 bins] with a pitch of 16 A + 1: the read of one b
-//     covers 32 consecutive elements per half wavefront. Left at that, the write of one bin meets the same banks from the A parts of a
-//     row, two (L = 32) or four ways (64: 16 cycles instead of 4). SPREAD: the bins of part a at k ^ (16 / A) a, without conflicts, for
-//     A write addresses instead of one: the 1D kernels at L = 64 (small grids, DY = 1024, K = 128, S = 16: 44.3 -> 38.7 us; first half, S =
-//     256, K = 32: 21.0 -> 19.7) and the one for small grids at L = 32 (22.3 -> 21.6); not where there are no registers for the addresses: the image
-//     kernels (16 images of 512 x 512: 588 -> 597 us) and the SIMT first half, which they take from 125 registers to 129, from four blocks
-//     on a CU to three (DY = 1024, K = 8, N = 64: S = 1000 25.3 -> 29.4 us);
+//     covers 32 consecutive elements per half wavefront. Left at that, the write of one bin meets the same banks from the A parts of
+//     a row, two (L = 32) or four ways (64: 16 cycles instead of 4). SPREAD: the bins of part a at k ^ (16 / A) a, without conflicts,
+//     for A write addresses instead of one: the 1D kernels at L = 64 (small grids, DY = 1024, K = 128, S = 16: 44.3 -> 38.7 us; first
+//     half, S = 256, K = 32: 21.0 -> 19.7) and the one for small grids at L = 32 (22.3 -> 21.6); not where there are no registers for the
+//     addresses: the image kernels (16 images of 512 x 512: 588 -> 597 us) and the SIMT first half, which they take from 125 registers
+//     to 129, from four blocks on a CU to three (DY = 1024, K = 8, N = 64, S = 1000: 25.3 -> 29.4 us);
 //   second exchange: [c][16 a' + r] with a pitch of L + 16: writes are consecutive, and the lanes a and a + 1 of a half
 //     wavefront, which read the rows c = a + A j and c + 1, land 16 elements apart modulo 32.
 // The powers w_L^e, e < L, come from the constant table, or (FROM_ARRAY) from an array of L values that the caller keeps

@@ -120,7 +120,8 @@ hipError_t launch_split_forward(int logDY, long S, int N, int K, const float2* x
                                 bool wide, hipStream_t stream);
 hipError_t launch_split_backward(int logDY, long S, int N, int K, const float2* A, const float2* W, float2* y, float2 alpha, hipStream_t stream);
 
-// Small grids, every length (layer1d_small.hip): one 512-thread block per (signal set, nt output channels), nt = 16, 32, 64; the layer and its halves.
+// Small grids, every length (layer1d_small.hip): one 512-thread block per (signal set, nt output channels), nt = 16, 32, 64; the
+// layer and its halves.
 hipError_t launch_fused_small(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* y, float2 alpha, int nt,
                               hipStream_t stream, int keep_y = 0);
 hipError_t launch_small_forward(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C, float2 alpha, float2 beta,

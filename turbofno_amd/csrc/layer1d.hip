@@ -555,33 +555,30 @@ static hipError_t launch_fused_wave(long S, int N, int K, const float2* x, const
 // (DY = 256, N = 64 / 128, small grids), 8 = as 3 with 128 output channels per block where N allows
 // The same rule holds where y is read again at once (middle stage of a 2D layer): the lines were drawn with x and y streamed, and of
 // 3166 2D layers in three stages, lengths 128 to 1024, none lost against a rule that treated that case apart.
-// The return value uses the same numbers (1 ... 8); chosen by size, 2 and 4 stand for blocks of 16, 32 or 64 output channels of the
-// small-grid kernel, 8 for blocks of 64 or of 128 output channels (tile_of_fused_1d_kernel). A selector
-// value that a kernel is not built for falls back to the choice by size.
+// The return value uses the same numbers (1 ... 8); chosen by size, 2 and 4 stand for blocks of 16, 32 or 64 output channels of
+// the small-grid kernel, 8 for blocks of 64 or of 128 (tile_of_fused_1d_kernel). A selector value that a kernel is not built for
+// falls back to the choice by size.
 //
-// By size (measured on MI355X, us):
-//  * while every block of 64 output channels has a CU to itself, every length: the small-grid kernel, with the fewest output channels per
-//    block that still give every block a CU (small_tile). Against the best of the other kernels here (the split kernel, and for long
-//    signals the SIMT kernel): N = 64, DY = 128: S = 160, K = 32: 7.8 / 9.3, S = 256, K = 128: 17.7 / 19.3; DY = 256: S = 128, K = 64: 11.3 / 16.9,
-//    S = 256, K = 64: 15.3 / 17.4; DY = 512, S = 128, K = 64: 18.7 / 28.9. Exceptions, all with nearly a block of 64 channels per CU, whose lines lie where the
-//    other kernel is level: the split kernel for DY = 256 with up to 16 channels (S = 256, K = 16: 10.5 / 9.9; N = 256: S = 52, K = 16 9.8 / 9.4, S = 54, K = 8 9.7 / 9.5), and for
-//    DY = 128 with 49 to 64 channels, of which the small-grid kernel leaves a sixth to a round of its own (N = 64, S = 200, K = 64: 11.6 / 11.5,
-//    S = 256: 12.2 / 11.9; N = 128, S = 100: 11.6 / 11.5), and with 32 or 40 channels and N no multiple of 128 (S = 256, K = 32: 9.0 / 8.8, S = 200: 8.3 / 8.5),
-//    16 to 40 channels with exactly one block per CU (S = 256, K = 16: 8.2 / 8.1); the SIMT kernel for DY = 1024 with eight channels on more than
-//    three quarters of the CUs (S = 200: 24.4 / 23.9, S = 245 28.5 / 27.3; as middle stage of three images with S = 192 the small-grid kernel is 4 us ahead);
-//  * DY = 256, more than 96 channels (a fourth round), blocks of 32 output channels for more than half of the CUs and at most one each: the
-//    K split, whose rounds have no barrier (small-grid kernel / K split: S = 64, N = 128: K = 104 15.8 / 15.2, K = 128: 17.6 / 17.1; S = 100,
-//    N = 64, K = 104: 14.5 / 13.9). Not with fewer channels or blocks (S = 64, N = 128: K = 64 11.7 / 13.2, K = 96: 14.6 / 15.3; S = 60, N = 64,
-//    K = 104: 13.0 / 13.5);
-//  * more than one block of 64 output channels per CU, lengths 128 / 256: the split kernel;
-//  * lengths 512 / 1024, more than one block per CU: the split kernel from the number of channels on where it is ahead of the SIMT
-//    kernel, which has less to do per channel (DY = 512, S = 2048, N = 64: K = 24 127 / 120, K = 40 185 / 170, K = 128 358 / 305; S = 512:
-//    K = 16 38 / 42, K = 40 52 / 51; N = 128, S = 1000: K = 32 144 / 123, K = 128 327 / 244; DY = 1024, N = 64: S = 2048, K = 32 325 / 318, S = 512,
-//    K = 16 68 / 68; N = 128, S = 1000: K = 32 246 / 257, K = 64 389 / 349). DY = 1024 with N no multiple of 128: the split kernel fits two
-//    blocks on a CU, the SIMT kernel three, so below 64 channels the latter is ahead where rounds of two per CU would be at most three
-//    quarters full (N = 64: S = 600: K = 32 98 / 102, K = 40 107 / 114, K = 64 159 / 143; S = 512, K = 40: 88 / 80; N = 192, K = 40: S = 200:
-//    104 / 113, S = 300: 147 / 139) and on large grids of three blocks or more per signal set (N = 192, S = 600: K = 40 242 / 259,
-//    K = 64 341 / 319).
+// By size (measured on MI355X, us; of two figures the second is the kernel named):
+//  * Every block of 64 output channels has a CU to itself, any length: the small-grid kernel, with the fewest output channels per
+//    block that leave it so (the best other kernel / this: N = 64: DY = 128, S = 256, K = 128 19.3 / 17.7; DY = 256, S = 128,
+//    K = 64 16.9 / 11.3; DY = 512, S = 128, K = 64 28.9 / 18.7). With nearly a block per CU others take over where they are ahead:
+//      DY = 256, up to 16 channels: split kernel (N = 256: S = 52, K = 16 9.8 / 9.4, S = 54, K = 8 9.7 / 9.5);
+//      DY = 128, 49 to 64 channels, where a round of 48 leaves a short one: split kernel (N = 64, S = 256, K = 64 12.2 / 11.9);
+//      DY = 128, 32 or 40 channels, N no multiple of 128: split kernel (S = 256, K = 32 9.0 / 8.8, S = 200 8.3 / 8.5); with 16 to
+//      40 channels and exactly one block per CU in the layout for two per CU (S = 256, K = 16 8.2 / 8.1);
+//      DY = 1024, eight channels, more than three quarters of the CUs: SIMT kernel (N = 64: S = 200 24.4 / 23.9, S = 245 28.5 /
+//      27.3; with 192 blocks it is 4 us behind as the middle stage of three images).
+//  * DY = 256, more than 96 channels (a fourth round), blocks of 32 output channels for more than half of the CUs and at most one
+//    each: the K split, whose rounds have no barrier (S = 64, N = 128: K = 104 15.8 / 15.2, K = 128 17.6 / 17.1). Not with fewer
+//    channels or blocks (S = 64, N = 128, K = 96: 14.6 / 15.3; S = 60, N = 64, K = 104: 13.0 / 13.5).
+//  * More than one block of 64 output channels per CU, lengths 128 / 256: the split kernel.
+//  * Lengths 512 / 1024, more than one block per CU: the SIMT kernel with few channels, the split kernel from where it is ahead
+//    (SIMT / split: DY = 512: N = 64, S = 2048: K = 24 120 / 127, K = 40 185 / 170; N = 128, S = 1000: K = 32 144 / 123; DY = 1024:
+//    N = 64, S = 2048, K = 32 325 / 318; N = 128, S = 1000: K = 32 246 / 257, K = 64 389 / 349). At DY = 1024 with N no multiple of
+//    128 the split kernel fits two blocks on a CU, the SIMT kernel three: below 64 channels the latter stays where rounds of two
+//    per CU would be at most three quarters full (N = 64, S = 600: K = 32 98 / 102, K = 64 159 / 143; S = 512, K = 40 88 / 80), and
+//    on large grids with three blocks or more per signal set (N = 192, S = 600: K = 40 242 / 259, K = 64 341 / 319).
 int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, long cus, bool exchange_attached)
 {
     const bool built = logDY >= 7 && logDY <= 10;
@@ -654,10 +651,10 @@ static bool wide_tiles(int logDY, long S, int N, int K, int algo, long cus)
     default: return K >= 64 ? blocks >= cus : blocks <= cus;
     }
 }
-// Output channels per block of the small-grid kernel: the fewest that leave every block a CU to itself. The blocks of a signal set repeat
-// each other's forward transforms, but they run side by side, and each has fewer backward transforms to do one after the other (us, 16 / 32 / 64
-// channels, N = 64: S = 1, K = 32: DY = 128 5.3 / 5.9 / 7.0, DY = 1024 13.8 / 18.0 / 23.5; S = 64, K = 8: DY = 512 8.3 / 8.6 / 12.4; S = 100: 12.9 / 8.5 / 9.4 at
-// DY = 256, K = 24; DY = 256, K = 8: S = 1 5.3 / 5.9, S = 64 6.1 / 6.6).
+// Output channels per block of the small-grid kernel: the fewest that leave every block a CU to itself. The blocks of a signal set
+// repeat each other's forward transforms, but side by side, and each has fewer backward transforms to do one after the other (us,
+// 16 / 32 / 64 channels, N = 64: S = 1, K = 32: DY = 128 5.3 / 5.9 / 7.0, DY = 1024 13.8 / 18.0 / 23.5; S = 64, K = 8: DY = 256 6.1 /
+// 6.6 for 16 / 32, DY = 512 8.3 / 8.6 / 12.4; but with more blocks than CUs, S = 100, DY = 256, K = 24: 12.9 / 8.5 / 9.4).
 static int small_tile(long S, int N, long cus)
 {
     if (S * (N / 16) <= cus) return 16;
@@ -716,20 +713,21 @@ hipError_t launch_fused_fft_cgemm_ifft(int logDY, long S, int N, int K, const fl
     }
 }
 
-// The halves of the layer. While every block of 64 output channels has a CU to itself: the small-grid kernel (us, split kernel / small-grid
-// kernel with 16, 32 or 64 output channels). First half: the fewest output channels pay from 32 input channels on and up to half of the CUs
-// (DY = 256, N = 64, K = 128: S = 1: 20.3 / 11.3, 12.5, 15.1, S = 64: 21.5 / 12.9, 13.5, 16.0; DY = 1024, K = 128, S = 64: 65.8 / 39.4, 36.7, 37.8; DY = 256, K = 8, S = 1:
-// 4.4 / 3.8, 4.0, 4.2); a block of 64 on every CU: DY = 128, K = 64, S = 256: 10.4 / 10.2, DY = 1024, K = 32: 21.0 / 16.1. Not with 49 to 64 channels
-// of length 128 in blocks of 64 outputs, whose rounds hold 48 (S = 200: K = 48 8.8 / 7.6, K = 56 9.5 / 9.8, K = 64 9.8 / 9.9, K = 72 11.8 / 10.5; S = 128,
-// N = 128, K = 56: 9.8 / 10.1). Second half: DY = 256, K = 32, S = 1: 8.4 / 4.5, 5.3, 7.1;
-// DY = 1024, K = 8, S = 1: 19.4 / 6.3, 9.6, 15.8, S = 64: 21.1 / 9.2, 11.1, 17.3, S = 200: 25.7 / 22.4 with 64; but a block of 64 on every CU: DY = 256, N = 64, K = 8: 8.7 / 9.1 (N = 128:
-// 9.4 / 9.1), DY = 512: 14.8 / 15.4, DY = 1024: 26.8 / 28.1. Few channels and more than 64 outputs: up to three quarters of the CUs (DY = 256, K = 16:
-// S = 50, N = 256 level, S = 54 8.8 / 9.1; DY = 512, K = 8 (SIMT kernel): S = 62, N = 192 0.98, S = 70 12.8 / 13.4); DY = 1024 with more than 128
-// outputs up to 13 of 16 (N = 256, K = 48: S = 52 0.98, S = 56 27.3 / 28.8), and so DY = 512, K = 8, N = 64 (S = 222: 12.9 / 13.4).
-// Larger grids: the SIMT kernel with few channels at lengths 512 / 1024; with eight a round of 16 would be half padding (second
-// half, us, split / SIMT: DY = 512, S = 1000: 58.5 / 54.8. First half, with blocks of 64 output
-// channels: DY = 512, S = 4096: 54.2 / 50.8, DY = 1024, N = 64: S = 2048: 49.4 / 46.4, S = 700: 20.2 / 21.7). Otherwise the split kernel: halves,
-// geometric mean of 1232 shapes against the SIMT kernel 0.66.
+// The halves of the layer. While every block of 64 output channels has a CU to itself: the small-grid kernel (us, split kernel /
+// small-grid kernel with 16, 32, 64 output channels per block).
+//   First half: DY = 256, N = 64, K = 128: S = 1 20.3 / 11.3, 12.5, 15.1, S = 64 21.5 / 12.9, 13.5, 16.0; DY = 1024, K = 128, S = 64 65.8 /
+//     39.4, 36.7, 37.8: blocks of 16 from 32 channels on and up to half of the CUs. Not with 49 to 64 channels of length 128 in
+//     blocks of 64, whose rounds hold 48 (S = 200: K = 48 8.8 / 7.6, K = 56 9.5 / 9.8, K = 64 9.8 / 9.9, K = 72 11.8 / 10.5; with one
+//     block on every CU only for multiples of 128: S = 128, N = 128, K = 56 9.8 / 10.1).
+//   Second half (small_second_half): DY = 256, K = 32, S = 1 8.4 / 4.5, 5.3, 7.1; DY = 1024, K = 8: S = 1 19.4 / 6.2, 9.6, 15.8, S = 64
+//     21.1 / 9.2, 11.1, 17.3. Length 128, and 256 with N a multiple of 128, up to one block per CU; else up to seven eighths (a block
+//     of 64 on every CU: DY = 256, N = 64, K = 8 8.7 / 9.1; DY = 512 14.8 / 15.4; DY = 1024 26.8 / 28.1). Few channels: up to three
+//     quarters with more than 64 outputs (DY = 256, K = 16, N = 256: S = 50 level, S = 54 8.8 / 9.1; DY = 512, K = 8, N = 192, against the
+//     SIMT kernel: S = 62 0.98, S = 70 12.8 / 13.4), 13 of 16 at DY = 512 with 64; DY = 1024 with more than 128 outputs: 13 of 16 (N =
+//     256, K = 48: S = 52 0.98, S = 56 27.3 / 28.8).
+// Larger grids: the SIMT kernel with eight channels at lengths 512 / 1024, where a round of 16 would be half padding (split / SIMT:
+// second half, DY = 512, S = 1000 58.5 / 54.8; first half with blocks of 64, DY = 1024, N = 64: S = 2048 49.4 / 46.4, S = 700 20.2 / 21.7);
+// otherwise the split kernel (1232 shapes against the SIMT kernel: 0.66 of its time).
 hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2* x, const float2* W, float2* C,
                                   float2 alpha, float2 beta, hipStream_t stream)
 {
@@ -745,7 +743,8 @@ hipError_t launch_fused_fft_cgemm(int logDY, long S, int N, int K, const float2*
     const bool wide = N % 128 == 0 && 2 * S * (N / 128) >= 3 * cus;
     if (K <= 8 && !wide) {
         if (logDY == 9) return launch_fused_1d_k<9, true, false, false>(S, N, K, x, W, C, alpha, beta, stream);
-        if (logDY == 10 && N % 128 != 0 && items > 3 * cus && items <= 8 * cus) return launch_fused_1d_k<10, true, false, false>(S, N, K, x, W, C, alpha, beta, stream);
+        if (logDY == 10 && N % 128 != 0 && items > 3 * cus && items <= 8 * cus)
+            return launch_fused_1d_k<10, true, false, false>(S, N, K, x, W, C, alpha, beta, stream);
     }
     return launch_split_forward(logDY, S, N, K, x, W, C, alpha, beta, wide, stream);
 }

@@ -4,16 +4,18 @@
 // Same operands and result as fused_fft_cgemm_ifft_{7,8} of the reference
 // (fusion_variants/1D_D_exp_fused_fft_cgemm_ifft/fused_fft_cgemm_ifft_7.cuh:9-222: (S, N/64) blocks that each traverse K).
 // What bounds it is the chain of latencies and instructions of one block, not memory: few blocks run, each with a CU to itself. So
-//   * the output channels of a signal set are spread over as many blocks as there are CUs for (NT = 16, 32, 64), although each of them repeats
-//     the forward transforms: 2 or 4 backward transforms in a row per lane group become one;
-//   * the weights (16 to 128 channels at a time) are split and laid out in LDS once, while x is on its way: done per round they cost every
-//     wave 76 vector instructions next to the 380 of a transform;
-//   * a round (one transform per lane group) has one barrier: spectra go to one of two LDS tiles in operand order, every wave multiplies its m tile with
-//     its tiles of output channels, and the accumulators of all rounds meet in LDS once before the backward transforms.
-// Rounds are bound by instruction issue, two waves per SIMD (vector ALUs 56 % busy; two rounds of x in flight instead of one: 3 - 10 % slower).
-// Measured (us, before / now: a kernel with fp32 matrix instructions, three barriers per round, 32 or 64 output channels): S = 1, K = 8, N = 64, DY = 128: 5.6 / 5.0;
-// S = 64, K = 16, N = 64, DY = 256: 7.4 / 6.4; S = 1, K = 64, N = 64: DY = 128 8.8 / 6.4, DY = 256 10.9 / 8.6, DY = 512 23.0 / 13.2, DY = 1024 38.1 / 22.0; S = 64, K = 128,
-// N = 128, DY = 1024: 64.9 / 48.8; S = 256, K = 64, N = 64, DY = 512: 32.7 / 27.2. Halves: first, DY = 256, K = 128, N = 64, S = 1: 20.3 / 11.3; second, DY = 1024, K = 8: 19.4 / 6.3.
+//   * the output channels of a signal set are spread over as many blocks as there are CUs for (NT = 16, 32, 64), although each of
+//     them repeats the forward transforms: 2 or 4 backward transforms in a row per lane group become one;
+//   * the weights (32 to 128 channels at a time) are split and laid out in LDS once, while x is on its way: done per round they
+//     cost every wave 76 vector instructions next to the 380 of a transform;
+//   * a round (one transform per lane group) has one barrier: spectra go to one of two LDS tiles in operand order, every wave
+//     multiplies its m tile with its tiles of output channels, and the accumulators of all rounds meet in LDS once before the
+//     backward transforms. Two signals of 128 samples per group fill a tile of 48 or 64 channels, of which the LDS holds one: with
+//     a forward transform at DY = 128 a round has two barriers.
+// Rounds are bound by instruction issue, two waves per SIMD (vector ALUs 56 % busy; two rounds of x in flight: 3 - 10 % slower).
+// Measured, N = 64 (us, a kernel with fp32 matrix instructions, three barriers per round, 32 or 64 output channels / this): S = 1,
+// K = 8, DY = 128 5.6 / 5.0; S = 1, K = 64: DY = 128 8.8 / 6.4, DY = 256 10.9 / 8.6, DY = 512 23.0 / 13.2, DY = 1024 38.1 / 21.8; S = 256,
+// K = 64, DY = 512 32.7 / 27.2. Halves: first, S = 1, DY = 256, K = 128 20.3 / 11.3; second, S = 1, DY = 1024, K = 8 19.4 / 6.2.
 // Error against 64 bits as for the split kernel (layer1d_split.hip), over the whole range of floats: operands that the split does not hold are
 // noticed as they are split or in the accumulators, and small_product_fp32() stands in.
 #include "bf16_split.h"

@@ -68,10 +68,10 @@ template <int LOGX, int LOGY> struct Geo2D {
 //     columns are read (32 lanes: LX rows of 2 or 4 columns): a pitch of 2 modulo 32 for 16 rows, of 4 modulo 32 for 8 rows;
 //   backward: columns are written (16 lanes: LX rows of 1 or 2 columns): an odd pitch for 16 rows, 2 modulo 16 for 8; rows are read (32 lanes: two
 //     groups, whose rows have to lie 16 elements apart modulo 32, and 8 for the rows of a pair).
-// One pitch of 66 for all cases put the writes of the backward kernel of 256 rows and the reads of the forward kernel of 128 rows on the same banks two by
-// two (us per layer, before / now: 16 images of 256 x 256, K = N = 64: 211.6 / 204.8; 36 images, K = 56: 444.9 / 425.4; 40 of 128 x 128, K = 72: 194.2 / 189.9; 16 of
-// 512 x 128: 237.9 / 233.1). Backward kernels of decimated images other than 512 x 128 keep 66 and its order of the rows, which lie 2 or 4 rows apart
-// in memory there (8 images of 1024 x 256: 312 / 331 with 65).
+// With one pitch of 66 for all cases the writes of the backward kernel of 256 rows and the reads of the forward kernel of 128 rows
+// met the same banks two by two (us per layer, before / now: 16 images of 256 x 256, K = N = 64: 211.6 / 204.8; 40 of 128 x 128, K = 72:
+// 194.2 / 189.9; 16 of 512 x 128: 237.9 / 233.1). Backward kernels of decimated images other than 512 x 128 keep 66 and its order of
+// the rows, which lie 2 or 4 rows apart in memory there (8 images of 1024 x 256: 312 / 331 with 65).
 //   PAIR:    rows of 128: group g owns the rows a and a + PAIR (lanes 0-7 / 8-15 finish one each), a enumerating the rows in question;
 //   PARTNER: rows between the first rows of the groups 2j and 2j + 1. Rows of 512 / 1024: a group is at least half a wavefront: any order.
 template <int LOGX, int LOGY, int LOGR, bool FORWARD> struct TileMap {
@@ -404,8 +404,8 @@ __global__ __launch_bounds__(1024) void ifft2d_pad_kernel(const float2* __restri
 // Rows of a tile are 16 output channels n, columns 16 consecutive m, contraction in steps of 32 channels (eight per lane
 // of a quarter wavefront). A wave owns 16 m and all 16 NT output channels of its block: an element of A is loaded and split
 // once per block, and its parts meet NT fragments of W read from LDS. The W tile holds the parts of alpha W as fragments
-// in lane order, 6 x 1 KiB per (step, 16 channels): an operand is one conflict-free 16-byte read. With HALVES a step is two of 16 channels whose
-// (re, im) pairs share one instruction, so that a last step of at most 16 channels costs half (gemm_steps.h).
+// in lane order, 6 x 1 KiB per (step, 16 channels): an operand is one conflict-free 16-byte read. With HALVES a step is two of 16
+// channels whose (re, im) pairs share one instruction, so that a last step of at most 16 channels costs half (gemm_steps.h).
 // Blocks are persistent over column blocks (XCD j takes the j-th eighth of them, so that an XCD keeps to one part of the
 // memory system); the strip of the next step - of the next column block after the last - is requested before the matrix
 // work of the current one, and nothing in the walk waits at a barrier, so loads, matrix work and stores of the waves overlap.
@@ -634,7 +634,8 @@ __global__ __launch_bounds__(THREADS, THREADS == 1024 ? 4 : 2) void cgemm_modes_
     }
 }
 
-// Few channels on some large products (K <= 16; K <= 32 in one range of sizes, see launch_cgemm_modes): fp32 matrix instructions over groups of four channels instead, three real products per complex one:
+// Few channels on some large products (K <= 16; K <= 32 in one range of sizes, see launch_cgemm_modes): fp32 matrix instructions
+// over groups of four channels instead, three real products per complex one:
 //   P1 = c (a + b),  P2 = (d - c) a,  P3 = (c + d) b   =>   re = P1 - P3,  im = P1 + P2      (alpha W = c + i d, A = a + i b)
 // A block is 16 waves; wave w owns the 16-m strip w and 64 output channels; the strip sits in NG float2 registers per
 // lane, all loads in flight while the W'' tile is built, and every n tile is stored as soon as it is complete.
@@ -869,21 +870,18 @@ hipError_t launch_ifft2d_pad(int logDX, int logDY, const float2* spec, float2* y
     return dispatch_image_kernel(true, logDX, logDY, spec, y, nimg, stream);
 }
 
-// Which kernel (times for the stand-alone product on operands that come from HBM, in us, column of the kernel before /
-// this one):
-//  * K <= 16: the split kernel (half a step) up to five blocks of 256 columns x 64 output channels per CU for N = 64 and multiples of 128, two for
-//    others, and for multiples of 128 from sixteen on (fp32 / split: K = 16, M = 4,096, N = 64, with beta: 9.5 / 7.4; M = 98,304: N = 64 16.0 / 13.1, N = 128
-//    23.1 / 20.5; M = 163,840, N = 128: 35.6 / 32.0; M = 524,288, N = 128: 157 / 136). Between, fp32 matrix instructions, with
-//    several column blocks per CU the persistent kernel (M = 262,144: N = 128 55.3 / 64.7, N = 192 78.8 / 114; M = 524,288, N = 64: 75.8 / 77.7; M =
-//    65,536, N = 192: 23.0 / 23.7). K <= 32 as well for N >= 128 and 8 to 16 such blocks
-//    per CU (M = 262,144, N = 128, K = 32: 77 against 88 us; from 16 on the 128-channel tile below is ahead).
+// Which kernel (times of the stand-alone product on operands that come from HBM, us, the kernel before / this one):
+//  * K <= 16: the split kernel (half a step) up to five blocks of 256 columns x 64 output channels per CU for N = 64 and multiples of
+//    128, two for others, and for multiples of 128 from sixteen on (fp32 / split, K = 16: M = 4,096, N = 64, with beta, in tiles of
+//    16 outputs 9.3 / 4.2; M = 98,304, N = 128 23.1 / 20.5; M = 163,840, N = 128 35.6 / 32.0; M = 524,288, N = 128 157 / 136).
+//    Between, fp32 matrix instructions (M = 262,144, N = 128 55.3 / 64.7, N = 192 78.8 / 114; M = 524,288, N = 64 75.8 / 77.7), the
+//    persistent kernel with several column blocks per CU. K <= 32 as well for N >= 128 and 8 to 16 such blocks per CU (M = 262,144,
+//    N = 128, K = 32: 77 against 88; from 16 on the 128-channel tile below is ahead).
 //  * otherwise the split kernel. Small products: blocks of 128 columns and the fewest output channels whose grid still fits one
-//    block per CU (K = 64, N = 64, tiles of 64 / 32 / 16 output channels: M = 64: 7.5 / 5.5 / 4.7; M = 8,192: 8.5 / 6.3 / 5.5; M = 16,384:
-//    9.1 / 6.9; N = 192, M = 4,096: 9.0 / 7.1).
-//    At most half a block of 256 columns x 64 output channels per CU: blocks of 128 columns
-//    (M = 16,384, N = 64, K = 64: fp32 18.6, 256 columns 14.0, 128 columns 11.1); also for N = 64 with one to two blocks per
-//    CU and more than 32 channels, where two blocks of 128 columns on a CU overlap each other's phases (M = 65,536, K = 64:
-//    22.7 / 21.5 / 19.6; M = 98,304: 36.2 / 26.9 / 24.2).
+//    block per CU (K = 64, N = 64, tiles of 64 / 32 / 16 output channels: M = 64: 7.5 / 5.5 / 4.7; M = 8,192: 8.5 / 6.3 / 5.5).
+//    At most half a block of 256 columns x 64 output channels per CU: blocks of 128 columns (M = 16,384, N = 64, K = 64: fp32 18.6,
+//    256 columns 14.0, 128 columns 11.1); also for N = 64 with one to two blocks per CU and more than 32 channels, where two blocks
+//    of 128 columns on a CU overlap each other's phases (M = 65,536, K = 64: 22.7 / 21.5 / 19.6).
 //    N a multiple of 128, up to 96 channels and 8 or more blocks per CU: tiles of 128 output channels, A is read once
 //    (M = 524,288, K = 64: 271 / 214 / 197).
 //    Else blocks of 256 columns, tiles of 64 (M = 163,840, N = 128, K = 72: 136 -> 90; M = 262,144, N = 128, K = 128: 259 -> 182).

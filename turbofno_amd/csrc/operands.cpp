@@ -1,10 +1,11 @@
-// Python extension `_operands`: the operand checks of the binding (turbofno_amd/api.py) and the two layer calls without a trip through
-// Python per tensor attribute. A call through the ctypes binding spent 6.7 us on the host, 2.5 of them on checks and conversions in
-// Python, for kernels of 5 us; through this module it spends 3.5 (S = 1, K = 8, N = 64, DY = 128, call after call: 7.3 -> 5.0 us).
+// Python extension `_operands`: the operand checks of the binding (turbofno_amd/api.py) and the two layer calls without a trip
+// through Python per tensor attribute. A call through the ctypes binding spent 6.7 us on the host, 2.5 of them on checks and
+// conversions in Python, for kernels of 5 us; through this module it spends 3.5 (S = 1, K = 8, N = 64, DY = 128, call after call:
+// 6.84 -> 4.91 us).
 //
-// Nothing here decides that a call is wrong: whatever does not pass is handed back (None, or -1) and takes the checks in Python, which
-// raise. Only plain torch.Tensor / Parameter objects are looked at, so subclasses and wrappers keep their own behaviour, and nothing is kept
-// from one call to the next.
+// Nothing here decides that a call is wrong: whatever does not pass is handed back (None, or -1) and takes the checks in Python,
+// which raise. Only plain torch.Tensor / Parameter objects are looked at, so subclasses and wrappers keep their own behaviour, and
+// nothing is kept from one call to the next.
 #include <torch/csrc/autograd/python_variable.h>
 #include <climits>
 
@@ -98,11 +99,11 @@ PyObject* layer_1d(PyObject*, PyObject* const* args, Py_ssize_t count)
                              *y = gpu_tensor(args[3], at::kComplexFloat, device);
             float re, im;
             long long dimX;
-            if (ok_f && call && ok_s && x && W && y && complex_value(args[4], re, im) && integer_value(args[5], dimX) && x->dim() == 3 && W->dim() == 2 &&
-                y->dim() == 3) {
+            if (ok_f && call && ok_s && x && W && y && complex_value(args[4], re, im) && integer_value(args[5], dimX) &&
+                x->dim() == 3 && W->dim() == 2 && y->dim() == 3) {
                 const int64_t K = x->size(0), S = x->size(1), DY = x->size(2), N = W->size(0);
-                if (W->size(1) == K && y->size(0) == N && y->size(1) == S && y->size(2) == DY && dimX > 0 && S % dimX == 0 && fits_int(K) && fits_int(S) &&
-                    fits_int(DY) && fits_int(N) && fits_int(dimX)) {
+                if (W->size(1) == K && y->size(0) == N && y->size(1) == S && y->size(2) == DY && dimX > 0 && S % dimX == 0 &&
+                    fits_int(K) && fits_int(S) && fits_int(DY) && fits_int(N) && fits_int(dimX)) {
                     void *px = x->data_ptr(), *pW = W->data_ptr(), *py = y->data_ptr();
                     const WithoutLock unlocked;
                     rc = call((int)(S / dimX), (int)dimX, (int)DY, (int)K, (int)N, px, pW, py, re, im, stream);
@@ -129,8 +130,8 @@ PyObject* layer_2d(PyObject*, PyObject* const* args, Py_ssize_t count)
                              *y = gpu_tensor(args[3], at::kComplexFloat, device), *ws = gpu_tensor(args[5], at::kByte, device);
             float re, im;
             long long algo;
-            if (ok_f && call && ok_s && x && W && y && ws && complex_value(args[4], re, im) && integer_value(args[6], algo) && fits_int(algo) && x->dim() == 4 &&
-                W->dim() == 2 && y->dim() == 4) {
+            if (ok_f && call && ok_s && x && W && y && ws && complex_value(args[4], re, im) && integer_value(args[6], algo) &&
+                fits_int(algo) && x->dim() == 4 && W->dim() == 2 && y->dim() == 4) {
                 const int64_t K = x->size(0), bs = x->size(1), DX = x->size(2), DY = x->size(3), N = W->size(0);
                 if (W->size(1) == K && y->size(0) == N && y->size(1) == bs && y->size(2) == DX && y->size(3) == DY && fits_int(K) && fits_int(bs) &&
                     fits_int(DX) && fits_int(DY) && fits_int(N)) {

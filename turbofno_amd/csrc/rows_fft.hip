@@ -112,18 +112,18 @@ static hipError_t launch_rows_k(const float2* in, float2* out, int DX, long nimg
     if constexpr (INVERSE) {
         hipLaunchKernelGGL((ifft_rows_pad_kernel<LOGDY, ROWS>), dim3((unsigned)blocks), dim3(256), R::LDS_BYTES, stream, in, out, DX);
     } else {
-        // as many blocks as the CUs hold at once (LDS: 43-52 KiB per block)
+        // as many blocks as the CUs hold at once (LDS: 38-52 KiB per block)
         const long resident = (long)cu_count() * (long)((160 * 1024) / R::LDS_BYTES);
         hipLaunchKernelGGL((fft_rows_trunc_kernel<LOGDY, ROWS>), dim3((unsigned)(blocks < resident ? blocks : resident)), dim3(256),
                            R::LDS_BYTES, stream, in, out, DX, blocks);
     }
     return hipGetLastError();
 }
-// Rows per block: 32, whose transposed accesses are two cache lines long; fewer on small grids, so that more blocks (and CUs) share the rows and
-// each has fewer batches one after the other. The limits are rows of the call per CU. Whole layers of one image, rows first, 32 rows / the rule (us):
-// 128 x 256, K = 8, N = 64 19.6 / 17.7 (4 and 32 rows per CU), 128 x 512 24.7 / 21.3, 128 x 1024 34.6 / 28.7; two of 256 x 1024, K = 8: 80 / 75. Beyond them: DY =
-// 256, backward with 64 rows per CU 24.3 / 25.9, 256: 55.7 / 60.9; DY = 512, backward, 64: 34.1 / 34.9, forward with 8 rows per block, 32: 38.8 / 38.9;
-// DY = 1024, backward, 256: 147.8 / 149.8.
+// Rows per block: 32, whose transposed accesses are two cache lines long; fewer on small grids, so that more blocks (and CUs) share
+// the rows and each has fewer batches one after the other. The limits are rows of the call per CU. Whole layers of one image, K = 8,
+// N = 64, rows first, 32 rows / the rule (us): 128 x 256 19.6 / 17.7, 128 x 512 24.7 / 21.3, 128 x 1024 34.6 / 28.7. Beyond the limits: DY
+// = 256, backward with 64 rows per CU 24.3 / 25.9; DY = 512, backward with 64 34.1 / 34.9, forward with 32 and eight rows per block
+// 38.8 / 38.9; DY = 1024, backward with 256 147.8 / 149.8.
 template <int LOGDY, bool INVERSE> struct RowsPerBlock {
     static constexpr int EIGHT_TO = LOGDY == 10 ? (INVERSE ? 128 : 64) : LOGDY == 9 && !INVERSE ? 16 : 0;
     static constexpr int SIXTEEN_TO = LOGDY == 10 ? (INVERSE ? 0 : 128) : LOGDY == 9 ? (INVERSE ? 32 : 64) : LOGDY == 8 ? 32 : 0;
