@@ -599,6 +599,9 @@ int pick_fused_1d_kernel(int logDY, long S, int N, int K, int algo, long cus, bo
     }
     // small grids, 64 channels or more, N = 64 / 128: a cluster of blocks per signal set, no forward transform twice.
     // Only for streams that have an exchange buffer attached; without one the kernels below take over.
+    // The line was drawn against the K split. The small-grid kernel has overtaken the cluster on part of this range (us, with / without
+    // a buffer, S = 64: N = 128: K = 64 12.7 / 11.9, K = 96 15.7 / 14.8, K = 128 16.2 / 16.6; N = 64: K = 64 9.7 / 9.6, K = 128 11.4 / 13.9,
+    // and 1.2 to 1.3 where K is no multiple of 32, which makes clusters of two): such streams are better off without one.
     if (algo == 7 || (algo == 0 && logDY == 8 && K >= 64)) {
         if (exchange_attached && cluster_size_1d(logDY, S, N, K, cus) > 0) return kFused1dCluster;
         if (algo == 7) algo = 0;                                // not applicable here: by size, as for every other value
