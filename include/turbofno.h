@@ -98,8 +98,9 @@ int turbofno_layer_1d(int bs, int dimX, int DY, int K, int N, const void* x, con
  * output, depending on the lengths, and earlier with many channels, else ROWS_FIRST or THREE_KERNEL); the workspace
  * query with the same arguments, and turbofno_query_2d_algo, make the same choice. Every algorithm takes every pair of
  * lengths in {128, 256, 512, 1024} (WHOLE_IMAGE handles images of 512 or 1024 rows as two or four interleaved parts of
- * 256 rows that the contraction sums over). ROWS_FIRST is the three-stage structure with the axes exchanged (the contiguous axis is transformed first and last, so that x and y move as whole rows): same result, the 2D
- * transform being separable; its intermediates are [images][64][DX].
+ * 256 rows that the contraction sums over). ROWS_FIRST is the three-stage structure with the axes exchanged (the
+ * contiguous axis is transformed first and last, so that x and y move as whole rows): same result, the 2D transform being
+ * separable; its intermediates are [images][64][DX].
  */
 size_t turbofno_layer_2d_workspace_bytes(int bs, int DX, int DY, int K, int N, int algo);
 int turbofno_layer_2d(int bs, int DX, int DY, int K, int N, const void* x, const void* W, void* y,
@@ -169,9 +170,9 @@ int turbofno_layer_2d_noalloc(int bs, int DX, int DY, int K, int N, const void* 
  * of the three-kernel 2D path (their reference-shaped signatures have no room for a selector): 0 = by problem size
  * (default), 1 = SIMT contraction, 2 = matrix cores with 512-thread blocks of 64 output channels, 3 = matrix cores with
  * 256-thread blocks of 64 output channels, 4 = as 2 with 32-channel output tiles (DY = 128 / 256), 5 = as 3, laid out for
- * four blocks per compute unit (DY = 128 with eight input channels: one wavefront per signal set and output tile), 6 = matrix cores, the K channels of an item split over
- * the waves of a block, 7 = matrix cores, the K channels of a signal set split over a cluster of blocks (see below), 8 = as 3
- * with 128 output channels per block where N is a multiple of 128.
+ * four blocks per compute unit (DY = 128 with eight input channels: one wavefront per signal set and output tile), 6 =
+ * matrix cores, the K channels of an item split over the waves of a block, 7 = matrix cores, the K channels of a signal set
+ * split over a cluster of blocks (see below), 8 = as 3 with 128 output channels per block where N is a multiple of 128.
  * A value a kernel is not built for falls back to the choice by size. Meant for tests and measurements; set returns
  * TURBOFNO_ERR_INVALID_ARG outside 0..TURBOFNO_1D_ALGO_MAX.
  */
