@@ -169,11 +169,18 @@ def test_1d_kernels_with_nearly_a_block_per_cu():
         assert tf.query_1d_kernel(1024, CUS // tiles, N, 16, CUS) == 2
 
 
-def test_mode_gemm_steps(tmp_path):
-    """half steps follow the run that is walked, not the period of the weights: with R parts per image a run mostly covers all R of them"""
+def _gemm_steps(tmp_path, lines):
+    """answers of the rules in turbofno_amd/csrc/gemm_steps.h, as tuples"""
     exe = str(tmp_path / "gemm_steps_check")
     source = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host", "gemm_steps_check.cpp")
     subprocess.run(["g++", "-O1", "-std=c++17", source, "-o", exe], check=True)
+    text = "".join(" ".join(map(str, line)) + "\n" for line in lines)
+    out = subprocess.run([exe], input=text, check=True, capture_output=True, text=True).stdout.splitlines()
+    return [tuple(map(int, ln.split())) for ln in out]
+
+
+def test_mode_gemm_steps(tmp_path):
+    """half steps follow the run that is walked, not the period of the weights: with R parts per image a run mostly covers all R of them"""
     wide, narrow, small = (4, 1024, 6), (4, 512, 6), (1, 512, 6)
     cases = [   # parts, channels per part, kernel -> channels per run, half steps
         (1, 8, wide, 8, 1), (1, 16, wide, 16, 1), (1, 24, wide, 24, 0), (1, 32, wide, 32, 0), (1, 72, wide, 72, 1), (1, 64, wide, 64, 0),
@@ -185,6 +192,13 @@ def test_mode_gemm_steps(tmp_path):
         (1, 48, small, 48, 1), (1, 72, small, 72, 0), (2, 24, small, 48, 1), (2, 40, small, 80, 0), (4, 72, small, 72, 0),
         (1, 112, narrow, 112, 1), (1, 136, narrow, 136, 0), (1, 136, wide, 136, 1), (1, 200, wide, 200, 0), (2, 72, narrow, 144, 0), (2, 72, wide, 144, 1),
     ]
-    lines = "".join("%d %d %d %d %d\n" % ((r * k, k) + kernel) for r, k, kernel, _, _ in cases)
-    out = subprocess.run([exe], input=lines, check=True, capture_output=True, text=True).stdout.splitlines()
-    assert [tuple(map(int, ln.split())) for ln in out] == [c[3:] for c in cases]
+    assert _gemm_steps(tmp_path, [(0, r * k, k) + kernel for r, k, kernel, _, _ in cases]) == [c[3:] for c in cases]
+
+
+def test_mode_gemm_persistent_blocks(tmp_path):
+    """blocks of columns, blocks that the CUs hold, channels -> blocks launched: whole groups of eight, unless with few channels they make two
+    rounds of one"""
+    cases = [(1, 256, 16, 1), (80, 85, 16, 80), (81, 85, 16, 81), (85, 85, 8, 85), (86, 85, 16, 80), (81, 85, 24, 80), (85, 85, 64, 80), (170, 85, 16, 80),
+             (42, 42, 16, 42), (43, 42, 16, 40), (51, 51, 8, 51), (1000, 51, 16, 48), (256, 256, 72, 256), (300, 256, 16, 256), (7, 7, 72, 7),
+             (1000, 7, 16, 7), (5, 0, 16, 1)]
+    assert _gemm_steps(tmp_path, [(1,) + c[:3] for c in cases]) == [c[3:] for c in cases]

@@ -20,6 +20,7 @@ pytestmark = pytest.mark.gpu
     (131072 + 64, 16, 192, 0.5),                         # more: fp32 matrix instructions
     (163840, 8, 128, 0.0), (163840 + 64, 16, 128, 0.0),  # five, and just above: fp32, persistent
     (524288, 16, 128, 0.0),                              # sixteen: tiles of 128 output channels
+    (21120, 16, 192, 0.5), (12800, 8, 320, 0.0), (10624, 16, 384, 0.0),     # one round of 83, 50 and 42 blocks: no groups of eight
     (16384, 104, 128, 0.0), (65536 + 64, 48, 64, 1.0),   # three whole steps and a quarter, one and a half
 ])
 def test_cgemm_with_a_short_last_step(M, K, N, beta):

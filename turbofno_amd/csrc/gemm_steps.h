@@ -1,5 +1,5 @@
-// How the mode GEMM (layer2d.hip) walks its contraction: channels per run over the tile of weights, and whole or half steps. Plain
-// arithmetic on the sizes, so that it can be checked without a GPU.
+// How the mode GEMM (layer2d.hip) walks its contraction: channels per run over the tile of weights, whole or half steps, and
+// its persistent blocks. Plain arithmetic on the sizes, so that it can be checked without a GPU.
 #pragma once
 
 namespace tfno {
@@ -25,6 +25,16 @@ inline GemmWalk gemm_walk(int K, int Kw, int nt, int threads, int cap)
     const int run = periods ? Kw : K, last = run % GEMM_KSTEP;
     const int longest = nt < 4 ? 48 : (nt == 4 && threads == 512 ? 128 : GEMM_KSTEP * cap);
     return { run, last > 0 && last <= GEMM_KSTEP / 2 && run <= longest };
+}
+
+// Persistent blocks per tile of outputs, of `most` that the CUs hold: whole groups of eight, every XCD the same share. With up to 16
+// channels not where the blocks left out make two rounds of one (us, whole groups / this: K = 16: N = 192, M = 21,120 11.6 / 9.4, N =
+// 320, M = 12,800 11.8 / 9.6; 14 numbers of columns with N = 192 ... 576, beta or not: 0.83 of the time on average). With K = 24 and 32
+// and beta the two rounds are ahead (N = 192, M = 20,608, K = 24 15.3 / 18.4).
+inline long gemm_persistent_blocks(long nblocks, long most, int K)
+{
+    const long groups = most >= 8 ? most - most % 8 : (most > 0 ? most : 1);
+    return nblocks <= (K <= 16 ? most : groups) ? nblocks : groups;
 }
 
 }  // namespace tfno

@@ -875,8 +875,12 @@ hipError_t launch_ifft2d_pad(int logDX, int logDY, const float2* spec, float2* y
 //    128, two for others, and for multiples of 128 from sixteen on (fp32 / split, K = 16: M = 4,096, N = 64, with beta, in tiles of
 //    16 outputs 9.3 / 4.2; M = 98,304, N = 128 23.1 / 20.5; M = 163,840, N = 128 35.6 / 32.0; M = 524,288, N = 128 157 / 136).
 //    Between, fp32 matrix instructions (M = 262,144, N = 128 55.3 / 64.7, N = 192 78.8 / 114; M = 524,288, N = 64 75.8 / 77.7), the
-//    persistent kernel with several column blocks per CU. K <= 32 as well for N >= 128 and 8 to 16 such blocks per CU (M = 262,144,
-//    N = 128, K = 32: 77 against 88; from 16 on the 128-channel tile below is ahead).
+//    persistent kernel with several column blocks per CU. The split kernel is not the faster one everywhere on its side: N = 256 and
+//    more from sixteen on with fewer than about six columns of blocks per CU (N = 256, K = 16: M = 262,144 102 / 123, M = 327,680
+//    147 / 157, M = 508,416 334 / 240), inside 2D layers with N = 128 and 256 at three to five (1 to 3 % of the layer), M = 64 (3.5 /
+//    3.6). It stays there for its error against 64 bits: 3.7e-8 (K = 16) and 3.2e-8 (K = 8), the three fp32 products 1.12e-7 and 8.7e-8.
+//    K <= 32 goes to fp32 as well for N >= 128 and 8 to 16 such blocks per CU (M = 262,144, N = 128, K = 32: 77 against 88; from 16 on
+//    the 128-channel tile below is ahead).
 //  * otherwise the split kernel. Small products: blocks of 128 columns and the fewest output channels whose grid still fits one
 //    block per CU (K = 64, N = 64, tiles of 64 / 32 / 16 output channels: M = 64: 7.5 / 5.5 / 4.7; M = 8,192: 8.5 / 6.3 / 5.5).
 //    At most half a block of 256 columns x 64 output channels per CU: blocks of 128 columns (M = 16,384, N = 64, K = 64: fp32 18.6,
@@ -928,10 +932,7 @@ hipError_t launch_cgemm_modes(const float2* A, const float2* W, float2* C, long 
             return e;
         const long nblocks = (Mtot + THREADS / 4 - 1) / (THREADS / 4), tiles = N / (16 * NT);
         if (lds_bytes * per_cu > 160 * 1024) per_cu = 1;
-        long g = per_cu * cus / tiles;
-        if (g >= 8) g -= g % 8;
-        if (g < 1) g = 1;
-        if (g > nblocks) g = nblocks;
+        const long g = gemm_persistent_blocks(nblocks, per_cu * cus / tiles, K);
         hipLaunchKernelGGL((cgemm_modes_split_kernel<NT, THREADS, HALVES>), dim3((unsigned)g, (unsigned)tiles, 1), dim3(THREADS), lds_bytes, stream,
                            A, W, C, Mtot, K, alpha, beta, nblocks, Kw, Kp, cap);
         return hipGetLastError();
